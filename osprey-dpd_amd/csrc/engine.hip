@@ -518,7 +518,8 @@ __global__ __launch_bounds__(256) void k_permute(int n, Buffers S, Buffers D, fl
     }
     Moved m;
     advance(o, c, img, d, B, m);
-    D.pos[dst] = make_float4(m.o[0], m.o[1], m.o[2], p.w);
+    const int w = (__float_as_int(p.w) & ~kCellXBits) | ((m.c[0] & 3) << kCellXShift);
+    D.pos[dst] = make_float4(m.o[0], m.o[1], m.o[2], __int_as_float(w));
     if (MODE == kRebin) {
         D.vel[dst] = v;
         D.fold[dst] = f;
@@ -808,11 +809,11 @@ void set_schedule(dpd_engine* e, int s)
     e->pair_kernel = kSchedule[s].kernel;
 }
 
-// the automatic choice: the hit-list kernel's default schedule for every engine whose slots
-// fit its 26-bit list entries, the full-shell kernel beyond
+// the automatic choice: the hit-list kernel's schedule for the engine's size where its slots
+// fit the 26-bit list entries, the full-shell kernel beyond
 int default_schedule(const dpd_engine* e)
 {
-    return e->n <= (int64_t)kHitSlotMask ? kDefaultSchedule : kFullShellSchedule;
+    return e->n <= (int64_t)kHitSlotMask ? size_schedule(e->n) : kFullShellSchedule;
 }
 
 void set_step_constants(BoxHost& b)
@@ -950,15 +951,13 @@ int launch_pair(dpd_engine* e, bool obs, bool* bonded = nullptr, bool epi = fals
 {
     if (bonded) *bonded = false;
     PairArgs a;
-    {
-        const Buffers S = bufs(e, e->cur);
-        a.vel = S.vel;
-        a.nkey = e->nkey;
-        a.rank = e->rank;
-        a.cnt = e->cnt;
-        a.gcnt = e->gcnt;
-        a.flags = e->flags;
-    }
+    const Buffers S = bufs(e, e->cur);
+    a.vel = S.vel;
+    a.nkey = e->nkey;
+    a.rank = e->rank;
+    a.cnt = e->cnt;
+    a.gcnt = e->gcnt;
+    a.flags = e->flags;
     a.n = (int)e->n;
     a.nbox = (int)e->boxes.size();
     a.ngroups = e->ngroups;
@@ -968,7 +967,7 @@ int launch_pair(dpd_engine* e, bool obs, bool* bonded = nullptr, bool epi = fals
     // stored half steps (k_permute did not write vp)
     a.vp = (in_seq && vp_is_vel(e)) ? e->vel[e->cur] : e->vp;
     a.key = e->key[e->cur];
-    a.code = e->code[e->cur];
+    a.code = S.code;
     a.cstart = e->cstart;
     a.table = e->table;
     a.step = e->dstep;
@@ -982,7 +981,6 @@ int launch_pair(dpd_engine* e, bool obs, bool* bonded = nullptr, bool epi = fals
     // 256 replicas)
     if (bonded && nq > 0 && e->pair_kernel == DPD_PAIR_HITLIST && a.n <= (int)kHitSlotMask && !multi(e)) {
         const BoxDev B0 = e->boxes[0].B;
-        const Buffers S = bufs(e, e->cur);
         // (never with the epilogue: epilogue_ok excludes engines with bonded terms)
         if (obs) launch_hitlist_bonded<true, false>(e->sched, a, B0, nq, S, e->slot_of, topo(e), e->stream);
         else launch_hitlist_bonded<false, false>(e->sched, a, B0, nq, S, e->slot_of, topo(e), e->stream);
@@ -1160,7 +1158,7 @@ int commit_beads(dpd_engine* e, int64_t step0)
     if (nbr != e->ngroups) {
         e->ngroups = nbr;
         e->nkeys = nbr * kGroupKeys;
-        if ((rc = dalloc(e, &e->cnt, e->nkeys)) || (rc = dalloc(e, &e->cstart, e->nkeys + 1)) ||
+        if ((rc = dalloc(e, &e->cnt, e->nkeys)) || (rc = dalloc(e, &e->cstart, e->nkeys + 1 + kCstartPad)) ||
             (rc = dalloc(e, &e->gcnt, e->ngroups)) || (rc = dalloc(e, &e->gstart, e->ngroups)))
             return rc;
         HIPCHK(hipMemsetAsync(e->cnt, 0, sizeof(int) * e->nkeys, e->stream));
@@ -1492,6 +1490,17 @@ int dpd_create_batch(int32_t nbox, const dpd_params* p, dpd_engine** out)
         for (int d = 0; d < 2; ++d) B.inv[d] = 1.0f / (float)B.n[d];
         B.wd[0] = p[b].wx; B.wd[1] = p[b].wy; B.wd[2] = p[b].wz;
         for (int d = 0; d < 3; ++d) B.w[d] = (float)B.wd[d];
+        {
+            // the scan's cut-off 1 + m, m = 1.01 |w| / 256 + 1e-5 (code_dist2), in code units
+            float s2 = 0.f, umax = 0.f;
+            for (int d = 0; d < 3; ++d) {
+                B.qinv[d] = 256.0f / B.w[d];
+                s2 += B.w[d] * B.w[d];
+                umax = std::max(umax, B.qinv[d]);
+            }
+            const float tu = (1.0f + std::sqrt(s2) * (1.01f / 256.0f) + 1e-5f) * umax;
+            B.qthr = (int)(tu * tu) + 1;
+        }
         B.ntypes = nt;
         B.seed0 = (uint32_t)p[b].seed;
         B.seed1 = (uint32_t)(p[b].seed >> 32);
@@ -1881,7 +1890,8 @@ int dpd_set_pair_kernel(dpd_engine* e, int32_t kernel)
     e->pair_auto = kernel == DPD_PAIR_AUTO;
     if (e->pair_auto) set_schedule(e, e->committed ? default_schedule(e) : kFullShellSchedule);
     else if (kernel == DPD_PAIR_FULLSHELL) set_schedule(e, kFullShellSchedule);
-    else if (kSchedule[e->sched].kernel != DPD_PAIR_HITLIST) set_schedule(e, kDefaultSchedule);
+    else if (kSchedule[e->sched].kernel != DPD_PAIR_HITLIST)
+        set_schedule(e, e->committed ? size_schedule(e->n) : kDefaultSchedule);
     return DPD_OK;
 }
 
@@ -2030,14 +2040,15 @@ int tune_trials(dpd_engine* e, int32_t nsteps, const std::vector<int>& trials, d
 int dpd_autotune(dpd_engine* e, int32_t nsteps, int32_t* chosen, double* ms_per_step)
 {
     if (!e) return DPD_ERR_PARAM;
-    const std::vector<int> trials = {kDefaultSchedule, kFullShellSchedule};
+    const int hit = size_schedule(e->n);
+    const std::vector<int> trials = {hit, kFullShellSchedule};
     double ms[2] = {0.0, 0.0};
     int best = 0;
     int rc = tune_trials(e, nsteps, trials, ms, &best);
     if (rc) return rc;
     if (ms_per_step) {
         for (int k = 0; k < DPD_PAIR_KINDS; ++k) ms_per_step[k] = 0.0;
-        ms_per_step[kSchedule[kDefaultSchedule].kernel - 1] = ms[0];
+        ms_per_step[kSchedule[hit].kernel - 1] = ms[0];
         ms_per_step[kSchedule[kFullShellSchedule].kernel - 1] = ms[1];
     }
     if (chosen) *chosen = kSchedule[best].kernel;

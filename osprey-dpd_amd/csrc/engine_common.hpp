@@ -35,6 +35,8 @@ struct BoxDev {
     double wd[3];
     float dt, hdt, hdt2, lamdt;   // dt, dt/2, dt^2/2, lambda*dt
     float invrootdt;              // sqrt(24 kT / dt)
+    float qinv[3];                // 256 / w: scan-code units
+    int qthr;                     // square of the scan's widened cut-off in the smallest of them
     int ntypes;
     uint32_t seed0, seed1;        // key of the pair stream
     int koff;                     // first global cell key of this box (a multiple of 64)
@@ -73,8 +75,10 @@ __host__ __device__ inline int floordiv(int a, int n)
     return (a >= 0) ? a / n : -((-a + n - 1) / n);
 }
 
-// bead word packing: pos.w = type | box << 8
-__host__ __device__ inline int bead_type(int w) { return w & 0xFF; }
+// bead word packing: pos.w = type | (x index of the cell mod 4) << 4 | box << 8
+__host__ __device__ inline int bead_type(int w) { return w & (kMaxTypes - 1); }
+constexpr int kCellXShift = 4;
+constexpr int kCellXBits = 3 << kCellXShift;
 __host__ __device__ inline int bead_box(int w) { return (w >> 8) & 0x3FFFFF; }
 // bit 30 of a position's w: the bead has bonds or angles (set from the topology)
 constexpr int kBondedBit = 1 << 30;
@@ -136,18 +140,32 @@ __device__ inline float pair_scalar(float dr2, float dxdv, float a, float sg, fl
     return (con + diss + rnd) * inv;
 }
 
+// pair_scalar with the random amplitude sgr = sqrt(gamma) sqrt(24kT/dt) as one factor
+__device__ inline float pair_scalar_t(float dr2, float dxdv, float a, float sgr, float g, uint32_t idi, uint32_t idj,
+                                      const RngKey& K, float* pe)
+{
+    const float inv = __builtin_amdgcn_rsqf(dr2);
+    const float dr = dr2 * inv;
+    const float wr = 1.0f - dr;
+    const float con = a * wr;
+    const float diss = -(g * wr * wr) * (dxdv * inv);
+    const float u = pair_uniform(idi, idj, K);
+    const float rnd = sgr * wr * (0.5f - u);
+    if (pe) *pe = 0.5f * a * wr * wr;
+    return (con + diss + rnd) * inv;
+}
+
 // Scan code of a bead: its offsets in the cell to 8 bits each, q = floor(256 o / w), with
 // byte 0 the x offset, byte 1 the cell's x index modulo 256, byte 2 the y offset and byte 3
 // the z offset.  The hit-list kernel tests candidates on these 4 bytes instead of the
-// 16-byte position: bytes 0-1 read as one 16-bit number less 256 times a row segment's
-// first cell index give the x position in that segment in units of w/256, so a row of
-// three cells is scanned as one range.  q is the floor of the offset in units of w/256, so
-// the offset lies in [q, q + 1) units.
+// 16-byte position: bytes 0-1 read as one 16-bit number give the x position along the row in
+// units of w/256 (mod 2^16), so a row of three cells is scanned as one range.  q is the floor
+// of the offset in units of w/256, so the offset lies in [q, q + 1) units.
 __device__ inline uint32_t scan_code(const float o[3], int cx, const BoxDev& B)
 {
     uint32_t q[3];
 #pragma unroll
-    for (int a = 0; a < 3; ++a) q[a] = (uint32_t)min(max((int)(o[a] * (256.0f / B.w[a])), 0), 255);
+    for (int a = 0; a < 3; ++a) q[a] = (uint32_t)min(max((int)(o[a] * B.qinv[a]), 0), 255);
     return q[0] | ((uint32_t)(cx & 0xFF) << 8) | (q[1] << 16) | (q[2] << 24);
 }
 

@@ -14,6 +14,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "dpd_engine.h"
 #include "engine_common.hpp"
 
@@ -127,21 +129,30 @@ __global__ __launch_bounds__(256) void k_pair_fullshell(PairArgs A, BoxDev B0, i
     }
 }
 
-// Hit-list kernel: thread per bead in two passes.  The scan of the 27 neighbour cells
-// appends every partner in range to a per-thread list in LDS (slot | neighbour-cell code
-// << 26); the list is then evaluated in one dense loop.  In the one-pass kernel a
-// wavefront runs the whole pair evaluation (random stream, force) whenever any of its
-// lanes has a partner in range -- on nearly every candidate iteration, with ~8% of the
-// lanes busy -- while here the evaluation loop runs max(partners per lane) ~20 times per
-// wavefront.  Partners are evaluated in candidate order with the same expressions as
-// k_pair_fullshell; the compiler contracts multiply-adds differently in the two code
-// shapes, so the forces agree to ~1 ulp per term, not bitwise.  Slots must fit in 26 bits.
+// Hit-list kernel: thread per bead in two passes.  The scan of the nine neighbour rows appends
+// every partner that may be in range to a per-thread list in LDS (slot | segment code << 26);
+// the wavefront then evaluates its lists together (evaluate_lists).  In the one-pass kernel a
+// wavefront runs the whole pair evaluation (random stream, force) whenever any of its lanes
+// has a partner in range -- on nearly every candidate iteration, with ~8% of the lanes busy.
+// Partners are evaluated with the same expressions as k_pair_fullshell; the compiler contracts
+// multiply-adds differently in the two code shapes, so the forces agree to ~1 ulp per term, not
+// bitwise.  Slots must fit in 26 bits.
+//
+// What bounds it: instruction issue (rocprofv3: VALU active 87% of the cycles, 41M wavefront
+// instructions on the condensate box of 64^3 cells), of which the scan is two thirds.  The scan
+// costs 42 VALU instructions per pass of four candidates: the codes of the next pass are loaded
+// into the same registers as soon as these are subtracted, the x image of a partner is left to
+// the evaluation (cell indices mod 4 in the beads' words), and a bead beside an x face goes on
+// to the cell across it within the row's loop, so the wavefront's other lanes do not wait for a
+// second one.  Pair launch, relaxed boxes, with 58 instructions per pass, a second loop at the
+// faces and lists evaluated lane by lane -> now: condensate 64^3 95 -> 80 us, water 96^3 332 ->
+// 263, binary 40^3 38 -> 31, bilayer 48x48x32 40 -> 31, 64 water/lipid replicas 141 -> 105.
+// (The z offsets in an array of their own, 38 instructions per pass, were slower: 89 us, the
+// second load; so were two passes per turn, 85 us.)
 // A schedule of the hit-list kernel: threads per workgroup, list entries per thread (4 B of
 // LDS each) and the flush threshold (after each row segment the wavefront evaluates its
 // lists together once any of them holds this many; FLUSH = CAP never flushes).
 // dpd_autotune_schedules picks among these by timing them.
-constexpr int kHitThreads = 512;   // the default schedule's
-constexpr int kHitCap = 24;
 constexpr int kHitSlotBits = 26;
 constexpr uint32_t kHitSlotMask = (1u << kHitSlotBits) - 1u;
 // slots of padding after the last scan code: the scan reads candidates four (or two) at a
@@ -157,22 +168,24 @@ typedef uint32_t code2_t __attribute__((ext_vector_type(2), aligned(4)));
 // four scan codes from one 4-byte-aligned 16-byte load
 typedef uint32_t code4_t __attribute__((ext_vector_type(4), aligned(4)));
 // two 16-bit integers in one register (v_pk_sub_i16, v_dot2_i32_i16)
+// cell starts: a row's four and two, from 4-byte-aligned loads
+typedef int int4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef int int2u __attribute__((ext_vector_type(2), aligned(4)));
+// entries of padding after the cell starts (a row's four are loaded at once)
+constexpr int kCstartPad = 4;
 typedef short short2_t __attribute__((ext_vector_type(2)));
 
-// The candidate test of cubic cells in integer code units (u = w / 256): dx and dy as one
-// packed pair, dz apart, |d|^2 by one two-term dot product plus dz^2.  QXY holds the bead's
-// x (plus the segment's first cell index times 256, mod 2^16) and y in code units, Qz its z:
-// floors of its position seen from the row, as the codes are floors of the candidates'.  Each
-// axis is then within one unit of the true difference, so every pair inside the cut-off
+// The candidate test in integer code units (u = w / 256): |d|^2 from dx and dy as one packed
+// pair (one two-term dot product) and dz.  code_dxy: QXY holds the bead's x (with its cell
+// index, mod 2^16) and y in code units, floors of its position seen from the row as the codes
+// are floors of the candidates'; one v_perm_b32 gathers the candidate's x field and y byte.
+// Each axis is then within one unit of the true difference, so every pair inside the cut-off
 // passes |d| < (1 + m) / u with m = 1.01 |w| / 256 + 1e-5; the evaluation drops the rest.
-__device__ inline int code_dist2(uint32_t cj, uint32_t QXY, int Qz)
+__device__ inline short2_t code_dxy(uint32_t cj, uint32_t QXY)
 {
-    // bytes 0, 1 (x16 of the row segment, before the first cell's offset) and 2 (y) of the code
-    const uint32_t p = __builtin_amdgcn_perm(0u, cj, 0x0c020100u);
-    const short2_t d = __builtin_bit_cast(short2_t, QXY) - __builtin_bit_cast(short2_t, p);
-    const int dz = Qz - (int)(cj >> 24);
-    return __builtin_amdgcn_sdot2(d, d, __mul24(dz, dz), false);
+    return __builtin_bit_cast(short2_t, QXY) - __builtin_bit_cast(short2_t, __builtin_amdgcn_perm(0u, cj, 0x0c020100u));
 }
+__device__ inline int code_dist2(short2_t d, int dz) { return __builtin_amdgcn_sdot2(d, d, __mul24(dz, dz), false); }
 // beads per workgroup of THREADS threads with SPLIT lanes per bead (21 per wavefront for 3,
 // 7 for 9; lane 63 idle)
 constexpr int hit_beads(int threads, int split) { return split == 1 ? threads : (threads / 64) * (63 / split); }
@@ -236,7 +249,7 @@ __device__ __attribute__((always_inline)) inline void hitlist_body(const PairArg
     static_assert(CAP > PASS, "room for a pass");
     static_assert(!(OBS && EPI), "the observing launch ends a sequence of steps");
     __shared__ uint32_t hits[CAP][THREADS];
-    __shared__ float stab[kTableStride];
+    __shared__ float4 stab[kTypeStride];   // a, gamma, sqrt(gamma) sqrt(24 kT / dt) per type pair
     const int blk = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
     if (blk >= nblocks) return;   // whole workgroups
     int box = 0, i0 = blk * hit_beads(THREADS, SPLIT), i1 = A.n;
@@ -245,13 +258,16 @@ __device__ __attribute__((always_inline)) inline void hitlist_body(const PairArg
         box = hb.x; i0 = hb.y; i1 = hb.z;
     }
     const BoxDev& B = MULTI ? A.boxes[box] : B0;
-    // the box's interaction table in LDS, and the shift of each neighbour-cell code
+    // the box's interaction table in LDS, and for each segment code the image of x in cells
+    // (mod 4, in the place of the cell index in a bead's word) and the shifts of y and z
     __shared__ float4 shtab[64];
     const float* gtab = A.table + (size_t)box * kTableStride;
-    for (int q = threadIdx.x; q < kTableStride; q += THREADS) stab[q] = gtab[q];
+    for (int q = threadIdx.x; q < kTypeStride; q += THREADS)
+        stab[q] = make_float4(gtab[q], gtab[kTypeStride + q], gtab[2 * kTypeStride + q] * B.invrootdt, 0.f);
     if (threadIdx.x < 64) {
-        const int q = threadIdx.x;
-        shtab[q] = make_float4((float)(1 - (q & 3)) * B.w[0], (float)(1 - ((q >> 2) & 3)) * B.w[1],
+        const int q = threadIdx.x, im = q & 3;
+        const int s = im == 1 ? -B.n[0] : (im == 2 ? B.n[0] : 0);
+        shtab[q] = make_float4(__int_as_float((s & 3) << kCellXShift), (float)(1 - ((q >> 2) & 3)) * B.w[1],
                                (float)(1 - (q >> 4)) * B.w[2], 0.f);
     }
     __syncthreads();
@@ -268,39 +284,46 @@ __device__ __attribute__((always_inline)) inline void hitlist_body(const PairArg
     if (OBS)
         for (int q = 0; q < 10; ++q) vir[q] = 0.0;
     float fx = 0.f, fy = 0.f, fz = 0.f;
-    if (valid) {
-        const float4 pi = A.pos[i];
-        const int wi = __float_as_int(pi.w);
+    // every lane of a wavefront with a bead runs the scan (lanes without one find nothing)
+    if (__ballot(valid) != 0) {
+        const int ii = min(i, i1 - 1);
+        const float4 pi = A.pos[ii];
         const RngKey K = rng_key(B, *A.step);
-        const float* tab = stab;
-        const float4 vi = A.vp[i];
-        const int ti = bead_type(wi);
+        const float4 vi = A.vp[ii];
         const uint32_t idi = (uint32_t)__float_as_int(vi.w);
+        const int key = A.key[ii];
         int c[3];
-        key_cell(A.key[i] - B.koff, B, c);
+        key_cell(key - B.koff, B, c);
+        // the bead's word for the evaluation: its row of the interaction table and, in the
+        // place of the cell index, minus its cell's x index mod 4
+        const int hw = (bead_type(__float_as_int(pi.w)) * kMaxTypes << 8) | ((-c[0] & 3) << kCellXShift);
         float sv[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
         // this thread's list: column t of hits, entry e at hits[e][t]; wp is the next free one
         lds_u32* const lbase = (lds_u32*)&hits[0][t];
         const uint32_t laddr = (uint32_t)(size_t)lbase;   // its LDS byte address
         uint32_t wp = laddr;
-        // one listed partner: slot | neighbour-cell code, its position and velocity
-        auto eval = [&](uint32_t e, const float4& pj, const float4& vj) {
+        // one listed partner of a bead (offset bx, by, bz, word bw, velocity and id bv): the
+        // entry is slot | segment code, pj and vj the partner's position and velocity
+        auto force = [&](uint32_t e, const float4& pj, const float4& vj, float bx, float by, float bz, int bw,
+                         float bvx, float bvy, float bvz, uint32_t bid, float& Fx, float& Fy, float& Fz) {
             const float4 sh = shtab[e >> kHitSlotBits];
-            const float ddx = (pi.x + sh.x) - pj.x;
-            const float ddy = (pi.y + sh.y) - pj.y;
-            const float ddz = (pi.z + sh.z) - pj.z;
+            // the partner's cell less the bead's along x (-1, 0 or 1) from the indices mod 4
+            const int wj = __float_as_int(pj.w);
+            const int dc = __builtin_amdgcn_sbfe(wj + bw + __float_as_int(sh.x), kCellXShift, 2);
+            const float ddx = fmaf(-(float)dc, B.w[0], bx) - pj.x;
+            const float ddy = (by + sh.y) - pj.y;
+            const float ddz = (bz + sh.z) - pj.z;
             const float dr2 = ddx * ddx + ddy * ddy + ddz * ddz;
-            const int tt = ti * kMaxTypes + bead_type(__float_as_int(pj.w));
-            const float dxdv = ddx * (vi.x - vj.x) + ddy * (vi.y - vj.y) + ddz * (vi.z - vj.z);
+            const float dxdv = ddx * (bvx - vj.x) + ddy * (bvy - vj.y) + ddz * (bvz - vj.z);
+            const float4 tab = stab[(bw >> 8) + bead_type(wj)];
             float pe;
-            float s = pair_scalar(dr2, dxdv, tab[tt], tab[2 * kTypeStride + tt], tab[kTypeStride + tt], idi,
-                                  (uint32_t)__float_as_int(vj.w), B.invrootdt, K, OBS ? &pe : nullptr);
+            float s = pair_scalar_t(dr2, dxdv, tab.x, tab.z, tab.y, bid, (uint32_t)__float_as_int(vj.w), K,
+                                    OBS ? &pe : nullptr);
             // the scan lists a superset: the bead itself and partners just past the cut-off
             const bool in_range = pair_in_range(dr2);
             s = in_range ? s : 0.f;
             if (OBS) pe = in_range ? pe : 0.f;
-            const float Fx = s * ddx, Fy = s * ddy, Fz = s * ddz;
-            fx += Fx; fy += Fy; fz += Fz;
+            Fx = s * ddx; Fy = s * ddy; Fz = s * ddz;
             if (OBS) {
                 sv[0] += ddx * Fx; sv[1] += ddy * Fx; sv[2] += ddz * Fx;
                 sv[3] += ddx * Fy; sv[4] += ddy * Fy; sv[5] += ddz * Fy;
@@ -308,10 +331,14 @@ __device__ __attribute__((always_inline)) inline void hitlist_body(const PairArg
                 sv[9] += pe;
             }
         };
+        auto eval = [&](uint32_t e, const float4& pj, const float4& vj) {
+            float Fx, Fy, Fz;
+            force(e, pj, vj, pi.x, pi.y, pi.z, hw, vi.x, vi.y, vi.z, idi, Fx, Fy, Fz);
+            fx += Fx; fy += Fy; fz += Fz;
+        };
         // evaluate and clear this thread's list, two entries per pass (both loads in
         // flight, two independent random-stream chains), in list order
-        auto drain = [&]() {
-            const int nh = (int)(wp - laddr) / (4 * THREADS);
+        auto drain_to = [&](int nh) {
             int h = 0;
             for (; h + 1 < nh; h += 2) {
                 const uint32_t ea = lbase[h * THREADS], eb = lbase[(h + 1) * THREADS];
@@ -328,105 +355,185 @@ __device__ __attribute__((always_inline)) inline void hitlist_body(const PairArg
             }
             wp = laddr;
         };
+        auto drain = [&]() { drain_to((int)(wp - laddr) / (4 * THREADS)); };
+        // The lists of a wavefront's 64 beads.  Their lengths differ (13.0 partners at density
+        // 3, the longest of 64 lists 17), and a loop over the longest leaves a quarter of the
+        // lanes idle.  So every lane evaluates its first R entries, R the mean length less
+        // one or two, and the entries past R of all lanes are packed and evaluated 64 at a
+        // time, each lane taking whichever bead's partner comes next (the bead's data by lane
+        // permutes), the forces handed back through LDS and added by the bead's own lane in
+        // list order (list by list to the longest: condensate 64^3 84 us per launch, this way 82;
+        // and where a list fills up within a row, all are evaluated this way instead of that
+        // lane's alone: the box's unrelaxed start 163 -> 99 us).  The LDS rows below R, evaluated by then, hold the packed entries, their
+        // beads and the forces, three rows per 64.
+        auto evaluate_lists = [&]() {
+            const int n = (int)(wp - laddr) / (4 * THREADS);
+            int R = max((__builtin_amdgcn_readlane(wave_incl_scan(n), 63) >> 6) - 1, 0) & ~1;
+            int ex, incl, total, nb;
+            while (true) {
+                ex = max(n - R, 0);
+                incl = wave_incl_scan(ex);
+                total = __builtin_amdgcn_readlane(incl, 63);
+                nb = (total + 63) >> 6;
+                if (3 * nb <= R) break;
+                R += 2;   // (room for the packed entries; none are left at the longest list)
+            }
+            drain_to(min(n, R));
+            if (nb == 0) return;
+            lds_u32* const wbase = lbase - lane;   // the wavefront's column 0
+            const int off = incl - ex;
+            for (int k = 0; k < ex; ++k) {
+                const int q = off + k;
+                lds_u32* const to = wbase + (q >> 6) * (3 * THREADS) + (q & 63);
+                to[0] = lbase[(R + k) * THREADS];
+                to[THREADS] = (uint32_t)lane;
+            }
+            __builtin_amdgcn_wave_barrier();
+            for (int b = 0; b < nb; ++b) {
+                lds_u32* const row = lbase + b * (3 * THREADS);
+                const bool act = 64 * b + lane < total;
+                const uint32_t e = row[0];
+                const int o = (int)row[THREADS] & 63;
+                const float bx = __shfl(pi.x, o), by = __shfl(pi.y, o), bz = __shfl(pi.z, o);
+                const float bvx = __shfl(vi.x, o), bvy = __shfl(vi.y, o), bvz = __shfl(vi.z, o);
+                const int bw = __shfl(hw, o);
+                const uint32_t bid = (uint32_t)__shfl((int)idi, o);
+                if (act) {
+                    const int j = (int)(e & kHitSlotMask);
+                    float Fx, Fy, Fz;
+                    force(e, A.pos[j], A.vp[j], bx, by, bz, bw, bvx, bvy, bvz, bid, Fx, Fy, Fz);
+                    row[0] = __float_as_uint(Fx);
+                    row[THREADS] = __float_as_uint(Fy);
+                    row[2 * THREADS] = __float_as_uint(Fz);
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
+            for (int k = 0; k < ex; ++k) {
+                const int q = off + k;
+                lds_u32* const at = wbase + (q >> 6) * (3 * THREADS) + (q & 63);
+                fx += __uint_as_float(at[0]);
+                fy += __uint_as_float(at[THREADS]);
+                fz += __uint_as_float(at[2 * THREADS]);
+            }
+        };
         // candidate test on the scan codes in integer code units (code_dist2): each axis of
         // the tested difference is within one unit u_a = w_a / 256 of the true one, so the
         // distance is within m = 1.01 |w| / 256 + 1e-5 of it and, with the sum of squares taken
         // in units of the smallest u_a, every pair inside the cut-off passes
-        // sum d_a^2 < ((1 + m) / u_min)^2 (exact for cubic cells, a wider superset for
+        // sum d_a^2 < ((1 + m) / u_min)^2 = thr (exact for cubic cells, a wider superset for
         // others); the evaluation drops the rest (the bead itself among them).
-        const float inv_ux = 256.0f / B.w[0], inv_uy = 256.0f / B.w[1], inv_uz = 256.0f / B.w[2];
-        const float m = sqrtf(B.w[0] * B.w[0] + B.w[1] * B.w[1] + B.w[2] * B.w[2]) * (1.01f / 256.0f) + 1e-5f;
-        const float tu = (1.0f + m) * fmaxf(inv_ux, fmaxf(inv_uy, inv_uz));
-        const uint32_t thr = (uint32_t)(tu * tu) + 1u;
+        const int thr = B.qthr;
         const char* cbase = reinterpret_cast<const char*>(A.code);
-        // a row wraps through the periodic x face only for beads in the first or last cell of
-        // their row: wavefronts without such a bead scan one segment per row
-        const int nseg = __ballot(c[0] == 0 || c[0] == B.n[0] - 1) != 0 ? 2 : 1;
+        const char* sbase = reinterpret_cast<const char*>(A.cstart);
+        // the bead's position in code units, floored as the codes are: x with its cell index
+        // and y in one register, z apart.  A row dy, dz sees them 256 dy and 256 dz lower.
+        const int Qx = (int)floorf(pi.x * B.qinv[0]) + (c[0] << 8);
+        const uint32_t QXY0 = ((uint32_t)Qx & 0xFFFFu) | ((uint32_t)(int)floorf(pi.y * B.qinv[1]) << 16);
+        const int Qz0 = (int)floorf(pi.z * B.qinv[2]);
+        // A row's cells are consecutive keys: cells cx-1 .. cx+1 are one range of slots, or,
+        // where the row wraps through the periodic x face, two cells and the one across the
+        // face, a second segment of that lane.
+        const int nx = B.n[0], nxy = B.n[0] * B.n[1], nall = nxy * B.n[2];
+        const bool xl = c[0] == 0, edge = xl || c[0] == nx - 1;
+        const bool across = __ballot(edge) != 0;
+        const int ym = c[1] == 0 ? nxy - nx : -nx, yp = c[1] == B.n[1] - 1 ? nx - nxy : nx;
+        const int zm = c[2] == 0 ? nall - nxy : -nxy, zp = c[2] == B.n[2] - 1 ? nxy - nall : nxy;
+        const int pa = xl ? key : key - 1, pb = pa + (edge ? 2 : 3);
+        // (the bead's own cell where there is none: its starts are loaded and not used)
+        const int pe = xl ? key + nx - 1 : (edge ? key + 1 - nx : key);
+        // code and x of the second segment: the cell across the face, at -1 or nx
+        const uint32_t img = xl ? 1u : 2u;
+        const int qimg = (xl ? nx : -nx) << 8;
         // the neighbour rows of this lane: all nine, one z layer (SPLIT 3) or one row (SPLIT 9)
-        const int dz0 = SPLIT == 1 ? -1 : (SPLIT == 3 ? part - 1 : part / 3 - 1);
-        const int dz1 = SPLIT == 1 ? 1 : dz0;
-        const int dy0 = SPLIT == 9 ? part % 3 - 1 : -1, dy1 = SPLIT == 9 ? dy0 : 1;
-        for (int dz = dz0; dz <= dz1; ++dz) {
-            int cz = c[2] + dz;
-            cz += (cz < 0) ? B.n[2] : ((cz >= B.n[2]) ? -B.n[2] : 0);
-            for (int dy = dy0; dy <= dy1; ++dy) {
-                int cy = c[1] + dy;
-                cy += (cy < 0) ? B.n[1] : ((cy >= B.n[1]) ? -B.n[1] : 0);
-                // the row's cells are consecutive keys: cells cx-1 .. cx+1 are one range, or two
-                // where the row wraps through the periodic x face.  Segment s covers the cells
-                // fx .. lx (wrapped indices), the first of them at fu = -1, 0 or +1 cells from
-                // the bead's along x (unwrapped).  Candidates come in the order of a cell-by-cell
-                // walk (x innermost).
-                const int krow = B.koff + B.n[0] * (cy + B.n[1] * cz);
-                const uint32_t qrow = (uint32_t)(((dy + 1) << 2) | ((dz + 1) << 4));
-                // the bead's y and z seen from this row (the shifts of the evaluation), in code
-                // units, floored as the codes are
-                const int Qy = (int)floorf((pi.y - (float)dy * B.w[1]) * inv_uy);
-                const int Qz = (int)floorf((pi.z - (float)dz * B.w[2]) * inv_uz);
-                const int cx = c[0], nx = B.n[0];
-                for (int sgm = 0; sgm < nseg; ++sgm) {
-                    int fx, lx, fu;
-                    if (cx >= 1 && cx <= nx - 2) { fx = cx - 1; lx = sgm ? cx - 2 : cx + 1; fu = -1; }
-                    else if (cx == 0) { fx = sgm ? 0 : nx - 1; lx = sgm ? 1 : nx - 1; fu = sgm ? 0 : -1; }
-                    else { fx = sgm ? 0 : nx - 2; lx = sgm ? 0 : nx - 1; fu = sgm ? 1 : -1; }
-                    const int j0 = A.cstart[krow + fx], j1 = (lx >= fx) ? A.cstart[krow + lx + 1] : j0;
-                    const uint32_t fxbits = (uint32_t)(fx & 0xFF) << 8;
-                    const uint32_t code = ((uint32_t)(fu + 1) | qrow) << kHitSlotBits;
-                    // the bead's x in the segment (code units) plus fxbits, mod 2^16: code bytes
-                    // 0-1 less fxbits are r * 256 + q_x, r the candidate's cell counted from the
-                    // segment's first one, so the packed difference is x less that
-                    const int Qx = (int)floorf((pi.x - (float)fu * B.w[0]) * inv_ux) + (int)fxbits;
-                    const uint32_t QXY = ((uint32_t)Qx & 0xFFFFu) | ((uint32_t)Qy << 16);
-                    // list entry of slot j: (j | code) + (r << 26), the neighbour-cell code of
-                    // the candidate's cell; r = (code byte 1 - fx) mod 64 = ((bits 8-13 of the
-                    // code) - fx) mod 64, and e0 - j0 holds the parts that do not depend on the
-                    // candidate
-                    const uint32_t e0 = ((uint32_t)j0 | code) - ((uint32_t)(fx & 0xFF) << kHitSlotBits);
-                    // PASS consecutive candidates per pass from one 16-byte (4) or 8-byte (2)
-                    // load, the next pass's loaded before these are tested.  (A wavefront
-                    // runs each segment to its lanes' longest count rounded up to the pass
-                    // width.)  The loads run up to seven codes past the segment (the next
-                    // cells' beads, or the padding after the last slot); none of those is
-                    // listed.  Slots are below 2^26, so byte offsets fit 32 bits and the loads
-                    // address from the array base.  Every candidate is stored at the list's
-                    // write pointer, which advances on a hit only (a miss is overwritten by
-                    // the next store).
-                    uint32_t e = e0;
-                    // one candidate: stored at the write pointer, which advances on a hit
-                    auto put = [&](uint32_t cj, uint32_t ej, bool in_seg) {
-                        const bool hit = ((uint32_t)code_dist2(cj, QXY, Qz) < thr) & in_seg;
-                        *(lds_u32*)(size_t)wp = ej + (((cj >> 8) & 63u) << kHitSlotBits);
-                        wp += hit ? 4 * THREADS : 0;
-                    };
-                    if constexpr (PASS == 4) {
-                        code4_t c4 = *reinterpret_cast<const code4_t*>(cbase + ((uint32_t)j0 << 2));
-                        for (int j = j0; j < j1; j += 4, e += 4) {
-                            const code4_t cn = *reinterpret_cast<const code4_t*>(cbase + ((uint32_t)j << 2) + 16);
-                            // room for the pass: a list past CAP - 4 entries is evaluated first
-                            // (overflow inside a segment: this lane alone)
-                            if (wp > laddr + 4 * (CAP - 4) * THREADS) drain();
-                            put(c4.x, e, true);
-                            put(c4.y, e + 1u, j + 1 < j1);
-                            put(c4.z, e + 2u, j + 2 < j1);
-                            put(c4.w, e + 3u, j + 3 < j1);
-                            c4 = cn;
-                        }
-                    } else {
-                        code2_t c2 = *reinterpret_cast<const code2_t*>(cbase + ((uint32_t)j0 << 2));
-                        for (int j = j0; j < j1; j += 2, e += 2) {
-                            const code2_t cn = *reinterpret_cast<const code2_t*>(cbase + ((uint32_t)j << 2) + 8);
-                            if (wp > laddr + 4 * (CAP - 2) * THREADS) drain();
-                            put(c2.x, e, true);
-                            put(c2.y, e + 1u, j + 1 < j1);
-                            c2 = cn;
-                        }
-                    }
-                    if (FLUSH < CAP && __ballot(wp >= laddr + 4 * FLUSH * THREADS) != 0) drain();
+        constexpr int NR = 9 / SPLIT;
+        auto row_key = [&](int r) {
+            const int dz = r / 3, dy = r - 3 * dz;   // 0, 1, 2
+            return (dy == 0 ? ym : (dy == 2 ? yp : 0)) + (dz == 0 ? zm : (dz == 2 ? zp : 0));
+        };
+        using code_t = typename std::conditional<PASS == 4, code4_t, code2_t>::type;
+        auto start_of = [&](int k) { return *reinterpret_cast<const int*>(sbase + ((uint32_t)k << 2)); };
+        auto codes_at = [&](uint32_t b) { return *reinterpret_cast<const code_t*>(cbase + b); };
+        // (a row's starts are loaded one row ahead)
+        int jn0 = start_of(pa + row_key(part * NR)), jn1 = start_of(pb + row_key(part * NR));
+        for (int q = 0; q < NR; ++q) {
+            const int r = part * NR + q;
+            const int dz = r / 3, dy = r - 3 * dz;
+            const int j0 = jn0, j1 = jn1;
+            code_t cc = codes_at((uint32_t)j0 << 2);
+            if (q + 1 < NR) {
+                const int d = row_key(r + 1);
+                jn0 = start_of(pa + d);
+                jn1 = start_of(pb + d);
+            }
+            const int krow = row_key(r);
+            const uint32_t code = (uint32_t)((dy << 2) | (dz << 4)) << kHitSlotBits;
+            uint32_t QXY = QXY0 + ((uint32_t)(1 - dy) << 24);
+            const int Qz = Qz0 + ((1 - dz) << 8);
+            // list entries of the segment's first candidate and of its end
+            uint32_t e = (uint32_t)j0 | code, e1 = valid ? (uint32_t)j1 | code : e;
+            uint32_t jb = (uint32_t)j0 << 2;
+            int2u ce = {0, 0};
+            if (across) ce = *reinterpret_cast<const int2u*>(sbase + ((uint32_t)(pe + krow) << 2));
+            bool more = valid && edge;
+            // PASS consecutive candidates per pass, the next pass's codes loaded as soon as
+            // these are subtracted.  The loads run up to seven codes past the segment (the next
+            // cells' beads, or the padding after the last slot); none of those is listed.
+            // Slots are below 2^26, so byte offsets fit 32 bits and the loads address from the
+            // array base.  Every candidate is stored at the list's write pointer, which
+            // advances on a hit only (a miss is overwritten by the next store).
+            auto put = [&](int d2, uint32_t ej, bool in_seg) {
+                *(lds_u32*)(size_t)wp = ej;
+                wp += (d2 < thr) & in_seg ? 4 * THREADS : 0;
+            };
+            // one pass
+            auto pass = [&]() {
+                short2_t d[PASS];
+                int z[PASS];
+#pragma unroll
+                for (int k = 0; k < PASS; ++k) {
+                    d[k] = code_dxy(cc[k], QXY);
+                    z[k] = Qz - (int)(cc[k] >> 24);
                 }
+                jb += 4 * PASS;
+                cc = codes_at(jb);
+                put(code_dist2(d[0], z[0]), e, true);
+#pragma unroll
+                for (int k = 1; k < PASS; ++k) put(code_dist2(d[k], z[k]), e + k, e + k < e1);
+                e += PASS;
+            };
+            const uint32_t full = laddr + 4 * (CAP - PASS) * THREADS;   // no room for a pass beyond
+            while (true) {
+                if (!across) {
+                    while (e < e1 && wp <= full) pass();
+                } else {
+                    while (true) {
+                        if (e >= e1) {
+                            // the cell across the x face, for a bead beside it
+                            if (!more) break;
+                            more = false;
+                            e = (uint32_t)ce.x | code | (img << kHitSlotBits);
+                            e1 = (uint32_t)ce.y | code | (img << kHitSlotBits);
+                            jb = (uint32_t)ce.x << 2;
+                            QXY = (QXY & 0xFFFF0000u) | (uint32_t)((Qx + qimg) & 0xFFFF);
+                            if (e >= e1) break;
+                            cc = codes_at(jb);
+                        }
+                        if (wp > full) break;
+                        pass();
+                    }
+                }
+                // a lane whose list is full leaves the loop before its segment's end: the
+                // wavefront then evaluates all its lists, as after the last row
+                const bool full_lists = __ballot(e < e1 || more) != 0;
+                if (full_lists || q == NR - 1 || (FLUSH < CAP && __ballot(wp >= laddr + 4 * FLUSH * THREADS) != 0)) {
+                    if constexpr (SPLIT == 1) evaluate_lists();
+                    else drain();
+                }
+                if (!full_lists) break;
+                cc = codes_at(jb);
             }
         }
-        drain();
-        if (SPLIT == 1) A.frc[i] = make_float4(fx, fy, fz, 0.f);
+        if (SPLIT == 1 && valid) A.frc[i] = make_float4(fx, fy, fz, 0.f);
         if (OBS)
             for (int q = 0; q < 10; ++q) vir[q] = 0.5 * (double)sv[q];
     }
@@ -448,19 +555,20 @@ __device__ __attribute__((always_inline)) inline void hitlist_body(const PairArg
     }
     if (EPI) pair_epilogue(A, B, i, valid && part == 0, fx, fy, fz);
     if (OBS) {
-        accumulate_boxes<10, THREADS / 64>(vir, valid ? box : -1, box, kObsVir, A.acc);
+        // (lanes without a bead too: they evaluate pairs of the wavefront's others)
+        accumulate_boxes<10, THREADS / 64>(vir, box, box, kObsVir, A.acc);
     }
 }
 
-// Six wavefronts per SIMD (three 512-thread or six 256-thread workgroups per CU, which the
-// LDS of the 24-entry lists also allows) need at most 80 VGPRs: the force-only kernel is held
-// to that; the kernel with observables runs once per batch of steps and is left freer.
-// wavefronts per SIMD that the LDS of a schedule allows (160 KB per CU, four SIMDs), at most 6
+// Wavefronts per SIMD that the LDS of a schedule allows (160 KB per CU, four SIMDs), at most
+// 5: the kernel needs 92 VGPRs (96 with the epilogue), and held to the 80 of six wavefronts it
+// spills (condensate 64^3: 123 us against 80 us per launch for 512 and 256 threads with 24
+// entries).  512-thread workgroups then fit twice, four wavefronts per SIMD.
 constexpr int hit_waves(int threads, int cap)
 {
-    const int lds = cap * threads * 4 + kTableStride * 4 + 64 * 16;
-    const int w = (160 * 1024 / lds) * (threads / 64) / 4;
-    return w < 6 ? w : 6;
+    const int lds = cap * threads * 4 + kTypeStride * 16 + 64 * 16;
+    const int per = threads / 64, w = (160 * 1024 / lds) * per / 4;
+    return w < 5 ? w : 20 / per * per / 4;
 }
 // the occupancy a kernel is held to: the split schedules run small boxes, which never fill
 // the SIMDs, and get the registers of four wavefronts (no spills)
@@ -495,7 +603,13 @@ constexpr Schedule kSchedule[kSchedules] = {
     {DPD_PAIR_HITLIST, 256, 12, 12, 3, "hitlist-split3-t256-c12"},
     {DPD_PAIR_HITLIST, 256, 8, 8, 9, "hitlist-split9-t256-c8"},
 };
-constexpr int kDefaultSchedule = 0;
+constexpr int kDefaultSchedule = 2;
+// The automatic choice for n beads: nine lanes per bead while one thread per bead would leave
+// most of the 1024 SIMDs without a wavefront, three lanes while it would leave them one or two,
+// then one (microseconds per step at 9, 3 and 1 lanes, density 3: chains 24.0k beads 28.6, 32.5,
+// 40.1; 41k 34.1, 35.6, 42.9; 66k 37.7, 37.4, 42.6; 98k 47.3, 43.5, 45.6; 140k 55.8, 52.8, 50.2;
+// water 5.2k 21.9, 25.6, 34.9; 41k 33.7, 32.2, 39.5; 98k 48.1, 39.0, 40.6; 140k 58.9, 49.7, 44.9).
+constexpr int size_schedule(int64_t n) { return n <= 45000 ? 6 : (n <= 105000 ? 5 : kDefaultSchedule); }
 constexpr int kFullShellSchedule = 4;
 
 // hit-list launch of schedule S on a grid of workgroups of its thread count
@@ -545,7 +659,7 @@ inline hipError_t launch_pair_kernel(int sched, const PairArgs& a, const BoxDev&
 {
     const bool multi = a.nbox > 1;
     if (sched < 0 || sched >= kSchedules) sched = kDefaultSchedule;
-    if (kSchedule[sched].kernel == DPD_PAIR_HITLIST && a.n <= (int)kHitSlotMask && (!multi || a.hitblk)) {
+    if (kSchedule[sched].kernel == DPD_PAIR_HITLIST && a.n <= (int)kHitSlotMask && a.ngroups < (1 << 24) && (!multi || a.hitblk)) {
         const int nb = kSchedule[sched].beads();
         const int gh = multi ? a.nhitblk : (a.n + nb - 1) / nb;
         if (obs) {
