@@ -1448,6 +1448,7 @@ int slice_tables(dpd_engine* e, int32_t box, int32_t nslices, double* tab, size_
     a.ang_bead = e->ang_bead;
     a.ang_par = e->ang_par;
     a.a0 = a.a1 = 0;
+    a.nbeads = (int)h.n;
     a.nslice = nslices;
     a.ntypes = nt;
     a.nidx = nt * nt;

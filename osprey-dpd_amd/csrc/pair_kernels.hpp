@@ -483,7 +483,7 @@ __device__ __attribute__((always_inline)) inline void hitlist_body(const PairArg
             // advances on a hit only (a miss is overwritten by the next store).
             auto put = [&](int d2, uint32_t ej, bool in_seg) {
                 *(lds_u32*)(size_t)wp = ej;
-                wp += (d2 < thr) & in_seg ? 4 * THREADS : 0;
+                wp += ((d2 < thr) & in_seg) ? 4 * THREADS : 0;
             };
             // one pass
             auto pass = [&]() {

@@ -7,10 +7,18 @@
 // beads.  Here the tables are produced on demand for the engine's current state: the pair
 // forces are re-evaluated with the same arithmetic and the same counter-based random
 // draws as the step kernels, so right after dpd_step they are the last step's forces.
-// Thread per bead walks the 27 neighbour cells (each pair is seen from both sides and
-// adds half of its share under each ordered type pair); thread per bond adds the bond's
-// share under (head type, tail type).  FP64 tables are accumulated in LDS per workgroup
-// when they fit, and with global FP64 atomics otherwise.
+// Pair and bond forces are parallel to dx, so F (x) dx is symmetric: six sums, mirrored when
+// they leave LDS.
+//
+// What bounds it: FP64 atomics (global ones at ~3e9 per second, whatever the addresses; a
+// wavefront's LDS ones serialise lane by lane).  So every table entry is summed in LDS first:
+// pairs in a window of the slices that one layer of cells reaches (a workgroup takes slots of
+// one z layer at a time, and the slots are sorted by z), bonds and bond pairs in windows of
+// the whole table.  Bilayer 48x48x32, 221k beads, 64 slices (global atomics per pair and bond
+// -> now): pairs 13,700 -> 177 us, bonds 715 -> 15, bond pairs 1,767 -> 28.
+#include <algorithm>
+#include <cmath>
+
 #include "pair_kernels.hpp"
 #include "slice_stress.hpp"
 
@@ -18,16 +26,13 @@ namespace dpd {
 
 namespace {
 
-// the z-slice split of one interaction (see orc_slice_add for the rule); tab is
-// [nslice][nidx][9]
-__device__ inline void slice_add(double* tab, int nslice, double Lz, int idx, int nidx, double z1, double z2,
-                                 const double F[3], const double dx[3], double wgt)
+// The z-slice split of one interaction (see orc_slice_add for the rule) between z1 and z2,
+// dz = z1 - z2 unwrapped: add(slice, share) for every slice spanned.
+template <class Add>
+__device__ inline void slice_split(int nslice, double Lz, double z1, double z2, double dz, const Add& add)
 {
     const double width = Lz / nslice, inv = nslice / Lz;
-    double fdx[9];
-    for (int a = 0; a < 3; ++a)
-        for (int b = 0; b < 3; ++b) fdx[3 * a + b] = F[a] * dx[b] * wgt;
-    double zd = dx[2], zu, zl;
+    double zd = dz, zu, zl;
     if (zd > 0.00001) { zu = z1 * inv; zl = z2 * inv; }
     else if (zd < -0.00001) { zd = -zd; zu = z2 * inv; zl = z1 * inv; }
     else { zu = zl = z1 * inv; }
@@ -35,10 +40,6 @@ __device__ inline void slice_add(double* tab, int nslice, double Lz, int idx, in
     // the table against a position rounded onto Lz
     int iu = min(max((int)zu, 0), nslice - 1), il = min(max((int)zl, 0), nslice - 1);
     const double ru = zu - (double)iu, rl = zl - (double)il;
-    auto add = [&](int sl, double share) {
-        double* t = tab + ((size_t)sl * nidx + idx) * 9;
-        for (int q = 0; q < 9; ++q) atomicAdd(t + q, fdx[q] * share);
-    };
     if (iu == il) {
         if (zu != zl || ru > 0.00001) {
             add(il, 1.0);
@@ -59,6 +60,10 @@ __device__ inline void slice_add(double* tab, int nslice, double Lz, int idx, in
     }
 }
 
+// the six sums of a symmetric tensor and where the nine components read them
+__device__ constexpr int kSym[9] = {0, 1, 2, 1, 3, 4, 2, 4, 5};
+__device__ constexpr int kTri[6] = {0, 1, 2, 4, 5, 8};   // their components 3a + b, a <= b
+
 __device__ inline double wrapped_z(const SliceArgs& A, int slot)
 {
     int c[3];
@@ -66,91 +71,235 @@ __device__ inline double wrapped_z(const SliceArgs& A, int slot)
     return (double)c[2] * A.B.wd[2] + (double)A.pos[slot].z;
 }
 
-template <bool SHARED>
-__global__ __launch_bounds__(256) void k_slice_pairs(SliceArgs A, double* __restrict__ out)
+// The pair table, each pair once (half shell: the cell's later beads, the cell after it in the
+// row and the nine and three cells of the rows after).  Workgroup b takes slots [b, b + 1) per,
+// one z layer of cells after the other; lds holds `copies` tables [win][types][6] (types: unordered
+// pairs) of the slices from s0 on, lane l adding to copy l mod copies.  The sums of types ti <= tj
+// go to their components a <= b of out; k_slice_mirror spreads them afterwards.  Without WIN
+// (no window fits LDS) the pairs add to out themselves.
+constexpr int kSliceList = 12;   // listed partners per thread
+template <bool WIN>
+__global__ __launch_bounds__(256) void k_slice_pairs(SliceArgs A, double* __restrict__ out, int per, int win, int copies)
 {
     extern __shared__ double lt[];
-    const int ntab = A.nslice * A.nidx * 9;
-    double* tab = SHARED ? lt : out;
-    if (SHARED) {
-        for (int q = threadIdx.x; q < ntab; q += blockDim.x) lt[q] = 0.0;
-        __syncthreads();
-    }
+    __shared__ int list[kSliceList][256];         // partner slots
+    __shared__ uint8_t row[kSliceList][256];      // and their row and image codes
     const BoxDev& B = A.B;
-    const double Lz = (double)B.n[2] * B.wd[2];
+    const int t = threadIdx.x;
+    const int ntri = A.ntypes * (A.ntypes + 1) / 2, tab = win * ntri * 6, stride = tab + 1;
+    const double Lz = (double)B.n[2] * B.wd[2], inv = A.nslice / Lz;
     const RngKey K = rng_key(B, *A.step);
     // the box's beads are the slots of its cell keys
-    const int s0 = A.cstart[B.koff], s1 = A.cstart[B.koff + B.ngroups * kGroupKeys];
-    for (int i = s0 + blockIdx.x * blockDim.x + threadIdx.x; i < s1; i += gridDim.x * blockDim.x) {
-        const float4 pi = A.pos[i], vi = A.vp[i];
-        const int ti = bead_type(__float_as_int(pi.w));
-        const uint32_t idi = (uint32_t)__float_as_int(vi.w);
-        int c[3];
-        key_cell(A.key[i] - B.koff, B, c);
-        const double zi = (double)c[2] * B.wd[2] + (double)pi.z;
-        for (int nb = 0; nb < 27; ++nb) {
-            const int ox = nb % 3 - 1, oy = (nb / 3) % 3 - 1, oz = nb / 9 - 1;
-            int cx = c[0] + ox, cy = c[1] + oy, cz = c[2] + oz;
-            cx += (cx < 0) ? B.n[0] : ((cx >= B.n[0]) ? -B.n[0] : 0);
-            cy += (cy < 0) ? B.n[1] : ((cy >= B.n[1]) ? -B.n[1] : 0);
-            cz += (cz < 0) ? B.n[2] : ((cz >= B.n[2]) ? -B.n[2] : 0);
-            const int k = B.koff + cell_key(cx, cy, cz, B);
-            const float sx = (float)ox * B.w[0], sy = (float)oy * B.w[1], sz = (float)oz * B.w[2];
-            for (int j = A.cstart[k], j1 = A.cstart[k + 1]; j < j1; ++j) {
-                if (j == i) continue;
-                const float4 pj = A.pos[j];
-                const float dx = (pi.x - pj.x) - sx, dy = (pi.y - pj.y) - sy, dz = (pi.z - pj.z) - sz;
-                const float dr2 = dx * dx + dy * dy + dz * dz;
-                if (!(dr2 < 1.0f && dr2 > 1e-18f)) continue;
-                const float4 vj = A.vp[j];
-                const int tj = bead_type(__float_as_int(pj.w));
-                const int tt = ti * kMaxTypes + tj;
-                const float dxdv = dx * (vi.x - vj.x) + dy * (vi.y - vj.y) + dz * (vi.z - vj.z);
-                const float s = pair_scalar(dr2, dxdv, A.table[tt], A.table[2 * kTypeStride + tt],
-                                            A.table[kTypeStride + tt], idi, (uint32_t)__float_as_int(vj.w),
-                                            B.invrootdt, K, nullptr);
-                const double F[3] = {(double)(s * dx), (double)(s * dy), (double)(s * dz)};
-                const double d[3] = {(double)dx, (double)dy, (double)dz};
-                const double zj = (double)cz * B.wd[2] + (double)pj.z;
-                slice_add(tab, A.nslice, Lz, ti * A.ntypes + tj, A.nidx, zi, zj, F, d, 0.5);
+    const int s0b = A.cstart[B.koff], s1b = A.cstart[B.koff + B.ngroups * kGroupKeys];
+    const int nxy = B.n[0] * B.n[1];
+    int first = s0b + blockIdx.x * per;
+    const int last = min(s1b, first + per);
+    double* mine = lt + (t % copies) * stride;
+    while (first < last) {
+        int c0[3];
+        key_cell(A.key[first] - B.koff, B, c0);
+        const int layer = min(last, A.cstart[B.koff + nxy * (c0[2] + 1)]);
+        // the first slice of the window; one below the layer's, for beads on a slice border
+        const int s0 = win >= A.nslice ? 0 : (int)floor(c0[2] * B.wd[2] * inv) - 1;
+        if (WIN) {
+            for (int q = t; q < copies * stride; q += 256) lt[q] = 0.0;
+            __syncthreads();
+        }
+        for (int i0 = first; i0 < layer; i0 += 256) {
+            const int i = min(i0 + t, layer - 1);
+            const bool valid = i0 + t < layer;
+            const float4 pi = A.pos[i], vi = A.vp[i];
+            const int wi = __float_as_int(pi.w), ti = bead_type(wi);
+            const uint32_t idi = (uint32_t)__float_as_int(vi.w);
+            int c[3];
+            key_cell(A.key[i] - B.koff, B, c);
+            const double zi = (double)c[2] * B.wd[2] + (double)pi.z;
+            const int nci = (-c[0] & 3) << kCellXShift;
+            int n = 0;
+            // separation from a listed partner j in row code r = dy + 1 + 4 (dz + 1) with x image
+            // im (1: one box length below, 2: above)
+            auto shift_x = [&](int im) { return (((im == 1 ? -B.n[0] : (im == 2 ? B.n[0] : 0)) & 3) << kCellXShift); };
+            auto separation = [&](const float4& pj, int im, int dy, int dz, float d[3]) {
+                const int dc = __builtin_amdgcn_sbfe(__float_as_int(pj.w) + nci + shift_x(im), kCellXShift, 2);
+                d[0] = fmaf(-(float)dc, B.w[0], pi.x) - pj.x;
+                d[1] = (pi.y - (float)dy * B.w[1]) - pj.y;
+                d[2] = (pi.z - (float)dz * B.w[2]) - pj.z;
+                return d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
+            };
+            auto evaluate = [&]() {
+                for (int h = 0; h < n; ++h) {
+                    const int j = list[h][t], code = row[h][t];
+                    const int im = code & 3, dy = ((code >> 2) & 3) - 1, dz = code >> 4;
+                    const float4 pj = A.pos[j], vj = A.vp[j];
+                    float d[3];
+                    const float dr2 = separation(pj, im, dy, dz, d);
+                    const int tj = bead_type(__float_as_int(pj.w));
+                    const int tt = ti * kMaxTypes + tj;
+                    const float dxdv = d[0] * (vi.x - vj.x) + d[1] * (vi.y - vj.y) + d[2] * (vi.z - vj.z);
+                    const float s = pair_scalar(dr2, dxdv, A.table[tt], A.table[2 * kTypeStride + tt],
+                                                A.table[kTypeStride + tt], idi, (uint32_t)__float_as_int(vj.w),
+                                                B.invrootdt, K, nullptr);
+                    int cz = c[2] + dz;
+                    cz -= cz >= B.n[2] ? B.n[2] : 0;
+                    const double zj = (double)cz * B.wd[2] + (double)pj.z;
+                    const double sx = (double)s * d[0], sy = (double)s * d[1], sz = (double)s * d[2];
+                    const double f[6] = {sx * d[0], sx * d[1], sx * d[2], sy * d[1], sy * d[2], sz * d[2]};
+                    const int lo = min(ti, tj), hi = max(ti, tj);
+                    slice_split(A.nslice, Lz, zi, zj, (double)d[2], [&](int sl, double share) {
+                        if constexpr (WIN) {
+                            int w = sl - s0;
+                            w -= w >= A.nslice ? A.nslice : 0;
+                            w += w < 0 ? A.nslice : 0;
+                            w = min(w, win - 1);   // (holds: keeps a bad state's sums in the table)
+                            double* q = mine + (w * ntri + hi * (hi + 1) / 2 + lo) * 6;
+#pragma unroll
+                            for (int m = 0; m < 6; ++m) atomicAdd(q + m, f[m] * share);
+                        } else {
+                            double* q = out + ((size_t)sl * A.nidx + lo * A.ntypes + hi) * 9;
+#pragma unroll
+                            for (int m = 0; m < 6; ++m) atomicAdd(q + kTri[m], f[m] * share);
+                        }
+                    });
+                }
+                n = 0;
+            };
+            auto scan = [&](int j0, int j1, int im, int dy, int dz) {
+                for (int j = j0; j < j1; ++j) {
+                    float d[3];
+                    const float dr2 = separation(A.pos[j], im, dy, dz, d);
+                    if (dr2 < 1.0f && dr2 > 1e-18f) {
+                        if (n == kSliceList) evaluate();
+                        list[n][t] = j;
+                        row[n++][t] = (uint8_t)(im | ((dy + 1) << 2) | (dz << 4));
+                    }
+                }
+            };
+            if (valid) {
+                // the five rows: own (beads after i, and the next cell), (1, 0), (-1 .. 1, 1)
+                for (int r = 0; r < 5; ++r) {
+                    const int dz = r >= 2, dy = r < 2 ? r : r - 3;
+                    int cy = c[1] + dy, cz = c[2] + dz;
+                    cy += (cy < 0) ? B.n[1] : ((cy >= B.n[1]) ? -B.n[1] : 0);
+                    cz -= cz >= B.n[2] ? B.n[2] : 0;
+                    const int k = B.koff + B.n[0] * (cy + B.n[1] * cz);
+                    const int x0 = r == 0 ? c[0] : max(c[0] - 1, 0), x1 = min(c[0] + 1, B.n[0] - 1);
+                    scan(r == 0 ? i + 1 : A.cstart[k + x0], A.cstart[k + x1 + 1], 0, dy, dz);
+                    if (r > 0 && c[0] == 0) scan(A.cstart[k + B.n[0] - 1], A.cstart[k + B.n[0]], 1, dy, dz);
+                    if (c[0] == B.n[0] - 1) scan(A.cstart[k], A.cstart[k + 1], 2, dy, dz);
+                }
+                evaluate();
             }
         }
-    }
-    if (SHARED) {
-        __syncthreads();
-        for (int q = threadIdx.x; q < ntab; q += blockDim.x)
-            if (lt[q] != 0.0) atomicAdd(out + q, lt[q]);
+        if (WIN) {
+            __syncthreads();
+            for (int q = t; q < tab; q += 256) {
+                double v = 0.0;
+                for (int r = 0; r < copies; ++r) v += lt[r * stride + q];
+                if (v != 0.0) {
+                    int sl = s0 + q / (ntri * 6);
+                    sl += sl < 0 ? A.nslice : 0;
+                    sl -= sl >= A.nslice ? A.nslice : 0;
+                    int u = q / 6 % ntri, hi = 0;
+                    while ((hi + 1) * (hi + 2) / 2 <= u) ++hi;
+                    const int lo = u - hi * (hi + 1) / 2;
+                    atomicAdd(out + ((size_t)sl * A.nidx + lo * A.ntypes + hi) * 9 + kTri[q % 6], v);
+                }
+            }
+            __syncthreads();
+        }
+        first = layer;
     }
 }
 
-// bonds of the box: head - tail (unwrapped), force on the head, FP64
-__global__ __launch_bounds__(256) void k_slice_bonds(SliceArgs A, double* __restrict__ out)
+// the pair table's other halves: types (tj, ti) beside (ti, tj), half of the sum each, and the
+// components below the diagonal
+__global__ __launch_bounds__(256) void k_slice_mirror(SliceArgs A, double* __restrict__ out)
 {
-    const int q = A.b0 + blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= A.b1) return;
-    const BoxDev& B = A.B;
-    const int2 hb = A.bond_bead[q];
-    const int sh = A.slot_of[hb.x], st = A.slot_of[hb.y];
-    double uh[3], ut[3];
-    for (int e = 0; e < 2; ++e) {
-        const int slot = e ? st : sh;
-        int c[3];
-        key_cell(A.key[slot] - B.koff, B, c);
-        const float4 p = A.pos[slot];
-        const int4 a = A.img[e ? hb.y : hb.x];
-        double* u = e ? ut : uh;
-        u[0] = (double)(c[0] + a.x * B.n[0]) * B.wd[0] + (double)p.x;
-        u[1] = (double)(c[1] + a.y * B.n[1]) * B.wd[1] + (double)p.y;
-        u[2] = (double)(c[2] + a.z * B.n[2]) * B.wd[2] + (double)p.z;
+    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= (int64_t)A.nslice * A.nidx) return;
+    const int lo = (int)(q % A.nidx) / A.ntypes, hi = (int)(q % A.nidx) % A.ntypes;
+    if (lo > hi) return;
+    double* a = out + q * 9;
+    double* b = out + (q - lo * A.ntypes - hi + hi * A.ntypes + lo) * 9;
+    const double share = lo == hi ? 1.0 : 0.5;
+    double v[6];
+    for (int m = 0; m < 6; ++m) v[m] = a[kTri[m]] * share;
+    for (int m = 0; m < 9; ++m) a[m] = v[kSym[m]];
+    if (lo != hi)
+        for (int m = 0; m < 9; ++m) b[m] = v[kSym[m]];
+}
+
+// Tables of bonds and bond pairs: workgroup (b, w) adds the interactions it takes (every
+// gridDim.x-th 256) to the slices [w win, (w + 1) win) in LDS, NC sums per slice and index, and
+// then to out.  win 0: not even one slice fits LDS, out is added to directly.
+template <int NC>
+struct SliceTable {
+    double* lt;
+    double* out;
+    int nslice, nidx, win, w0;
+    __device__ SliceTable(const SliceArgs& A, double* lds, double* o, int win_)
+        : lt(lds), out(o), nslice(A.nslice), nidx(A.nidx), win(win_), w0((int)blockIdx.y * win_)
+    {
+        for (int q = threadIdx.x; q < win * nidx * NC; q += blockDim.x) lt[q] = 0.0;
+        __syncthreads();
     }
-    const double2 par = A.bond_par[q];
-    const double d[3] = {uh[0] - ut[0], uh[1] - ut[1], uh[2] - ut[2]};
-    const double L = sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
-    const double s = par.x * (par.y - L) / L;
-    const double F[3] = {s * d[0], s * d[1], s * d[2]};
-    const int th = bead_type(__float_as_int(A.pos[sh].w)), tt = bead_type(__float_as_int(A.pos[st].w));
-    slice_add(out, A.nslice, (double)B.n[2] * B.wd[2], th * A.ntypes + tt, A.nidx, wrapped_z(A, sh),
-              wrapped_z(A, st), F, d, 1.0);
+    __device__ static int sum_of(int m) { return NC == 6 ? kSym[m] : m; }
+    __device__ void add(int sl, int idx, const double (&f)[NC], double share)
+    {
+        if (win) {
+            const int w = sl - w0;
+            if (w < 0 || w >= win) return;
+            double* q = lt + ((size_t)w * nidx + idx) * NC;
+#pragma unroll
+            for (int m = 0; m < NC; ++m) atomicAdd(q + m, f[m] * share);
+        } else {
+            double* q = out + ((size_t)sl * nidx + idx) * 9;
+            for (int m = 0; m < 9; ++m) atomicAdd(q + m, f[sum_of(m)] * share);
+        }
+    }
+    __device__ void flush()
+    {
+        __syncthreads();
+        const int ns = min(win, nslice - w0);
+        for (int q = threadIdx.x; q < ns * nidx * 9; q += blockDim.x) {
+            const double v = lt[(q / 9) * NC + sum_of(q % 9)];
+            if (v != 0.0) atomicAdd(out + (size_t)w0 * nidx * 9 + q, v);
+        }
+    }
+};
+
+// bonds of the box: head - tail (unwrapped), force on the head, FP64
+__global__ __launch_bounds__(256) void k_slice_bonds(SliceArgs A, double* __restrict__ out, int win)
+{
+    extern __shared__ double lt[];
+    SliceTable<6> T(A, lt, out, win);
+    const BoxDev& B = A.B;
+    for (int q = A.b0 + blockIdx.x * 256 + threadIdx.x; q < A.b1; q += gridDim.x * 256) {
+        const int2 hb = A.bond_bead[q];
+        const int sh = A.slot_of[hb.x], st = A.slot_of[hb.y];
+        double uh[3], ut[3];
+        for (int e = 0; e < 2; ++e) {
+            const int slot = e ? st : sh;
+            int c[3];
+            key_cell(A.key[slot] - B.koff, B, c);
+            const float4 p = A.pos[slot];
+            const int4 a = A.img[e ? hb.y : hb.x];
+            double* u = e ? ut : uh;
+            u[0] = (double)(c[0] + a.x * B.n[0]) * B.wd[0] + (double)p.x;
+            u[1] = (double)(c[1] + a.y * B.n[1]) * B.wd[1] + (double)p.y;
+            u[2] = (double)(c[2] + a.z * B.n[2]) * B.wd[2] + (double)p.z;
+        }
+        const double2 par = A.bond_par[q];
+        const double d[3] = {uh[0] - ut[0], uh[1] - ut[1], uh[2] - ut[2]};
+        const double L = sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
+        const double s = par.x * (par.y - L) / L;
+        const double F[3] = {s * d[0], s * d[1], s * d[2]};
+        const double f[6] = {F[0] * d[0], F[0] * d[1], F[0] * d[2], F[1] * d[1], F[1] * d[2], F[2] * d[2]};
+        const int th = bead_type(__float_as_int(A.pos[sh].w)), tt = bead_type(__float_as_int(A.pos[st].w));
+        slice_split(A.nslice, (double)B.n[2] * B.wd[2], wrapped_z(A, sh), wrapped_z(A, st), d[2],
+                    [&](int sl, double share) { T.add(sl, th * A.ntypes + tt, f, share); });
+    }
+    T.flush();
 }
 
 __device__ inline void unwrapped(const SliceArgs& A, int bead, int slot, double u[3])
@@ -170,32 +319,38 @@ __device__ inline void unwrapped(const SliceArgs& A, int bead, int slot, double 
 // head -> second head -> first tail, each adding 0.33333333 (F[j+1] - F[j]) (x)
 // (u[j+1] - u[j]) over the slices it spans, keyed by the bead types (second head, first
 // head, first tail) where the reference keys by bond-pair type.
-__global__ __launch_bounds__(256) void k_slice_bondpairs(SliceArgs A, double* __restrict__ out)
+__global__ __launch_bounds__(256) void k_slice_bondpairs(SliceArgs A, double* __restrict__ out, int win)
 {
-    const int q = A.a0 + blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= A.a1) return;
-    const int4 abc = A.ang_bead[q];
-    const int sa = A.slot_of[abc.x], sb = A.slot_of[abc.y], sc = A.slot_of[abc.z];
-    double ua[3], ub[3], uc[3], f[3][3];
-    unwrapped(A, abc.x, sa, ua);
-    unwrapped(A, abc.y, sb, ub);
-    unwrapped(A, abc.z, sc, uc);
-    angle_forces(ua, ub, uc, A.ang_par[q], f, nullptr);   // f[0] on c, f[1] on b, f[2] on a
-    const double* u[4] = {uc, ub, ua, uc};
-    const double* F[4] = {f[0], f[1], f[2], f[0]};
-    const int slot[4] = {sc, sb, sa, sc};
-    const int nt = A.ntypes;
-    const int idx = (bead_type(__float_as_int(A.pos[sa].w)) * nt + bead_type(__float_as_int(A.pos[sb].w))) * nt +
-                    bead_type(__float_as_int(A.pos[sc].w));
-    const double Lz = (double)A.B.n[2] * A.B.wd[2];
-    for (int j = 0; j < 3; ++j) {
-        double dx[3], fj[3];
-        for (int d = 0; d < 3; ++d) {
-            dx[d] = u[j + 1][d] - u[j][d];
-            fj[d] = 0.33333333 * (F[j + 1][d] - F[j][d]);
+    extern __shared__ double lt[];
+    SliceTable<9> T(A, lt, out, win);
+    for (int q = A.a0 + blockIdx.x * 256 + threadIdx.x; q < A.a1; q += gridDim.x * 256) {
+        const int4 abc = A.ang_bead[q];
+        const int sa = A.slot_of[abc.x], sb = A.slot_of[abc.y], sc = A.slot_of[abc.z];
+        double ua[3], ub[3], uc[3], f[3][3];
+        unwrapped(A, abc.x, sa, ua);
+        unwrapped(A, abc.y, sb, ub);
+        unwrapped(A, abc.z, sc, uc);
+        angle_forces(ua, ub, uc, A.ang_par[q], f, nullptr);   // f[0] on c, f[1] on b, f[2] on a
+        const double* u[4] = {uc, ub, ua, uc};
+        const double* F[4] = {f[0], f[1], f[2], f[0]};
+        const int slot[4] = {sc, sb, sa, sc};
+        const int nt = A.ntypes;
+        const int idx = (bead_type(__float_as_int(A.pos[sa].w)) * nt + bead_type(__float_as_int(A.pos[sb].w))) * nt +
+                        bead_type(__float_as_int(A.pos[sc].w));
+        const double Lz = (double)A.B.n[2] * A.B.wd[2];
+        for (int j = 0; j < 3; ++j) {
+            double dx[3], fj[3];
+            for (int d = 0; d < 3; ++d) {
+                dx[d] = u[j + 1][d] - u[j][d];
+                fj[d] = 0.33333333 * (F[j + 1][d] - F[j][d]);
+            }
+            double f9[9];
+            for (int m = 0; m < 9; ++m) f9[m] = fj[m / 3] * dx[m % 3];
+            slice_split(A.nslice, Lz, wrapped_z(A, slot[j + 1]), wrapped_z(A, slot[j]), dx[2],
+                        [&](int sl, double share) { T.add(sl, idx, f9, share); });
         }
-        slice_add(out, A.nslice, Lz, idx, nt * nt * nt, wrapped_z(A, slot[j + 1]), wrapped_z(A, slot[j]), fj, dx, 1.0);
     }
+    T.flush();
 }
 
 // The 13 half-shell neighbours of the reference's cells (CSimBox::MakeCNTCells,
@@ -284,31 +439,56 @@ __global__ __launch_bounds__(256) void k_energy_bonded(SliceArgs A, double* __re
 
 hipError_t launch_energy_output(const SliceArgs& a, double* out3, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_energy_pairs, dim3(kSliceBlocks), dim3(256), 0, s, a, out3);
+    hipLaunchKernelGGL(k_energy_pairs, dim3(kEnergyBlocks), dim3(256), 0, s, a, out3);
     const int nq = (a.b1 - a.b0) + (a.a1 - a.a0);
     if (nq > 0) hipLaunchKernelGGL(k_energy_bonded, dim3((nq + 255) / 256), dim3(256), 0, s, a, out3);
     return hipGetLastError();
 }
 
+// slices of a bonded table that fit LDS (nc sums per index); 0: none, or too many windows
+static int slice_window(const SliceArgs& a, int nc)
+{
+    const int win = (int)std::min<size_t>((size_t)a.nslice, kSliceLdsBytes / (sizeof(double) * nc * a.nidx));
+    return win > 0 && (a.nslice + win - 1) / win <= 64 ? win : 0;
+}
+
 hipError_t launch_slice_bondpairs(const SliceArgs& a, double* tab, hipStream_t s)
 {
-    if (a.a1 > a.a0)
-        hipLaunchKernelGGL(k_slice_bondpairs, dim3((a.a1 - a.a0 + 255) / 256), dim3(256), 0, s, a, tab);
+    if (a.a1 > a.a0) {
+        const int win = slice_window(a, 9);
+        const dim3 grid(std::min((a.a1 - a.a0 + 255) / 256, win ? kSliceBondBlocks : 1 << 20),
+                        win ? (a.nslice + win - 1) / win : 1);
+        hipLaunchKernelGGL(k_slice_bondpairs, grid, dim3(256), sizeof(double) * win * a.nidx * 9, s, a, tab, win);
+    }
     return hipGetLastError();
 }
 
 hipError_t launch_slice_stress(const SliceArgs& a, double* pair_tab, double* bond_tab, hipStream_t s)
 {
-    const size_t tab_bytes = sizeof(double) * (size_t)a.nslice * a.nidx * 9;
     if (pair_tab) {
-        const int g = kSliceBlocks;
-        if (tab_bytes <= kSliceLdsBytes)
-            hipLaunchKernelGGL(k_slice_pairs<true>, dim3(g), dim3(256), tab_bytes, s, a, pair_tab);
+        // the slices that one layer of cells and the next reach, and one more at each end
+        const double Lz = (double)a.B.n[2] * a.B.wd[2];
+        const int win = (int)std::min<double>(a.nslice, std::ceil(2.0 * a.B.wd[2] * a.nslice / Lz) + 3.0);
+        const size_t tab = (size_t)(a.ntypes * (a.ntypes + 1) / 2) * 6 * win + 1;
+        int copies = 1;
+        while (copies < 16 && 2 * copies * tab * sizeof(double) <= kSliceCopyBytes) copies *= 2;
+        const int nb = std::max(1, a.nbeads);
+        // whole 256s of slots per workgroup, about kSliceBlocks workgroups
+        const int per = (nb + kSliceBlocks * 256 - 1) / (kSliceBlocks * 256) * 256;
+        if (tab * sizeof(double) <= kSliceLdsBytes)
+            hipLaunchKernelGGL(k_slice_pairs<true>, dim3((nb + per - 1) / per), dim3(256), copies * tab * sizeof(double),
+                               s, a, pair_tab, per, win, copies);
         else
-            hipLaunchKernelGGL(k_slice_pairs<false>, dim3(g), dim3(256), 0, s, a, pair_tab);
+            hipLaunchKernelGGL(k_slice_pairs<false>, dim3((nb + per - 1) / per), dim3(256), 0, s, a, pair_tab, per, 0, 1);
+        hipLaunchKernelGGL(k_slice_mirror, dim3((unsigned)(((size_t)a.nslice * a.nidx + 255) / 256)), dim3(256), 0, s, a,
+                           pair_tab);
     }
-    if (bond_tab && a.b1 > a.b0)
-        hipLaunchKernelGGL(k_slice_bonds, dim3((a.b1 - a.b0 + 255) / 256), dim3(256), 0, s, a, bond_tab);
+    if (bond_tab && a.b1 > a.b0) {
+        const int win = slice_window(a, 6);
+        const dim3 grid(std::min((a.b1 - a.b0 + 255) / 256, win ? kSliceBondBlocks : 1 << 20),
+                        win ? (a.nslice + win - 1) / win : 1);
+        hipLaunchKernelGGL(k_slice_bonds, grid, dim3(256), sizeof(double) * win * a.nidx * 6, s, a, bond_tab, win);
+    }
     return hipGetLastError();
 }
 

@@ -22,15 +22,24 @@ struct SliceArgs {
     const int4* ang_bead;     // (second head, first head, first tail) bead index per bond pair
     const double4* ang_par;   // (k, phi0, cos phi0, sin phi0) per bond pair
     int a0, a1;               // this box's bond pairs
+    int nbeads;               // this box's beads
     int nslice;
     int ntypes;
     int nidx;                 // ntypes * ntypes
 };
 
-// largest table kept in LDS per workgroup; larger tables go straight to global atomics
-constexpr size_t kSliceLdsBytes = 32768;
-// workgroups of the pair pass (grid-stride over the box's beads)
+// largest window of a table kept in LDS per workgroup; larger tables go straight to global
+// atomics
+constexpr size_t kSliceLdsBytes = 49152;
+// the pair window is repeated in LDS up to this size, for fewer lanes on one address
+constexpr size_t kSliceCopyBytes = 32768;
+// workgroups of the pair pass (each adds its window to the table once per z layer it touches;
+// 512, 1024, 2048 of them: 230, 198, 196 us a call on the 48x48x32 bilayer)
+// and of the bonded tables per window
 constexpr int kSliceBlocks = 1024;
+constexpr int kSliceBondBlocks = 48;
+// workgroups of the energy pass (grid-stride over the box's beads)
+constexpr int kEnergyBlocks = 1024;
 
 hipError_t launch_slice_stress(const SliceArgs& a, double* pair_tab, double* bond_tab, hipStream_t s);
 // the reference's energy-output sums: out3[0] pairs, [1] bonds, [2] bond pairs (added to)
