@@ -1,16 +1,36 @@
 // mlp.hip -- surrogate network: BF16 matrix-core forward/backward and FP32 Adam on gfx950.
 //
-// Every matrix product runs on v_mfma_f32_16x16x16_bf16 (BF16 operands, FP32 accumulation)
-// in LDS-staged workgroup tiles (k_gemm_tile).  Operand fragment layout of that instruction
-// for lane l (0..63): A holds A[l%16][4(l/16) .. 4(l/16)+3], B holds
-// B[4(l/16) .. 4(l/16)+3][l%16], and the accumulator holds C[4(l/16)+i][l%16], i = 0..3.
-// Strided operand addressing gives C = A B, A^T B and A B^T from one kernel.
+// Two kernels an iteration.  k_mlp_rows takes 16 rows of the batch through the whole forward
+// and backward chain (a workgroup, activations in registers and one LDS buffer) and leaves the
+// factors of the weight gradients; k_mlp_update makes every gradient entry and applies Adam to
+// it.  Every matrix product runs on v_mfma_f32_16x16x16_bf16 (BF16 operands, FP32
+// accumulation).  Operand fragment layout of that instruction for lane l (0..63): A holds
+// A[l%16][4(l/16) .. 4(l/16)+3], B holds B[4(l/16) .. 4(l/16)+3][l%16], and the accumulator
+// holds C[4(l/16)+i][l%16], i = 0..3.  Everything a product reads from memory is stored as
+// fragments: 64 lanes x 4 values, [16 columns][16 of k][lane][4], one 512-byte load per
+// wavefront.  A result leaves in that layout too, as the fragment of a product over its rows,
+// which is what the weight gradients are.  Weights are kept in BF16 as fragments of W and, for
+// the way back, of W transposed.
+//
+// What bounds it: the latency of a chain of small products (0.7 GFLOP an iteration at 1,638
+// rows and 256 hidden units), so what counts is the number of launches and of passes over
+// memory.  That iteration took 26 launches and 123 us with a kernel for each product, partial
+// sum, column sum and elementwise step; it takes 30 us, 14 of it in k_mlp_rows and 12 in
+// k_mlp_update.  With operands in [column][k] order, of which a wavefront's load touches 16
+// rows, the two took 25 and 20 us.  Many rows are bound by L2: 20,000 of 256 units 43 and
+// 61 us (k_mlp_update reads 330 MB of fragments at 5.4 TB/s), 429 us before.
+//
+// Sums are split over K in the same parts and added in the same order whatever the kernel
+// (split_k), and each part is one chain of matrix instructions, so results do not depend on
+// how the work is laid out over the chip.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <random>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "dpd_mlp.h"
@@ -19,7 +39,6 @@ namespace {
 
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
-
 
 __host__ __device__ inline uint16_t f2bf(float f)
 {
@@ -30,204 +49,380 @@ __host__ __device__ inline uint16_t f2bf(float f)
     return (uint16_t)(u >> 16);
 }
 
-// C[m][n] (ldc) = sum_k A(m,k) B(k,n);  A(m,k) = A[m*am + k*ak], B(k,n) = B[k*bk + n*bn],
-// with am or ak equal to 1 and bk or bn equal to 1 (each operand contiguous along one of its
-// dimensions).  A workgroup of GM x GN wavefronts computes a TM x TN tile, each wavefront
-// FM x FN fragments of 16 x 16.  K advances in chunks of kKC staged in LDS, both operands as
-// [row][k] rows (k contiguous, padded by 4 to spread the banks): the global loads are 8-byte
-// vectors along each operand's contiguous dimension (coalesced across the workgroup), and
-// each fragment operand is one 8-byte LDS read.  blockIdx.z takes the K range
-// [z kper, (z + 1) kper); with several, the tile goes to partial buffer z (C + z cstride) and
-// k_sum_partials adds them in order.  M, N, K, kper: multiples of 16.
-constexpr int kKC = 32;
-constexpr int kLDK = kKC + 4;
-template <int FM, int FN, int GM, int GN>
-__global__ __launch_bounds__(64 * GM * GN) void k_gemm_tile(int M, int N, int K, int kper,
-                                                            const uint16_t* __restrict__ A, int am, int ak,
-                                                            const uint16_t* __restrict__ B, int bk, int bn,
-                                                            float* __restrict__ C, int ldc, int64_t cstride)
+// How a product of M x N outputs over K is summed: `parts` parts of `per` terms (a multiple of
+// 16), each a chain over ascending k, added in order.  (Enough parts that 64 x 64 tiles of the
+// outputs would occupy 256 workgroups, with at least 64 terms each.)
+struct SplitK {
+    int parts, per;
+};
+inline SplitK split_k(int M, int N, int K)
 {
-    constexpr int TM = 16 * FM * GM, TN = 16 * FN * GN, NT = 64 * GM * GN;
-    __shared__ __align__(16) uint16_t As[TM][kLDK];
-    __shared__ __align__(16) uint16_t Bs[TN][kLDK];
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const int wm = w / GN, wn = w % GN;
-    const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
-    const int kz0 = blockIdx.z * kper, kz1 = min(K, kz0 + kper);
-    const int r = lane & 15, q = (lane >> 4) * 4;
-    floatx4 acc[FM][FN];
+    int TM = 64, TN = 64;
+    if (N < 64) TN = 16;
+    else if (M < 64) TM = 16;
+    const int tiles = ((N + TN - 1) / TN) * ((M + TM - 1) / TM);
+    int nz = 1;
+    while (tiles * nz < 256 && K / (2 * nz) >= 64) nz *= 2;
+    const int per = (K / 16 + nz - 1) / nz * 16;
+    return {(K + per - 1) / per, per};
+}
+
+__device__ inline uint2 pack4(const float (&v)[4])
+{
+    return make_uint2((uint32_t)f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16), (uint32_t)f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16));
+}
+__device__ inline bf16x4 frag(const uint16_t* p) { return *reinterpret_cast<const bf16x4*>(p); }
+// place of element (k, n) of a matrix stored as fragments, `steps` 16-row blocks of k
+__host__ __device__ inline int64_t frag_at(int64_t k, int64_t n, int64_t steps)
+{
+    return (((n >> 4) * steps + (k >> 4)) * 64 + ((k & 15) >> 2) * 16 + (n & 15)) * 4 + (k & 3);
+}
+__device__ inline floatx4 mfma(bf16x4 a, bf16x4 b, floatx4 c) { return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0); }
+
+// f(steps, k) over k = k0 .. k1 - 16 in ascending order, four, two or one 16-term steps at a
+// time (the operands of several steps are then loaded together)
+template <class F>
+__device__ inline void in_steps(int k0, int k1, const F& f)
+{
+    int k = k0;
+    for (; k + 64 <= k1; k += 64) f(std::integral_constant<int, 4>{}, k);
+    if (k + 32 <= k1) { f(std::integral_constant<int, 2>{}, k); k += 32; }
+    if (k < k1) f(std::integral_constant<int, 1>{}, k);
+}
+
+// standardisation of inputs and targets
+struct Scaling {
+    double in_mean[16], in_scale[16], out_mean[16], out_scale[16];
+};
+
+// Inputs standardised to BF16 as [row][16] and as fragments over the rows, targets to FP32
+// [row][nout] (y may be null); rows past n and columns past nin are zero.  One thread per
+// padded row and column.
+__global__ __launch_bounds__(256) void k_mlp_input(int n, int Mp, int nin, int nout, const double* __restrict__ x,
+                                                   const double* __restrict__ y, Scaling S, uint16_t* __restrict__ X,
+                                                   uint16_t* __restrict__ XF, float* __restrict__ T)
+{
+    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, i = t >> 4;
+    const int j = t & 15;
+    if (i >= Mp) return;
+    uint16_t v = 0;
+    if (i < n && j < nin) v = f2bf((float)((x[(size_t)i * nin + j] - S.in_mean[j]) / S.in_scale[j]));
+    X[(size_t)i * 16 + j] = v;
+    XF[frag_at(i, j, Mp >> 4)] = v;
+    if (y && j < nout)
+        T[(size_t)i * nout + j] = i < n ? (float)((y[(size_t)i * nout + j] - S.out_mean[j]) / S.out_scale[j]) : 0.0f;
+}
+
+struct RowArgs {
+    int n, Mp, H, nout;
+    SplitK k2, k3;               // sums of the hidden-to-hidden and hidden-to-output products
+    const uint16_t* X;           // [Mp][16]
+    const float* T;              // [Mp][nout]
+    const uint16_t *W1, *W2, *W3;      // fragments of W1, W2, W3
+    const uint16_t *W2t, *W3t;         // and of W2 and W3 transposed
+    const float *b1, *b2, *b3;
+    // training: the gradients' factors as fragments over the rows, and in FP32 for the biases
+    uint16_t *H1F, *H2F, *dZ1F, *dZ2F, *dYF;
+    float *dZ1, *dZ2, *dY;
+    double* loss;
+    // prediction: y[n][nout]
+    double* out;
+    Scaling S;
+};
+
+// Rows [16 b, 16 b + 16) through the network and, with TRAIN, back: WAVES wavefronts, wavefront
+// w computing the 16-column tiles w, w + WAVES, ... (TPW of them at most) of every hidden layer.
+// One LDS buffer holds the layer that the next product reads; the weights come from L2.
+template <int WAVES, int TPW, bool TRAIN>
+__global__ __launch_bounds__(64 * WAVES) void k_mlp_rows(RowArgs A)
+{
+    extern __shared__ __align__(16) uint16_t act[];   // [16][H + 4]
+    __shared__ __align__(16) float part[16][256];     // parts of the output layer's sums
+    __shared__ __align__(16) uint16_t dyb[16][20];
+    __shared__ double lsum[WAVES];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6, r = lane & 15, q = (lane >> 4) * 4;
+    const int H = A.H, nt = H >> 4, ld = H + 4, Mp = A.Mp;
+    const int row0 = blockIdx.x * 16;
+    const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+    float h1[TPW][4], h2[TPW][4];
+    // this lane's place in this workgroup's fragment of a tile of columns
+    auto mine = [&](int tile) { return (((size_t)tile * (Mp >> 4) + blockIdx.x) * 64 + lane) * 4; };
+    auto hidden = [&](int tile, const floatx4& z, const float* bias, float (&h)[4], uint16_t* HF) {
+        const int n = tile * 16 + r;
+        const float b = bias[n];
 #pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-    for (int kc = kz0; kc < kz1; kc += kKC) {
-        // stage A: TM x kKC, zero beyond M and kz1 (kz1 - kc is a multiple of 16)
-        for (int v = t; v < TM * kKC / 4; v += NT) {
-            int mm, kk;
-            if (ak == 1) { mm = v / (kKC / 4); kk = (v % (kKC / 4)) * 4; }
-            else { kk = v / (TM / 4); mm = (v % (TM / 4)) * 4; }
-            uint2 x = make_uint2(0u, 0u);
-            const int gm = m0 + mm, gk = kc + kk;
-            if (gm < M && gk < kz1) x = *reinterpret_cast<const uint2*>(A + (size_t)gm * am + (size_t)gk * ak);
-            if (ak == 1) {
-                *reinterpret_cast<uint2*>(&As[mm][kk]) = x;
-            } else {
-                As[mm][kk] = (uint16_t)(x.x & 0xFFFFu); As[mm + 1][kk] = (uint16_t)(x.x >> 16);
-                As[mm + 2][kk] = (uint16_t)(x.y & 0xFFFFu); As[mm + 3][kk] = (uint16_t)(x.y >> 16);
-            }
+        for (int i = 0; i < 4; ++i) {
+            h[i] = row0 + q + i < A.n ? tanhf(z[i] + b) : 0.0f;
+            act[(q + i) * ld + n] = f2bf(h[i]);
         }
-        // stage B: kKC x TN as [n][k]
-        for (int v = t; v < TN * kKC / 4; v += NT) {
-            int nn, kk;
-            if (bk == 1) { nn = v / (kKC / 4); kk = (v % (kKC / 4)) * 4; }
-            else { kk = v / (TN / 4); nn = (v % (TN / 4)) * 4; }
-            uint2 x = make_uint2(0u, 0u);
-            const int gn = n0 + nn, gk = kc + kk;
-            if (gn < N && gk < kz1) x = *reinterpret_cast<const uint2*>(B + (size_t)gk * bk + (size_t)gn * bn);
-            if (bk == 1) {
-                *reinterpret_cast<uint2*>(&Bs[nn][kk]) = x;
-            } else {
-                Bs[nn][kk] = (uint16_t)(x.x & 0xFFFFu); Bs[nn + 1][kk] = (uint16_t)(x.x >> 16);
-                Bs[nn + 2][kk] = (uint16_t)(x.y & 0xFFFFu); Bs[nn + 3][kk] = (uint16_t)(x.y >> 16);
-            }
+        if (TRAIN) *reinterpret_cast<uint2*>(HF + mine(tile)) = pack4(h);
+    };
+    // act (16 x H) times a weight matrix's fragments: this wavefront's tiles
+    auto product = [&](const uint16_t* WF, floatx4 (&s)[TPW]) {
+        for (int z = 0; z < A.k2.parts; ++z) {
+            floatx4 acc[TPW];
+#pragma unroll
+            for (int j = 0; j < TPW; ++j) acc[j] = zero;
+            in_steps(z * A.k2.per, min(H, (z + 1) * A.k2.per), [&](auto steps, int k) {
+                constexpr int U = decltype(steps)::value;
+                bf16x4 b[U][TPW];
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+#pragma unroll
+                    for (int j = 0; j < TPW; ++j) {
+                        // (a wavefront without this tile repeats the last one)
+                        const int tile = min(w + WAVES * j, nt - 1);
+                        b[u][j] = frag(WF + (((size_t)tile * nt + (k >> 4) + u) * 64 + lane) * 4);
+                    }
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const bf16x4 a = frag(act + r * ld + k + 16 * u + q);
+#pragma unroll
+                    for (int j = 0; j < TPW; ++j) acc[j] = mfma(a, b[u][j], acc[j]);
+                }
+            });
+#pragma unroll
+            for (int j = 0; j < TPW; ++j) s[j] = z ? s[j] + acc[j] : acc[j];
         }
-        __syncthreads();
+    };
+    // hidden layer 1
+    {
+        const bf16x4 a = frag(A.X + (size_t)(row0 + r) * 16 + q);
 #pragma unroll
-        for (int ks = 0; ks < kKC; ks += 16) {
-            bf16x4 a[FM], b[FN];
-#pragma unroll
-            for (int i = 0; i < FM; ++i)
-                a[i] = *reinterpret_cast<const bf16x4*>(&As[(wm * FM + i) * 16 + r][ks + q]);
-#pragma unroll
-            for (int j = 0; j < FN; ++j)
-                b[j] = *reinterpret_cast<const bf16x4*>(&Bs[(wn * FN + j) * 16 + r][ks + q]);
-#pragma unroll
-            for (int i = 0; i < FM; ++i)
-#pragma unroll
-                for (int j = 0; j < FN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[i], b[j], acc[i][j], 0, 0, 0);
+        for (int j = 0; j < TPW; ++j) {
+            const int tile = w + WAVES * j;
+            if (tile < nt) hidden(tile, mfma(a, frag(A.W1 + (tile * 64 + lane) * 4), zero), A.b1, h1[j], A.H1F);
         }
-        __syncthreads();
     }
-    float* Cz = C + (int64_t)blockIdx.z * cstride;
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-            const int gn = n0 + (wn * FN + j) * 16 + r;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int gm = m0 + (wm * FM + i) * 16 + q + e;
-                if (gm < M && gn < N) Cz[(size_t)gm * ldc + gn] = acc[i][j][e];
-            }
-        }
-}
-
-// C[m][n] (row stride ldc) = sum over z = 0 .. nz-1 of P[z][m][n] (M x N each), in that order
-__global__ void k_sum_partials(int M, int N, int nz, const float* __restrict__ P, int64_t pstride,
-                               float* __restrict__ C, int ldc)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= M * N) return;
-    float s = 0.f;
-    for (int z = 0; z < nz; ++z) s += P[(int64_t)z * pstride + i];
-    C[(size_t)(i / N) * ldc + i % N] = s;
-}
-
-// H = tanh(Z + b) for rows < rows_valid (0 beyond), FP32 and BF16 copies
-__global__ void k_bias_tanh(int M, int N, int rows_valid, const float* __restrict__ Z, const float* __restrict__ b,
-                            float* __restrict__ H, uint16_t* __restrict__ Hb)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= M * N) return;
-    const int m = i / N, n = i % N;
-    const float h = m < rows_valid ? tanhf(Z[i] + b[n]) : 0.0f;
-    H[i] = h;
-    Hb[i] = f2bf(h);
-}
-
-// Y = Z + b3 on the valid block; dY = (Y - T) / (n nout) there and 0 elsewhere; loss
-__global__ void k_output(int M, int N, int rows_valid, int nout, const float* __restrict__ Z,
-                         const float* __restrict__ b, const float* __restrict__ T, float* __restrict__ Y,
-                         float* __restrict__ dY, uint16_t* __restrict__ dYb, double* __restrict__ loss)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    double l = 0.0;
-    if (i < M * N) {
-        const int m = i / N, n = i % N;
-        const bool valid = m < rows_valid && n < nout;
-        const float y = Z[i] + b[n];
-        Y[i] = y;
-        const float e = valid ? (y - T[i]) : 0.0f;
-        const float g = e / (float)(rows_valid * nout);
-        dY[i] = g;
-        dYb[i] = f2bf(g);
-        l = valid ? 0.5 * (double)e * (double)e / (double)(rows_valid * nout) : 0.0;
-    }
-    if (loss) {
-        for (int off = 32; off > 0; off >>= 1) l += __shfl_down(l, off, 64);
-        if ((threadIdx.x & 63) == 0 && l != 0.0) atomicAdd(loss, l);
-    }
-}
-
-// dZ = dH * (1 - H^2), FP32 and BF16
-__global__ void k_tanh_grad(int total, const float* __restrict__ dH, const float* __restrict__ H,
-                            float* __restrict__ dZ, uint16_t* __restrict__ dZb)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= total) return;
-    const float g = dH[i] * (1.0f - H[i] * H[i]);
-    dZ[i] = g;
-    dZb[i] = f2bf(g);
-}
-
-// Column sums of dZ (M x N) for the bias gradients, in two ordered passes: workgroup (b, z)
-// takes columns 64b .. 64b+63 and the rows of slab z (kColSlab of them), wavefront w of 16
-// the slab's rows m = w (mod 16) (coalesced rows of 64 columns), and writes the slab's sum
-// P[z][n] (its 16 wavefront sums added in order through LDS); k_sum_partials then adds the
-// slabs in order.
-constexpr int kColSlab = 128;
-__global__ __launch_bounds__(1024) void k_colsum(int M, int N, const float* __restrict__ dZ, float* __restrict__ P)
-{
-    __shared__ float part[16][64];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int n = blockIdx.x * 64 + lane;
-    const int m1 = min(M, (int)(blockIdx.y + 1) * kColSlab);
-    float s = 0.f;
-    if (n < N)
-        for (int m = blockIdx.y * kColSlab + w; m < m1; m += 16) s += dZ[(size_t)m * N + n];
-    part[w][lane] = s;
     __syncthreads();
-    if (w == 0 && n < N) {
-        float t = 0.f;
-        for (int q = 0; q < 16; ++q) t += part[q][lane];
-        P[(size_t)blockIdx.y * N + n] = t;
+    floatx4 s[TPW];
+    product(A.W2, s);
+    __syncthreads();   // act is read no more
+#pragma unroll
+    for (int j = 0; j < TPW; ++j)
+        if (w + WAVES * j < nt) hidden(w + WAVES * j, s[j], A.b2, h2[j], A.H2F);
+    __syncthreads();
+    // output layer: a part of its sum per wavefront
+    for (int z = w; z < A.k3.parts; z += WAVES) {
+        floatx4 acc = zero;
+        in_steps(z * A.k3.per, min(H, (z + 1) * A.k3.per), [&](auto steps, int k) {
+            constexpr int U = decltype(steps)::value;
+            bf16x4 b[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) b[u] = frag(A.W3 + (((k >> 4) + u) * 64 + lane) * 4);
+#pragma unroll
+            for (int u = 0; u < U; ++u) acc = mfma(frag(act + r * ld + k + 16 * u + q), b[u], acc);
+        });
+        *reinterpret_cast<floatx4*>(&part[z][lane * 4]) = acc;
+    }
+    __syncthreads();
+    double l = 0.0;
+    if (t < 256) {
+        float y = part[0][t];
+        for (int z = 1; z < A.k3.parts; ++z) y += part[z][t];
+        const int m = 4 * (t >> 6) + (t & 3), n = (t >> 2) & 15, row = row0 + m;
+        y += A.b3[n];
+        const bool valid = row < A.n && n < A.nout;
+        if (TRAIN) {
+            const float e = valid ? y - A.T[(size_t)row * A.nout + n] : 0.0f;
+            const float g = e / (float)(A.n * A.nout);
+            dyb[m][n] = f2bf(g);
+            A.dYF[(size_t)blockIdx.x * 256 + t] = f2bf(g);
+            A.dY[(size_t)blockIdx.x * 256 + t] = g;
+            l = valid ? 0.5 * (double)e * (double)e / (double)(A.n * A.nout) : 0.0;
+        } else if (valid) {
+#pragma clang fp contract(off)
+            const double scaled = A.S.out_scale[n] * (double)y;
+            A.out[(size_t)row * A.nout + n] = A.S.out_mean[n] + scaled;
+        }
+    }
+    if (!TRAIN) return;
+    for (int off = 32; off > 0; off >>= 1) l += __shfl_down(l, off, 64);
+    if (lane == 0) lsum[w] = l;
+    __syncthreads();
+    if (t == 0) {
+        double v = 0.0;
+        for (int i = 0; i < WAVES; ++i) v += lsum[i];
+        atomicAdd(A.loss, v);
+    }
+    // back through the output layer
+    auto back = [&](int tile, const floatx4& dh, const float (&h)[4], bool keep, uint16_t* dZF, float* dZ) {
+        const int n = tile * 16 + r;
+        float g[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            g[i] = dh[i] * (1.0f - h[i] * h[i]);
+            if (keep) act[(q + i) * ld + n] = f2bf(g[i]);
+        }
+        *reinterpret_cast<uint2*>(dZF + mine(tile)) = pack4(g);
+        *reinterpret_cast<float4*>(dZ + mine(tile)) = make_float4(g[0], g[1], g[2], g[3]);
+    };
+    {
+        const bf16x4 a = frag(&dyb[r][q]);
+#pragma unroll
+        for (int j = 0; j < TPW; ++j) {
+            const int tile = w + WAVES * j;
+            if (tile < nt) back(tile, mfma(a, frag(A.W3t + (tile * 64 + lane) * 4), zero), h2[j], true, A.dZ2F, A.dZ2);
+        }
+    }
+    __syncthreads();
+    product(A.W2t, s);
+#pragma unroll
+    for (int j = 0; j < TPW; ++j)
+        if (w + WAVES * j < nt) back(w + WAVES * j, s[j], h1[j], false, A.dZ1F, A.dZ1);
+}
+
+struct UpdateArgs {
+    int Mp, H;
+    SplitK g1, g2, g3;           // sums of the weight gradients
+    const uint16_t *XF, *H1F, *H2F, *dZ1F, *dZ2F, *dYF;
+    const float *dZ1, *dZ2, *dY;
+    int64_t w1, b1, w2, b2, w3, b3;   // parameter offsets
+    float* grad;                 // with it: store the gradients and leave the parameters
+    float *w, *mo, *ve;
+    const uint8_t* mask;
+    uint16_t *wf, *wt;           // BF16 fragments of the weights and of the weights transposed
+    float lr, c1, c2;
+};
+
+// BF16 copies of weight (k, n) of the matrix at parameter offset o with K x N entries
+__device__ inline void store_weight(uint16_t* wf, uint16_t* wt, int64_t o, int k, int n, int K, int N, float v)
+{
+    const uint16_t b = f2bf(v);
+    wf[o + frag_at(k, n, K >> 4)] = b;
+    wt[o + frag_at(n, k, N >> 4)] = b;
+}
+
+// Adam on parameter i with gradient g; entries with mask 0 (padding) stay zero.  Returns the
+// new value.
+__device__ inline float adam(const UpdateArgs& A, int64_t i, float g)
+{
+    float wi = 0.f;
+    if (A.mask[i]) {
+        const float m = 0.9f * A.mo[i] + 0.1f * g;
+        const float v = 0.999f * A.ve[i] + 0.001f * g * g;
+        A.mo[i] = m;
+        A.ve[i] = v;
+        wi = A.w[i] - A.lr * (m / A.c1) / (sqrtf(v / A.c2) + 1e-8f);
+    }
+    A.w[i] = wi;
+    return wi;
+}
+
+// The gradients of 16 x 16 blocks of a weight matrix, or of 16 biases, and their update:
+// blocks of W2, of W3, of W1, then tiles of b2, b1, b3.  Of the 16 wavefronts P share a block (P
+// the parts of its sum over the rows, as a power of two up to 16) and take parts p, p + P, ...;
+// 16 / P blocks side by side share a workgroup.  The parts are added in order through LDS.
+// Bias gradients are column sums in slabs of kColSlab rows: in each, 16 sums over every 16th
+// row, added in order, and the slabs in order.
+constexpr int kColSlab = 128;
+inline __host__ __device__ int update_share(const SplitK& k)
+{
+    int P = 1;
+    while (P < k.parts && P < 16) P *= 2;
+    return P;
+}
+inline __host__ __device__ int update_groups(const SplitK& k, int blocks) { return (blocks + 16 / update_share(k) - 1) / (16 / update_share(k)); }
+__global__ __launch_bounds__(1024) void k_mlp_update(UpdateArgs A)
+{
+    __shared__ __align__(16) float part[16][256];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6, r = lane & 15;
+    const int H = A.H, nt = H >> 4, nb = A.Mp >> 4;
+    const int n2 = update_groups(A.g2, nt * nt), n3 = update_groups(A.g3, nt), n1 = update_groups(A.g1, nt);
+    int job = blockIdx.x;
+    if (job < n2 + n3 + n1) {
+        const bool is2 = job < n2, is3 = !is2 && job < n2 + n3;
+        const SplitK k = is2 ? A.g2 : (is3 ? A.g3 : A.g1);
+        job -= is2 ? 0 : (is3 ? n2 : n2 + n3);
+        const int P = update_share(k), per = 16 / P, blocks = is2 ? nt * nt : nt;
+        // block x of the matrix: k tile tm, n tile tn
+        auto tm = [&](int x) { return is2 ? x / nt : (is3 ? x : 0); };
+        auto tn = [&](int x) { return is2 ? x % nt : (is3 ? 0 : x); };
+        const int x = min(job * per + w / P, blocks - 1);   // (past the last: it again, not stored)
+        const uint16_t* a = (is2 ? A.H1F : (is3 ? A.H2F : A.XF)) + ((size_t)tm(x) * nb * 64 + lane) * 4;
+        const uint16_t* b = (is2 ? A.dZ2F : (is3 ? A.dYF : A.dZ1F)) + ((size_t)tn(x) * nb * 64 + lane) * 4;
+        float g[4] = {0.f, 0.f, 0.f, 0.f};   // entries t % 256 of blocks t / 256 + 4 v
+        for (int z0 = 0; z0 < k.parts; z0 += P) {
+            const int z = z0 + w % P;
+            if (z < k.parts) {
+                floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+                in_steps(z * k.per, min(A.Mp, (z + 1) * k.per), [&](auto steps, int kk) {
+                    constexpr int U = decltype(steps)::value;
+                    bf16x4 fa[U], fb[U];
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        fa[u] = frag(a + (size_t)((kk >> 4) + u) * 256);
+                        fb[u] = frag(b + (size_t)((kk >> 4) + u) * 256);
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; ++u) acc = mfma(fa[u], fb[u], acc);
+                });
+                *reinterpret_cast<floatx4*>(&part[w][lane * 4]) = acc;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int c = t / 256 + 4 * v;
+                if (c < per)
+                    for (int u = 0; u < min(P, k.parts - z0); ++u) g[v] += part[c * P + u][t % 256];
+            }
+            __syncthreads();
+        }
+        const int e = t % 256, m = 4 * (e >> 6) + (e & 3), n = (e >> 2) & 15;
+        const int64_t o = is2 ? A.w2 : (is3 ? A.w3 : A.w1);
+        const int K = is2 || is3 ? H : 16, N = is3 ? 16 : H;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int c = t / 256 + 4 * v, y = job * per + c;
+            if (c >= per || y >= blocks) continue;
+            const int row = tm(y) * 16 + m, col = tn(y) * 16 + n;
+            const int64_t i = o + (int64_t)row * N + col;
+            if (A.grad) A.grad[i] = g[v];
+            else store_weight(A.wf, A.wt, o, row, col, K, N, adam(A, i, g[v]));
+        }
+        return;
+    }
+    job -= n2 + n3 + n1;
+    const float* d = job < nt ? A.dZ2 : (job < 2 * nt ? A.dZ1 : A.dY);
+    const int64_t i0 = job < nt ? A.b2 + job * 16 : (job < 2 * nt ? A.b1 + (job - nt) * 16 : A.b3);
+    d += ((size_t)(job < 2 * nt ? job % nt : 0) * nb * 64 + lane) * 4;
+    const int slabs = (A.Mp + kColSlab - 1) / kColSlab;
+    float g = 0.f;
+    for (int z0 = 0; z0 < slabs; z0 += 16) {
+        const int z = z0 + w;
+        if (z < slabs) {
+            // lane (q, r): rows 4q .. 4q+3 of every 16, column r
+            float s[4] = {0.f, 0.f, 0.f, 0.f};
+            const int b1 = min(nb, (z + 1) * (kColSlab / 16));
+#pragma unroll 8
+            for (int b = z * (kColSlab / 16); b < b1; ++b) {
+                const float4 v = *reinterpret_cast<const float4*>(d + (size_t)b * 256);
+                s[0] += v.x; s[1] += v.y; s[2] += v.z; s[3] += v.w;
+            }
+            float p = 0.f;
+#pragma unroll
+            for (int u = 0; u < 16; ++u) p += __shfl(s[u & 3], (u >> 2) * 16 + r);
+            if (lane < 16) part[w][lane] = p;
+        }
+        __syncthreads();
+        if (t < 16)
+            for (int u = 0; u < min(16, slabs - z0); ++u) g += part[u][t];
+        __syncthreads();
+    }
+    if (t < 16) {
+        if (A.grad) A.grad[i0 + t] = g;
+        else adam(A, i0 + t, g);
     }
 }
 
-// Adam on the parameter array; entries with mask 0 (padding) stay zero.  Also refreshes the
-// BF16 copy (same layout) the matrix products read.
-__global__ void k_adam(int total, float* __restrict__ w, const float* __restrict__ g, float* __restrict__ mo,
-                       float* __restrict__ ve, const uint8_t* __restrict__ mask, float lr, float c1, float c2,
-                       uint16_t* __restrict__ wb)
+// the weights' BF16 fragments
+__global__ void k_to_bf16(int H, int64_t w1, int64_t b1, int64_t w2, int64_t b2, int64_t w3, int64_t b3,
+                          const float* __restrict__ w, uint16_t* __restrict__ wf, uint16_t* __restrict__ wt)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= total) return;
-    if (mask && !mask[i]) { w[i] = 0.f; wb[i] = 0; return; }
-    const float gi = g[i];
-    const float m = 0.9f * mo[i] + 0.1f * gi;
-    const float v = 0.999f * ve[i] + 0.001f * gi * gi;
-    mo[i] = m;
-    ve[i] = v;
-    const float wi = w[i] - lr * (m / c1) / (sqrtf(v / c2) + 1e-8f);
-    w[i] = wi;
-    wb[i] = f2bf(wi);
-}
-
-__global__ void k_to_bf16(int total, const float* __restrict__ w, uint16_t* __restrict__ wb)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < total) wb[i] = f2bf(w[i]);
+    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (i < b1) store_weight(wf, wt, w1, (int)((i - w1) / H), (int)((i - w1) % H), 16, H, w[i]);
+    else if (i >= w2 && i < b2) store_weight(wf, wt, w2, (int)((i - w2) / H), (int)((i - w2) % H), H, H, w[i]);
+    else if (i >= w3 && i < b3) store_weight(wf, wt, w3, (int)((i - w3) / 16), (int)((i - w3) % 16), H, 16, w[i]);
 }
 
 inline int blocks(int64_t n, int b = 256) { return (int)((n + b - 1) / b); }
@@ -239,26 +434,21 @@ struct dpd_mlp {
     int nin = 0, H = 0, nout = 0, kin = 16, kout = 16;
     int device = 0;
     hipStream_t stream = nullptr;
-    // FP32 parameters (padded): W1[kin][H], b1[H], W2[H][H], b2[H], W3[H][kout], b3[kout]
-    float *W1 = nullptr, *b1 = nullptr, *W2 = nullptr, *b2 = nullptr, *W3 = nullptr, *b3 = nullptr;
-    uint16_t* Wb = nullptr;   // BF16 copy of the parameter array (same layout)
-    uint16_t *W1b = nullptr, *W2b = nullptr, *W3b = nullptr;   // its weight blocks
-    // gradients and Adam moments, same shapes
-    float *gW1 = nullptr, *gb1 = nullptr, *gW2 = nullptr, *gb2 = nullptr, *gW3 = nullptr, *gb3 = nullptr;
-    float* mom = nullptr;     // all parameters: first moment
-    float* var = nullptr;     // second moment
+    // FP32 parameters (padded): W1[kin][H], b1[H], W2[H][H], b2[H], W3[H][kout], b3[kout]; their
+    // gradients and Adam moments, and the weights' BF16 fragments, plain and transposed
+    float *w = nullptr, *grad = nullptr, *mom = nullptr, *var = nullptr;
+    uint16_t *wf = nullptr, *wt = nullptr;
     uint8_t* mask = nullptr;  // 1 where a parameter is real (not padding)
     int64_t nparam_pad = 0;
     int64_t adam_t = 0;
-    // activations for up to cap rows
-    int cap = 0;
-    uint16_t *Xb = nullptr, *H1b = nullptr, *H2b = nullptr, *dYb = nullptr, *dZ2b = nullptr, *dZ1b = nullptr;
-    float *Z1 = nullptr, *H1 = nullptr, *Z2 = nullptr, *H2 = nullptr, *Z3 = nullptr, *Y = nullptr, *T = nullptr;
-    float *dY = nullptr, *dH2 = nullptr, *dZ2 = nullptr, *dH1 = nullptr, *dZ1 = nullptr;
+    // the batch, for up to cap rows: inputs [row][16] and as fragments, targets, and what the
+    // gradients are made of; its raw rows
+    int cap = 0, train_cap = 0;
+    uint16_t *X = nullptr, *XF = nullptr, *H1F = nullptr, *H2F = nullptr, *dZ1F = nullptr, *dZ2F = nullptr, *dYF = nullptr;
+    float *T = nullptr, *dZ1 = nullptr, *dZ2 = nullptr, *dY = nullptr;
+    double *raw = nullptr, *out = nullptr;
     double* loss = nullptr;
     int loss_cap = 0;
-    float* part = nullptr;    // split-K partial tiles
-    int64_t part_cap = 0;
     std::vector<double> in_mean, in_scale, out_mean, out_scale;
     std::string err;
 };
@@ -305,165 +495,135 @@ Layout layout(const dpd_mlp* m)
     return L;
 }
 
-int ensure_rows(dpd_mlp* m, int rows)
+// room for `rows` padded rows; what only training needs when it is first asked for
+int ensure_rows(dpd_mlp* m, int rows, bool train)
 {
-    if (rows <= m->cap) return 0;
-    const int c = rows;
-    const size_t h = (size_t)c * m->H, o = (size_t)c * m->kout, x = (size_t)c * m->kin;
     int rc = 0;
-    if ((rc = malloc_dev(m, &m->Xb, x)) || (rc = malloc_dev(m, &m->H1b, h)) || (rc = malloc_dev(m, &m->H2b, h)) ||
-        (rc = malloc_dev(m, &m->dYb, o)) || (rc = malloc_dev(m, &m->dZ2b, h)) || (rc = malloc_dev(m, &m->dZ1b, h)) ||
-        (rc = malloc_dev(m, &m->Z1, h)) || (rc = malloc_dev(m, &m->H1, h)) || (rc = malloc_dev(m, &m->Z2, h)) ||
-        (rc = malloc_dev(m, &m->H2, h)) || (rc = malloc_dev(m, &m->Z3, o)) || (rc = malloc_dev(m, &m->Y, o)) ||
-        (rc = malloc_dev(m, &m->T, o)) || (rc = malloc_dev(m, &m->dY, o)) || (rc = malloc_dev(m, &m->dH2, h)) ||
-        (rc = malloc_dev(m, &m->dZ2, h)) || (rc = malloc_dev(m, &m->dH1, h)) || (rc = malloc_dev(m, &m->dZ1, h)))
-        return rc;
-    m->cap = c;
-    return 0;
-}
-
-// the partial-sum buffer (split-K tiles, column-sum slabs), grown to `need` floats
-int ensure_part(dpd_mlp* m, int64_t need)
-{
-    if (need <= m->part_cap) return 0;
-    int rc;
-    if ((rc = malloc_dev(m, &m->part, need))) return rc;
-    m->part_cap = need;
-    return 0;
-}
-
-// db[n] = sum over the M rows of dZ[m][n] (N columns), in slabs of kColSlab rows
-int colsum(dpd_mlp* m, int M, int N, const float* dZ, float* db)
-{
-    const int nslab = (M + kColSlab - 1) / kColSlab;
-    int rc;
-    if ((rc = ensure_part(m, (int64_t)nslab * N))) return rc;
-    hipLaunchKernelGGL(k_colsum, dim3(blocks(N, 64), nslab), dim3(1024), 0, m->stream, M, N, dZ, m->part);
-    hipLaunchKernelGGL(k_sum_partials, dim3(blocks(N)), dim3(256), 0, m->stream, 1, N, nslab, m->part, (int64_t)N,
-                       db, N);
-    return 0;
-}
-
-// tile shapes: 64 x 64 (four wavefronts of 2 x 2 fragments), 64 x 16 for N = 16 outputs,
-// 16 x 64 for M = 16 (a fragment per wavefront); K split over workgroups (at least 64 each)
-// when the tiles alone would leave CUs idle
-int gemm(dpd_mlp* m, int M, int N, int K, const uint16_t* A, int am, int ak, const uint16_t* B, int bk, int bn,
-         float* C, int ldc)
-{
-    if ((am != 1 && ak != 1) || (bk != 1 && bn != 1) || M % 16 || N % 16 || K % 16)
-        return mfail(m, "gemm: operands must be contiguous along one dimension, sizes multiples of 16");
-    int TM = 64, TN = 64;
-    if (N < 64) TN = 16;
-    else if (M < 64) TM = 16;
-    const int gx = (N + TN - 1) / TN, gy = (M + TM - 1) / TM;
-    int nz = 1;
-    while (gx * gy * nz < 256 && K / (2 * nz) >= 2 * kKC) nz *= 2;
-    const int kper = (K / 16 + nz - 1) / nz * 16;
-    nz = (K + kper - 1) / kper;
-    float* out = C;
-    int ldo = ldc;
-    int64_t cstride = 0;
-    if (nz > 1) {
-        int rc;
-        if ((rc = ensure_part(m, (int64_t)nz * M * N))) return rc;
-        out = m->part;
-        ldo = N;
-        cstride = (int64_t)M * N;
+    if (rows > m->cap) {
+        m->cap = 0;
+        const size_t c = rows;
+        if ((rc = malloc_dev(m, &m->X, c * 16)) || (rc = malloc_dev(m, &m->XF, c * 16)) || (rc = malloc_dev(m, &m->T, c * 16)) ||
+            (rc = malloc_dev(m, &m->raw, c * (m->nin + m->nout))) || (rc = malloc_dev(m, &m->out, c * m->nout)))
+            return rc;
+        m->cap = rows;
     }
-    const dim3 grid(gx, gy, nz);
-    if (TN == 16)
-        hipLaunchKernelGGL((k_gemm_tile<1, 1, 4, 1>), grid, dim3(256), 0, m->stream, M, N, K, kper, A, am, ak, B, bk,
-                           bn, out, ldo, cstride);
-    else if (TM == 16)
-        hipLaunchKernelGGL((k_gemm_tile<1, 1, 1, 4>), grid, dim3(256), 0, m->stream, M, N, K, kper, A, am, ak, B, bk,
-                           bn, out, ldo, cstride);
-    else
-        hipLaunchKernelGGL((k_gemm_tile<2, 2, 2, 2>), grid, dim3(256), 0, m->stream, M, N, K, kper, A, am, ak, B, bk,
-                           bn, out, ldo, cstride);
-    if (nz > 1)
-        hipLaunchKernelGGL(k_sum_partials, dim3(blocks((int64_t)M * N)), dim3(256), 0, m->stream, M, N, nz, m->part,
-                           cstride, C, ldc);
+    if (train && rows > m->train_cap) {
+        m->train_cap = 0;
+        const size_t h = (size_t)rows * m->H, o = (size_t)rows * 16;
+        if ((rc = malloc_dev(m, &m->H1F, h)) || (rc = malloc_dev(m, &m->H2F, h)) || (rc = malloc_dev(m, &m->dZ1F, h)) ||
+            (rc = malloc_dev(m, &m->dZ2F, h)) || (rc = malloc_dev(m, &m->dYF, o)) || (rc = malloc_dev(m, &m->dZ1, h)) ||
+            (rc = malloc_dev(m, &m->dZ2, h)) || (rc = malloc_dev(m, &m->dY, o)))
+            return rc;
+        m->train_cap = rows;
+    }
     return 0;
 }
 
-// standardised inputs (bf16, padded to kin) and targets (fp32, padded to kout)
+Scaling scaling(const dpd_mlp* m)
+{
+    Scaling S{};
+    std::copy(m->in_mean.begin(), m->in_mean.end(), S.in_mean);
+    std::copy(m->in_scale.begin(), m->in_scale.end(), S.in_scale);
+    std::copy(m->out_mean.begin(), m->out_mean.end(), S.out_mean);
+    std::copy(m->out_scale.begin(), m->out_scale.end(), S.out_scale);
+    return S;
+}
+
+// the batch's rows (y may be null) to the device, standardised there
 int upload_batch(dpd_mlp* m, int64_t n, const double* x, const double* y, int Mp)
 {
-    std::vector<uint16_t> xb((size_t)Mp * m->kin, 0);
-    for (int64_t i = 0; i < n; ++i)
-        for (int j = 0; j < m->nin; ++j)
-            xb[(size_t)i * m->kin + j] = f2bf((float)((x[i * m->nin + j] - m->in_mean[j]) / m->in_scale[j]));
-    MCHK(hipMemcpyAsync(m->Xb, xb.data(), sizeof(uint16_t) * xb.size(), hipMemcpyHostToDevice, m->stream));
-    if (y) {
-        std::vector<float> t((size_t)Mp * m->kout, 0.f);
-        for (int64_t i = 0; i < n; ++i)
-            for (int j = 0; j < m->nout; ++j)
-                t[(size_t)i * m->kout + j] = (float)((y[i * m->nout + j] - m->out_mean[j]) / m->out_scale[j]);
-        MCHK(hipMemcpyAsync(m->T, t.data(), sizeof(float) * t.size(), hipMemcpyHostToDevice, m->stream));
-    }
+    double* ry = m->raw + (size_t)n * m->nin;
+    MCHK(hipMemcpyAsync(m->raw, x, sizeof(double) * n * m->nin, hipMemcpyHostToDevice, m->stream));
+    if (y) MCHK(hipMemcpyAsync(ry, y, sizeof(double) * n * m->nout, hipMemcpyHostToDevice, m->stream));
+    hipLaunchKernelGGL(k_mlp_input, dim3(blocks((int64_t)Mp * 16)), dim3(256), 0, m->stream, (int)n, Mp, m->nin, m->nout,
+                       m->raw, y ? ry : nullptr, scaling(m), m->X, m->XF, m->T);
     return 0;
 }
 
-int forward(dpd_mlp* m, int n, int Mp, double* loss)
+template <int WAVES, int TPW>
+void launch_rows_t(const RowArgs& a, bool train, hipStream_t s)
 {
-    const int H = m->H, ko = m->kout;
-    int rc;
-    if ((rc = gemm(m, Mp, H, m->kin, m->Xb, m->kin, 1, m->W1b, H, 1, m->Z1, H))) return rc;
-    hipLaunchKernelGGL(k_bias_tanh, dim3(blocks((int64_t)Mp * H)), dim3(256), 0, m->stream, Mp, H, n, m->Z1, m->b1,
-                       m->H1, m->H1b);
-    if ((rc = gemm(m, Mp, H, H, m->H1b, H, 1, m->W2b, H, 1, m->Z2, H))) return rc;
-    hipLaunchKernelGGL(k_bias_tanh, dim3(blocks((int64_t)Mp * H)), dim3(256), 0, m->stream, Mp, H, n, m->Z2, m->b2,
-                       m->H2, m->H2b);
-    if ((rc = gemm(m, Mp, ko, H, m->H2b, H, 1, m->W3b, ko, 1, m->Z3, ko))) return rc;
-    hipLaunchKernelGGL(k_output, dim3(blocks((int64_t)Mp * ko)), dim3(256), 0, m->stream, Mp, ko, n, m->nout, m->Z3,
-                       m->b3, m->T, m->Y, m->dY, m->dYb, loss);
-    return 0;
+    const dim3 grid(a.Mp / 16), block(64 * WAVES);
+    const size_t lds = sizeof(uint16_t) * 16 * (a.H + 4);
+    if (train) hipLaunchKernelGGL((k_mlp_rows<WAVES, TPW, true>), grid, block, lds, s, a);
+    else hipLaunchKernelGGL((k_mlp_rows<WAVES, TPW, false>), grid, block, lds, s, a);
 }
 
-int backward(dpd_mlp* m, int Mp)
+// forward (and with `loss` backward) over the uploaded batch
+void launch_rows(dpd_mlp* m, int n, int Mp, double* loss)
 {
-    const int H = m->H, ko = m->kout, ki = m->kin;
-    int rc;
-    // dW3 = H2^T dY, db3 = colsum dY
-    if ((rc = gemm(m, H, ko, Mp, m->H2b, 1, H, m->dYb, ko, 1, m->gW3, ko))) return rc;
-    if ((rc = colsum(m, Mp, ko, m->dY, m->gb3))) return rc;
-    // dH2 = dY W3^T
-    if ((rc = gemm(m, Mp, H, ko, m->dYb, ko, 1, m->W3b, 1, ko, m->dH2, H))) return rc;
-    hipLaunchKernelGGL(k_tanh_grad, dim3(blocks((int64_t)Mp * H)), dim3(256), 0, m->stream, Mp * H, m->dH2, m->H2,
-                       m->dZ2, m->dZ2b);
-    // dW2 = H1^T dZ2, db2
-    if ((rc = gemm(m, H, H, Mp, m->H1b, 1, H, m->dZ2b, H, 1, m->gW2, H))) return rc;
-    if ((rc = colsum(m, Mp, H, m->dZ2, m->gb2))) return rc;
-    // dH1 = dZ2 W2^T
-    if ((rc = gemm(m, Mp, H, H, m->dZ2b, H, 1, m->W2b, 1, H, m->dH1, H))) return rc;
-    hipLaunchKernelGGL(k_tanh_grad, dim3(blocks((int64_t)Mp * H)), dim3(256), 0, m->stream, Mp * H, m->dH1, m->H1,
-                       m->dZ1, m->dZ1b);
-    // dW1 = X^T dZ1, db1
-    if ((rc = gemm(m, ki, H, Mp, m->Xb, 1, ki, m->dZ1b, H, 1, m->gW1, H))) return rc;
-    if ((rc = colsum(m, Mp, H, m->dZ1, m->gb1))) return rc;
-    return 0;
+    const Layout L = layout(m);
+    RowArgs a{};
+    a.n = n; a.Mp = Mp; a.H = m->H; a.nout = m->nout;
+    a.k2 = split_k(Mp, m->H, m->H);
+    a.k3 = split_k(Mp, m->kout, m->H);
+    a.X = m->X; a.T = m->T;
+    a.W1 = m->wf + L.w1; a.W2 = m->wf + L.w2; a.W3 = m->wf + L.w3;
+    a.W2t = m->wt + L.w2; a.W3t = m->wt + L.w3;
+    a.b1 = m->w + L.b1; a.b2 = m->w + L.b2; a.b3 = m->w + L.b3;
+    a.H1F = m->H1F; a.H2F = m->H2F; a.dZ1F = m->dZ1F; a.dZ2F = m->dZ2F; a.dYF = m->dYF;
+    a.dZ1 = m->dZ1; a.dZ2 = m->dZ2; a.dY = m->dY;
+    a.loss = loss;
+    a.out = m->out;
+    a.S = scaling(m);
+    // Eight wavefronts a workgroup where there is one tile of columns for each, or where
+    // workgroups wait for a compute unit anyway; otherwise sixteen, which halve the chain of
+    // each (training, 16 against 8: 1,638 rows of 256 13.8 / 16.1 us, 500 of 512 25.5 / 30.1,
+    // 300 of 1,024 74 / 78; 20,000 of 256 45.6 / 43.3, 6,000 of 512 51.7 / 45.1).
+    const int tiles = m->H / 16;
+    const bool train = loss != nullptr, many = Mp / 16 > 256;
+    if (tiles <= 8) launch_rows_t<8, 1>(a, train, m->stream);
+    else if (tiles <= 16) many ? launch_rows_t<8, 2>(a, train, m->stream) : launch_rows_t<16, 1>(a, train, m->stream);
+    else if (tiles <= 32) many ? launch_rows_t<8, 4>(a, train, m->stream) : launch_rows_t<16, 2>(a, train, m->stream);
+    else many ? launch_rows_t<8, 8>(a, train, m->stream) : launch_rows_t<16, 4>(a, train, m->stream);
+}
+
+// every gradient of the batch: stored (store), or Adam's step with it
+void launch_update(dpd_mlp* m, int Mp, bool store, float lr, float c1, float c2)
+{
+    const Layout L = layout(m);
+    UpdateArgs a{};
+    a.Mp = Mp; a.H = m->H;
+    a.g1 = split_k(m->kin, m->H, Mp);
+    a.g2 = split_k(m->H, m->H, Mp);
+    a.g3 = split_k(m->H, m->kout, Mp);
+    a.XF = m->XF; a.H1F = m->H1F; a.H2F = m->H2F; a.dZ1F = m->dZ1F; a.dZ2F = m->dZ2F; a.dYF = m->dYF;
+    a.dZ1 = m->dZ1; a.dZ2 = m->dZ2; a.dY = m->dY;
+    a.w1 = L.w1; a.b1 = L.b1; a.w2 = L.w2; a.b2 = L.b2; a.w3 = L.w3; a.b3 = L.b3;
+    a.grad = store ? m->grad : nullptr;
+    a.w = m->w; a.mo = m->mom; a.ve = m->var;
+    a.mask = m->mask;
+    a.wf = m->wf; a.wt = m->wt;
+    a.lr = lr; a.c1 = c1; a.c2 = c2;
+    const int nt = m->H / 16;
+    const int groups = update_groups(a.g2, nt * nt) + update_groups(a.g3, nt) + update_groups(a.g1, nt);
+    hipLaunchKernelGGL(k_mlp_update, dim3(groups + 2 * nt + 1), dim3(1024), 0, m->stream, a);
 }
 
 void refresh_bf16(dpd_mlp* m)
 {
     const Layout L = layout(m);
-    hipLaunchKernelGGL(k_to_bf16, dim3(blocks(L.total)), dim3(256), 0, m->stream, (int)L.total, m->W1, m->Wb);
+    hipLaunchKernelGGL(k_to_bf16, dim3(blocks(L.total)), dim3(256), 0, m->stream, m->H, L.w1, L.b1, L.w2, L.b2,
+                       L.w3, L.b3, m->w, m->wf, m->wt);
 }
 
-// copy between the padded device layout and the compact parameter order of the ABI
-void compact_order(const dpd_mlp* m, std::vector<std::pair<int64_t, int64_t>>& map)
+// The compact parameter order of the ABI leaves out the padding: W1's rows past nin and the
+// columns of W3 and b3 past nout; blocks of it in both orders (f(padded offset, compact offset,
+// count)).
+template <class F>
+void compact_blocks(const dpd_mlp* m, const F& f)
 {
     const Layout L = layout(m);
-    map.clear();
-    for (int i = 0; i < m->nin; ++i)
-        for (int j = 0; j < m->H; ++j) map.push_back({L.w1 + (int64_t)i * m->H + j, 0});
-    for (int j = 0; j < m->H; ++j) map.push_back({L.b1 + j, 0});
-    for (int64_t i = 0; i < (int64_t)m->H * m->H; ++i) map.push_back({L.w2 + i, 0});
-    for (int j = 0; j < m->H; ++j) map.push_back({L.b2 + j, 0});
-    for (int i = 0; i < m->H; ++i)
-        for (int j = 0; j < m->nout; ++j) map.push_back({L.w3 + (int64_t)i * m->kout + j, 0});
-    for (int j = 0; j < m->nout; ++j) map.push_back({L.b3 + j, 0});
-    for (size_t q = 0; q < map.size(); ++q) map[q].second = (int64_t)q;
+    const int64_t H = m->H;
+    int64_t c = 0;
+    auto block = [&](int64_t at, int64_t count) {
+        f(at, c, count);
+        c += count;
+    };
+    block(L.w1, m->nin * H);
+    block(L.b1, H + H * H + H);   // b1, W2, b2
+    for (int64_t i = 0; i < H; ++i) block(L.w3 + i * m->kout, m->nout);
+    block(L.b3, m->nout);
 }
 
 }  // namespace
@@ -484,19 +644,11 @@ int dpd_mlp_create(int32_t nin, int32_t hidden, int32_t nout, uint64_t seed, int
     MCHK(hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking));
     const Layout L = layout(m);
     m->nparam_pad = L.total;
-    float* params = nullptr;
     int rc;
-    if ((rc = malloc_dev(m, &params, L.total)) || (rc = malloc_dev(m, &m->mom, L.total)) ||
+    if ((rc = malloc_dev(m, &m->w, L.total)) || (rc = malloc_dev(m, &m->grad, L.total)) || (rc = malloc_dev(m, &m->mom, L.total)) ||
         (rc = malloc_dev(m, &m->var, L.total)) || (rc = malloc_dev(m, &m->mask, L.total)))
         return rc;
-    m->W1 = params + L.w1; m->b1 = params + L.b1; m->W2 = params + L.w2;
-    m->b2 = params + L.b2; m->W3 = params + L.w3; m->b3 = params + L.b3;
-    float* grads = nullptr;
-    if ((rc = malloc_dev(m, &grads, L.total))) return rc;
-    m->gW1 = grads + L.w1; m->gb1 = grads + L.b1; m->gW2 = grads + L.w2;
-    m->gb2 = grads + L.b2; m->gW3 = grads + L.w3; m->gb3 = grads + L.b3;
-    if ((rc = malloc_dev(m, &m->Wb, L.total))) return rc;
-    m->W1b = m->Wb + L.w1; m->W2b = m->Wb + L.w2; m->W3b = m->Wb + L.w3;
+    if ((rc = malloc_dev(m, &m->wf, L.total)) || (rc = malloc_dev(m, &m->wt, L.total))) return rc;
     // Glorot-uniform weights, zero biases, padding masked out
     std::mt19937_64 rng(seed);
     std::vector<float> w(L.total, 0.f);
@@ -516,7 +668,7 @@ int dpd_mlp_create(int32_t nin, int32_t hidden, int32_t nout, uint64_t seed, int
     fill(L.b2, 1, hidden, hidden, 1, 1, false);
     fill(L.w3, hidden, nout, m->kout, hidden, nout, true);
     fill(L.b3, 1, nout, m->kout, 1, 1, false);
-    MCHK(hipMemcpyAsync(params, w.data(), sizeof(float) * L.total, hipMemcpyHostToDevice, m->stream));
+    MCHK(hipMemcpyAsync(m->w, w.data(), sizeof(float) * L.total, hipMemcpyHostToDevice, m->stream));
     MCHK(hipMemcpyAsync(m->mask, mk.data(), L.total, hipMemcpyHostToDevice, m->stream));
     refresh_bf16(m);
     m->in_mean.assign(nin, 0.0); m->in_scale.assign(nin, 1.0);
@@ -529,9 +681,8 @@ void dpd_mlp_destroy(dpd_mlp* m)
 {
     if (!m) return;
     if (m->stream) (void)hipStreamSynchronize(m->stream);
-    void* ptrs[] = {m->W1, m->gW1, m->mom, m->var, m->mask, m->Wb, m->Xb, m->H1b, m->H2b, m->dYb,
-                    m->dZ2b, m->dZ1b, m->Z1, m->H1, m->Z2, m->H2, m->Z3, m->Y, m->T, m->dY, m->dH2, m->dZ2,
-                    m->dH1, m->dZ1, m->loss, m->part};
+    void* ptrs[] = {m->w, m->grad, m->mom, m->var, m->mask, m->wf, m->wt, m->X, m->XF, m->T, m->raw, m->out, m->H1F,
+                    m->H2F, m->dZ1F, m->dZ2F, m->dYF, m->dZ1, m->dZ2, m->dY, m->loss};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     if (m->stream) (void)hipStreamDestroy(m->stream);
@@ -561,11 +712,9 @@ int dpd_mlp_get_params(dpd_mlp* m, float* params)
 {
     if (!m || !params) return 1;
     std::vector<float> w(m->nparam_pad);
-    MCHK(hipMemcpyAsync(w.data(), m->W1, sizeof(float) * w.size(), hipMemcpyDeviceToHost, m->stream));
+    MCHK(hipMemcpyAsync(w.data(), m->w, sizeof(float) * w.size(), hipMemcpyDeviceToHost, m->stream));
     MCHK(hipStreamSynchronize(m->stream));
-    std::vector<std::pair<int64_t, int64_t>> map;
-    compact_order(m, map);
-    for (auto& p : map) params[p.second] = w[p.first];
+    compact_blocks(m, [&](int64_t at, int64_t c, int64_t n) { std::copy_n(w.data() + at, n, params + c); });
     return 0;
 }
 
@@ -573,10 +722,8 @@ int dpd_mlp_set_params(dpd_mlp* m, const float* params)
 {
     if (!m || !params) return 1;
     std::vector<float> w(m->nparam_pad, 0.f);
-    std::vector<std::pair<int64_t, int64_t>> map;
-    compact_order(m, map);
-    for (auto& p : map) w[p.first] = params[p.second];
-    MCHK(hipMemcpyAsync(m->W1, w.data(), sizeof(float) * w.size(), hipMemcpyHostToDevice, m->stream));
+    compact_blocks(m, [&](int64_t at, int64_t c, int64_t n) { std::copy_n(params + c, n, w.data() + at); });
+    MCHK(hipMemcpyAsync(m->w, w.data(), sizeof(float) * w.size(), hipMemcpyHostToDevice, m->stream));
     refresh_bf16(m);
     MCHK(hipStreamSynchronize(m->stream));
     m->adam_t = 0;
@@ -592,25 +739,22 @@ int dpd_mlp_gradients(dpd_mlp* m, int64_t n, const double* x, const double* y, d
     MCHK(hipSetDevice(m->device));
     const int Mp = pad16(n);
     int rc;
-    if ((rc = ensure_rows(m, Mp)) || (rc = upload_batch(m, n, x, y, Mp))) return rc;
+    if ((rc = ensure_rows(m, Mp, true)) || (rc = upload_batch(m, n, x, y, Mp))) return rc;
     if (m->loss_cap < 1) {
         if ((rc = malloc_dev(m, &m->loss, 1))) return rc;
         m->loss_cap = 1;
     }
     MCHK(hipMemsetAsync(m->loss, 0, sizeof(double), m->stream));
-    if ((rc = forward(m, (int)n, Mp, m->loss)) || (rc = backward(m, Mp))) return rc;
+    launch_rows(m, (int)n, Mp, m->loss);
+    launch_update(m, Mp, true, 0.f, 1.f, 1.f);
     MCHK(hipGetLastError());
     double l = 0;
     MCHK(hipMemcpyAsync(&l, m->loss, sizeof(double), hipMemcpyDeviceToHost, m->stream));
     std::vector<float> g(m->nparam_pad);
-    MCHK(hipMemcpyAsync(g.data(), m->gW1, sizeof(float) * g.size(), hipMemcpyDeviceToHost, m->stream));
+    MCHK(hipMemcpyAsync(g.data(), m->grad, sizeof(float) * g.size(), hipMemcpyDeviceToHost, m->stream));
     MCHK(hipStreamSynchronize(m->stream));
     if (loss) *loss = l;
-    if (grads) {
-        std::vector<std::pair<int64_t, int64_t>> map;
-        compact_order(m, map);
-        for (auto& p : map) grads[p.second] = g[p.first];
-    }
+    if (grads) compact_blocks(m, [&](int64_t at, int64_t c, int64_t k) { std::copy_n(g.data() + at, k, grads + c); });
     return 0;
 }
 
@@ -620,20 +764,18 @@ int dpd_mlp_train(dpd_mlp* m, int64_t n, const double* x, const double* y, int32
     MCHK(hipSetDevice(m->device));
     const int Mp = pad16(n);
     int rc;
-    if ((rc = ensure_rows(m, Mp)) || (rc = upload_batch(m, n, x, y, Mp))) return rc;
+    if ((rc = ensure_rows(m, Mp, true)) || (rc = upload_batch(m, n, x, y, Mp))) return rc;
     if (m->loss_cap < iters) {
         if ((rc = malloc_dev(m, &m->loss, iters))) return rc;
         m->loss_cap = iters;
     }
     MCHK(hipMemsetAsync(m->loss, 0, sizeof(double) * std::max(iters, 1), m->stream));
-    const int64_t tot = m->nparam_pad;
     for (int32_t it = 0; it < iters; ++it) {
-        if ((rc = forward(m, (int)n, Mp, m->loss + it)) || (rc = backward(m, Mp))) return rc;
+        launch_rows(m, (int)n, Mp, m->loss + it);
         m->adam_t += 1;
         const float c1 = 1.0f - std::pow(0.9f, (float)m->adam_t);
         const float c2 = 1.0f - std::pow(0.999f, (float)m->adam_t);
-        hipLaunchKernelGGL(k_adam, dim3(blocks(tot)), dim3(256), 0, m->stream, (int)tot, m->W1, m->gW1, m->mom,
-                           m->var, m->mask, (float)lr, c1, c2, m->Wb);
+        launch_update(m, Mp, false, (float)lr, c1, c2);
     }
     MCHK(hipGetLastError());
     if (loss_out && iters > 0)
@@ -648,15 +790,11 @@ int dpd_mlp_predict(dpd_mlp* m, int64_t n, const double* x, double* y)
     MCHK(hipSetDevice(m->device));
     const int Mp = pad16(n);
     int rc;
-    if ((rc = ensure_rows(m, Mp)) || (rc = upload_batch(m, n, x, nullptr, Mp))) return rc;
-    if ((rc = forward(m, (int)n, Mp, nullptr))) return rc;
+    if ((rc = ensure_rows(m, Mp, false)) || (rc = upload_batch(m, n, x, nullptr, Mp))) return rc;
+    launch_rows(m, (int)n, Mp, nullptr);
     MCHK(hipGetLastError());
-    std::vector<float> out((size_t)Mp * m->kout);
-    MCHK(hipMemcpyAsync(out.data(), m->Y, sizeof(float) * out.size(), hipMemcpyDeviceToHost, m->stream));
+    MCHK(hipMemcpyAsync(y, m->out, sizeof(double) * n * m->nout, hipMemcpyDeviceToHost, m->stream));
     MCHK(hipStreamSynchronize(m->stream));
-    for (int64_t i = 0; i < n; ++i)
-        for (int j = 0; j < m->nout; ++j)
-            y[i * m->nout + j] = m->out_mean[j] + m->out_scale[j] * (double)out[(size_t)i * m->kout + j];
     return 0;
 }
 
