@@ -4,17 +4,16 @@
 //
 // One step (the reference's CSimBox::Evolve, src/SimBox.cpp:977-1120) runs as:
 //   k_advance   UpdateMom of the previous step fused with UpdatePos of this one
-//               (src/CNTCell.cpp:2280-2310, :1704-1757); computes each bead's new cell
-//               key and its rank in that cell
-//   cell starts  counting-sort prefix sums, one launch up to 8192 groups of 64 keys
-//               (k_cell_scan_small, k_cell_start_direct), else k_group_scan + k_cell_start
-//   k_place / k_permute   counting-sort placement into the new cell-sorted SoA buffers,
-//               beads of a cell in ascending bead index (deterministic layout)
+//               (src/CNTCell.cpp:2280-2310, :1704-1757); files each bead under its new cell
+//               (without bonded terms the previous pair launch's epilogue does this)
+//   k_sort      the counting sort and the move into the new cell-sorted SoA buffers, beads
+//               of a cell in ascending bead index (deterministic layout); above 8192 groups
+//               of 64 cell keys k_group_scan goes before it
 //   pair kernel DPD pair forces (src/CNTCell.cpp:1144-1555)
 //   k_bonded / k_bonded_sum   bonds and angles (src/Bond.cpp:111-162,
 //               src/BondPair.cpp:138-286), each once, summed into the bonded beads' forces
 // and a last k_finish closes the final step (UpdateMom + FP64 observables).
-// The simulation time lives in device memory (bumped by k_advance), so a captured
+// The simulation time lives in device memory (bumped by k_sort), so a captured
 // sequence of steps replays as a hipGraph without re-capture.
 #include <hip/hip_runtime.h>
 
@@ -273,12 +272,9 @@ __global__ __launch_bounds__(256) void k_bonded_sum(Topo T, const int* __restric
 template <int MODE, bool MULTI>
 __global__ __launch_bounds__(256) void k_advance(int n, Buffers S, float4* __restrict__ frc, Topo T,
                                                  const BoxDev* boxes,
-                                                 BoxDev B0, int* __restrict__ cnt, int* __restrict__ gcnt,
-                                                 int* __restrict__ nkey, int* __restrict__ rank,
-                                                 int* __restrict__ flags, int64_t* __restrict__ step)
+                                                 BoxDev B0, Intake I, int* __restrict__ flags)
 {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (MODE != kRebin && s == 0) *step += 1;   // simulation time of the coming force evaluation
     const bool active = s < n;
     int k = 0;
     if (active) {
@@ -293,7 +289,7 @@ __global__ __launch_bounds__(256) void k_advance(int n, Buffers S, float4* __res
             frc[s] = f;
         }
         if (MODE == kEndBegin) {
-            // UpdateMom: the stored velocity is v + dt/2 F_old; k_permute repeats this sum
+            // UpdateMom: the stored velocity is v + dt/2 F_old; k_sort repeats this sum
             v.x = kick(v.x, f.x, B.hdt);
             v.y = kick(v.y, f.y, B.hdt);
             v.z = kick(v.z, f.z, B.hdt);
@@ -303,7 +299,7 @@ __global__ __launch_bounds__(256) void k_advance(int n, Buffers S, float4* __res
         int c[3];
         key_cell(S.key[s] - B.koff, B, c);
         const float o[3] = {p.x, p.y, p.z};
-        const int img[3] = {0, 0, 0};   // the image change is applied by k_permute
+        const int img[3] = {0, 0, 0};   // the image change is applied by k_sort
         float d[3] = {0.f, 0.f, 0.f};
         if (MODE != kRebin) {
             d[0] = drift(v.x, f.x, B);
@@ -313,22 +309,10 @@ __global__ __launch_bounds__(256) void k_advance(int n, Buffers S, float4* __res
         Moved m;
         advance(o, c, img, d, B, m);
         k = B.koff + cell_key(m.c[0], m.c[1], m.c[2], B);
-        nkey[s] = k;
         if (m.jump) atomicAdd(flags + 1, 1);
         if (m.bad) atomicAdd(flags + 0, 1);
     }
-    // Counting-sort ranks.  Beads arrive cell-sorted, so a wavefront's keys repeat: one
-    // atomic per distinct cell (and per distinct scan group) instead of one per bead, which
-    // would serialise ~192 same-address atomics per group counter.
-    const int lane = threadIdx.x & 63;
-    int r, size, leader;
-    wave_groups(k, active, r, size, leader);
-    int base = 0;
-    if (active && lane == leader) base = atomicAdd(cnt + k, size);
-    base = __shfl(base, leader, 64);
-    if (active) rank[s] = base + r;
-    wave_groups(k >> 6, active, r, size, leader);
-    if (active && lane == leader) atomicAdd(gcnt + (k >> 6), size);
+    file_bead(I, k, s, active);
 }
 
 // Exclusive scan of in[0, m) into out, in[] cleared, by one workgroup of 1024 threads: in
@@ -382,172 +366,195 @@ __device__ inline void scan_block(int* in, int* __restrict__ out, int m, int* ex
 }
 
 // exclusive scan of the scan groups' counts (one workgroup), clears the counts
-// `step` (may be null): the simulation time to advance, when the epilogue of the previous
-// pair launch did the work of k_advance
-__global__ __launch_bounds__(1024) void k_group_scan(int ngroups, int* __restrict__ gcnt, int* __restrict__ gstart,
-                                                     int64_t* __restrict__ step)
+__global__ __launch_bounds__(1024) void k_group_scan(int ngroups, int* __restrict__ gcnt, int* __restrict__ gstart)
 {
     __shared__ int ex[kScanRound];
     __shared__ int wsum[16];
     __shared__ int carry;
-    if (step && threadIdx.x == 0) *step += 1;
     scan_block(gcnt, gstart, ngroups, ex, wsum, &carry);
 }
 
-// Engines of up to kSmallScanKeys cell keys: the cell starts in one launch (scan_block over
-// the cell counts), which replaces k_group_scan + k_cell_start; clears the cell and group
-// counts.
-constexpr int kSmallScanKeys = 16384;
-__global__ __launch_bounds__(1024) void k_cell_scan_small(int nkeys, int ngroups, int n, int* __restrict__ cnt,
-                                                          int* __restrict__ gcnt, int* __restrict__ cstart,
-                                                          int64_t* __restrict__ step)
+// The counting sort and the move in one launch: workgroup g takes the 64 cell keys of scan
+// group g, finds where its beads go (the counts of the groups before it, then a scan of its 64
+// cells), collects them from their bins and moves them there, in every cell by ascending bead
+// index: a function of the state alone (reruns, and a state downloaded and uploaded again, lay
+// the beads out identically).  The move recomputes the advance that filed the bead.
+// The beads before the group are gstart[g] (k_group_scan) or, with it null, the sum of gcnt.
+// Clears cnt; gcnt and nspill are read by other workgroups, so those of the sort before (`clear`)
+// are cleared instead.
+// Groups of more than kSortList beads, or with a spill, go through `order` in global memory.
+// What bounds it: in small boxes the three round trips to memory (counts, bins, beads), 4.8 us
+// where three launches (cell starts, placement by rank, move), each a chain of its own, took 14;
+// in large ones HBM, about 110 bytes a bead: 786,432 beads 19.8 us (4.4 TB/s) against 28,
+// 2,654,208 beads 56 us and 6 of k_group_scan against 82.  The spare places of the bins are
+// traffic too: with 2 c + 10 places 96^3 steps took 355 us, with 2 c + 6 351, with c + 5 348.
+// A workgroup takes one group: four wavefronts move its 192 beads (at three a cell) at once.
+// Workgroups are dealt to the XCDs in eight contiguous ranges, as the pair launch deals beads:
+// 96^3 342 us a step, dealt in turn 352.
+constexpr int kSortList = 1024;
+template <int MODE, bool MULTI>
+__global__ __launch_bounds__(256) void k_sort(int n, int ngroups, int per_xcd, Buffers S, Buffers D,
+                                              const float4* __restrict__ frc, float4* __restrict__ vp,
+                                              const BoxDev* boxes, BoxDev B0, Intake I, const int* __restrict__ gstart,
+                                              int* __restrict__ cstart, int* __restrict__ clear,
+                                              int* __restrict__ slot_of, int write_vp, int64_t* __restrict__ step,
+                                              int2* __restrict__ order)
 {
-    __shared__ int ex[kScanRound];
-    __shared__ int wsum[16];
-    __shared__ int carry;
-    if (step && threadIdx.x == 0) *step += 1;
-    scan_block(cnt, cstart, nkeys, ex, wsum, &carry);
-    for (int g = threadIdx.x; g < ngroups; g += 1024) gcnt[g] = 0;
-    if (threadIdx.x == 0) cstart[nkeys] = n;
-}
-
-// cell starts: one wavefront per scan group scans its 64 cell counts; clears the counts
-__global__ __launch_bounds__(256) void k_cell_start(int ngroups, int n, const int* __restrict__ gstart,
-                                                    int* __restrict__ cnt, int* __restrict__ cstart)
-{
-    const int g = blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
+    __shared__ int first[kGroupKeys + 1];   // of each cell among the group's beads
+    __shared__ int old[kGroupKeys];         // of each cell in the old order
+    __shared__ int slot[kSortList], ids[kSortList];
+    __shared__ int wsum[4], spilled;
+    const int g = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
     if (g >= ngroups) return;
-    const int k = g * 64 + lane;
-    const int c = cnt[k];
-    const int incl = wave_incl_scan(c);
-    cstart[k] = gstart[g] + incl - c;
-    cnt[k] = 0;
-    if (g == ngroups - 1 && lane == 63) cstart[ngroups * 64] = n;
-}
-
-// Engines of up to kDirectGroups scan groups: the cell starts in one launch without a scan of
-// the group counts.  Each workgroup (four groups, a wavefront each) sums the counts of every
-// group before its first itself, from L2 (at most kDirectGroups ints per workgroup, 8 MB
-// in all for 4096 groups), then each wavefront scans its 64 cell counts as k_cell_start does.
-// Clears the cell counts; the group counts stay for the other workgroups and k_place clears
-// them.  `step` (may be null): as for k_group_scan.
-constexpr int kDirectGroups = 8192;
-__global__ __launch_bounds__(256) void k_cell_start_direct(int ngroups, int n, const int* __restrict__ gcnt,
-                                                           int* __restrict__ cnt, int* __restrict__ cstart,
-                                                           int64_t* __restrict__ step)
-{
-    __shared__ int wsum[4];
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const int g0 = blockIdx.x * 4;
-    if (step && blockIdx.x == 0 && t == 0) *step += 1;
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6, k0 = g * kGroupKeys;
+    if (MODE != kRebin && g == 0 && t == 0) *step += 1;   // simulation time of the coming force evaluation
+    if (w == 0) {
+        const int c = I.cnt[k0 + lane];
+        const int a = I.cstart[k0 + lane], b = I.cstart[k0 + lane + 1];
+        old[lane] = a;
+        const bool over = __any(c > bin_room(b - a));
+        if (lane == 0) spilled = over;
+        const int incl = wave_incl_scan(c);
+        first[lane] = incl - c;
+        if (lane == 63) first[kGroupKeys] = incl;
+        if (c) I.cnt[k0 + lane] = 0;
+    } else if (w == 1 && lane == 0) {
+        clear[g] = 0;
+        if (g == 0) clear[ngroups] = 0;
+    }
     int p = 0;
+    if (!gstart) {
+        const int4* g4 = reinterpret_cast<const int4*>(I.gcnt);
 #pragma unroll 4
-    for (int i = t; i < g0; i += 256) p += gcnt[i];
+        for (int i = t; i < g >> 2; i += 256) {
+            const int4 c = g4[i];
+            p += (c.x + c.y) + (c.z + c.w);
+        }
+        if (t < (g & 3)) p += I.gcnt[(g & ~3) + t];
+    }
     p = __builtin_amdgcn_readlane(wave_incl_scan(p), 63);
     if (lane == 0) wsum[w] = p;
     __syncthreads();
-    const int g = g0 + w;
-    if (g >= ngroups) return;
-    int start = wsum[0] + wsum[1] + wsum[2] + wsum[3];
-    for (int j = g0; j < g; ++j) start += gcnt[j];
-    const int k = g * 64 + lane;
-    const int c = cnt[k];
-    const int incl = wave_incl_scan(c);
-    cstart[k] = start + incl - c;
-    cnt[k] = 0;
-    if (g == ngroups - 1 && lane == 63) cstart[ngroups * 64] = n;
-}
-
-// Counting-sort placement, first half: every source slot s writes (bead index, s) to the
-// position its rank gives it inside its new cell.  Ranks come from atomics, so the order
-// inside a cell is arbitrary here; k_permute restores a deterministic one.  gclear (may be
-// null): the group counts k_cell_start_direct left, cleared by threads s < ngroups (the grid
-// covers max(n, ngroups) threads).
-__global__ __launch_bounds__(256) void k_place(int n, const int* __restrict__ bead, const int* __restrict__ nkey,
-                                               const int* __restrict__ rank, const int* __restrict__ cstart,
-                                               int2* __restrict__ tmp, int* __restrict__ gclear, int ngroups)
-{
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (gclear && s < ngroups) gclear[s] = 0;
-    if (s >= n) return;
-    tmp[cstart[nkey[s]] + rank[s]] = make_int2(bead[s], s);
-}
-
-// Counting-sort placement, second half: the bead placed at d goes to the start of its cell
-// plus the number of the cell's beads with a smaller bead index, so the order inside every
-// cell is ascending bead index, a function of the state alone (reruns, and a state
-// downloaded and uploaded again, lay the beads out identically).  One pass over the cell's m
-// entries per bead, from L1.  Then the move itself (recomputing the same advance as
-// k_advance).
-template <int MODE, bool MULTI>
-__global__ __launch_bounds__(256) void k_permute(int n, Buffers S, Buffers D, float4* __restrict__ frc,
-                                                 float4* __restrict__ vp, const BoxDev* boxes, BoxDev B0,
-                                                 const int* __restrict__ nkey, const int2* __restrict__ tmp,
-                                                 const int* __restrict__ cstart, int* __restrict__ slot_of,
-                                                 int write_vp)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int2 t0 = tmp[i];
-    const int s = t0.y;
-    const int k = nkey[s];
-    const int c0 = cstart[k], c1 = cstart[k + 1];
-    int dst = c0;
-    for (int e = c0; e < c1; ++e) dst += tmp[e].x < t0.x;
-    const float4 p = S.pos[s];
-    const BoxDev& B = box_of<MULTI>(boxes, B0, __float_as_int(p.w));
-    const float4 f = (MODE == kRebin) ? S.fold[s] : frc[s];
-    float4 v = S.vel[s];
-    if (MODE == kEndBegin) {
-        // UpdateMom of the step that ends (the same sum as k_advance)
-        v.x = kick(v.x, f.x, B.hdt);
-        v.y = kick(v.y, f.y, B.hdt);
-        v.z = kick(v.z, f.z, B.hdt);
+    const int start = wsum[0] + wsum[1] + wsum[2] + wsum[3] + (gstart ? gstart[g] : 0);
+    const int total = first[kGroupKeys];
+    if (t < kGroupKeys) cstart[k0 + t] = start + first[t];
+    if (g == ngroups - 1 && t == 0) cstart[ngroups * kGroupKeys] = n;
+    // cell of the group's bead j
+    auto cell_of = [&](int j) {
+        int c = 0;
+#pragma unroll
+        for (int h = kGroupKeys / 2; h > 0; h >>= 1) c += first[c + h] <= j ? h : 0;
+        return c;
+    };
+    auto bin = [&](int c) { return I.bins + bin_at(old[c], k0 + c); };
+    struct Bead {
+        float4 p, v, f;
+        int key;
+    };
+    auto load = [&](int s) {
+        return Bead{S.pos[s], S.vel[s], MODE == kRebin ? S.fold[s] : frc[s], S.key[s]};
+    };
+    auto move = [&](const Bead& x, int k, int q, int dst) {
+        const float4 p = x.p, f = x.f;
+        float4 v = x.v;
+        const BoxDev& B = box_of<MULTI>(boxes, B0, __float_as_int(p.w));
+        if (MODE == kEndBegin) {
+            // UpdateMom of the step that ends (the same sum as k_advance)
+            v.x = kick(v.x, f.x, B.hdt);
+            v.y = kick(v.y, f.y, B.hdt);
+            v.z = kick(v.z, f.z, B.hdt);
+        }
+        int c[3];
+        key_cell(x.key - B.koff, B, c);
+        const float o[3] = {p.x, p.y, p.z};
+        const int img[3] = {0, 0, 0};   // m.img is the change of image this step
+        float d[3] = {0.f, 0.f, 0.f};
+        if (MODE != kRebin) {
+            d[0] = drift(v.x, f.x, B);
+            d[1] = drift(v.y, f.y, B);
+            d[2] = drift(v.z, f.z, B);
+        }
+        Moved m;
+        advance(o, c, img, d, B, m);
+        const int wd = (__float_as_int(p.w) & ~kCellXBits) | ((m.c[0] & 3) << kCellXShift);
+        D.pos[dst] = make_float4(m.o[0], m.o[1], m.o[2], __int_as_float(wd));
+        if (MODE == kRebin) {
+            D.vel[dst] = v;
+            D.fold[dst] = f;
+        } else {
+            // the first half of the next UpdateMom: v + dt/2 F, so the force need not be kept
+            D.vel[dst] = make_float4(kick(v.x, f.x, B.hdt), kick(v.y, f.y, B.hdt), kick(v.z, f.z, B.hdt), v.w);
+        }
+        D.bead[dst] = q;
+        // the image counts live by bead index: only a bead that crosses the box changes them,
+        // and only its own thread writes them
+        if (m.img[0] | m.img[1] | m.img[2]) {
+            int4 im = S.img[q];
+            im.x += m.img[0]; im.y += m.img[1]; im.z += m.img[2];
+            S.img[q] = im;
+        }
+        D.key[dst] = k;
+        D.code[dst] = scan_code(m.o, m.c[0], B);
+        if (MODE == kRebin) {
+            vp[dst] = v;
+        } else {
+            // (equal to the new velocity's bits when lambda dt = dt/2: the steps then read that)
+            if (write_vp)
+                vp[dst] = make_float4(kick(v.x, f.x, B.lamdt), kick(v.y, f.y, B.lamdt), kick(v.z, f.z, B.lamdt), v.w);
+        }
+        // the slot of each bead is read for bonded beads only (bond and angle terms); a scattered
+        // 4-byte store per bead costs a partial-line write each, so the others are skipped once
+        // the topology has flagged the bonded ones (an upload re-binning writes every bead)
+        if (MODE == kRebin || (__float_as_int(p.w) & kBondedBit)) slot_of[q] = dst;
+    };
+    if (total <= kSortList && !spilled) {
+        // the first 256 beads are loaded before their indices are exchanged
+        Bead b0;
+        int c0 = 0;
+        if (t < total) {
+            c0 = cell_of(t);
+            const int s = bin(c0)[t - first[c0]];
+            ids[t] = S.bead[s];
+            b0 = load(s);
+        }
+        for (int j = t + 256; j < total; j += 256) {
+            const int c = cell_of(j);
+            slot[j] = bin(c)[j - first[c]];
+            ids[j] = S.bead[slot[j]];
+        }
+        __syncthreads();
+        auto place = [&](int c, int q) {
+            int r = 0;
+            for (int e = first[c]; e < first[c + 1]; ++e) r += ids[e] < q;
+            return start + first[c] + r;
+        };
+        if (t < total) move(b0, k0 + c0, ids[t], place(c0, ids[t]));
+        for (int j = t + 256; j < total; j += 256) {
+            const int c = cell_of(j);
+            move(load(slot[j]), k0 + c, ids[j], place(c, ids[j]));
+        }
+        return;
     }
-    const int q = t0.x;   // bead index of the source slot
-    int c[3];
-    key_cell(S.key[s] - B.koff, B, c);
-    const float o[3] = {p.x, p.y, p.z};
-    const int img[3] = {0, 0, 0};   // m.img is the change of image this step
-    float d[3] = {0.f, 0.f, 0.f};
-    if (MODE != kRebin) {
-        d[0] = drift(v.x, f.x, B);
-        d[1] = drift(v.y, f.y, B);
-        d[2] = drift(v.z, f.z, B);
+    int2* list = order + start;   // (bead index, source slot)
+    for (int j = t; j < total; j += 256) {
+        const int c = cell_of(j), r = j - first[c];
+        if (r >= bin_room(I.cstart[k0 + c + 1] - old[c])) continue;
+        const int s = bin(c)[r];
+        list[j] = make_int2(S.bead[s], s);
     }
-    Moved m;
-    advance(o, c, img, d, B, m);
-    const int w = (__float_as_int(p.w) & ~kCellXBits) | ((m.c[0] & 3) << kCellXShift);
-    D.pos[dst] = make_float4(m.o[0], m.o[1], m.o[2], __int_as_float(w));
-    if (MODE == kRebin) {
-        D.vel[dst] = v;
-        D.fold[dst] = f;
-    } else {
-        // the first half of the next UpdateMom: v + dt/2 F, so the force need not be kept
-        D.vel[dst] = make_float4(kick(v.x, f.x, B.hdt), kick(v.y, f.y, B.hdt), kick(v.z, f.z, B.hdt), v.w);
+    for (int i = t, m = spilled ? min(*I.nspill, I.cap) : 0; i < m; i += 256) {
+        const int4 x = I.spill[i];
+        if ((x.x >> 6) == g) list[first[x.x & 63] + x.y] = make_int2(S.bead[x.z], x.z);
     }
-    D.bead[dst] = q;
-    // the image counts live by bead index: only a bead that crosses the box changes them,
-    // and only its own thread writes them
-    if (m.img[0] | m.img[1] | m.img[2]) {
-        int4 im = S.img[q];
-        im.x += m.img[0]; im.y += m.img[1]; im.z += m.img[2];
-        S.img[q] = im;
+    __threadfence_block();
+    __syncthreads();
+    for (int j = t; j < total; j += 256) {
+        const int c = cell_of(j);
+        const int2 x = list[j];
+        int r = 0;
+        for (int e = first[c]; e < first[c + 1]; ++e) r += list[e].x < x.x;
+        move(load(x.y), k0 + c, x.x, start + first[c] + r);
     }
-    D.key[dst] = k;
-    D.code[dst] = scan_code(m.o, m.c[0], B);
-    if (MODE == kRebin) {
-        vp[dst] = v;
-    } else {
-        // (equal to the new velocity's bits when lambda dt = dt/2: the steps then read that)
-        if (write_vp)
-            vp[dst] = make_float4(kick(v.x, f.x, B.lamdt), kick(v.y, f.y, B.lamdt), kick(v.z, f.z, B.lamdt), v.w);
-    }
-    // the slot of each bead is read for bonded beads only (bond and angle terms); a scattered
-    // 4-byte store per bead costs a partial-line write each, so the others are skipped once
-    // the topology has flagged the bonded ones (an upload re-binning writes every bead)
-    if (MODE == kRebin || (__float_as_int(p.w) & kBondedBit)) slot_of[q] = dst;
 }
 
 // REBIN leaves the uploaded force in fold; the canonical state needs it in frc too
@@ -719,9 +726,15 @@ struct dpd_engine {
     int* key[2] = {};
     uint32_t* code[2] = {};   // n + kCodePad: the hit-list scan reads up to 7 slots past the end
     float4 *frc = nullptr, *vp = nullptr;
-    int *slot_of = nullptr, *nkey = nullptr, *rank = nullptr;
-    int2* place = nullptr;    // counting-sort placement: (bead index, source slot) per new slot
-    int *cnt = nullptr, *gcnt = nullptr, *gstart = nullptr, *cstart = nullptr;
+    int* slot_of = nullptr;
+    // counting sort (Intake); cstart[cur] are the cell starts of buffer cur, counts[cur]
+    // (beads per scan group | spills) belong to the sort out of it and are zero at rest
+    // (all per cell key or group in `cells`, per bead in `filed`)
+    int *cstart[2] = {}, *counts[2] = {}, *cnt = nullptr, *gstart = nullptr, *bins = nullptr;
+    int4 *spill = nullptr, *filed = nullptr;
+    int2* order = nullptr;
+    int* cells = nullptr;
+    size_t cleared = 0;   // ints of `cells` (cnt and counts) that are zero at rest
     int* flags = nullptr;
     int64_t* dstep = nullptr;
     double* acc = nullptr;
@@ -746,7 +759,7 @@ struct dpd_engine {
     std::vector<dpd_obs> obs;
     bool obs_valid = false;
     int64_t jumps = 0;
-    // graphs (steps, observe) -> executable graph; valid while buffers stay put
+    // graphs (steps, observe | current buffer << 1) -> executable graph; valid while buffers stay put
     std::map<std::pair<int64_t, int>, hipGraphExec_t> graphs;
     std::map<std::pair<int64_t, int>, hipGraph_t> graph_src;
     // timing
@@ -784,7 +797,7 @@ int dalloc(dpd_engine* e, T** p, size_t count)
 
 // With lambda = 1/2 and the forces on, the predicted velocity v + lambda dt f and the stored
 // half step v + dt/2 f are the same FP32 expression (lambda dt and dt/2 round to the same
-// float): steps then read the predicted velocities from vel, k_permute does not write vp, and
+// float): steps then read the predicted velocities from vel, k_sort does not write vp, and
 // k_finish keeps the last step's in vp for the calls between steps.
 inline bool vp_is_vel(const dpd_engine* e)
 {
@@ -894,37 +907,43 @@ Topo topo(dpd_engine* e)
 inline int grid(int64_t n, int b) { return (int)((n + b - 1) / b); }
 inline bool multi(dpd_engine* e) { return e->boxes.size() > 1; }
 
+// the intake of the sort out of buffer `cur`
+Intake intake(dpd_engine* e)
+{
+    int* c = e->counts[e->cur];
+    return Intake{e->cstart[e->cur], e->bins, e->cnt, c, e->spill, c + e->ngroups, (int)e->n};
+}
+
+// the sort's counts to zero where steps have not left them so (outside captured sequences)
+int clear_counts(dpd_engine* e)
+{
+    HIPCHK(hipMemsetAsync(e->cells, 0, sizeof(int) * e->cleared, e->stream));
+    return DPD_OK;
+}
+
 // counting sort of buffer `cur` into buffer `cur^1`; MODE decides the move.  `advanced`: the
-// previous pair launch's epilogue already closed the step and computed the new keys and ranks
-// (MODE kEndBegin only), so k_advance is left out and the scan advances the simulation time.
+// previous pair launch's epilogue already closed the step and filed the beads (MODE kEndBegin
+// only), so k_advance is left out.
+// Up to kDirectGroups groups every workgroup of k_sort adds up the counts before its own; with
+// more the sum, quadratic in all, costs more than a launch of one workgroup that scans them
+// (a step of 4,096 groups 122.2 us, with the scan 123.7; of 13,824 355 us, with the scan 342).
+constexpr int kDirectGroups = 8192;
 template <int MODE, bool MULTI>
 void sort_step_t(dpd_engine* e, bool advanced)
 {
     const int n = (int)e->n;
     Buffers S = bufs(e, e->cur), D = bufs(e, e->cur ^ 1);
     const BoxDev B0 = e->boxes[0].B;
+    const Intake I = intake(e);
     if (!advanced)
         hipLaunchKernelGGL((k_advance<MODE, MULTI>), dim3(grid(n, 256)), dim3(256), 0, e->stream, n, S, e->frc,
-                           topo(e), e->dboxes, B0, e->cnt, e->gcnt, e->nkey, e->rank, e->flags, e->dstep);
-    int64_t* bump = advanced ? e->dstep : nullptr;
-    int* gclear = nullptr;
-    if (e->nkeys <= kSmallScanKeys) {
-        hipLaunchKernelGGL(k_cell_scan_small, dim3(1), dim3(1024), 0, e->stream, e->nkeys, e->ngroups, n, e->cnt,
-                           e->gcnt, e->cstart, bump);
-    } else if (e->ngroups <= kDirectGroups) {
-        hipLaunchKernelGGL(k_cell_start_direct, dim3(grid(e->ngroups, 4)), dim3(256), 0, e->stream, e->ngroups, n,
-                           e->gcnt, e->cnt, e->cstart, bump);
-        gclear = e->gcnt;
-    } else {
-        hipLaunchKernelGGL(k_group_scan, dim3(1), dim3(1024), 0, e->stream, e->ngroups, e->gcnt, e->gstart, bump);
-        hipLaunchKernelGGL(k_cell_start, dim3(grid(e->ngroups, 4)), dim3(256), 0, e->stream, e->ngroups, n, e->gstart,
-                           e->cnt, e->cstart);
-    }
-    hipLaunchKernelGGL(k_place, dim3(grid(std::max<int64_t>(n, gclear ? e->ngroups : 0), 256)), dim3(256), 0,
-                       e->stream, n, S.bead, e->nkey, e->rank, e->cstart, e->place, gclear, (int)e->ngroups);
-    hipLaunchKernelGGL((k_permute<MODE, MULTI>), dim3(grid(n, 256)), dim3(256), 0, e->stream, n, S, D, e->frc,
-                       e->vp, e->dboxes, B0, e->nkey, e->place, e->cstart, e->slot_of,
-                       (MODE == kRebin || !vp_is_vel(e)) ? 1 : 0);
+                           topo(e), e->dboxes, B0, I, e->flags);
+    const bool scan = e->ngroups > kDirectGroups;
+    if (scan) hipLaunchKernelGGL(k_group_scan, dim3(1), dim3(1024), 0, e->stream, e->ngroups, I.gcnt, e->gstart);
+    const int per = grid(e->ngroups, 8);
+    hipLaunchKernelGGL((k_sort<MODE, MULTI>), dim3(8 * per), dim3(256), 0, e->stream, n, e->ngroups, per, S, D, e->frc,
+                       e->vp, e->dboxes, B0, I, scan ? e->gstart : nullptr, e->cstart[e->cur ^ 1],
+                       e->counts[e->cur ^ 1], e->slot_of, (MODE == kRebin || !vp_is_vel(e)) ? 1 : 0, e->dstep, e->order);
     e->cur ^= 1;
 }
 
@@ -947,16 +966,16 @@ inline bool epilogue_ok(const dpd_engine* e) { return e->nbonded == 0 && epilogu
 // Pair forces of this step.  With the hit-list kernel the bond and angle terms run in the
 // same launch (k_pair_hitlist_bonded); `bonded` then tells launch_bonded to add only the sums.
 // `epi` (epilogue_ok): the launch also closes the step and starts the next one (pair_epilogue).
-int launch_pair(dpd_engine* e, bool obs, bool* bonded = nullptr, bool epi = false, bool in_seq = false)
+// `spills` false: the launch is repeated on one state, and what overfills the sort's bins is dropped.
+int launch_pair(dpd_engine* e, bool obs, bool* bonded = nullptr, bool epi = false, bool in_seq = false,
+                bool spills = true)
 {
     if (bonded) *bonded = false;
     PairArgs a;
     const Buffers S = bufs(e, e->cur);
     a.vel = S.vel;
-    a.nkey = e->nkey;
-    a.rank = e->rank;
-    a.cnt = e->cnt;
-    a.gcnt = e->gcnt;
+    a.intake = intake(e);
+    if (!spills) a.intake.cap = 0;
     a.flags = e->flags;
     a.n = (int)e->n;
     a.nbox = (int)e->boxes.size();
@@ -964,11 +983,11 @@ int launch_pair(dpd_engine* e, bool obs, bool* bonded = nullptr, bool epi = fals
     a.boxes = e->dboxes;
     a.pos = e->pos[e->cur];
     // inside a sequence of steps with lambda dt = dt/2 the predicted velocities are the
-    // stored half steps (k_permute did not write vp)
+    // stored half steps (k_sort did not write vp)
     a.vp = (in_seq && vp_is_vel(e)) ? e->vel[e->cur] : e->vp;
     a.key = e->key[e->cur];
     a.code = S.code;
-    a.cstart = e->cstart;
+    a.cstart = e->cstart[e->cur];
     a.table = e->table;
     a.step = e->dstep;
     a.frc = e->frc;
@@ -1155,14 +1174,29 @@ int commit_beads(dpd_engine* e, int64_t step0)
             e->nhitblk[tb] = (int)hb.size();
         }
     }
-    if (nbr != e->ngroups) {
+    const bool new_cells = nbr != e->ngroups || !e->cells;
+    if (new_cells) {
         e->ngroups = nbr;
         e->nkeys = nbr * kGroupKeys;
-        if ((rc = dalloc(e, &e->cnt, e->nkeys)) || (rc = dalloc(e, &e->cstart, e->nkeys + 1 + kCstartPad)) ||
-            (rc = dalloc(e, &e->gcnt, e->ngroups)) || (rc = dalloc(e, &e->gstart, e->ngroups)))
-            return rc;
-        HIPCHK(hipMemsetAsync(e->cnt, 0, sizeof(int) * e->nkeys, e->stream));
-        HIPCHK(hipMemsetAsync(e->gcnt, 0, sizeof(int) * e->ngroups, e->stream));
+        // (each part starts at a multiple of four: the counts are read four at a time)
+        const size_t nk = (size_t)e->nkeys, ng = (size_t)(nbr + 4) / 4 * 4, nc = (nk + 1 + kCstartPad + 3) / 4 * 4;
+        if ((rc = dalloc(e, &e->cells, nk + 3 * ng + 2 * nc))) return rc;
+        e->cnt = e->cells;
+        e->counts[0] = e->cells + nk;
+        e->counts[1] = e->counts[0] + ng;
+        e->gstart = e->counts[1] + ng;
+        e->cstart[0] = e->gstart + ng;
+        e->cstart[1] = e->cstart[0] + nc;
+        e->cleared = nk + 2 * ng;
+        if ((rc = clear_counts(e))) return rc;
+    }
+    if (new_cells || n != e->n || !e->filed) {
+        // spill (int4 a bead), order (int2 a bead), bins
+        const size_t nbins = bin_at((int)n, e->nkeys);
+        if ((rc = dalloc(e, &e->filed, (6 * (size_t)n + nbins + 3) / 4))) return rc;
+        e->spill = e->filed;
+        e->order = reinterpret_cast<int2*>(e->filed + n);
+        e->bins = reinterpret_cast<int*>(e->order + n);
     }
     if (n != e->n) {
         for (int b = 0; b < 2; ++b)
@@ -1173,7 +1207,6 @@ int commit_beads(dpd_engine* e, int64_t step0)
         if ((rc = dalloc(e, &e->img, n))) return rc;
         for (int b = 0; b < 2; ++b) HIPCHK(hipMemsetAsync(e->code[b] + n, 0, sizeof(uint32_t) * kCodePad, e->stream));
         if ((rc = dalloc(e, &e->frc, n)) || (rc = dalloc(e, &e->vp, n)) || (rc = dalloc(e, &e->slot_of, n)) ||
-            (rc = dalloc(e, &e->nkey, n)) || (rc = dalloc(e, &e->rank, n)) || (rc = dalloc(e, &e->place, n)) ||
             (rc = dalloc(e, &e->gather, 12 * n)))
             return rc;
         e->n = n;
@@ -1182,7 +1215,7 @@ int commit_beads(dpd_engine* e, int64_t step0)
     std::vector<float4> hp(n), hv(n), hf(n);
     std::vector<int> hb(n);
     std::vector<int4> hi(n);
-    std::vector<int> hk(n);
+    std::vector<int> hk(n), hc(e->nkeys + 1, 0);   // cell keys and, for the bins, their cell starts
     for (size_t b = 0; b < e->boxes.size(); ++b) {
         const BoxHost& h = e->boxes[b];
         const BoxDev& B = h.B;
@@ -1213,8 +1246,10 @@ int commit_beads(dpd_engine* e, int64_t step0)
             hb[g] = (int)g;
             hi[g] = make_int4(im[0], im[1], im[2], 0);
             hk[g] = B.koff + cell_key(c[0], c[1], c[2], B);
+            ++hc[hk[g] + 1];
         }
     }
+    for (int k = 0; k < e->nkeys; ++k) hc[k + 1] += hc[k];
     const int src = e->cur;
     HIPCHK(hipMemcpyAsync(e->pos[src], hp.data(), sizeof(float4) * n, hipMemcpyHostToDevice, e->stream));
     HIPCHK(hipMemcpyAsync(e->vel[src], hv.data(), sizeof(float4) * n, hipMemcpyHostToDevice, e->stream));
@@ -1222,6 +1257,7 @@ int commit_beads(dpd_engine* e, int64_t step0)
     HIPCHK(hipMemcpyAsync(e->bead[src], hb.data(), sizeof(int) * n, hipMemcpyHostToDevice, e->stream));
     HIPCHK(hipMemcpyAsync(e->img, hi.data(), sizeof(int4) * n, hipMemcpyHostToDevice, e->stream));
     HIPCHK(hipMemcpyAsync(e->key[src], hk.data(), sizeof(int) * n, hipMemcpyHostToDevice, e->stream));
+    HIPCHK(hipMemcpyAsync(e->cstart[src], hc.data(), sizeof(int) * hc.size(), hipMemcpyHostToDevice, e->stream));
     launch_zero(e, true);
     if ((rc = sort_step<kRebin>(e))) return rc;
     hipLaunchKernelGGL(k_copy_force, dim3(grid(n, 256)), dim3(256), 0, e->stream, (int)n, e->fold[e->cur], e->frc);
@@ -1436,7 +1472,7 @@ int slice_tables(dpd_engine* e, int32_t box, int32_t nslices, double* tab, size_
     a.vp = e->vp;
     a.img = e->img;
     a.key = e->key[e->cur];
-    a.cstart = e->cstart;
+    a.cstart = e->cstart[e->cur];
     a.table = e->table + (size_t)box * kTableStride;
     a.step = e->dstep;
     a.slot_of = e->slot_of;
@@ -1533,9 +1569,8 @@ void dpd_destroy(dpd_engine* e)
     if (e->stream) (void)hipStreamSynchronize(e->stream);
     drop_graphs(e);
     void* ptrs[] = {e->pos[0], e->pos[1], e->vel[0], e->vel[1], e->fold[0], e->fold[1], e->bead[0], e->bead[1], e->img,
-                    e->key[0], e->key[1], e->code[0], e->code[1], e->frc, e->vp, e->slot_of, e->nkey, e->rank,
-                    e->place, e->cnt, e->gcnt,
-                    e->gstart, e->cstart, e->flags, e->dstep, e->acc, e->table, e->gather, e->bond_ptr,
+                    e->key[0], e->key[1], e->code[0], e->code[1], e->frc, e->vp, e->slot_of,
+                    e->cells, e->filed, e->flags, e->dstep, e->acc, e->table, e->gather, e->bond_ptr,
                     e->ang_ptr, e->bond_csr, e->bond_par, e->ang_csr, e->ang_bead, e->ang_par, e->bond_bead,
                     e->fbond, e->fang, e->bonded, e->dboxes, e->slice, e->madj};
     for (void* q : ptrs)
@@ -1635,7 +1670,7 @@ int dpd_step(dpd_engine* e, int64_t nsteps, uint32_t flags)
         int64_t done = 0;
         while (chunk >= 2 && nsteps - done >= chunk) {
             const bool last_obs = obs && (nsteps - done == chunk);
-            const auto keyg = std::make_pair(chunk, (int)last_obs);
+            const auto keyg = std::make_pair(chunk, (int)last_obs | e->cur << 1);
             auto it = e->graphs.find(keyg);
             if (it == e->graphs.end()) {
                 const int cur0 = e->cur;
@@ -1857,22 +1892,21 @@ int dpd_time_pair(dpd_engine* e, int32_t nlaunch, double* ms_per_launch)
     float4* keep = e->fold[e->cur ^ 1];
     HIPCHK(hipMemcpyAsync(keep, e->frc, f4, hipMemcpyDeviceToDevice, e->stream));
     // the launch a step that another follows uses: with the epilogue where the schedule has
-    // one, which also writes new cell keys and ranks, counts the counting sort's cells and
-    // may raise the flags (restored below)
+    // one, which also files the beads for the counting sort and may raise the flags (both
+    // restored below)
     const bool epi = epilogue_ok(e);
     int flags0[2] = {0, 0};
     if (epi) HIPCHK(hipMemcpyAsync(flags0, e->flags, sizeof(flags0), hipMemcpyDeviceToHost, e->stream));
     bool terms_done = false;
-    if ((rc = launch_pair(e, false, &terms_done, epi))) return rc;   // untimed first launch
+    if ((rc = launch_pair(e, false, &terms_done, epi, false, false))) return rc;   // untimed first launch
     HIPCHK(hipEventRecord(e->ev[0], e->stream));
     for (int32_t i = 0; i < nlaunch; ++i)
-        if ((rc = launch_pair(e, false, &terms_done, epi))) return rc;
+        if ((rc = launch_pair(e, false, &terms_done, epi, false, false))) return rc;
     HIPCHK(hipEventRecord(e->ev[1], e->stream));
     HIPCHK(hipMemcpyAsync(e->frc, keep, f4, hipMemcpyDeviceToDevice, e->stream));
     if (epi) {
         HIPCHK(hipMemcpyAsync(e->flags, flags0, sizeof(flags0), hipMemcpyHostToDevice, e->stream));
-        HIPCHK(hipMemsetAsync(e->cnt, 0, sizeof(int) * (size_t)e->nkeys, e->stream));
-        HIPCHK(hipMemsetAsync(e->gcnt, 0, sizeof(int) * (size_t)e->ngroups, e->stream));
+        if ((rc = clear_counts(e))) return rc;
     }
     HIPCHK(hipStreamSynchronize(e->stream));
     float ms = 0.f;
@@ -1993,7 +2027,7 @@ int tune_trials(dpd_engine* e, int32_t nsteps, const std::vector<int>& trials, d
             HIPCHK(hipMemcpyAsync(sk, e->key[c0], sizeof(int) * n, k, e->stream));
             HIPCHK(hipMemcpyAsync(scd, e->code[c0], sizeof(uint32_t) * n, k, e->stream));
             HIPCHK(hipMemcpyAsync(sso, e->slot_of, sizeof(int) * n, k, e->stream));
-            HIPCHK(hipMemcpyAsync(scs, e->cstart, sizeof(int) * (e->nkeys + 1), k, e->stream));
+            HIPCHK(hipMemcpyAsync(scs, e->cstart[c0], sizeof(int) * (e->nkeys + 1), k, e->stream));
         } else {
             HIPCHK(hipMemcpyAsync(e->pos[c0], sp, f4, k, e->stream));
             HIPCHK(hipMemcpyAsync(e->vel[c0], sv, f4, k, e->stream));
@@ -2005,10 +2039,11 @@ int tune_trials(dpd_engine* e, int32_t nsteps, const std::vector<int>& trials, d
             HIPCHK(hipMemcpyAsync(e->key[c0], sk, sizeof(int) * n, k, e->stream));
             HIPCHK(hipMemcpyAsync(e->code[c0], scd, sizeof(uint32_t) * n, k, e->stream));
             HIPCHK(hipMemcpyAsync(e->slot_of, sso, sizeof(int) * n, k, e->stream));
-            HIPCHK(hipMemcpyAsync(e->cstart, scs, sizeof(int) * (e->nkeys + 1), k, e->stream));
+            HIPCHK(hipMemcpyAsync(e->cstart[c0], scs, sizeof(int) * (e->nkeys + 1), k, e->stream));
             hipLaunchKernelGGL(k_set_step, dim3(1), dim3(64), 0, e->stream, e->dstep, step0);
             e->cur = c0;
             e->step = step0;
+            if (int rc = clear_counts(e)) return rc;   // (an odd number of steps left those of buffer c0)
         }
         HIPCHK(hipStreamSynchronize(e->stream));
         return DPD_OK;
@@ -2177,7 +2212,7 @@ int dpd_energy_output(dpd_engine* e, int32_t box, double* out3)
     a.vp = e->vp;
     a.img = e->img;
     a.key = e->key[e->cur];
-    a.cstart = e->cstart;
+    a.cstart = e->cstart[e->cur];
     a.table = e->table + (size_t)box * kTableStride;
     a.slot_of = e->slot_of;
     a.bond_bead = e->bond_bead;

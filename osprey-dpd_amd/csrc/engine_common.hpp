@@ -170,7 +170,7 @@ __device__ inline uint32_t scan_code(const float o[3], int cx, const BoxDev& B)
 }
 
 // The integration arithmetic with its rounding fixed by explicit fused multiply-adds, so
-// that kernels repeating a sum (k_advance and k_permute, the pair epilogue, the last step's
+// that kernels repeating a sum (k_advance and k_sort, the pair epilogue, the last step's
 // k_finish) get the same bits however the compiler contracts the rest: kick is v + h f (the
 // halves of UpdateMom, the predicted velocity), drift the displacement dt v + dt^2/2 f.
 __device__ inline float kick(float v, float f, float h) { return fmaf(h, f, v); }
@@ -304,6 +304,51 @@ __device__ inline void wave_groups(int key, bool active, int& rank, int& size, i
             leader = first;
         }
         todo &= ~m;
+    }
+}
+
+// Intake of the counting sort: every bead is filed under its new cell key while the beads
+// still lie in the old order.  The source slots of new cell k go to its bin, with room for five
+// more than the beads it holds (a step moves few beads to another cell).  What finds no room is
+// spilled to a list with its key and rank, in any state at most all beads.
+struct Intake {
+    const int* cstart;   // cell starts of the old order
+    int* bins;
+    int* cnt;            // beads per new cell key
+    int* gcnt;           // per scan group
+    int4* spill;         // (key, rank, source slot, 0)
+    int* nspill;
+    int cap;             // room for spills (0: they are dropped)
+};
+constexpr int kBinSpare = 5;
+__host__ __device__ inline size_t bin_at(int start, int k) { return (size_t)start + kBinSpare * (size_t)k; }
+__host__ __device__ inline int bin_room(int beads) { return beads + kBinSpare; }
+
+// the bead of slot s (where `act`) under key k; reached by the whole wavefront.  Beads arrive
+// cell-sorted, so a wavefront's keys repeat: one atomic per distinct cell and group instead of
+// one per bead, which would serialise ~192 same-address atomics per group counter.  (An atomic
+// on a shared address costs about 100 ns in turn: without the grouping the pair launch of 96^3
+// cells takes 451 us instead of 268, and a counter per 64 groups 30 us more in k_advance.)
+__device__ inline void file_bead(const Intake& I, int k, int s, bool act)
+{
+    int start = 0, room = 0;
+    if (act) {
+        start = I.cstart[k];
+        room = bin_room(I.cstart[k + 1] - start);
+    }
+    const int lane = threadIdx.x & 63;
+    int r, size, leader, base = 0, rg;
+    wave_groups(k, act, r, size, leader);
+    if (act && lane == leader) base = atomicAdd(I.cnt + k, size);
+    r += __shfl(base, leader, 64);
+    wave_groups(k >> 6, act, rg, size, leader);
+    if (act && lane == leader) atomicAdd(I.gcnt + (k >> 6), size);
+    if (act) {
+        if (r < room) I.bins[bin_at(start, k) + r] = s;
+        else if (I.cap > 0) {
+            const int i = atomicAdd(I.nspill, 1);
+            if (i < I.cap) I.spill[i] = make_int4(k, r, s, 0);
+        }
     }
 }
 

@@ -38,13 +38,9 @@ struct PairArgs {
     const int4* hitblk;    // hit-list workgroups of a batch: (box, first slot, end slot)
     int nhitblk;
     // the epilogue of a step that another follows (hit-list kernels, engines without bonded
-    // terms): UpdateMom of this step, UpdatePos of the next, the new cell key and
-    // counting-sort rank
+    // terms): UpdateMom of this step, UpdatePos of the next, the bead filed under its new cell
     const float4* vel;     // v + dt/2 F of the previous step
-    int* nkey;             // new cell key per slot
-    int* rank;             // rank inside the new cell
-    int* cnt;              // beads per cell key (counting sort)
-    int* gcnt;             // beads per scan group
+    Intake intake;
     int* flags;            // [0] non-finite force or velocity, [1] moves of more than one cell
 };
 
@@ -203,7 +199,7 @@ __device__ inline void pair_epilogue(const PairArgs& A, const BoxDev& B, int i, 
         const float4 p = A.pos[i];
         act = !(__float_as_int(p.w) & kBondedBit);
         if (act) {
-            // UpdateMom (k_permute repeats the sum and stores the next half step)
+            // UpdateMom (k_sort repeats the sum and stores the next half step)
             float4 v = A.vel[i];
             v.x = kick(v.x, Fx, B.hdt);
             v.y = kick(v.y, Fy, B.hdt);
@@ -213,25 +209,16 @@ __device__ inline void pair_epilogue(const PairArgs& A, const BoxDev& B, int i, 
             int c[3];
             key_cell(A.key[i] - B.koff, B, c);
             const float o[3] = {p.x, p.y, p.z};
-            const int img[3] = {0, 0, 0};   // the image change is applied by k_permute
+            const int img[3] = {0, 0, 0};   // the image change is applied by k_sort
             const float d[3] = {drift(v.x, Fx, B), drift(v.y, Fy, B), drift(v.z, Fz, B)};
             Moved m;
             advance(o, c, img, d, B, m);
             k = B.koff + cell_key(m.c[0], m.c[1], m.c[2], B);
-            A.nkey[i] = k;
             if (m.jump) atomicAdd(A.flags + 1, 1);
             if (m.bad) atomicAdd(A.flags + 0, 1);
         }
     }
-    const int lane = threadIdx.x & 63;
-    int r, size, leader;
-    wave_groups(k, act, r, size, leader);
-    int base = 0;
-    if (act && lane == leader) base = atomicAdd(A.cnt + k, size);
-    base = __shfl(base, leader, 64);
-    if (act) A.rank[i] = base + r;
-    wave_groups(k >> 6, act, r, size, leader);
-    if (act && lane == leader) atomicAdd(A.gcnt + (k >> 6), size);
+    file_bead(A.intake, k, i, act);
 }
 
 // body of the hit-list kernel for workgroup blockIdx.x (< 8 * per_xcd); also called by the
