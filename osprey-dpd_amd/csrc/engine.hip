@@ -276,6 +276,7 @@ __global__ __launch_bounds__(256) void k_advance(int n, Buffers S, float4* __res
 {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     const bool active = s < n;
+    const int from = S.key[min(s, n - 1)];
     int k = 0;
     if (active) {
         const float4 p = S.pos[s];
@@ -297,7 +298,7 @@ __global__ __launch_bounds__(256) void k_advance(int n, Buffers S, float4* __res
                 atomicAdd(flags + 0, 1);
         }
         int c[3];
-        key_cell(S.key[s] - B.koff, B, c);
+        key_cell(from - B.koff, B, c);
         const float o[3] = {p.x, p.y, p.z};
         const int img[3] = {0, 0, 0};   // the image change is applied by k_sort
         float d[3] = {0.f, 0.f, 0.f};
@@ -312,7 +313,7 @@ __global__ __launch_bounds__(256) void k_advance(int n, Buffers S, float4* __res
         if (m.jump) atomicAdd(flags + 1, 1);
         if (m.bad) atomicAdd(flags + 0, 1);
     }
-    file_bead(I, k, s, active);
+    file_bead(I, from, k, s, active);
 }
 
 // Exclusive scan of in[0, m) into out, in[] cleared, by one workgroup of 1024 threads: in

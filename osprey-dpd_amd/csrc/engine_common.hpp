@@ -283,30 +283,6 @@ __device__ inline int wave_incl_scan(int x)
     return x;
 }
 
-// Active lanes of a wavefront holding equal keys form a group: this lane's rank in its
-// group, the group's size and its lowest lane.  Must be reached by the whole wavefront.
-// One pass per distinct key, with wave-uniform bookkeeping; a wavefront of cell-sorted
-// beads holds ~20 distinct cells.
-__device__ inline void wave_groups(int key, bool active, int& rank, int& size, int& leader)
-{
-    uint64_t todo = __ballot(active);
-    rank = 0;
-    size = 0;
-    leader = 0;
-    while (todo) {
-        const int first = __builtin_ctzll(todo);
-        const int k0 = __builtin_amdgcn_readlane(key, first);
-        const bool mine = active && key == k0;
-        const uint64_t m = __ballot(mine);
-        if (mine) {
-            rank = lane_prefix(m);
-            size = __popcll(m);
-            leader = first;
-        }
-        todo &= ~m;
-    }
-}
-
 // Intake of the counting sort: every bead is filed under its new cell key while the beads
 // still lie in the old order.  The source slots of new cell k go to its bin, with room for five
 // more than the beads it holds (a step moves few beads to another cell).  What finds no room is
@@ -324,30 +300,55 @@ constexpr int kBinSpare = 5;
 __host__ __device__ inline size_t bin_at(int start, int k) { return (size_t)start + kBinSpare * (size_t)k; }
 __host__ __device__ inline int bin_room(int beads) { return beads + kBinSpare; }
 
-// the bead of slot s (where `act`) under key k; reached by the whole wavefront.  Beads arrive
-// cell-sorted, so a wavefront's keys repeat: one atomic per distinct cell and group instead of
-// one per bead, which would serialise ~192 same-address atomics per group counter.  (An atomic
-// on a shared address costs about 100 ns in turn: without the grouping the pair launch of 96^3
-// cells takes 451 us instead of 268, and a counter per 64 groups 30 us more in k_advance.)
-__device__ inline void file_bead(const Intake& I, int k, int s, bool act)
+// Runs of equal values over the lanes of a wavefront: `starts` has the first lane of each.
+__device__ inline uint64_t run_starts(int v)
+{
+    const int before = __builtin_amdgcn_update_dpp(v, v, 0x138, 0xf, 0xf, false);   // wave_shr:1
+    return __ballot((threadIdx.x & 63) == 0 || before != v);
+}
+// the lanes of this lane's run
+__device__ inline uint64_t run_lanes(uint64_t starts)
+{
+    const uint64_t upto = ~0ull >> (63 - (threadIdx.x & 63));
+    const uint64_t next = starts & ~upto;
+    const uint64_t below = next ? (next & -next) - 1 : ~0ull;   // lanes before the next run
+    return below & (~0ull << (63 - __builtin_clzll(starts & upto)));
+}
+
+// The bead of slot s (where `act`), of cell key `from` so far, under key `to`; reached by the
+// whole wavefront, by every lane with the `from` of a slot of its own or its neighbours.  Slots
+// are cell-sorted and few beads leave their cell, so the lanes of a run of equal `from` whose
+// bead stays are counted with one atomic, and so are those of a run of equal groups; a bead that
+// leaves counts by itself.  (One atomic per bead would serialise: an atomic on a shared address
+// costs about 100 ns in turn.  The pair launch of 96^3 cells took 451 us that way against 268
+// with a loop over the wavefront's distinct keys, whose 300 instructions were 8% of the launch;
+// 252 us with runs.)
+__device__ inline void file_bead(const Intake& I, int from, int to, int s, bool act)
 {
     int start = 0, room = 0;
     if (act) {
-        start = I.cstart[k];
-        room = bin_room(I.cstart[k + 1] - start);
+        start = I.cstart[to];
+        room = bin_room(I.cstart[to + 1] - start);
     }
     const int lane = threadIdx.x & 63;
-    int r, size, leader, base = 0, rg;
-    wave_groups(k, act, r, size, leader);
-    if (act && lane == leader) base = atomicAdd(I.cnt + k, size);
-    r += __shfl(base, leader, 64);
-    wave_groups(k >> 6, act, rg, size, leader);
-    if (act && lane == leader) atomicAdd(I.gcnt + (k >> 6), size);
+    const bool stays = act && from == to;
+    const uint64_t cell = __ballot(stays) & run_lanes(run_starts(from));
+    const int first = __builtin_ctzll(cell | (1ull << 63));
+    int n = act, r = 0;
+    if (stays) n = lane == first ? __popcll(cell) : 0;
+    if (n) r = atomicAdd(I.cnt + to, n);
+    const int base = __shfl(r, first, 64);
+    if (stays) r = base + lane_prefix(cell);
+    const bool same = act && from >> 6 == to >> 6;
+    const uint64_t group = __ballot(same) & run_lanes(run_starts(from >> 6));
+    n = act;
+    if (same) n = lane_prefix(group) ? 0 : __popcll(group);
+    if (n) atomicAdd(I.gcnt + (to >> 6), n);
     if (act) {
-        if (r < room) I.bins[bin_at(start, k) + r] = s;
+        if (r < room) I.bins[bin_at(start, to) + r] = s;
         else if (I.cap > 0) {
             const int i = atomicAdd(I.nspill, 1);
-            if (i < I.cap) I.spill[i] = make_int4(k, r, s, 0);
+            if (i < I.cap) I.spill[i] = make_int4(to, r, s, 0);
         }
     }
 }

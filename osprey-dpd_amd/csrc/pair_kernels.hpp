@@ -189,11 +189,12 @@ constexpr int hit_beads(int threads, int split) { return split == 1 ? threads : 
 // The step's end and the next step's start for slot i, whose force (Fx, Fy, Fz) this launch
 // computed: the arithmetic of k_advance (MODE kEndBegin).  Used for engines without bonded
 // terms (a bonded bead's force is not complete here); a bead flagged bonded is left alone.
-// Every lane of the wavefront calls it (the counting-sort ranks group the wavefront's keys);
+// Every lane of the wavefront calls it (file_bead counts the wavefront's keys);
 // `act` marks the lanes that hold a finished bead.
 __device__ inline void pair_epilogue(const PairArgs& A, const BoxDev& B, int i, bool act, float Fx, float Fy,
                                      float Fz)
 {
+    const int from = A.key[min(i, A.n - 1)];
     int k = 0;
     if (act) {
         const float4 p = A.pos[i];
@@ -207,7 +208,7 @@ __device__ inline void pair_epilogue(const PairArgs& A, const BoxDev& B, int i, 
             if (!(fabsf(Fx) + fabsf(Fy) + fabsf(Fz) < 1e30f) || !(fabsf(v.x) + fabsf(v.y) + fabsf(v.z) < 1e30f))
                 atomicAdd(A.flags + 0, 1);
             int c[3];
-            key_cell(A.key[i] - B.koff, B, c);
+            key_cell(from - B.koff, B, c);
             const float o[3] = {p.x, p.y, p.z};
             const int img[3] = {0, 0, 0};   // the image change is applied by k_sort
             const float d[3] = {drift(v.x, Fx, B), drift(v.y, Fy, B), drift(v.z, Fz, B)};
@@ -218,7 +219,7 @@ __device__ inline void pair_epilogue(const PairArgs& A, const BoxDev& B, int i, 
             if (m.bad) atomicAdd(A.flags + 0, 1);
         }
     }
-    file_bead(A.intake, k, i, act);
+    file_bead(A.intake, from, k, i, act);
 }
 
 // body of the hit-list kernel for workgroup blockIdx.x (< 8 * per_xcd); also called by the
