@@ -10,8 +10,9 @@
 //               of a cell in ascending bead index (deterministic layout); above 8192 groups
 //               of 64 cell keys k_group_scan goes before it
 //   pair kernel DPD pair forces (src/CNTCell.cpp:1144-1555)
-//   k_bonded / k_bonded_sum   bonds and angles (src/Bond.cpp:111-162,
-//               src/BondPair.cpp:138-286), each once, summed into the bonded beads' forces
+//               and in the same launch the bonded terms (k_bonded with the full-shell kernel):
+//               bonds and angles (src/Bond.cpp:111-162, src/BondPair.cpp:138-286) summed for
+//               each bonded bead, which k_advance or k_finish adds to its force
 // and a last k_finish closes the final step (UpdateMom + FP64 observables).
 // The simulation time lives in device memory (bumped by k_sort), so a captured
 // sequence of steps replays as a hipGraph without re-capture.
@@ -41,20 +42,18 @@ enum AdvanceMode { kRebin = 0, kBegin = 1, kEndBegin = 2 };
 enum ObsSlot { O_V2 = 0, O_MOM = 3, O_VIR = 6, O_PEP = 15, O_PEB = 16, O_PEA = 17, O_N = 18 };
 static_assert(O_VIR == kObsVir && O_PEP == kObsPEP, "accumulator layout");
 
+// Bonds and angles by bonded bead: thread t of the bonded launch takes bonded[t] and evaluates
+// every term that bead is in.
 struct Topo {
-    const int* bond_ptr;      // [n+1] bond entries of each bead index (all boxes)
-    const int2* bond_csr;     // per bond: the entries of its head and of its tail
-    const int2* bond_bead;    // (head, tail) bead index per bond
-    const double2* bond_par;  // (k, l0) per bond
-    const int* ang_ptr;       // [n+1] angle entries of each bead index
-    const int4* ang_csr;      // per angle: the entries of roles 0 (c), 1 (b), 2 (a)
-    const int4* ang_bead;     // (a, b, c, 0) per angle
-    const double4* ang_par;   // (k, phi0, cos phi0, sin phi0)
-    double4* fbond;           // per bond entry: the bond's force on that entry's bead
-    double4* fang;            // per angle entry: the angle's force on that entry's bead
     const int* bonded;        // bead indices with at least one bond or angle
-    int nbonds, nangles, nbonded;
-    int has_bonds, has_angles;
+    const int4* span;         // its bond entries [x, y) and angle entries [z, w)
+    const int2* bond;         // (the other bead, bond << 1 | this bead is the tail)
+    const int4* angle;        // (the other two in the order a, b, c; angle; role: 0 c, 1 b, 2 a)
+    const double2* bond_par;  // (k, l0) per bond
+    const double4* ang_par;   // (k, phi0, cos phi0, sin phi0)
+    double4* upos;            // (batches) unwrapped position and box by bead index, kept for bonded beads
+    float4* force;            // by slot: the bonded beads' sums of this step
+    int nbonded;
 };
 
 struct Buffers {
@@ -84,148 +83,136 @@ __device__ inline void unwrapped_pos(int slot, int bead, const Buffers& S, const
     u[2] = (double)(c[2] + a.z * B.n[2]) * B.wd[2] + (double)p.z;
 }
 
-// Sum of the bonded forces on bead index q, gathered from the per-bond and per-angle
-// forces of this step (each bond and angle is evaluated once, by k_bonded).
-__device__ inline void bonded_gather(int q, const Topo& T, double f[3])
-{
-    f[0] = f[1] = f[2] = 0.0;
-    if (T.has_bonds) {
-        for (int e = T.bond_ptr[q], e1 = T.bond_ptr[q + 1]; e < e1; ++e) {
-            const double4 fb = T.fbond[e];
-            f[0] += fb.x; f[1] += fb.y; f[2] += fb.z;
-        }
-    }
-    if (T.has_angles) {
-        for (int e = T.ang_ptr[q], e1 = T.ang_ptr[q + 1]; e < e1; ++e) {
-            const double4 fa = T.fang[e];
-            f[0] += fa.x; f[1] += fa.y; f[2] += fa.z;
-        }
-    }
-}
-
 // ---------------------------------------------------------------- kernels ------
 
-// CBond::AddForce (src/Bond.cpp:111-162) and CBondPair::AddForce for every bond and angle
-// of this step, in FP64: thread q < nbonds takes bond q, the rest take angles.  The force
-// goes to fbond / fang, from where k_advance / k_finish gather each bead's sum.  OBS adds
-// the bond virial (to the head bead's box, as CBond::AddForce adds its stress to the head)
-// and the bond and angle potential energies.  Bonds and angles never cross boxes.
-// q = this thread's bond or angle, q0 = the workgroup's first (its box receives the
-// workgroup's observables); workgroups of up to 64 * WAVES threads
+// CBond::AddForce (src/Bond.cpp:111-162) and CBondPair::AddForce of this step in FP64, summed
+// over the terms of bonded bead t (bonds first, each in the order of upload) and rounded once;
+// k_advance and k_finish add the sum to the bead's pair force.  OBS adds the bond virial (to the
+// head bead's box, as CBond::AddForce adds its stress to the head) and the bond and angle
+// potential energies, each from one of its beads (the head, the shared bead).  Bonds and angles
+// never cross boxes; t0 is the workgroup's first bead, whose box receives the workgroup's sums.
+// What bounds it: traffic and its latency.  Each term is evaluated once for each of its beads
+// (a bond's force and its negative have the same bits), so a sum stays in registers; with a
+// thread per bond and angle the forces went through memory, 160 bytes written and read for each
+// bead of a chain.  Positions of a batch come unwrapped from k_sort, in bead order (the
+// neighbours along a chain are the neighbouring threads' own): 64 replicas 14.0 us, with a thread
+// per term 16.4, and 163 us a step where positions looked up by slot take 171.  One box's bonded
+// terms run beside the pair launch and the look-ups are hidden there, k_sort's extra 36 bytes a
+// bead are not (48x48x32 bilayer 48.4 us a step against 49.8).
 template <bool OBS, bool MULTI, int WAVES>
-__device__ __attribute__((always_inline)) inline void bonded_body(const Buffers& S, const int* __restrict__ slot_of,
-                                                                  const Topo& T, const BoxDev* boxes, const BoxDev& B0,
-                                                                  double* __restrict__ acc, int q, int q0)
+__device__ __attribute__((always_inline)) inline void bonded_body(const Buffers& S, const BoxDev& B0, const Topo& T,
+                                                                  const int* __restrict__ slot_of,
+                                                                  double* __restrict__ acc, int t, int t0)
 {
     double ob[12];
     if (OBS)
         for (int i = 0; i < 12; ++i) ob[i] = 0.0;
     int box = -1;
-    if (q < T.nbonds) {
-        const int2 hb = T.bond_bead[q];
-        const int sh = slot_of[hb.x], st = slot_of[hb.y];
-        const int w = __float_as_int(S.pos[sh].w);
-        box = bead_box(w);
-        const BoxDev& B = box_of<MULTI>(boxes, B0, w);
-        double uh[3], ut[3];
-        unwrapped_pos(sh, hb.x, S, B, uh);
-        unwrapped_pos(st, hb.y, S, B, ut);
-        const double2 par = T.bond_par[q];
-        const double d[3] = {uh[0] - ut[0], uh[1] - ut[1], uh[2] - ut[2]};
-        const double L = sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
-        const double s = par.x * (par.y - L) / L;
-        const double fb[3] = {s * d[0], s * d[1], s * d[2]};
-        // straight into the two beads' entries (negation is exact: the sums are those of
-        // one force per bond added with its sign)
-        const int2 ent = T.bond_csr[q];
-        T.fbond[ent.x] = make_double4(fb[0], fb[1], fb[2], 0.0);
-        T.fbond[ent.y] = make_double4(-fb[0], -fb[1], -fb[2], 0.0);
-        if (OBS) {
-            for (int a = 0; a < 3; ++a)
-                for (int b = 0; b < 3; ++b) ob[3 * a + b] = d[b] * fb[a];
-            ob[10] = 0.5 * par.x * (L - par.y) * (L - par.y);
+    auto where = [&](int q) {
+        if (MULTI) return T.upos[q];
+        double u[3];
+        unwrapped_pos(slot_of[q], q, S, B0, u);
+        return make_double4(u[0], u[1], u[2], 0.0);
+    };
+    if (t < T.nbonded) {
+        const int q = T.bonded[t];
+        const int4 sp = T.span[t];
+        const int s = slot_of[q];
+        const double4 me = where(q);
+        const double u[3] = {me.x, me.y, me.z};
+        double F[3] = {0.0, 0.0, 0.0};
+        if (OBS) box = (int)me.w;
+        for (int e = sp.x; e < sp.y; ++e) {
+            const int2 en = T.bond[e];
+            const double2 par = T.bond_par[en.y >> 1];
+            const double4 o = where(en.x);
+            const bool tail = en.y & 1;
+            const double x[3] = {o.x, o.y, o.z};
+            double d[3];   // head - tail
+            for (int a = 0; a < 3; ++a) d[a] = tail ? x[a] - u[a] : u[a] - x[a];
+            const double L = sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
+            const double f = par.x * (par.y - L) / L;
+            const double fb[3] = {f * d[0], f * d[1], f * d[2]};
+            for (int a = 0; a < 3; ++a) F[a] += tail ? -fb[a] : fb[a];
+            if (OBS && !tail) {
+                for (int a = 0; a < 3; ++a)
+                    for (int b = 0; b < 3; ++b) ob[3 * a + b] += d[b] * fb[a];
+                ob[10] += 0.5 * par.x * (L - par.y) * (L - par.y);
+            }
         }
-    } else if (q < T.nbonds + T.nangles) {
-        const int g = q - T.nbonds;
-        const int4 abc = T.ang_bead[g];
-        const int sa = slot_of[abc.x], sb = slot_of[abc.y], sc = slot_of[abc.z];
-        const int w = __float_as_int(S.pos[sb].w);
-        box = bead_box(w);
-        const BoxDev& B = box_of<MULTI>(boxes, B0, w);
-        double ua[3], ub[3], uc[3], f[3][3], pe = 0.0;
-        unwrapped_pos(sa, abc.x, S, B, ua);
-        unwrapped_pos(sb, abc.y, S, B, ub);
-        unwrapped_pos(sc, abc.z, S, B, uc);
-        angle_forces(ua, ub, uc, T.ang_par[g], f, OBS ? &pe : nullptr);
-        const int4 ent = T.ang_csr[g];
-        T.fang[ent.x] = make_double4(f[0][0], f[0][1], f[0][2], 0.0);
-        T.fang[ent.y] = make_double4(f[1][0], f[1][1], f[1][2], 0.0);
-        T.fang[ent.z] = make_double4(f[2][0], f[2][1], f[2][2], 0.0);
-        if (OBS) ob[11] = pe;
+        for (int e = sp.z; e < sp.w; ++e) {
+            const int4 en = T.angle[e];
+            const double4 par = T.ang_par[en.z];
+            const double4 g = where(en.x), h = where(en.y);
+            const double ug[3] = {g.x, g.y, g.z}, uh[3] = {h.x, h.y, h.z};
+            double ua[3], ub[3], uc[3], f[3][3], pe = 0.0;
+            for (int a = 0; a < 3; ++a) {
+                ua[a] = en.w == 2 ? u[a] : ug[a];
+                ub[a] = en.w == 1 ? u[a] : (en.w == 2 ? ug[a] : uh[a]);
+                uc[a] = en.w == 0 ? u[a] : uh[a];
+            }
+            angle_forces(ua, ub, uc, par, f, OBS ? &pe : nullptr);
+            for (int a = 0; a < 3; ++a) F[a] += en.w == 0 ? f[0][a] : (en.w == 1 ? f[1][a] : f[2][a]);
+            if (OBS && en.w == 1) ob[11] += pe;
+        }
+        T.force[s] = make_float4((float)F[0], (float)F[1], (float)F[2], 0.f);
     }
     if (OBS) {
         // slots O_VIR .. O_PEA: virial (9), pair PE (untouched here), bond PE, angle PE
-        int box0 = 0;
-        if (MULTI) {
-            const int s0 = q0 < T.nbonds ? slot_of[T.bond_bead[q0].x] : slot_of[T.ang_bead[q0 - T.nbonds].y];
-            box0 = bead_box(__float_as_int(S.pos[s0].w));
-        } else {
-            box = box < 0 ? -1 : 0;
-        }
+        const int box0 = MULTI ? (int)T.upos[T.bonded[t0]].w : 0;
         accumulate_boxes<12, WAVES>(ob, box, box0, kObsVir, acc);
     }
 }
 
 template <bool OBS, bool MULTI>
-__global__ __launch_bounds__(256) void k_bonded(Buffers S, const int* __restrict__ slot_of, Topo T,
-                                                const BoxDev* boxes, BoxDev B0, double* __restrict__ acc)
+__global__ __launch_bounds__(256) void k_bonded(Buffers S, BoxDev B0, Topo T, const int* __restrict__ slot_of,
+                                                double* __restrict__ acc)
 {
-    const int q0 = blockIdx.x * blockDim.x;
-    bonded_body<OBS, MULTI, 4>(S, slot_of, T, boxes, B0, acc, q0 + threadIdx.x, q0);
+    const int t0 = blockIdx.x * blockDim.x;
+    bonded_body<OBS, MULTI, 4>(S, B0, T, slot_of, acc, t0 + threadIdx.x, t0);
 }
 
 // The hit-list pair kernel and the bonded terms of the same step in one launch: the pair
-// workgroups come first, the bond and angle workgroups after them, so the bonded work fills
-// the CUs the pair kernel's last workgroups leave idle (the two write disjoint buffers).
-// (one box; held to 80 VGPRs like the hit-list kernel, six wavefronts per SIMD)
-template <bool OBS, int THREADS, int CAP, int FLUSH, int SPLIT, bool EPI>
+// workgroups come first, the bonded workgroups after them, so the bonded work fills the CUs the
+// pair kernel's last workgroups leave idle (the two write disjoint buffers).  One box.
+template <bool OBS, int THREADS, int CAP, int FLUSH, int SPLIT>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(hit_waves_eu(OBS, THREADS, CAP, SPLIT))))
-void k_pair_hitlist_bonded(PairArgs A, BoxDev B0, int nblocks, int per_xcd, Buffers S,
-                           const int* __restrict__ slot_of, Topo T)
+void k_pair_hitlist_bonded(PairArgs A, BoxDev B0, int nblocks, int per_xcd, Buffers S, Topo T,
+                           const int* __restrict__ slot_of)
 {
     const int npair = 8 * per_xcd;
     if ((int)blockIdx.x >= npair) {
-        const int q0 = ((int)blockIdx.x - npair) * THREADS;
-        bonded_body<OBS, false, THREADS / 64>(S, slot_of, T, A.boxes, B0, A.acc, q0 + (int)threadIdx.x, q0);
+        const int t0 = ((int)blockIdx.x - npair) * THREADS;
+        bonded_body<OBS, false, THREADS / 64>(S, B0, T, slot_of, A.acc, t0 + (int)threadIdx.x, t0);
         return;
     }
-    hitlist_body<OBS, false, THREADS, CAP, FLUSH, SPLIT, EPI>(A, B0, nblocks, per_xcd);
+    hitlist_body<OBS, false, THREADS, CAP, FLUSH, SPLIT, false>(A, B0, nblocks, per_xcd);
 }
 
-// the fused launch of hit-list schedule S with `nq` bonds and angles
-template <int S, bool OBS, bool EPI>
-void launch_hitlist_bonded_s(const PairArgs& a, const BoxDev& B0, int nq, const Buffers& Sb, const int* slot_of,
-                             const Topo& T, hipStream_t st)
+// the fused launch of hit-list schedule S
+template <int S, bool OBS>
+void launch_hitlist_bonded_s(const PairArgs& a, const BoxDev& B0, const Buffers& Sb, const Topo& T, const int* slot_of,
+                             hipStream_t st)
 {
     constexpr Schedule q = kSchedule[S];
     const int gh = (a.n + q.beads() - 1) / q.beads();
     const int ph = (gh + 7) / 8;
-    const dim3 gr(8 * ph + (nq + q.threads - 1) / q.threads), bl(q.threads);
-    hipLaunchKernelGGL((k_pair_hitlist_bonded<OBS, q.threads, q.cap, q.flush, q.split, EPI>), gr, bl, 0, st,
-                       a, B0, gh, ph, Sb, slot_of, T);
+    const dim3 gr(8 * ph + (T.nbonded + q.threads - 1) / q.threads), bl(q.threads);
+    hipLaunchKernelGGL((k_pair_hitlist_bonded<OBS, q.threads, q.cap, q.flush, q.split>), gr, bl, 0, st, a, B0, gh, ph,
+                       Sb, T, slot_of);
 }
 
-template <bool OBS, bool EPI>
-void launch_hitlist_bonded(int sched, const PairArgs& a, const BoxDev& B0, int nq, const Buffers& Sb,
-                           const int* slot_of, const Topo& T, hipStream_t st)
+template <bool OBS>
+void launch_hitlist_bonded(int sched, const PairArgs& a, const BoxDev& B0, const Buffers& Sb, const Topo& T,
+                           const int* slot_of, hipStream_t st)
 {
     switch (sched) {
-    case 1: launch_hitlist_bonded_s<1, OBS, EPI>(a, B0, nq, Sb, slot_of, T, st); break;
-    case 2: launch_hitlist_bonded_s<2, OBS, EPI>(a, B0, nq, Sb, slot_of, T, st); break;
-    case 3: launch_hitlist_bonded_s<3, OBS, EPI>(a, B0, nq, Sb, slot_of, T, st); break;
-    case 5: launch_hitlist_bonded_s<5, OBS, EPI>(a, B0, nq, Sb, slot_of, T, st); break;
-    case 6: launch_hitlist_bonded_s<6, OBS, EPI>(a, B0, nq, Sb, slot_of, T, st); break;
-    default: launch_hitlist_bonded_s<0, OBS, EPI>(a, B0, nq, Sb, slot_of, T, st); break;
+    case 1: launch_hitlist_bonded_s<1, OBS>(a, B0, Sb, T, slot_of, st); break;
+    case 2: launch_hitlist_bonded_s<2, OBS>(a, B0, Sb, T, slot_of, st); break;
+    case 3: launch_hitlist_bonded_s<3, OBS>(a, B0, Sb, T, slot_of, st); break;
+    case 5: launch_hitlist_bonded_s<5, OBS>(a, B0, Sb, T, slot_of, st); break;
+    case 6: launch_hitlist_bonded_s<6, OBS>(a, B0, Sb, T, slot_of, st); break;
+    default: launch_hitlist_bonded_s<0, OBS>(a, B0, Sb, T, slot_of, st); break;
     }
 }
 
@@ -240,35 +227,25 @@ __global__ __launch_bounds__(256) void k_clear_bonded_flag(int n, float4* __rest
     slot_of[bead[s]] = s;
 }
 
-__global__ __launch_bounds__(256) void k_set_bonded_flag(int nbonded, const int* __restrict__ bonded,
-                                                         const int* __restrict__ slot_of, float4* __restrict__ pos)
-{
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nbonded) return;
-    const int s = slot_of[bonded[t]];
-    pos[s].w = __int_as_float(__float_as_int(pos[s].w) | kBondedBit);
-}
-
-// Add each bonded bead's bond and angle forces of this step to its pair force, in place
-// (one thread per bead that has bonds; its sum in FP64, rounded once).
-__global__ __launch_bounds__(256) void k_bonded_sum(Topo T, const int* __restrict__ slot_of,
-                                                    float4* __restrict__ frc)
+// (and, in a batch, the unwrapped positions, which k_sort keeps from then on)
+__global__ __launch_bounds__(256) void k_set_bonded_flag(Topo T, const int* __restrict__ slot_of, Buffers S,
+                                                         const BoxDev* boxes)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= T.nbonded) return;
-    const int q = T.bonded[t];
-    double fb[3];
-    bonded_gather(q, T, fb);
-    const int s = slot_of[q];
-    float4 f = frc[s];
-    f.x += (float)fb[0]; f.y += (float)fb[1]; f.z += (float)fb[2];
-    frc[s] = f;
+    const int q = T.bonded[t], s = slot_of[q];
+    const int w = __float_as_int(S.pos[s].w) | kBondedBit;
+    S.pos[s].w = __int_as_float(w);
+    if (!T.upos) return;
+    double u[3];
+    unwrapped_pos(s, q, S, boxes[bead_box(w)], u);
+    T.upos[q] = make_double4(u[0], u[1], u[2], (double)bead_box(w));
 }
 
 // Close the previous step (kEndBegin) and start the next one: new cell key and rank.
 // kEndBegin also adds the previous step's bond and angle forces of bonded beads (flagged in
 // pos.w) to their pair force, in place: within a sequence of steps the bonded sum of every
-// step but the last is left to the next step's k_advance (same arithmetic as k_bonded_sum).
+// step but the last is left to the next step's k_advance (the last one's to k_finish).
 template <int MODE, bool MULTI>
 __global__ __launch_bounds__(256) void k_advance(int n, Buffers S, float4* __restrict__ frc, Topo T,
                                                  const BoxDev* boxes,
@@ -284,9 +261,8 @@ __global__ __launch_bounds__(256) void k_advance(int n, Buffers S, float4* __res
         float4 v = S.vel[s];
         float4 f = (MODE == kRebin) ? S.fold[s] : frc[s];
         if (MODE == kEndBegin && (__float_as_int(p.w) & kBondedBit)) {
-            double fb[3];
-            bonded_gather(S.bead[s], T, fb);
-            f.x += (float)fb[0]; f.y += (float)fb[1]; f.z += (float)fb[2];
+            const float4 b = T.force[s];
+            f.x += b.x; f.y += b.y; f.z += b.z;
             frc[s] = f;
         }
         if (MODE == kEndBegin) {
@@ -398,8 +374,8 @@ __global__ __launch_bounds__(256) void k_sort(int n, int ngroups, int per_xcd, B
                                               const float4* __restrict__ frc, float4* __restrict__ vp,
                                               const BoxDev* boxes, BoxDev B0, Intake I, const int* __restrict__ gstart,
                                               int* __restrict__ cstart, int* __restrict__ clear,
-                                              int* __restrict__ slot_of, int write_vp, int64_t* __restrict__ step,
-                                              int2* __restrict__ order)
+                                              int* __restrict__ slot_of, double4* __restrict__ upos,
+                                              int write_vp, int64_t* __restrict__ step, int2* __restrict__ order)
 {
     __shared__ int first[kGroupKeys + 1];   // of each cell among the group's beads
     __shared__ int old[kGroupKeys];         // of each cell in the old order
@@ -489,10 +465,16 @@ __global__ __launch_bounds__(256) void k_sort(int n, int ngroups, int per_xcd, B
         D.bead[dst] = q;
         // the image counts live by bead index: only a bead that crosses the box changes them,
         // and only its own thread writes them
-        if (m.img[0] | m.img[1] | m.img[2]) {
+        const bool bonded = __float_as_int(p.w) & kBondedBit, crosses = m.img[0] | m.img[1] | m.img[2];
+        if ((MULTI && bonded) || crosses) {
             int4 im = S.img[q];
             im.x += m.img[0]; im.y += m.img[1]; im.z += m.img[2];
-            S.img[q] = im;
+            if (crosses) S.img[q] = im;
+            if (MULTI && bonded)
+                upos[q] = make_double4((double)(m.c[0] + im.x * B.n[0]) * B.wd[0] + (double)m.o[0],
+                                       (double)(m.c[1] + im.y * B.n[1]) * B.wd[1] + (double)m.o[1],
+                                       (double)(m.c[2] + im.z * B.n[2]) * B.wd[2] + (double)m.o[2],
+                                       (double)bead_box(wd));
         }
         D.key[dst] = k;
         D.code[dst] = scan_code(m.o, m.c[0], B);
@@ -506,7 +488,7 @@ __global__ __launch_bounds__(256) void k_sort(int n, int ngroups, int per_xcd, B
         // the slot of each bead is read for bonded beads only (bond and angle terms); a scattered
         // 4-byte store per bead costs a partial-line write each, so the others are skipped once
         // the topology has flagged the bonded ones (an upload re-binning writes every bead)
-        if (MODE == kRebin || (__float_as_int(p.w) & kBondedBit)) slot_of[q] = dst;
+        if (MODE == kRebin || bonded) slot_of[q] = dst;
     };
     if (total <= kSortList && !spilled) {
         // the first 256 beads are loaded before their indices are exchanged
@@ -565,11 +547,11 @@ __global__ void k_copy_force(int n, const float4* __restrict__ fold, float4* __r
     if (s < n) frc[s] = fold[s];
 }
 
-// Close the last step: UpdateMom (UPDATE_V) and the FP64 sums of v^2 and momentum (the
-// force already holds the bonded terms; the virial and energies come from the pair and
+// Close the last step: the bonded beads' sums added to their force, UpdateMom (UPDATE_V) and
+// the FP64 sums of v^2 and momentum (the virial and energies come from the pair and
 // bonded kernels).
 template <bool UPDATE_V, bool OBS, bool MULTI>
-__global__ __launch_bounds__(256) void k_finish(int n, Buffers S, const float4* __restrict__ frc,
+__global__ __launch_bounds__(256) void k_finish(int n, Buffers S, float4* __restrict__ frc, Topo T,
                                                 const BoxDev* boxes, BoxDev B0, int* __restrict__ flags,
                                                 double* __restrict__ acc, float4* __restrict__ vp_keep)
 {
@@ -583,8 +565,13 @@ __global__ __launch_bounds__(256) void k_finish(int n, Buffers S, const float4* 
         const int w = __float_as_int(S.pos[s].w);
         box = bead_box(w);
         const BoxDev& B = box_of<MULTI>(boxes, B0, w);
-        const float4 f = frc[s];
+        float4 f = frc[s];
         float4 v = S.vel[s];
+        if (T.nbonded > 0 && (w & kBondedBit)) {
+            const float4 b = T.force[s];
+            f.x += b.x; f.y += b.y; f.z += b.z;
+            frc[s] = f;
+        }
         if (UPDATE_V) {
             // the last step's predicted velocity, which the steps read from vel (vp_is_vel)
             if (vp_keep) vp_keep[s] = v;
@@ -747,15 +734,13 @@ struct dpd_engine {
     int nhitblk[kSchedules] = {};    // per schedule (its beads per workgroup)
     size_t slice_cap = 0;
     // topology
-    int *bond_ptr = nullptr, *ang_ptr = nullptr;
-    int2 *bond_csr = nullptr, *bond_bead = nullptr;
-    int4* ang_csr = nullptr;
+    int2 *bond_bead = nullptr, *bond_ent = nullptr;
+    int4 *ang_bead = nullptr, *ang_ent = nullptr, *span = nullptr;
     double2* bond_par = nullptr;
-    int4* ang_bead = nullptr;
-    double4 *ang_par = nullptr, *fbond = nullptr, *fang = nullptr;
+    double4 *ang_par = nullptr, *upos = nullptr;
+    float4* bforce = nullptr;
     int* bonded = nullptr;
     int nbonds = 0, nangles = 0, nbonded = 0;
-    int has_bonds = 0, has_angles = 0;
     // observables
     std::vector<dpd_obs> obs;
     bool obs_valid = false;
@@ -900,9 +885,7 @@ Buffers bufs(dpd_engine* e, int i)
 
 Topo topo(dpd_engine* e)
 {
-    return Topo{e->bond_ptr, e->bond_csr, e->bond_bead, e->bond_par, e->ang_ptr, e->ang_csr, e->ang_bead,
-                e->ang_par, e->fbond, e->fang, e->bonded, e->nbonds, e->nangles, e->nbonded, e->has_bonds,
-                e->has_angles};
+    return Topo{e->bonded, e->span, e->bond_ent, e->ang_ent, e->bond_par, e->ang_par, e->upos, e->bforce, e->nbonded};
 }
 
 inline int grid(int64_t n, int b) { return (int)((n + b - 1) / b); }
@@ -944,7 +927,7 @@ void sort_step_t(dpd_engine* e, bool advanced)
     const int per = grid(e->ngroups, 8);
     hipLaunchKernelGGL((k_sort<MODE, MULTI>), dim3(8 * per), dim3(256), 0, e->stream, n, e->ngroups, per, S, D, e->frc,
                        e->vp, e->dboxes, B0, I, scan ? e->gstart : nullptr, e->cstart[e->cur ^ 1],
-                       e->counts[e->cur ^ 1], e->slot_of, (MODE == kRebin || !vp_is_vel(e)) ? 1 : 0, e->dstep, e->order);
+                       e->counts[e->cur ^ 1], e->slot_of, e->upos, (MODE == kRebin || !vp_is_vel(e)) ? 1 : 0, e->dstep, e->order);
     e->cur ^= 1;
 }
 
@@ -962,10 +945,10 @@ int sort_step(dpd_engine* e, bool advanced = false)
 // the bond and angle forces are known: measured on the condensate box, the epilogue added
 // 14 us to the pair launch and that pass took 20 us, against the 25 us of k_advance it
 // replaced.)
-inline bool epilogue_ok(const dpd_engine* e) { return e->nbonded == 0 && epilogue_available(e->sched, e->n); }
+inline bool epilogue_ok(const dpd_engine* e) { return e->nbonded == 0 && epilogue_available(e->sched, e->n, e->ngroups); }
 
 // Pair forces of this step.  With the hit-list kernel the bond and angle terms run in the
-// same launch (k_pair_hitlist_bonded); `bonded` then tells launch_bonded to add only the sums.
+// same launch (k_pair_hitlist_bonded); `bonded` then tells that they are done.
 // `epi` (epilogue_ok): the launch also closes the step and starts the next one (pair_epilogue).
 // `spills` false: the launch is repeated on one state, and what overfills the sort's bins is dropped.
 int launch_pair(dpd_engine* e, bool obs, bool* bonded = nullptr, bool epi = false, bool in_seq = false,
@@ -995,15 +978,14 @@ int launch_pair(dpd_engine* e, bool obs, bool* bonded = nullptr, bool epi = fals
     a.acc = e->acc;
     a.hitblk = e->hitblk[e->sched];
     a.nhitblk = e->nhitblk[e->sched];
-    const int nq = e->nbonds + e->nangles;
-    // one box only: in a batch the bonded path's per-lane box raises the fused kernel to 87
-    // VGPRs and costs more than the launch it saves (3.59e9 against 3.72e9 bead-steps/s for
-    // 256 replicas)
-    if (bonded && nq > 0 && e->pair_kernel == DPD_PAIR_HITLIST && a.n <= (int)kHitSlotMask && !multi(e)) {
-        const BoxDev B0 = e->boxes[0].B;
+    // one box only: a batch's pair kernel leaves no registers for the bonded terms (held to its 96
+    // it spills 18: 202 us a step of 64 replicas, 163 with the bonded terms in their own launch)
+    if (bonded && e->nbonded > 0 && e->pair_kernel == DPD_PAIR_HITLIST && hitlist_fits(a.n, a.ngroups) && !multi(e)) {
         // (never with the epilogue: epilogue_ok excludes engines with bonded terms)
-        if (obs) launch_hitlist_bonded<true, false>(e->sched, a, B0, nq, S, e->slot_of, topo(e), e->stream);
-        else launch_hitlist_bonded<false, false>(e->sched, a, B0, nq, S, e->slot_of, topo(e), e->stream);
+        const BoxDev B0 = e->boxes[0].B;
+        const Topo T = topo(e);
+        if (obs) launch_hitlist_bonded<true>(e->sched, a, B0, S, T, e->slot_of, e->stream);
+        else launch_hitlist_bonded<false>(e->sched, a, B0, S, T, e->slot_of, e->stream);
         *bonded = true;
         return hipGetLastError() == hipSuccess ? DPD_OK : fail(e, DPD_ERR_HIP, "pair kernel launch failed");
     }
@@ -1020,32 +1002,22 @@ void launch_finish(dpd_engine* e)
     float4* keep = (UPDATE_V && vp_is_vel(e)) ? e->vp : nullptr;
     if (multi(e))
         hipLaunchKernelGGL((k_finish<UPDATE_V, OBS, true>), dim3(grid(n, 256)), dim3(256), 0, e->stream, n,
-                           bufs(e, e->cur), e->frc, e->dboxes, B0, e->flags, e->acc, keep);
+                           bufs(e, e->cur), e->frc, topo(e), e->dboxes, B0, e->flags, e->acc, keep);
     else
         hipLaunchKernelGGL((k_finish<UPDATE_V, OBS, false>), dim3(grid(n, 256)), dim3(256), 0, e->stream, n,
-                           bufs(e, e->cur), e->frc, e->dboxes, B0, e->flags, e->acc, keep);
+                           bufs(e, e->cur), e->frc, topo(e), e->dboxes, B0, e->flags, e->acc, keep);
 }
 
-// bonds and angles of this step (unless the pair launch ran them) and each bonded bead's
-// sum added to its force
-// `sum` false: the bonded sum is left to the next step's k_advance (kEndBegin)
+// bonds and angles of this step, where the pair launch did not run them
 template <bool OBS>
-void launch_bonded(dpd_engine* e, bool terms_done = false, bool sum = true)
+void launch_bonded(dpd_engine* e)
 {
-    const int nq = e->nbonds + e->nangles;
-    if (nq == 0) return;
+    if (e->nbonded == 0) return;
+    const dim3 gr(grid(e->nbonded, 256)), bl(256);
+    const Buffers S = bufs(e, e->cur);
     const BoxDev B0 = e->boxes[0].B;
-    if (terms_done)
-        ;
-    else if (multi(e))
-        hipLaunchKernelGGL((k_bonded<OBS, true>), dim3(grid(nq, 256)), dim3(256), 0, e->stream, bufs(e, e->cur),
-                           e->slot_of, topo(e), e->dboxes, B0, e->acc);
-    else
-        hipLaunchKernelGGL((k_bonded<OBS, false>), dim3(grid(nq, 256)), dim3(256), 0, e->stream, bufs(e, e->cur),
-                           e->slot_of, topo(e), e->dboxes, B0, e->acc);
-    if (sum)
-        hipLaunchKernelGGL(k_bonded_sum, dim3(grid(e->nbonded, 256)), dim3(256), 0, e->stream, topo(e),
-                           e->slot_of, e->frc);
+    if (multi(e)) hipLaunchKernelGGL((k_bonded<OBS, true>), gr, bl, 0, e->stream, S, B0, topo(e), e->slot_of, e->acc);
+    else hipLaunchKernelGGL((k_bonded<OBS, false>), gr, bl, 0, e->stream, S, B0, topo(e), e->slot_of, e->acc);
 }
 
 // clear the observable accumulators (and, when `flags`, the error flags)
@@ -1126,9 +1098,10 @@ int enqueue_steps(dpd_engine* e, int64_t nsteps, bool obs, int timing)
         bool terms_done = false;
         if ((rc = launch_pair(e, obs && last, &terms_done, epi, true))) return rc;
         if (timed) HIPCHK(hipEventRecord(e->pev[2 * ti++ + 1], e->stream));
-        // the bonded sum of every step but the last is added by the next step's k_advance
-        if (obs && last) launch_bonded<true>(e, terms_done);
-        else launch_bonded<false>(e, terms_done, last);
+        if (!terms_done) {
+            if (obs && last) launch_bonded<true>(e);
+            else launch_bonded<false>(e);
+        }
         advanced = epi;
     }
     if (obs) launch_finish<true, true>(e);
@@ -1276,6 +1249,13 @@ int commit_beads(dpd_engine* e, int64_t step0)
 }
 
 // Global CSR topology from the staged per-box bonds and bond pairs.
+void mark_bonded(dpd_engine* e)
+{
+    if (e->nbonded > 0)
+        hipLaunchKernelGGL(k_set_bonded_flag, dim3(grid(e->nbonded, 256)), dim3(256), 0, e->stream, topo(e), e->slot_of,
+                           bufs(e, e->cur), e->dboxes);
+}
+
 int commit_topology(dpd_engine* e)
 {
     const int64_t n = e->n;
@@ -1305,62 +1285,59 @@ int commit_topology(dpd_engine* e)
         ap[a + 1]++; ap[bm + 1]++; ap[c + 1]++;
     }
     for (int64_t i = 0; i < n; ++i) { bp[i + 1] += bp[i]; ap[i + 1] += ap[i]; }
-    // each bead's entries in bond order (then angle order): the bonded kernels write every
-    // bond's and angle's forces into its beads' entries, and a bead's sum reads its entries
-    std::vector<int2> bcsr(std::max<int64_t>(nbonds, 1)), bbead(std::max<int64_t>(nbonds, 1));
+    // each bead's entries in bond order (then angle order)
+    std::vector<int2> bent(std::max<int>(bp[n], 1)), bbead(std::max<int64_t>(nbonds, 1));
     std::vector<double2> bpar(std::max<int64_t>(nbonds, 1));
-    std::vector<int4> acsr(std::max<int64_t>(npairs, 1));
+    std::vector<int4> aent(std::max<int>(ap[n], 1));
     std::vector<int> fill(bp.begin(), bp.end() - 1);
     for (int64_t b = 0; b < nbonds; ++b) {
         const int h = H[b], t = Tl[b];
         bbead[b] = make_int2(h, t);
         bpar[b] = make_double2(K[b], L0[b]);
-        const int eh = fill[h]++;
-        const int et = fill[t]++;
-        bcsr[b] = make_int2(eh, et);
+        bent[fill[h]++] = make_int2(t, (int)b << 1);
+        bent[fill[t]++] = make_int2(h, (int)b << 1 | 1);
     }
-    std::vector<int> bonded;
-    for (int64_t i = 0; i < n; ++i)
-        if (bp[i + 1] > bp[i] || ap[i + 1] > ap[i]) bonded.push_back((int)i);
     std::vector<int> afill(ap.begin(), ap.end() - 1);
     for (int64_t q = 0; q < npairs; ++q) {
         const int4 abc = abead[q];
-        const int ec = afill[abc.z]++;
-        const int eb = afill[abc.y]++;
-        const int ea = afill[abc.x]++;
-        acsr[q] = make_int4(ec, eb, ea, 0);
+        aent[afill[abc.z]++] = make_int4(abc.x, abc.y, (int)q, 0);
+        aent[afill[abc.y]++] = make_int4(abc.x, abc.z, (int)q, 1);
+        aent[afill[abc.x]++] = make_int4(abc.y, abc.z, (int)q, 2);
     }
+    std::vector<int> bonded;
+    std::vector<int4> span;
+    for (int64_t i = 0; i < n; ++i)
+        if (bp[i + 1] > bp[i] || ap[i + 1] > ap[i]) {
+            bonded.push_back((int)i);
+            span.push_back(make_int4(bp[i], bp[i + 1], ap[i], ap[i + 1]));
+        }
     drop_graphs(e);
     int rc;
-    if ((rc = dalloc(e, &e->bond_ptr, n + 1)) || (rc = dalloc(e, &e->ang_ptr, n + 1)) ||
-        (rc = dalloc(e, &e->bond_csr, bcsr.size())) || (rc = dalloc(e, &e->bond_par, bpar.size())) ||
-        (rc = dalloc(e, &e->bond_bead, bbead.size())) ||
-        (rc = dalloc(e, &e->fbond, std::max<int64_t>(bp[n], 1))) ||
-        (rc = dalloc(e, &e->fang, std::max<int64_t>(ap[n], 1))) || (rc = dalloc(e, &e->bonded, bonded.size())) ||
-        (rc = dalloc(e, &e->ang_csr, acsr.size())) || (rc = dalloc(e, &e->ang_bead, abead.size())) ||
-        (rc = dalloc(e, &e->ang_par, apar.size())))
+    e->nbonded = 0;
+    const size_t nb = bonded.size();
+    if ((rc = dalloc(e, &e->bond_ent, bent.size())) || (rc = dalloc(e, &e->bond_par, bpar.size())) ||
+        (rc = dalloc(e, &e->bond_bead, bbead.size())) || (rc = dalloc(e, &e->ang_ent, aent.size())) ||
+        (rc = dalloc(e, &e->ang_bead, abead.size())) || (rc = dalloc(e, &e->ang_par, apar.size())) ||
+        (rc = dalloc(e, &e->bonded, nb)) || (rc = dalloc(e, &e->span, nb)) ||
+        (multi(e) && (rc = dalloc(e, &e->upos, nb ? n : 0))) || (rc = dalloc(e, &e->bforce, nb ? n : 0)))
         return rc;
-    HIPCHK(hipMemcpyAsync(e->bond_ptr, bp.data(), sizeof(int) * (n + 1), hipMemcpyHostToDevice, e->stream));
-    HIPCHK(hipMemcpyAsync(e->ang_ptr, ap.data(), sizeof(int) * (n + 1), hipMemcpyHostToDevice, e->stream));
-    HIPCHK(hipMemcpyAsync(e->bond_csr, bcsr.data(), sizeof(int2) * bcsr.size(), hipMemcpyHostToDevice, e->stream));
+    HIPCHK(hipMemcpyAsync(e->bond_ent, bent.data(), sizeof(int2) * bent.size(), hipMemcpyHostToDevice, e->stream));
     HIPCHK(hipMemcpyAsync(e->bond_bead, bbead.data(), sizeof(int2) * bbead.size(), hipMemcpyHostToDevice, e->stream));
-    if (!bonded.empty())
-        HIPCHK(hipMemcpyAsync(e->bonded, bonded.data(), sizeof(int) * bonded.size(), hipMemcpyHostToDevice, e->stream));
+    if (nb) {
+        HIPCHK(hipMemcpyAsync(e->bonded, bonded.data(), sizeof(int) * nb, hipMemcpyHostToDevice, e->stream));
+        HIPCHK(hipMemcpyAsync(e->span, span.data(), sizeof(int4) * nb, hipMemcpyHostToDevice, e->stream));
+    }
     HIPCHK(hipMemcpyAsync(e->bond_par, bpar.data(), sizeof(double2) * bpar.size(), hipMemcpyHostToDevice, e->stream));
-    HIPCHK(hipMemcpyAsync(e->ang_csr, acsr.data(), sizeof(int4) * acsr.size(), hipMemcpyHostToDevice, e->stream));
+    HIPCHK(hipMemcpyAsync(e->ang_ent, aent.data(), sizeof(int4) * aent.size(), hipMemcpyHostToDevice, e->stream));
     HIPCHK(hipMemcpyAsync(e->ang_bead, abead.data(), sizeof(int4) * abead.size(), hipMemcpyHostToDevice, e->stream));
     HIPCHK(hipMemcpyAsync(e->ang_par, apar.data(), sizeof(double4) * apar.size(), hipMemcpyHostToDevice, e->stream));
     HIPCHK(hipStreamSynchronize(e->stream));
     e->nbonds = (int)nbonds;
     e->nangles = (int)npairs;
-    e->nbonded = (int)bonded.size();
-    e->has_bonds = nbonds > 0;
-    e->has_angles = npairs > 0;
+    e->nbonded = (int)nb;
     hipLaunchKernelGGL(k_clear_bonded_flag, dim3(grid(n, 256)), dim3(256), 0, e->stream, (int)n, e->pos[e->cur],
                        e->bead[e->cur], e->slot_of);
-    if (e->nbonded > 0)
-        hipLaunchKernelGGL(k_set_bonded_flag, dim3(grid(e->nbonded, 256)), dim3(256), 0, e->stream, e->nbonded,
-                           e->bonded, e->slot_of, e->pos[e->cur]);
+    mark_bonded(e);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(e->stream));
     return DPD_OK;
@@ -1571,9 +1548,9 @@ void dpd_destroy(dpd_engine* e)
     drop_graphs(e);
     void* ptrs[] = {e->pos[0], e->pos[1], e->vel[0], e->vel[1], e->fold[0], e->fold[1], e->bead[0], e->bead[1], e->img,
                     e->key[0], e->key[1], e->code[0], e->code[1], e->frc, e->vp, e->slot_of,
-                    e->cells, e->filed, e->flags, e->dstep, e->acc, e->table, e->gather, e->bond_ptr,
-                    e->ang_ptr, e->bond_csr, e->bond_par, e->ang_csr, e->ang_bead, e->ang_par, e->bond_bead,
-                    e->fbond, e->fang, e->bonded, e->dboxes, e->slice, e->madj};
+                    e->cells, e->filed, e->flags, e->dstep, e->acc, e->table, e->gather, e->bond_ent,
+                    e->ang_ent, e->span, e->bond_par, e->ang_bead, e->ang_par, e->bond_bead,
+                    e->upos, e->bforce, e->bonded, e->dboxes, e->slice, e->madj};
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
     for (void* q : e->hitblk)
@@ -1596,7 +1573,6 @@ int dpd_upload_beads(dpd_engine* e, int64_t n, const int32_t* id, const int32_t*
     if ((rc = stage_beads(e, 0, n, id, type, x, unpbc, v, f))) return rc;
     if ((rc = commit_beads(e, step0))) return rc;
     if (keep_topo) return commit_topology(e);
-    e->has_bonds = e->has_angles = 0;
     e->nbonds = e->nangles = e->nbonded = 0;
     return DPD_OK;
 }
@@ -1745,7 +1721,7 @@ int dpd_compute_forces(dpd_engine* e, int64_t step, uint32_t flags, double* f_ou
     // last step's predicted velocity)
     bool terms_done = false;
     if ((rc = launch_pair(e, true, &terms_done))) return rc;
-    launch_bonded<true>(e, terms_done);
+    if (!terms_done) launch_bonded<true>(e);
     launch_finish<false, true>(e);
     HIPCHK(hipGetLastError());
     if ((rc = read_flags(e))) return rc;
@@ -2044,6 +2020,7 @@ int tune_trials(dpd_engine* e, int32_t nsteps, const std::vector<int>& trials, d
             hipLaunchKernelGGL(k_set_step, dim3(1), dim3(64), 0, e->stream, e->dstep, step0);
             e->cur = c0;
             e->step = step0;
+            mark_bonded(e);   // (the unwrapped positions)
             if (int rc = clear_counts(e)) return rc;   // (an odd number of steps left those of buffer c0)
         }
         HIPCHK(hipStreamSynchronize(e->stream));

@@ -623,11 +623,13 @@ inline void launch_hitlist(int sched, const PairArgs& a, const BoxDev& B0, int n
     }
 }
 
+// whether the hit-list kernel's list entries and row addresses hold an engine's slots and keys
+inline bool hitlist_fits(int64_t n, int64_t ngroups) { return n <= (int64_t)kHitSlotMask && ngroups < (1 << 24); }
+
 // whether schedule `sched` can carry the step's epilogue (hit-list kernels only)
-inline bool epilogue_available(int sched, int64_t n)
+inline bool epilogue_available(int sched, int64_t n, int64_t ngroups)
 {
-    return sched >= 0 && sched < kSchedules && kSchedule[sched].kernel == DPD_PAIR_HITLIST &&
-           n <= (int64_t)kHitSlotMask;
+    return sched >= 0 && sched < kSchedules && kSchedule[sched].kernel == DPD_PAIR_HITLIST && hitlist_fits(n, ngroups);
 }
 
 // The automatic choice: the hit-list kernel for every engine whose slots fit its 26-bit list
@@ -647,7 +649,7 @@ inline hipError_t launch_pair_kernel(int sched, const PairArgs& a, const BoxDev&
 {
     const bool multi = a.nbox > 1;
     if (sched < 0 || sched >= kSchedules) sched = kDefaultSchedule;
-    if (kSchedule[sched].kernel == DPD_PAIR_HITLIST && a.n <= (int)kHitSlotMask && a.ngroups < (1 << 24) && (!multi || a.hitblk)) {
+    if (kSchedule[sched].kernel == DPD_PAIR_HITLIST && hitlist_fits(a.n, a.ngroups) && (!multi || a.hitblk)) {
         const int nb = kSchedule[sched].beads();
         const int gh = multi ? a.nhitblk : (a.n + nb - 1) / nb;
         if (obs) {
