@@ -101,8 +101,8 @@ __device__ inline void unwrapped_pos(int slot, int bead, const Buffers& S, const
 // bead are not (48x48x32 bilayer 48.4 us a step against 49.8).
 template <bool OBS, bool MULTI, int WAVES>
 __device__ __attribute__((always_inline)) inline void bonded_body(const Buffers& S, const BoxDev& B0, const Topo& T,
-                                                                  const int* __restrict__ slot_of,
-                                                                  double* __restrict__ acc, int t, int t0)
+                                                                  const int* __restrict__ slot_of, const Sums& sums,
+                                                                  int t, int t0)
 {
     double ob[12];
     if (OBS)
@@ -160,16 +160,16 @@ __device__ __attribute__((always_inline)) inline void bonded_body(const Buffers&
     if (OBS) {
         // slots O_VIR .. O_PEA: virial (9), pair PE (untouched here), bond PE, angle PE
         const int box0 = MULTI ? (int)T.upos[T.bonded[t0]].w : 0;
-        accumulate_boxes<12, WAVES>(ob, box, box0, kObsVir, acc);
+        accumulate_boxes<12, WAVES>(ob, box, box0, kObsVir, sums);
     }
 }
 
 template <bool OBS, bool MULTI>
 __global__ __launch_bounds__(256) void k_bonded(Buffers S, BoxDev B0, Topo T, const int* __restrict__ slot_of,
-                                                double* __restrict__ acc)
+                                                Sums sums)
 {
     const int t0 = blockIdx.x * blockDim.x;
-    bonded_body<OBS, MULTI, 4>(S, B0, T, slot_of, acc, t0 + threadIdx.x, t0);
+    bonded_body<OBS, MULTI, 4>(S, B0, T, slot_of, sums, t0 + threadIdx.x, t0);
 }
 
 // The hit-list pair kernel and the bonded terms of the same step in one launch: the pair
@@ -183,7 +183,7 @@ void k_pair_hitlist_bonded(PairArgs A, BoxDev B0, int nblocks, int per_xcd, Buff
     const int npair = 8 * per_xcd;
     if ((int)blockIdx.x >= npair) {
         const int t0 = ((int)blockIdx.x - npair) * THREADS;
-        bonded_body<OBS, false, THREADS / 64>(S, B0, T, slot_of, A.acc, t0 + (int)threadIdx.x, t0);
+        bonded_body<OBS, false, THREADS / 64>(S, B0, T, slot_of, A.sums, t0 + (int)threadIdx.x, t0);
         return;
     }
     hitlist_body<OBS, false, THREADS, CAP, FLUSH, SPLIT, false>(A, B0, nblocks, per_xcd);
@@ -553,7 +553,7 @@ __global__ void k_copy_force(int n, const float4* __restrict__ fold, float4* __r
 template <bool UPDATE_V, bool OBS, bool MULTI>
 __global__ __launch_bounds__(256) void k_finish(int n, Buffers S, float4* __restrict__ frc, Topo T,
                                                 const BoxDev* boxes, BoxDev B0, int* __restrict__ flags,
-                                                double* __restrict__ acc, float4* __restrict__ vp_keep)
+                                                Sums sums, float4* __restrict__ vp_keep)
 {
     static_assert(O_V2 == 0 && O_MOM == 3, "kinetic slots first");
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
@@ -594,13 +594,13 @@ __global__ __launch_bounds__(256) void k_finish(int n, Buffers S, float4* __rest
     }
     if (OBS) {
         const int box0 = MULTI ? bead_box(__float_as_int(S.pos[blockIdx.x * blockDim.x].w)) : 0;
-        accumulate_boxes<6>(ob, MULTI ? box : (s < n ? 0 : -1), box0, 0, acc);
+        accumulate_boxes<6>(ob, MULTI ? box : (s < n ? 0 : -1), box0, 0, sums);
     }
 }
 
-// FP64 sums per box of v and v^2 and the bead count: acc[box][0..4]
+// FP64 sums per box of v and v^2 and the bead count, slots 0..4
 template <bool MULTI>
-__global__ __launch_bounds__(256) void k_mom_sums(int n, Buffers S, double* __restrict__ acc)
+__global__ __launch_bounds__(256) void k_mom_sums(int n, Buffers S, Sums sums)
 {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     double ob[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
@@ -613,7 +613,7 @@ __global__ __launch_bounds__(256) void k_mom_sums(int n, Buffers S, double* __re
         ob[4] = 1.0;
     }
     const int box0 = MULTI ? bead_box(__float_as_int(S.pos[blockIdx.x * blockDim.x].w)) : 0;
-    accumulate_boxes<5>(ob, box, box0, 0, acc);
+    accumulate_boxes<5>(ob, box, box0, 0, sums);
 }
 
 // v <- (v - shift) * scale with adj[box] = (shift x, y, z, scale), in FP64
@@ -631,7 +631,7 @@ __global__ __launch_bounds__(256) void k_mom_apply(int n, Buffers S, const doubl
     S.vel[s] = v;
 }
 
-// state back to upload order in FP64
+// state back to upload order in FP64 (of x, u, v, f those that are not null)
 template <bool MULTI>
 __global__ __launch_bounds__(256) void k_gather(int n, Buffers S, const float4* __restrict__ frc,
                                                 const BoxDev* boxes, BoxDev B0, double* __restrict__ x,
@@ -640,32 +640,62 @@ __global__ __launch_bounds__(256) void k_gather(int n, Buffers S, const float4* 
 {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= n) return;
-    const float4 p = S.pos[s];
-    const BoxDev& B = box_of<MULTI>(boxes, B0, __float_as_int(p.w));
-    int c[3];
-    key_cell(S.key[s] - B.koff, B, c);
-    const int q = S.bead[s];
-    const int4 a = S.img[q];
-    const float4 vv = S.vel[s];
-    const float4 ff = frc[s];
-    const double o[3] = {p.x, p.y, p.z};
-    const int im[3] = {a.x, a.y, a.z};
-    for (int d = 0; d < 3; ++d) {
-        const double xa = (double)c[d] * B.wd[d] + o[d];
-        x[3 * q + d] = xa;
-        u[3 * q + d] = xa + (double)im[d] * (double)B.n[d] * B.wd[d];
+    const int64_t q = S.bead[s];
+    if (x || u) {
+        const float4 p = S.pos[s];
+        const BoxDev& B = box_of<MULTI>(boxes, B0, __float_as_int(p.w));
+        int c[3];
+        key_cell(S.key[s] - B.koff, B, c);
+        const int4 a = u ? S.img[q] : make_int4(0, 0, 0, 0);
+        const double o[3] = {p.x, p.y, p.z};
+        const int im[3] = {a.x, a.y, a.z};
+        for (int d = 0; d < 3; ++d) {
+            const double xa = (double)c[d] * B.wd[d] + o[d];
+            if (x) x[3 * q + d] = xa;
+            if (u) u[3 * q + d] = xa + (double)im[d] * (double)B.n[d] * B.wd[d];
+        }
     }
-    v[3 * q + 0] = vv.x; v[3 * q + 1] = vv.y; v[3 * q + 2] = vv.z;
-    f[3 * q + 0] = ff.x; f[3 * q + 1] = ff.y; f[3 * q + 2] = ff.z;
+    if (v) {
+        const float4 vv = S.vel[s];
+        v[3 * q + 0] = vv.x; v[3 * q + 1] = vv.y; v[3 * q + 2] = vv.z;
+    }
+    if (f) {
+        const float4 ff = frc[s];
+        f[3 * q + 0] = ff.x; f[3 * q + 1] = ff.y; f[3 * q + 2] = ff.z;
+    }
 }
 
-// clears the FP64 accumulators and error flags (a kernel rather than a memset, so that
-// it can sit inside a captured graph)
-__global__ void k_zero(double* acc, int nacc, int* flags, int nflags)
+// The end of a call: its flags and (with hacc) the sums of box blockIdx.x to page-locked host
+// memory, and both cleared for the next call (they are zero at rest, so that a call starts with
+// its first kernel and a captured graph needs no clearing).  What bounds it, and a call of few
+// steps: the host's round trip.  With two clearing launches before the steps and a copy to
+// pageable memory after them, a second one for the sums, a call of one step in a 37x23x29 box of
+// chains took 104 us, of which 48 were kernels; it takes 66.
+__global__ __launch_bounds__(64) void k_report(Sums S, int* __restrict__ flags, double* __restrict__ hacc,
+                                               int* __restrict__ hflags)
+{
+    const int t = threadIdx.x, i = t & (kObsStride - 1);
+    if (hacc) {
+        double* a = S.acc + (size_t)blockIdx.x * (S.spread + 1) * kObsStride;
+        double s = 0.0;
+        for (int r = t / kObsStride; r <= S.spread; r += 64 / kObsStride) {
+            s += a[r * kObsStride + i];
+            a[r * kObsStride + i] = 0.0;
+        }
+        s += __shfl_down(s, kObsStride, 64);
+        if (t < kObsStride) hacc[(size_t)blockIdx.x * kObsStride + i] = s;
+    }
+    if (blockIdx.x == 0 && t < 4) {
+        hflags[t] = flags[t];
+        flags[t] = 0;
+    }
+}
+
+// clears a table (a kernel rather than a memset, so that it can sit inside a captured graph)
+__global__ void k_zero(double* tab, int n)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < nacc) acc[i] = 0.0;
-    if (i < nflags) flags[i] = 0;
+    if (i < n) tab[i] = 0.0;
 }
 
 __global__ void k_set_step(int64_t* step, int64_t value)
@@ -707,6 +737,7 @@ struct dpd_engine {
     bool pair_auto = false;   // choose by bead count at each commit
     bool committed = false;
     // device buffers
+    char *per_box = nullptr, *per_bead = nullptr;   // what the arrays by box and by bead lie in
     BoxDev* dboxes = nullptr;
     float4 *pos[2] = {}, *vel[2] = {}, *fold[2] = {};
     int* bead[2] = {};
@@ -724,8 +755,10 @@ struct dpd_engine {
     int* cells = nullptr;
     size_t cleared = 0;   // ints of `cells` (cnt and counts) that are zero at rest
     int* flags = nullptr;
-    int64_t* dstep = nullptr;
-    double* acc = nullptr;
+    int64_t* dstep = nullptr;   // the simulation time, and that of dpd_compute_forces
+    double* acc = nullptr;      // Sums, zero at rest as the flags are
+    double* hacc = nullptr;     // page-locked: a call's sums per box, then its flags
+    int* hflags = nullptr;
     float* table = nullptr;
     double* gather = nullptr;   // 12n doubles for downloads
     double* slice = nullptr;    // slice stress tables (pair | bond)
@@ -778,6 +811,26 @@ int dalloc(dpd_engine* e, T** p, size_t count)
     if (count == 0) count = 1;
     hipError_t st = hipMalloc((void**)p, sizeof(T) * count);
     if (st != hipSuccess) return fail(e, DPD_ERR_OOM, std::string("hipMalloc: ") + hipGetErrorString(st));
+    return DPD_OK;
+}
+
+// several arrays in one allocation, each on a 256-byte boundary
+struct Part {
+    void** p;
+    size_t bytes;
+};
+template <class T>
+Part part(T** p, size_t count) { return {(void**)p, (sizeof(T) * count + 255) / 256 * 256}; }
+int dalloc_parts(dpd_engine* e, char** block, const std::vector<Part>& parts)
+{
+    size_t total = 0;
+    for (const Part& q : parts) total += q.bytes;
+    if (int rc = dalloc(e, block, total)) return rc;
+    char* at = *block;
+    for (const Part& q : parts) {
+        *q.p = at;
+        at += q.bytes;
+    }
     return DPD_OK;
 }
 
@@ -888,6 +941,11 @@ Topo topo(dpd_engine* e)
     return Topo{e->bonded, e->span, e->bond_ent, e->ang_ent, e->bond_par, e->ang_par, e->upos, e->bforce, e->nbonded};
 }
 
+inline Sums sums(const dpd_engine* e) { return Sums{e->acc, (int)e->boxes.size() <= kSpreadBoxes ? kSpread : 0}; }
+
+// where an evaluation beside the trajectory leaves its force (scratch between calls)
+inline float4* aside_force(dpd_engine* e) { return e->fold[e->cur ^ 1]; }
+
 inline int grid(int64_t n, int b) { return (int)((n + b - 1) / b); }
 inline bool multi(dpd_engine* e) { return e->boxes.size() > 1; }
 
@@ -951,8 +1009,9 @@ inline bool epilogue_ok(const dpd_engine* e) { return e->nbonded == 0 && epilogu
 // same launch (k_pair_hitlist_bonded); `bonded` then tells that they are done.
 // `epi` (epilogue_ok): the launch also closes the step and starts the next one (pair_epilogue).
 // `spills` false: the launch is repeated on one state, and what overfills the sort's bins is dropped.
+// `aside`: an evaluation beside the trajectory, force to aside_force(e), time from dstep[1].
 int launch_pair(dpd_engine* e, bool obs, bool* bonded = nullptr, bool epi = false, bool in_seq = false,
-                bool spills = true)
+                bool spills = true, bool aside = false)
 {
     if (bonded) *bonded = false;
     PairArgs a;
@@ -973,9 +1032,9 @@ int launch_pair(dpd_engine* e, bool obs, bool* bonded = nullptr, bool epi = fals
     a.code = S.code;
     a.cstart = e->cstart[e->cur];
     a.table = e->table;
-    a.step = e->dstep;
-    a.frc = e->frc;
-    a.acc = e->acc;
+    a.step = e->dstep + (aside ? 1 : 0);
+    a.frc = aside ? aside_force(e) : e->frc;
+    a.sums = sums(e);
     a.hitblk = e->hitblk[e->sched];
     a.nhitblk = e->nhitblk[e->sched];
     // one box only: a batch's pair kernel leaves no registers for the bonded terms (held to its 96
@@ -995,17 +1054,17 @@ int launch_pair(dpd_engine* e, bool obs, bool* bonded = nullptr, bool epi = fals
 }
 
 template <bool UPDATE_V, bool OBS>
-void launch_finish(dpd_engine* e)
+void launch_finish(dpd_engine* e, float4* frc)
 {
     const int n = (int)e->n;
     const BoxDev B0 = e->boxes[0].B;
     float4* keep = (UPDATE_V && vp_is_vel(e)) ? e->vp : nullptr;
     if (multi(e))
         hipLaunchKernelGGL((k_finish<UPDATE_V, OBS, true>), dim3(grid(n, 256)), dim3(256), 0, e->stream, n,
-                           bufs(e, e->cur), e->frc, topo(e), e->dboxes, B0, e->flags, e->acc, keep);
+                           bufs(e, e->cur), frc, topo(e), e->dboxes, B0, e->flags, sums(e), keep);
     else
         hipLaunchKernelGGL((k_finish<UPDATE_V, OBS, false>), dim3(grid(n, 256)), dim3(256), 0, e->stream, n,
-                           bufs(e, e->cur), e->frc, topo(e), e->dboxes, B0, e->flags, e->acc, keep);
+                           bufs(e, e->cur), frc, topo(e), e->dboxes, B0, e->flags, sums(e), keep);
 }
 
 // bonds and angles of this step, where the pair launch did not run them
@@ -1016,37 +1075,28 @@ void launch_bonded(dpd_engine* e)
     const dim3 gr(grid(e->nbonded, 256)), bl(256);
     const Buffers S = bufs(e, e->cur);
     const BoxDev B0 = e->boxes[0].B;
-    if (multi(e)) hipLaunchKernelGGL((k_bonded<OBS, true>), gr, bl, 0, e->stream, S, B0, topo(e), e->slot_of, e->acc);
-    else hipLaunchKernelGGL((k_bonded<OBS, false>), gr, bl, 0, e->stream, S, B0, topo(e), e->slot_of, e->acc);
+    if (multi(e)) hipLaunchKernelGGL((k_bonded<OBS, true>), gr, bl, 0, e->stream, S, B0, topo(e), e->slot_of, sums(e));
+    else hipLaunchKernelGGL((k_bonded<OBS, false>), gr, bl, 0, e->stream, S, B0, topo(e), e->slot_of, sums(e));
 }
 
-// clear the observable accumulators (and, when `flags`, the error flags)
-void launch_zero(dpd_engine* e, bool flags)
+// the end of a call: waits for it, takes its flags and (`obs`) its sums to hacc
+int report(dpd_engine* e, bool obs)
 {
-    const int nacc = (int)e->boxes.size() * kObsStride;
-    hipLaunchKernelGGL(k_zero, dim3(grid(std::max(nacc, 4), 256)), dim3(256), 0, e->stream, e->acc, nacc, e->flags,
-                       flags ? 4 : 0);
-}
-
-int read_flags(dpd_engine* e)
-{
-    int h[4];
-    HIPCHK(hipMemcpyAsync(h, e->flags, sizeof(h), hipMemcpyDeviceToHost, e->stream));
+    hipLaunchKernelGGL(k_report, dim3(obs ? e->boxes.size() : 1), dim3(64), 0, e->stream, sums(e), e->flags,
+                       obs ? e->hacc : nullptr, e->hflags);
+    HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(e->stream));
-    e->jumps += h[1];
-    if (h[0]) return fail(e, DPD_ERR_NAN, "non-finite force, velocity or position detected");
+    e->jumps += e->hflags[1];
+    if (e->hflags[0]) return fail(e, DPD_ERR_NAN, "non-finite force, velocity or position detected");
     return DPD_OK;
 }
 
 int finish_obs(dpd_engine* e)
 {
     const size_t nb = e->boxes.size();
-    std::vector<double> h(nb * kObsStride);
-    HIPCHK(hipMemcpyAsync(h.data(), e->acc, sizeof(double) * h.size(), hipMemcpyDeviceToHost, e->stream));
-    HIPCHK(hipStreamSynchronize(e->stream));
     e->obs.assign(nb, dpd_obs{});
     for (size_t b = 0; b < nb; ++b) {
-        const double* a = h.data() + b * kObsStride;
+        const double* a = e->hacc + b * kObsStride;
         const dpd_params& p = e->boxes[b].p;
         dpd_obs& o = e->obs[b];
         o.step = e->step;
@@ -1085,7 +1135,6 @@ inline int64_t timed_steps(int64_t nsteps, int timing)
 int enqueue_steps(dpd_engine* e, int64_t nsteps, bool obs, int timing)
 {
     int rc;
-    launch_zero(e, false);
     int64_t ti = 0;   // timed launches so far (event pair 2 ti, 2 ti + 1)
     bool advanced = false;   // the previous pair launch carried the step's epilogue
     for (int64_t t = 0; t < nsteps; ++t) {
@@ -1104,8 +1153,8 @@ int enqueue_steps(dpd_engine* e, int64_t nsteps, bool obs, int timing)
         }
         advanced = epi;
     }
-    if (obs) launch_finish<true, true>(e);
-    else launch_finish<true, false>(e);
+    if (obs) launch_finish<true, true>(e, e->frc);
+    else launch_finish<true, false>(e, e->frc);
     HIPCHK(hipGetLastError());
     return DPD_OK;
 }
@@ -1173,16 +1222,16 @@ int commit_beads(dpd_engine* e, int64_t step0)
         e->bins = reinterpret_cast<int*>(e->order + n);
     }
     if (n != e->n) {
+        std::vector<Part> parts;
         for (int b = 0; b < 2; ++b)
-            if ((rc = dalloc(e, &e->pos[b], n)) || (rc = dalloc(e, &e->vel[b], n)) ||
-                (rc = dalloc(e, &e->fold[b], n)) || (rc = dalloc(e, &e->bead[b], n)) ||
-                (rc = dalloc(e, &e->key[b], n)) || (rc = dalloc(e, &e->code[b], n + kCodePad)))
-                return rc;
-        if ((rc = dalloc(e, &e->img, n))) return rc;
+            for (const Part& q : {part(&e->pos[b], n), part(&e->vel[b], n), part(&e->fold[b], n), part(&e->bead[b], n),
+                                  part(&e->key[b], n), part(&e->code[b], n + kCodePad)})
+                parts.push_back(q);
+        for (const Part& q : {part(&e->img, n), part(&e->frc, n), part(&e->vp, n), part(&e->slot_of, n),
+                              part(&e->gather, 12 * n)})
+            parts.push_back(q);
+        if ((rc = dalloc_parts(e, &e->per_bead, parts))) return rc;
         for (int b = 0; b < 2; ++b) HIPCHK(hipMemsetAsync(e->code[b] + n, 0, sizeof(uint32_t) * kCodePad, e->stream));
-        if ((rc = dalloc(e, &e->frc, n)) || (rc = dalloc(e, &e->vp, n)) || (rc = dalloc(e, &e->slot_of, n)) ||
-            (rc = dalloc(e, &e->gather, 12 * n)))
-            return rc;
         e->n = n;
     }
     if ((rc = upload_boxes(e))) return rc;
@@ -1232,7 +1281,6 @@ int commit_beads(dpd_engine* e, int64_t step0)
     HIPCHK(hipMemcpyAsync(e->img, hi.data(), sizeof(int4) * n, hipMemcpyHostToDevice, e->stream));
     HIPCHK(hipMemcpyAsync(e->key[src], hk.data(), sizeof(int) * n, hipMemcpyHostToDevice, e->stream));
     HIPCHK(hipMemcpyAsync(e->cstart[src], hc.data(), sizeof(int) * hc.size(), hipMemcpyHostToDevice, e->stream));
-    launch_zero(e, true);
     if ((rc = sort_step<kRebin>(e))) return rc;
     hipLaunchKernelGGL(k_copy_force, dim3(grid(n, 256)), dim3(256), 0, e->stream, (int)n, e->fold[e->cur], e->frc);
     hipLaunchKernelGGL(k_set_step, dim3(1), dim3(64), 0, e->stream, e->dstep, step0);
@@ -1244,8 +1292,7 @@ int commit_beads(dpd_engine* e, int64_t step0)
     if (e->pair_auto) {
         set_schedule(e, default_schedule(e));
     }
-    HIPCHK(hipStreamSynchronize(e->stream));
-    return read_flags(e);
+    return report(e, false);
 }
 
 // Global CSR topology from the staged per-box bonds and bond pairs.
@@ -1528,12 +1575,15 @@ int dpd_create_batch(int32_t nbox, const dpd_params* p, dpd_engine** out)
     HIPCHK(hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking));
     for (auto& ev : e->ev) HIPCHK(hipEventCreate(&ev));
     if ((rc = dpd_set_pair_kernel(e, p[0].pair_kernel))) return rc;
-    if ((rc = dalloc(e, &e->flags, 4)) || (rc = dalloc(e, &e->dstep, 1)) ||
-        (rc = dalloc(e, &e->acc, (size_t)nbox * kObsStride)) || (rc = dalloc(e, &e->table, (size_t)nbox * kTableStride)) ||
-        (rc = dalloc(e, &e->dboxes, nbox)))
+    const size_t nacc = (size_t)nbox * (sums(e).spread + 1) * kObsStride;
+    if ((rc = dalloc_parts(e, &e->per_box, {part(&e->flags, 4), part(&e->dstep, 2), part(&e->acc, nacc),
+                                            part(&e->table, (size_t)nbox * kTableStride), part(&e->dboxes, nbox)})))
         return rc;
-    HIPCHK(hipMemsetAsync(e->flags, 0, sizeof(int) * 4, e->stream));
-    HIPCHK(hipMemsetAsync(e->dstep, 0, sizeof(int64_t), e->stream));
+    // (flags, times and sums)
+    HIPCHK(hipMemsetAsync(e->per_box, 0, (char*)e->table - e->per_box, e->stream));
+    const size_t nh = (size_t)nbox * kObsStride;
+    HIPCHK(hipHostMalloc((void**)&e->hacc, sizeof(double) * nh + sizeof(int) * 4, hipHostMallocDefault));
+    e->hflags = reinterpret_cast<int*>(e->hacc + nh);
     if ((rc = upload_tables(e))) return rc;
     e->err.clear();
     return DPD_OK;
@@ -1546,15 +1596,13 @@ void dpd_destroy(dpd_engine* e)
     if (!e) return;
     if (e->stream) (void)hipStreamSynchronize(e->stream);
     drop_graphs(e);
-    void* ptrs[] = {e->pos[0], e->pos[1], e->vel[0], e->vel[1], e->fold[0], e->fold[1], e->bead[0], e->bead[1], e->img,
-                    e->key[0], e->key[1], e->code[0], e->code[1], e->frc, e->vp, e->slot_of,
-                    e->cells, e->filed, e->flags, e->dstep, e->acc, e->table, e->gather, e->bond_ent,
-                    e->ang_ent, e->span, e->bond_par, e->ang_bead, e->ang_par, e->bond_bead,
-                    e->upos, e->bforce, e->bonded, e->dboxes, e->slice, e->madj};
+    void* ptrs[] = {e->per_box, e->per_bead, e->cells, e->filed, e->bond_ent, e->ang_ent, e->span, e->bond_par,
+                    e->ang_bead, e->ang_par, e->bond_bead, e->upos, e->bforce, e->bonded, e->slice, e->madj};
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
     for (void* q : e->hitblk)
         if (q) (void)hipFree(q);
+    if (e->hacc) (void)hipHostFree(e->hacc);
     for (auto& ev : e->ev)
         if (ev) (void)hipEventDestroy(ev);
     for (auto& ev : e->pev) (void)hipEventDestroy(ev);
@@ -1637,7 +1685,6 @@ int dpd_step(dpd_engine* e, int64_t nsteps, uint32_t flags)
             e->pev.push_back(ev);
         }
     }
-    launch_zero(e, true);
     HIPCHK(hipEventRecord(e->ev[0], e->stream));
     if (use_graph) {
         // whole calls of an even step count replay one captured graph: the two SoA buffers
@@ -1677,7 +1724,7 @@ int dpd_step(dpd_engine* e, int64_t nsteps, uint32_t flags)
         e->step += nsteps;
     }
     HIPCHK(hipEventRecord(e->ev[1], e->stream));
-    if ((rc = read_flags(e))) return rc;
+    if ((rc = report(e, obs))) return rc;
     float ms = 0.f;
     HIPCHK(hipEventElapsedTime(&ms, e->ev[0], e->ev[1]));
     e->t_total = ms;
@@ -1698,6 +1745,25 @@ int dpd_step(dpd_engine* e, int64_t nsteps, uint32_t flags)
     return DPD_OK;
 }
 
+}  // extern "C"
+
+namespace {
+
+void launch_gather(dpd_engine* e, const float4* frc, double* x, double* u, double* v, double* f)
+{
+    const int n = (int)e->n;
+    const dim3 gr(grid(n, 256)), bl(256);
+    const BoxDev B0 = e->boxes[0].B;
+    if (multi(e))
+        hipLaunchKernelGGL(k_gather<true>, gr, bl, 0, e->stream, n, bufs(e, e->cur), frc, e->dboxes, B0, x, u, v, f);
+    else
+        hipLaunchKernelGGL(k_gather<false>, gr, bl, 0, e->stream, n, bufs(e, e->cur), frc, e->dboxes, B0, x, u, v, f);
+}
+
+}  // namespace
+
+extern "C" {
+
 int dpd_compute_forces(dpd_engine* e, int64_t step, uint32_t flags, double* f_out, double* virial, double* pe)
 {
     if (!e) return DPD_ERR_PARAM;
@@ -1709,38 +1775,23 @@ int dpd_compute_forces(dpd_engine* e, int64_t step, uint32_t flags, double* f_ou
         for (auto& b : e->boxes) { saved.push_back(b.thermostat_on); b.thermostat_on = false; }
         if ((rc = upload_tables(e))) return rc;
     }
-    launch_zero(e, true);
-    // the force the next dpd_step starts from is kept aside (the inactive SoA buffers are
-    // scratch between calls) and restored below, so a diagnostic evaluation does not change
-    // the trajectory
-    const size_t f4 = sizeof(float4) * (size_t)e->n;
-    float4* keep = e->fold[e->cur ^ 1];
-    HIPCHK(hipMemcpyAsync(keep, e->frc, f4, hipMemcpyDeviceToDevice, e->stream));
-    hipLaunchKernelGGL(k_set_step, dim3(1), dim3(64), 0, e->stream, e->dstep, step);
+    // beside the trajectory: force and time of the next dpd_step stay as they are
+    hipLaunchKernelGGL(k_set_step, dim3(1), dim3(64), 0, e->stream, e->dstep + 1, step);
     // the uploaded state is sorted with vp = v: evaluate at it (after dpd_step, vp is the
     // last step's predicted velocity)
     bool terms_done = false;
-    if ((rc = launch_pair(e, true, &terms_done))) return rc;
+    if ((rc = launch_pair(e, true, &terms_done, false, false, true, true))) return rc;
     if (!terms_done) launch_bonded<true>(e);
-    launch_finish<false, true>(e);
+    launch_finish<false, false>(e, aside_force(e));
     HIPCHK(hipGetLastError());
-    if ((rc = read_flags(e))) return rc;
-    std::vector<double> h(e->boxes.size() * kObsStride);
-    HIPCHK(hipMemcpyAsync(h.data(), e->acc, sizeof(double) * h.size(), hipMemcpyDeviceToHost, e->stream));
-    const int n = (int)e->n;
+    double* g = e->gather;
+    if (f_out) launch_gather(e, aside_force(e), nullptr, nullptr, nullptr, g);
+    if ((rc = report(e, true))) return rc;
     if (f_out) {
-        double* g = e->gather;
-        if (multi(e))
-            hipLaunchKernelGGL(k_gather<true>, dim3(grid(n, 256)), dim3(256), 0, e->stream, n, bufs(e, e->cur), e->frc,
-                               e->dboxes, e->boxes[0].B, g, g + 3 * n, g + 6 * n, g + 9 * n);
-        else
-            hipLaunchKernelGGL(k_gather<false>, dim3(grid(n, 256)), dim3(256), 0, e->stream, n, bufs(e, e->cur),
-                               e->frc, e->dboxes, e->boxes[0].B, g, g + 3 * n, g + 6 * n, g + 9 * n);
-        HIPCHK(hipMemcpyAsync(f_out, g + 9 * n, sizeof(double) * 3 * n, hipMemcpyDeviceToHost, e->stream));
+        HIPCHK(hipMemcpyAsync(f_out, g, sizeof(double) * 3 * e->n, hipMemcpyDeviceToHost, e->stream));
+        HIPCHK(hipStreamSynchronize(e->stream));
     }
-    HIPCHK(hipMemcpyAsync(e->frc, keep, f4, hipMemcpyDeviceToDevice, e->stream));
-    hipLaunchKernelGGL(k_set_step, dim3(1), dim3(64), 0, e->stream, e->dstep, e->step);
-    HIPCHK(hipStreamSynchronize(e->stream));
+    const double* h = e->hacc;
     // totals over all boxes
     if (virial)
         for (int i = 0; i < 9; ++i) {
@@ -1776,14 +1827,9 @@ int dpd_download_box(dpd_engine* e, int32_t box, double* x, double* unpbc, doubl
     if (!e->committed) return fail(e, DPD_ERR_STATE, "no beads uploaded");
     if (box < -1 || box >= (int32_t)e->boxes.size()) return fail(e, DPD_ERR_PARAM, "box index out of range");
     HIPCHK(hipSetDevice(e->device));
-    const int n = (int)e->n;
+    const int64_t n = e->n;
     double* g = e->gather;
-    if (multi(e))
-        hipLaunchKernelGGL(k_gather<true>, dim3(grid(n, 256)), dim3(256), 0, e->stream, n, bufs(e, e->cur), e->frc,
-                           e->dboxes, e->boxes[0].B, g, g + 3 * n, g + 6 * n, g + 9 * n);
-    else
-        hipLaunchKernelGGL(k_gather<false>, dim3(grid(n, 256)), dim3(256), 0, e->stream, n, bufs(e, e->cur), e->frc,
-                           e->dboxes, e->boxes[0].B, g, g + 3 * n, g + 6 * n, g + 9 * n);
+    launch_gather(e, e->frc, x ? g : nullptr, unpbc ? g + 3 * n : nullptr, v ? g + 6 * n : nullptr, f ? g + 9 * n : nullptr);
     HIPCHK(hipGetLastError());
     const int64_t off = box < 0 ? 0 : e->boxes[box].bead_off;
     const int64_t cnt = box < 0 ? e->n : e->boxes[box].n;
@@ -1863,26 +1909,19 @@ int dpd_time_pair(dpd_engine* e, int32_t nlaunch, double* ms_per_launch)
     if (nlaunch < 1 || nlaunch > 100000) return fail(e, DPD_ERR_PARAM, "nlaunch must be in [1, 100000]");
     HIPCHK(hipSetDevice(e->device));
     int rc;
-    // the launches rewrite this step's pair force: the force the next step starts from is
-    // kept in the inactive SoA buffer (scratch between calls) and restored afterwards
-    const size_t f4 = sizeof(float4) * (size_t)e->n;
-    float4* keep = e->fold[e->cur ^ 1];
-    HIPCHK(hipMemcpyAsync(keep, e->frc, f4, hipMemcpyDeviceToDevice, e->stream));
     // the launch a step that another follows uses: with the epilogue where the schedule has
     // one, which also files the beads for the counting sort and may raise the flags (both
-    // restored below)
+    // cleared below)
     const bool epi = epilogue_ok(e);
-    int flags0[2] = {0, 0};
-    if (epi) HIPCHK(hipMemcpyAsync(flags0, e->flags, sizeof(flags0), hipMemcpyDeviceToHost, e->stream));
+    hipLaunchKernelGGL(k_set_step, dim3(1), dim3(64), 0, e->stream, e->dstep + 1, e->step);
     bool terms_done = false;
-    if ((rc = launch_pair(e, false, &terms_done, epi, false, false))) return rc;   // untimed first launch
+    if ((rc = launch_pair(e, false, &terms_done, epi, false, false, true))) return rc;   // untimed first launch
     HIPCHK(hipEventRecord(e->ev[0], e->stream));
     for (int32_t i = 0; i < nlaunch; ++i)
-        if ((rc = launch_pair(e, false, &terms_done, epi, false, false))) return rc;
+        if ((rc = launch_pair(e, false, &terms_done, epi, false, false, true))) return rc;
     HIPCHK(hipEventRecord(e->ev[1], e->stream));
-    HIPCHK(hipMemcpyAsync(e->frc, keep, f4, hipMemcpyDeviceToDevice, e->stream));
     if (epi) {
-        HIPCHK(hipMemcpyAsync(e->flags, flags0, sizeof(flags0), hipMemcpyHostToDevice, e->stream));
+        HIPCHK(hipMemsetAsync(e->flags, 0, sizeof(int) * 4, e->stream));
         if ((rc = clear_counts(e))) return rc;
     }
     HIPCHK(hipStreamSynchronize(e->stream));
@@ -2098,18 +2137,15 @@ int adjust_momenta(dpd_engine* e, int32_t box, bool renormalise)
     if (box < -1 || box >= nbox) return fail(e, DPD_ERR_PARAM, "box index out of range");
     HIPCHK(hipSetDevice(e->device));
     const int n = (int)e->n;
-    const int nacc = nbox * kObsStride;
-    hipLaunchKernelGGL(k_zero, dim3(grid(std::max(nacc, 4), 256)), dim3(256), 0, e->stream, e->acc, nacc, e->flags, 0);
-    if (multi(e)) hipLaunchKernelGGL(k_mom_sums<true>, dim3(grid(n, 256)), dim3(256), 0, e->stream, n, bufs(e, e->cur), e->acc);
-    else hipLaunchKernelGGL(k_mom_sums<false>, dim3(grid(n, 256)), dim3(256), 0, e->stream, n, bufs(e, e->cur), e->acc);
+    if (multi(e)) hipLaunchKernelGGL(k_mom_sums<true>, dim3(grid(n, 256)), dim3(256), 0, e->stream, n, bufs(e, e->cur), sums(e));
+    else hipLaunchKernelGGL(k_mom_sums<false>, dim3(grid(n, 256)), dim3(256), 0, e->stream, n, bufs(e, e->cur), sums(e));
     HIPCHK(hipGetLastError());
-    std::vector<double> h(nacc);
-    HIPCHK(hipMemcpyAsync(h.data(), e->acc, sizeof(double) * nacc, hipMemcpyDeviceToHost, e->stream));
-    HIPCHK(hipStreamSynchronize(e->stream));
+    int rc;
+    if ((rc = report(e, true))) return rc;
     std::vector<double4> adj(nbox, make_double4(0.0, 0.0, 0.0, 1.0));
     for (int b = 0; b < nbox; ++b) {
         if (box >= 0 && b != box) continue;
-        const double* a = h.data() + (size_t)b * kObsStride;
+        const double* a = e->hacc + (size_t)b * kObsStride;
         const double cnt = a[4];
         if (!(cnt > 0.0)) continue;
         if (renormalise) {
@@ -2121,7 +2157,6 @@ int adjust_momenta(dpd_engine* e, int32_t box, bool renormalise)
             adj[b] = make_double4(a[0] / cnt, a[1] / cnt, a[2] / cnt, 1.0);
         }
     }
-    int rc;
     if (!e->madj && (rc = dalloc(e, &e->madj, (size_t)nbox))) return rc;
     HIPCHK(hipMemcpyAsync(e->madj, adj.data(), sizeof(double4) * nbox, hipMemcpyHostToDevice, e->stream));
     if (multi(e)) hipLaunchKernelGGL(k_mom_apply<true>, dim3(grid(n, 256)), dim3(256), 0, e->stream, n, bufs(e, e->cur), e->madj);
@@ -2166,7 +2201,7 @@ int dpd_slice_stress_noalloc(dpd_engine* e, int32_t box, int32_t nslices, double
     // the scratch keeps the last call's tables: clear the part this call uses (a kernel,
     // not a memset node, so that the call may be captured)
     const int nclr = (int)(2 * ntab);
-    hipLaunchKernelGGL(k_zero, dim3(grid(std::max(nclr, 1), 256)), dim3(256), 0, e->stream, tab, nclr, e->flags, 0);
+    hipLaunchKernelGGL(k_zero, dim3(grid(std::max(nclr, 1), 256)), dim3(256), 0, e->stream, tab, nclr);
     HIPCHK(hipGetLastError());
     return slice_tables(e, box, nslices, tab, ntab, pair_out, bond_out);
 }

@@ -353,29 +353,46 @@ __device__ inline void file_bead(const Intake& I, int from, int to, int s, bool 
     }
 }
 
-// Add per-thread FP64 values v[0..N) into acc[box * kObsStride + base + i]: one
-// block-wide reduction for the threads of the block's first box, direct atomics for
-// threads of another box (only blocks straddling a box boundary have any).
+// Accumulators of a call's sums: each box has spread + 1 rows of kObsStride (spread + 1 a power
+// of two), of which a workgroup adds to one; k_report adds the rows up.  FP64 atomics on one
+// address take about 15 ns in turn: with one row the 10,368 workgroups of k_finish took 134 us in
+// a 96^3 box, 42 with sixteen.
+struct Sums {
+    double* acc;
+    int spread;
+};
+constexpr int kSpread = 15;   // (engines of up to kSpreadBoxes boxes; more share no rows anyway)
+constexpr int kSpreadBoxes = 16;
+
+// Add per-thread FP64 values v[0..N) to slots base .. base + N - 1 of the threads' boxes (< 0:
+// none): one block-wide reduction for the threads of the block's first box, then one
+// wavefront-wide for each other box (only blocks straddling a box boundary have any; an atomic
+// for each of their threads took such a block 50 us).
 template <int N, int WAVES = 4>
-__device__ inline void accumulate_boxes(const double (&v)[N], int box, int box0, int base, double* acc)
+__device__ inline void accumulate_boxes(const double (&v)[N], int box, int box0, int base, const Sums& S)
 {
     __shared__ double red[N][WAVES];   // workgroups of up to 64 * WAVES threads
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    const bool mine = box == box0;
+    auto row = [&](int b) { return S.acc + ((size_t)b * (S.spread + 1) + (blockIdx.x & S.spread)) * kObsStride + base; };
 #pragma unroll
     for (int i = 0; i < N; ++i) {
-        const double s = wave_sum(mine ? v[i] : 0.0);
+        const double s = wave_sum(box == box0 ? v[i] : 0.0);
         if (lane == 0) red[i][wid] = s;
     }
-    if (!mine && box >= 0)
-        for (int i = 0; i < N; ++i)
-            if (v[i] != 0.0) atomicAdd(acc + box * kObsStride + base + i, v[i]);
+    for (uint64_t todo = __ballot(box >= 0 && box != box0); todo;) {
+        const int b = __builtin_amdgcn_readlane(box, __builtin_ctzll(todo));
+        for (int i = 0; i < N; ++i) {
+            const double s = wave_sum(box == b ? v[i] : 0.0);
+            if (lane == 0 && s != 0.0) atomicAdd(row(b) + i, s);
+        }
+        todo &= ~__ballot(box == b);
+    }
     __syncthreads();
     if (threadIdx.x < N) {
         const int nw = (blockDim.x + 63) >> 6;
         double s = 0.0;
         for (int w = 0; w < nw; ++w) s += red[threadIdx.x][w];
-        atomicAdd(acc + box0 * kObsStride + base + threadIdx.x, s);
+        atomicAdd(row(box0) + threadIdx.x, s);
     }
 }
 

@@ -34,7 +34,7 @@ struct PairArgs {
     const float* table;    // per box: a | gamma | sqrt(gamma), kTypeStride each
     const int64_t* step;   // simulation time of this force evaluation (device)
     float4* frc;           // out: pair force per slot
-    double* acc;           // out (OBS): per box [6..14] virial sum dx_b F_a, [15] pair PE
+    Sums sums;             // out (OBS): per box [6..14] virial sum dx_b F_a, [15] pair PE
     const int4* hitblk;    // hit-list workgroups of a batch: (box, first slot, end slot)
     int nhitblk;
     // the epilogue of a step that another follows (hit-list kernels, engines without bonded
@@ -121,7 +121,7 @@ __global__ __launch_bounds__(256) void k_pair_fullshell(PairArgs A, BoxDev B0, i
     }
     if (OBS) {
         const int box0 = MULTI ? bead_box(__float_as_int(A.pos[blk * 256].w)) : 0;
-        accumulate_boxes<10>(vir, box, box0, kObsVir, A.acc);
+        accumulate_boxes<10>(vir, box, box0, kObsVir, A.sums);
     }
 }
 
@@ -544,7 +544,7 @@ __device__ __attribute__((always_inline)) inline void hitlist_body(const PairArg
     if (EPI) pair_epilogue(A, B, i, valid && part == 0, fx, fy, fz);
     if (OBS) {
         // (lanes without a bead too: they evaluate pairs of the wavefront's others)
-        accumulate_boxes<10, THREADS / 64>(vir, box, box, kObsVir, A.acc);
+        accumulate_boxes<10, THREADS / 64>(vir, box, box, kObsVir, A.sums);
     }
 }
 
