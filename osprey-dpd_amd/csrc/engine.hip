@@ -477,7 +477,7 @@ __global__ __launch_bounds__(256) void k_sort(int n, int ngroups, int per_xcd, B
                                        (double)bead_box(wd));
         }
         D.key[dst] = k;
-        D.code[dst] = scan_code(m.o, m.c[0], B);
+        D.code[dst] = scan_code(m.o, m.c, B);
         if (MODE == kRebin) {
             vp[dst] = v;
         } else {
@@ -1553,15 +1553,15 @@ int dpd_create_batch(int32_t nbox, const dpd_params* p, dpd_engine** out)
         B.wd[0] = p[b].wx; B.wd[1] = p[b].wy; B.wd[2] = p[b].wz;
         for (int d = 0; d < 3; ++d) B.w[d] = (float)B.wd[d];
         {
-            // the scan's cut-off 1 + m, m = 1.01 |w| / 256 + 1e-5 (code_dist2), in code units
+            // the scan's cut-off 1 + m (code_dist2) in code units
             float s2 = 0.f, umax = 0.f;
             for (int d = 0; d < 3; ++d) {
-                B.qinv[d] = 256.0f / B.w[d];
-                s2 += B.w[d] * B.w[d];
+                B.qinv[d] = (float)kCodeUnits / B.w[d];
+                s2 += B.w[d] * B.w[d] * (d == 1 ? 2.25f : 1.0f);
                 umax = std::max(umax, B.qinv[d]);
             }
-            const float tu = (1.0f + std::sqrt(s2) * (1.01f / 256.0f) + 1e-5f) * umax;
-            B.qthr = (int)(tu * tu) + 1;
+            const float tu = (1.0f + std::sqrt(s2) * (1.01f / kCodeUnits) + 1e-5f) * umax;
+            B.qthr = (int)(tu * tu) + 2;
         }
         B.ntypes = nt;
         B.seed0 = (uint32_t)p[b].seed;

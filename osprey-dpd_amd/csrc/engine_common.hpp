@@ -35,7 +35,7 @@ struct BoxDev {
     double wd[3];
     float dt, hdt, hdt2, lamdt;   // dt, dt/2, dt^2/2, lambda*dt
     float invrootdt;              // sqrt(24 kT / dt)
-    float qinv[3];                // 256 / w: scan-code units
+    float qinv[3];                // kCodeUnits / w: scan-code units
     int qthr;                     // square of the scan's widened cut-off in the smallest of them
     int ntypes;
     uint32_t seed0, seed1;        // key of the pair stream
@@ -155,18 +155,16 @@ __device__ inline float pair_scalar_t(float dr2, float dxdv, float a, float sgr,
     return (con + diss + rnd) * inv;
 }
 
-// Scan code of a bead: its offsets in the cell to 8 bits each, q = floor(256 o / w), with
-// byte 0 the x offset, byte 1 the cell's x index modulo 256, byte 2 the y offset and byte 3
-// the z offset.  The hit-list kernel tests candidates on these 4 bytes instead of the
-// 16-byte position: bytes 0-1 read as one 16-bit number give the x position along the row in
-// units of w/256 (mod 2^16), so a row of three cells is scanned as one range.  q is the floor
-// of the offset in units of w/256, so the offset lies in [q, q + 1) units.
-__device__ inline uint32_t scan_code(const float o[3], int cx, const BoxDev& B)
+// Scan code of a bead: its x, y and z in units of w / kCodeUnits, with the cell and modulo 256,
+// in bytes 0, 1 and 3, and a one in byte 2 (code_dist2).
+constexpr int kCodeUnits = 84;
+__device__ inline uint32_t scan_code(const float o[3], const int c[3], const BoxDev& B)
 {
     uint32_t q[3];
 #pragma unroll
-    for (int a = 0; a < 3; ++a) q[a] = (uint32_t)min(max((int)(o[a] * B.qinv[a]), 0), 255);
-    return q[0] | ((uint32_t)(cx & 0xFF) << 8) | (q[1] << 16) | (q[2] << 24);
+    for (int a = 0; a < 3; ++a)
+        q[a] = (uint32_t)(min(max((int)(o[a] * B.qinv[a]), 0), kCodeUnits - 1) + kCodeUnits * c[a]) & 0xFF;
+    return q[0] | (q[1] << 8) | (1u << 16) | (q[2] << 24);
 }
 
 // The integration arithmetic with its rounding fixed by explicit fused multiply-adds, so
@@ -195,7 +193,10 @@ __device__ inline void advance(const float o[3], const int c[3], const int img[3
     for (int a = 0; a < 3; ++a) {
         float x = o[a] + d[a];
         if (!(fabsf(x) < 1.0e6f)) { m.bad = 1; x = 0.0f; }
-        int s = (int)floorf(x / B.w[a]);
+        // cells moved, floor(x / w): the division's rounding changes nothing up to one cell either
+        // way (x - w and x + w are then what its corrections below would leave)
+        int s = x < 0.0f ? -1 : (x >= B.w[a] ? 1 : 0);
+        if (!(x >= -B.w[a] && x < 2.0f * B.w[a])) s = (int)floorf(x / B.w[a]);
         x = x - (float)s * B.w[a];
         if (x < 0.0f) { x += B.w[a]; s -= 1; }
         if (x >= B.w[a]) x = B.w[a] * 0.99999994f;

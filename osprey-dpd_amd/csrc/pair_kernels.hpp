@@ -134,17 +134,22 @@ __global__ __launch_bounds__(256) void k_pair_fullshell(PairArgs A, BoxDev B0, i
 // multiply-adds differently in the two code shapes, so the forces agree to ~1 ulp per term, not
 // bitwise.  Slots must fit in 26 bits.
 //
-// What bounds it: instruction issue (rocprofv3: VALU active 87% of the cycles, 41M wavefront
-// instructions on the condensate box of 64^3 cells), of which the scan is two thirds.  The scan
-// costs 42 VALU instructions per pass of four candidates: the codes of the next pass are loaded
-// into the same registers as soon as these are subtracted, the x image of a partner is left to
-// the evaluation (cell indices mod 4 in the beads' words), and a bead beside an x face goes on
-// to the cell across it within the row's loop, so the wavefront's other lanes do not wait for a
-// second one.  Pair launch, relaxed boxes, with 58 instructions per pass, a second loop at the
-// faces and lists evaluated lane by lane -> now: condensate 64^3 95 -> 80 us, water 96^3 332 ->
-// 263, binary 40^3 38 -> 31, bilayer 48x48x32 40 -> 31, 64 water/lipid replicas 141 -> 105.
-// (The z offsets in an array of their own, 38 instructions per pass, were slower: 89 us, the
-// second load; so were two passes per turn, 85 us.)
+// What bounds it: instruction issue (rocprofv3: VALU active 85% of the cycles, 36M wavefront
+// instructions on the condensate box of 64^3 cells), of which the scan is a third, the
+// evaluation of 14 listed partners a bead (12.6 are in range) two fifths.  The scan costs 29 VALU
+// instructions per pass of four candidates: positions modulo 256 in bytes need one subtraction
+// and one dot product each (code_dist2), the codes of the next pass are loaded into the same
+// registers as soon as these are subtracted, the x image of a partner is left to the evaluation
+// (cell indices mod 4 in the beads' words), and a bead beside an x face goes on to the cell
+// across it within the row's loop, so the wavefront's other lanes do not wait for a second one.
+// Pair launch, relaxed boxes, with 58 instructions per pass, a second loop at the faces and lists
+// evaluated lane by lane -> with 42 and lists evaluated together -> now: condensate 64^3
+// 95 -> 79.4 -> 77 us, water 96^3 332 -> 252 -> 248, binary 40^3 38 -> 29.4 -> 29.1, bilayer
+// 48x48x32 40 -> 31.0 -> 29.7, 64 water/lipid replicas 141 -> 102.6 -> 100.
+// Slower: the z offsets in an array of their own (38 instructions per pass but a second load,
+// 89 us on the condensate), two passes per turn (85), a wavefront's row of codes staged in LDS
+// (98, the look-ups of each row and fewer registers), lists of 20 for a sixth wavefront (84 for
+// the lists, 89 to 104 with the registers of six), lists of 29 beside a smaller table (76).
 // A schedule of the hit-list kernel: threads per workgroup, list entries per thread (4 B of
 // LDS each) and the flush threshold (after each row segment the wavefront evaluates its
 // lists together once any of them holds this many; FLUSH = CAP never flushes).
@@ -163,25 +168,26 @@ typedef __attribute__((address_space(3))) uint32_t lds_u32;
 typedef uint32_t code2_t __attribute__((ext_vector_type(2), aligned(4)));
 // four scan codes from one 4-byte-aligned 16-byte load
 typedef uint32_t code4_t __attribute__((ext_vector_type(4), aligned(4)));
-// two 16-bit integers in one register (v_pk_sub_i16, v_dot2_i32_i16)
 // cell starts: a row's four and two, from 4-byte-aligned loads
 typedef int int4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef int int2u __attribute__((ext_vector_type(2), aligned(4)));
 // entries of padding after the cell starts (a row's four are loaded at once)
 constexpr int kCstartPad = 4;
-typedef short short2_t __attribute__((ext_vector_type(2)));
 
-// The candidate test in integer code units (u = w / 256): |d|^2 from dx and dy as one packed
-// pair (one two-term dot product) and dz.  code_dxy: QXY holds the bead's x (with its cell
-// index, mod 2^16) and y in code units, floors of its position seen from the row as the codes
-// are floors of the candidates'; one v_perm_b32 gathers the candidate's x field and y byte.
-// Each axis is then within one unit of the true difference, so every pair inside the cut-off
-// passes |d| < (1 + m) / u with m = 1.01 |w| / 256 + 1e-5; the evaluation drops the rest.
-__device__ inline short2_t code_dxy(uint32_t cj, uint32_t QXY)
+// The candidate test in integer code units (u = w / kCodeUnits): the four bytes of code minus
+// code, as one 32-bit difference, squared and added by one v_dot4_i32_i8.  Bytes hold positions
+// modulo 256, so differences are right from -128 to 127, more than the cut-off's 84 to 88; the
+// largest of a neighbour, 168, reads as -88 (and in cells of unequal sides, whose cut-off is
+// wider in some units, one may pass that is not near: the evaluation drops it).  A borrow of x
+// lowers y by one; it lowers the one of byte 2 instead of z, which adds at most one to the sum.
+// Positions are floored, the bead's y half a unit lower: the difference is then within 1, 1.5
+// and 1 units of the true one, so every pair inside the cut-off passes |d| < (1 + m) / u with
+// m = 1.01 |(w_x, 1.5 w_y, w_z)| / kCodeUnits + 1e-5.
+__device__ inline int code_dist2(uint32_t cj, uint32_t Q)
 {
-    return __builtin_bit_cast(short2_t, QXY) - __builtin_bit_cast(short2_t, __builtin_amdgcn_perm(0u, cj, 0x0c020100u));
+    const int d = (int)(cj - Q);
+    return __builtin_amdgcn_sdot4(d, d, 0, true);
 }
-__device__ inline int code_dist2(short2_t d, int dz) { return __builtin_amdgcn_sdot2(d, d, __mul24(dz, dz), false); }
 // beads per workgroup of THREADS threads with SPLIT lanes per bead (21 per wavefront for 3,
 // 7 for 9; lane 63 idle)
 constexpr int hit_beads(int threads, int split) { return split == 1 ? threads : (threads / 64) * (63 / split); }
@@ -404,20 +410,23 @@ __device__ __attribute__((always_inline)) inline void hitlist_body(const PairArg
                 fz += __uint_as_float(at[2 * THREADS]);
             }
         };
-        // candidate test on the scan codes in integer code units (code_dist2): each axis of
-        // the tested difference is within one unit u_a = w_a / 256 of the true one, so the
-        // distance is within m = 1.01 |w| / 256 + 1e-5 of it and, with the sum of squares taken
-        // in units of the smallest u_a, every pair inside the cut-off passes
-        // sum d_a^2 < ((1 + m) / u_min)^2 = thr (exact for cubic cells, a wider superset for
-        // others); the evaluation drops the rest (the bead itself among them).
+        // candidate test on the scan codes (code_dist2) with the sum of squares taken in units of
+        // the smallest u_a: every pair inside the cut-off passes sum d_a^2 < thr
+        // = ((1 + m) / u_min)^2 + 2 (a wider superset for cells of unequal sides); the evaluation
+        // drops the rest (the bead itself among them).
         const int thr = B.qthr;
         const char* cbase = reinterpret_cast<const char*>(A.code);
         const char* sbase = reinterpret_cast<const char*>(A.cstart);
-        // the bead's position in code units, floored as the codes are: x with its cell index
-        // and y in one register, z apart.  A row dy, dz sees them 256 dy and 256 dz lower.
-        const int Qx = (int)floorf(pi.x * B.qinv[0]) + (c[0] << 8);
-        const uint32_t QXY0 = ((uint32_t)Qx & 0xFFFFu) | ((uint32_t)(int)floorf(pi.y * B.qinv[1]) << 16);
-        const int Qz0 = (int)floorf(pi.z * B.qinv[2]);
+        // the bead's own position as its neighbours' codes have theirs; a row across a periodic
+        // face sees it a box's length away
+        const int Qx = (int)floorf(pi.x * B.qinv[0]) + kCodeUnits * c[0];
+        const int Qy = (int)floorf(pi.y * B.qinv[1] - 0.5f) + kCodeUnits * c[1];
+        const int Qz = (int)floorf(pi.z * B.qinv[2]) + kCodeUnits * c[2];
+        auto code_of = [](int x, int y, int z) {
+            return (uint32_t)(x & 0xFF) | ((uint32_t)(y & 0xFF) << 8) | ((uint32_t)z << 24);
+        };
+        const uint32_t Q0 = code_of(Qx, Qy, Qz);
+        const bool faces = __ballot(c[1] == 0 || c[1] == B.n[1] - 1 || c[2] == 0 || c[2] == B.n[2] - 1) != 0;
         // A row's cells are consecutive keys: cells cx-1 .. cx+1 are one range of slots, or,
         // where the row wraps through the periodic x face, two cells and the one across the
         // face, a second segment of that lane.
@@ -431,7 +440,7 @@ __device__ __attribute__((always_inline)) inline void hitlist_body(const PairArg
         const int pe = xl ? key + nx - 1 : (edge ? key + 1 - nx : key);
         // code and x of the second segment: the cell across the face, at -1 or nx
         const uint32_t img = xl ? 1u : 2u;
-        const int qimg = (xl ? nx : -nx) << 8;
+        const int qimg = (xl ? nx : -nx) * kCodeUnits;
         // the neighbour rows of this lane: all nine, one z layer (SPLIT 3) or one row (SPLIT 9)
         constexpr int NR = 9 / SPLIT;
         auto row_key = [&](int r) {
@@ -455,8 +464,12 @@ __device__ __attribute__((always_inline)) inline void hitlist_body(const PairArg
             }
             const int krow = row_key(r);
             const uint32_t code = (uint32_t)((dy << 2) | (dz << 4)) << kHitSlotBits;
-            uint32_t QXY = QXY0 + ((uint32_t)(1 - dy) << 24);
-            const int Qz = Qz0 + ((1 - dz) << 8);
+            uint32_t Q = Q0;
+            if (faces) {
+                const int sy = dy == 0 ? (c[1] == 0 ? B.n[1] : 0) : (dy == 2 && c[1] == B.n[1] - 1 ? -B.n[1] : 0);
+                const int sz = dz == 0 ? (c[2] == 0 ? B.n[2] : 0) : (dz == 2 && c[2] == B.n[2] - 1 ? -B.n[2] : 0);
+                Q = code_of(Qx, Qy + kCodeUnits * sy, Qz + kCodeUnits * sz);
+            }
             // list entries of the segment's first candidate and of its end
             uint32_t e = (uint32_t)j0 | code, e1 = valid ? (uint32_t)j1 | code : e;
             uint32_t jb = (uint32_t)j0 << 2;
@@ -475,18 +488,14 @@ __device__ __attribute__((always_inline)) inline void hitlist_body(const PairArg
             };
             // one pass
             auto pass = [&]() {
-                short2_t d[PASS];
-                int z[PASS];
+                int d2[PASS];
 #pragma unroll
-                for (int k = 0; k < PASS; ++k) {
-                    d[k] = code_dxy(cc[k], QXY);
-                    z[k] = Qz - (int)(cc[k] >> 24);
-                }
+                for (int k = 0; k < PASS; ++k) d2[k] = code_dist2(cc[k], Q);
                 jb += 4 * PASS;
                 cc = codes_at(jb);
-                put(code_dist2(d[0], z[0]), e, true);
+                put(d2[0], e, true);
 #pragma unroll
-                for (int k = 1; k < PASS; ++k) put(code_dist2(d[k], z[k]), e + k, e + k < e1);
+                for (int k = 1; k < PASS; ++k) put(d2[k], e + k, e + k < e1);
                 e += PASS;
             };
             const uint32_t full = laddr + 4 * (CAP - PASS) * THREADS;   // no room for a pass beyond
@@ -502,7 +511,7 @@ __device__ __attribute__((always_inline)) inline void hitlist_body(const PairArg
                             e = (uint32_t)ce.x | code | (img << kHitSlotBits);
                             e1 = (uint32_t)ce.y | code | (img << kHitSlotBits);
                             jb = (uint32_t)ce.x << 2;
-                            QXY = (QXY & 0xFFFF0000u) | (uint32_t)((Qx + qimg) & 0xFFFF);
+                            Q = (Q & 0xFFFFFF00u) | (uint32_t)((Qx + qimg) & 0xFF);
                             if (e >= e1) break;
                             cc = codes_at(jb);
                         }
@@ -549,9 +558,9 @@ __device__ __attribute__((always_inline)) inline void hitlist_body(const PairArg
 }
 
 // Wavefronts per SIMD that the LDS of a schedule allows (160 KB per CU, four SIMDs), at most
-// 5: the kernel needs 92 VGPRs (96 with the epilogue), and held to the 80 of six wavefronts it
-// spills (condensate 64^3: 123 us against 80 us per launch for 512 and 256 threads with 24
-// entries).  512-thread workgroups then fit twice, four wavefronts per SIMD.
+// 5: the kernel needs 92 VGPRs (96 with the epilogue, 12 bytes of them spilled: 248 us on water 96^3
+// against 281 with four wavefronts), and held to the 80 of six it spills more (condensate 64^3:
+// 123 us against 80 us per launch for 512 and 256 threads with 24 entries).  512-thread workgroups then fit twice, four wavefronts per SIMD.
 constexpr int hit_waves(int threads, int cap)
 {
     const int lds = cap * threads * 4 + kTypeStride * 16 + 64 * 16;
