@@ -246,50 +246,72 @@ __global__ __launch_bounds__(256) void k_set_bonded_flag(Topo T, const int* __re
 // kEndBegin also adds the previous step's bond and angle forces of bonded beads (flagged in
 // pos.w) to their pair force, in place: within a sequence of steps the bonded sum of every
 // step but the last is left to the next step's k_advance (the last one's to k_finish).
-template <int MODE, bool MULTI>
-__global__ __launch_bounds__(256) void k_advance(int n, Buffers S, float4* __restrict__ frc, Topo T,
+// What bounds it: latency (the bead, its bonded sum, the cells' starts and counts one after the
+// other), and with more wavefronts than the chip holds, its rounds.  Workgroups are dealt to the
+// XCDs as the pair launch and k_sort deal them (48x48x32 bilayer 47.2 -> 46.3 us a step, a
+// 37x23x29 box of chains 32.5 -> 31.4), and a thread takes BEADS = 2 beads, loaded together, in
+// engines of more than kAdvanceOnce beads (condensate 64^3 113.7 -> 111.1, 64 replicas 161.5 ->
+// 160.3; the chains' 74,000 beads, which one round holds, 32.5 -> 33.3).
+constexpr int kAdvanceOnce = 8192 * 64;
+template <int MODE, bool MULTI, int BEADS>
+__global__ __launch_bounds__(256) void k_advance(int n, int per_xcd, Buffers S, float4* __restrict__ frc, Topo T,
                                                  const BoxDev* boxes,
                                                  BoxDev B0, Intake I, int* __restrict__ flags)
 {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool active = s < n;
-    const int from = S.key[min(s, n - 1)];
-    int k = 0;
-    if (active) {
-        const float4 p = S.pos[s];
-        const BoxDev& B = box_of<MULTI>(boxes, B0, __float_as_int(p.w));
-        float4 v = S.vel[s];
-        float4 f = (MODE == kRebin) ? S.fold[s] : frc[s];
-        if (MODE == kEndBegin && (__float_as_int(p.w) & kBondedBit)) {
-            const float4 b = T.force[s];
-            f.x += b.x; f.y += b.y; f.z += b.z;
-            frc[s] = f;
-        }
-        if (MODE == kEndBegin) {
-            // UpdateMom: the stored velocity is v + dt/2 F_old; k_sort repeats this sum
-            v.x = kick(v.x, f.x, B.hdt);
-            v.y = kick(v.y, f.y, B.hdt);
-            v.z = kick(v.z, f.z, B.hdt);
-            if (!(fabsf(f.x) + fabsf(f.y) + fabsf(f.z) < 1e30f) || !(fabsf(v.x) + fabsf(v.y) + fabsf(v.z) < 1e30f))
-                atomicAdd(flags + 0, 1);
-        }
-        int c[3];
-        key_cell(from - B.koff, B, c);
-        const float o[3] = {p.x, p.y, p.z};
-        const int img[3] = {0, 0, 0};   // the image change is applied by k_sort
-        float d[3] = {0.f, 0.f, 0.f};
-        if (MODE != kRebin) {
-            d[0] = drift(v.x, f.x, B);
-            d[1] = drift(v.y, f.y, B);
-            d[2] = drift(v.z, f.z, B);
-        }
-        Moved m;
-        advance(o, c, img, d, B, m);
-        k = B.koff + cell_key(m.c[0], m.c[1], m.c[2], B);
-        if (m.jump) atomicAdd(flags + 1, 1);
-        if (m.bad) atomicAdd(flags + 0, 1);
+    const int s0 = ((blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3)) * 256 * BEADS;
+    if (s0 >= n) return;
+    float4 P[BEADS], V[BEADS], F[BEADS];
+    int key[BEADS];
+#pragma unroll
+    for (int u = 0; u < BEADS; ++u) {
+        const int s = min(s0 + 256 * u + (int)threadIdx.x, n - 1);
+        P[u] = S.pos[s];
+        V[u] = S.vel[s];
+        F[u] = (MODE == kRebin) ? S.fold[s] : frc[s];
+        key[u] = S.key[s];
     }
-    file_bead(I, from, k, s, active);
+#pragma unroll
+    for (int u = 0; u < BEADS; ++u) {
+        const int s = s0 + 256 * u + (int)threadIdx.x;
+        const bool active = s < n;
+        const int from = key[u];
+        int k = 0;
+        if (active) {
+            const float4 p = P[u];
+            const BoxDev& B = box_of<MULTI>(boxes, B0, __float_as_int(p.w));
+            float4 v = V[u];
+            float4 f = F[u];
+            if (MODE == kEndBegin && (__float_as_int(p.w) & kBondedBit)) {
+                const float4 b = T.force[s];
+                f.x += b.x; f.y += b.y; f.z += b.z;
+                frc[s] = f;
+            }
+            if (MODE == kEndBegin) {
+                // UpdateMom: the stored velocity is v + dt/2 F_old; k_sort repeats this sum
+                v.x = kick(v.x, f.x, B.hdt);
+                v.y = kick(v.y, f.y, B.hdt);
+                v.z = kick(v.z, f.z, B.hdt);
+                if (!(fabsf(f.x) + fabsf(f.y) + fabsf(f.z) < 1e30f) || !(fabsf(v.x) + fabsf(v.y) + fabsf(v.z) < 1e30f))
+                    atomicAdd(flags + 0, 1);
+            }
+            int c[3];
+            key_cell(from - B.koff, B, c);
+            const float o[3] = {p.x, p.y, p.z};
+            const int img[3] = {0, 0, 0};   // the image change is applied by k_sort
+            float d[3] = {0.f, 0.f, 0.f};
+            if (MODE != kRebin) {
+                d[0] = drift(v.x, f.x, B);
+                d[1] = drift(v.y, f.y, B);
+                d[2] = drift(v.z, f.z, B);
+            }
+            Moved m;
+            advance(o, c, img, d, B, m);
+            k = B.koff + cell_key(m.c[0], m.c[1], m.c[2], B);
+            if (m.jump) atomicAdd(flags + 1, 1);
+            if (m.bad) atomicAdd(flags + 0, 1);
+        }
+        file_bead(I, from, k, s, active);
+    }
 }
 
 // Exclusive scan of in[0, m) into out, in[] cleared, by one workgroup of 1024 threads: in
@@ -963,6 +985,14 @@ int clear_counts(dpd_engine* e)
     return DPD_OK;
 }
 
+template <int MODE, bool MULTI, int BEADS>
+void launch_advance(dpd_engine* e, const Buffers& S, const Intake& I)
+{
+    const int n = (int)e->n, per = grid(n, 8 * 256 * BEADS);
+    hipLaunchKernelGGL((k_advance<MODE, MULTI, BEADS>), dim3(8 * per), dim3(256), 0, e->stream, n, per, S, e->frc,
+                       topo(e), e->dboxes, e->boxes[0].B, I, e->flags);
+}
+
 // counting sort of buffer `cur` into buffer `cur^1`; MODE decides the move.  `advanced`: the
 // previous pair launch's epilogue already closed the step and filed the beads (MODE kEndBegin
 // only), so k_advance is left out.
@@ -978,8 +1008,7 @@ void sort_step_t(dpd_engine* e, bool advanced)
     const BoxDev B0 = e->boxes[0].B;
     const Intake I = intake(e);
     if (!advanced)
-        hipLaunchKernelGGL((k_advance<MODE, MULTI>), dim3(grid(n, 256)), dim3(256), 0, e->stream, n, S, e->frc,
-                           topo(e), e->dboxes, B0, I, e->flags);
+        n > kAdvanceOnce ? launch_advance<MODE, MULTI, 2>(e, S, I) : launch_advance<MODE, MULTI, 1>(e, S, I);
     const bool scan = e->ngroups > kDirectGroups;
     if (scan) hipLaunchKernelGGL(k_group_scan, dim3(1), dim3(1024), 0, e->stream, e->ngroups, I.gcnt, e->gstart);
     const int per = grid(e->ngroups, 8);

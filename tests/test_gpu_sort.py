@@ -67,3 +67,25 @@ def test_graphs_after_an_odd_number_of_steps():
         out.append(e.download())
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("n", [8192 * 64, 8192 * 64 + 1, 8192 * 64 + 257])
+def test_two_beads_a_thread(n):
+    """Engines of more beads than the chip's wavefronts hold take two beads a thread in
+    k_advance (every step's, with the full-shell kernel): at the line and one bead and one
+    workgroup past it."""
+    cells = (64, 56, 52)
+    print("two beads", n, flush=True)
+    ids, t, x, v = random_state(cells, n, 2, seed=n)
+    L = np.array(cells, dtype=float)
+    e = D.Engine(cells, A2, G2, dt=DT, seed=3, pair_kernel=D.PAIR_FULLSHELL)
+    e.upload(ids, t, x, v)
+    e.step(3)
+    X, U, V, _ = e.download()
+    # weak forces: three steps of free flight but for some 1e-3 of a cell
+    off = (X - x - 3 * DT * v + L / 2) % L - L / 2
+    assert np.abs(off).max() < 0.01 and np.abs(U - x - 3 * DT * v).max() < 0.01
+    f, _, _ = e.compute_forces(step=7, thermostat=False)
+    fresh = D.Engine(cells, A2, G2, dt=DT, seed=3, pair_kernel=D.PAIR_FULLSHELL)
+    fresh.upload(ids, t, X, V, unpbc=U)
+    assert np.array_equal(f, fresh.compute_forces(step=7, thermostat=False)[0])
