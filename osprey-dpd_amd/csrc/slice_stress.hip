@@ -15,7 +15,10 @@
 // pairs in a window of the slices that one layer of cells reaches (a workgroup takes slots of
 // one z layer at a time, and the slots are sorted by z), bonds and bond pairs in windows of
 // the whole table.  Bilayer 48x48x32, 221k beads, 64 slices (global atomics per pair and bond
-// -> now): pairs 13,700 -> 177 us, bonds 715 -> 15, bond pairs 1,767 -> 28.
+// -> now): pairs 13,700 -> 80 us, bonds 715 -> 15, bond pairs 1,767 -> 28.  The atomics are
+// then 30 us of the pairs; the rest is their scan and evaluation, with few wavefronts to hide a
+// load (177 us with one position loaded at a time and lists of 12 that a lane evaluated alone
+// whenever they were full).
 #include <algorithm>
 #include <cmath>
 
@@ -77,13 +80,18 @@ __device__ inline double wrapped_z(const SliceArgs& A, int slot)
 // pairs) of the slices from s0 on, lane l adding to copy l mod copies.  The sums of types ti <= tj
 // go to their components a <= b of out; k_slice_mirror spreads them afterwards.  Without WIN
 // (no window fits LDS) the pairs add to out themselves.
-constexpr int kSliceList = 12;   // listed partners per thread
-template <bool WIN>
+// LIST: listed partners per thread; when one of the lanes that scan has no room for four more,
+// they evaluate their lists together.  28 where they fit 64 KB beside the window, else 12 (a
+// call on the 48x48x32 bilayer with 64 slices, and one of 48x40x20 with 250: 108 and 151 us,
+// with 12 127 and 192; with 28 a lane alone 105 and 148, but 353 with 12).
+constexpr int kSliceListLong = 28, kSliceListShort = 12;
+constexpr size_t slice_list_bytes(int list) { return (size_t)list * 256 * (sizeof(int) + 1); }
+template <bool WIN, int LIST>
 __global__ __launch_bounds__(256) void k_slice_pairs(SliceArgs A, double* __restrict__ out, int per, int win, int copies)
 {
     extern __shared__ double lt[];
-    __shared__ int list[kSliceList][256];         // partner slots
-    __shared__ uint8_t row[kSliceList][256];      // and their row and image codes
+    __shared__ int list[LIST][256];         // partner slots
+    __shared__ uint8_t row[LIST][256];      // and their row and image codes
     const BoxDev& B = A.B;
     const int t = threadIdx.x;
     const int ntri = A.ntypes * (A.ntypes + 1) / 2, tab = win * ntri * 6, stride = tab + 1;
@@ -164,13 +172,19 @@ __global__ __launch_bounds__(256) void k_slice_pairs(SliceArgs A, double* __rest
                 n = 0;
             };
             auto scan = [&](int j0, int j1, int im, int dy, int dz) {
-                for (int j = j0; j < j1; ++j) {
-                    float d[3];
-                    const float dr2 = separation(A.pos[j], im, dy, dz, d);
-                    if (dr2 < 1.0f && dr2 > 1e-18f) {
-                        if (n == kSliceList) evaluate();
-                        list[n][t] = j;
-                        row[n++][t] = (uint8_t)(im | ((dy + 1) << 2) | (dz << 4));
+                for (int j = j0; j < j1; j += 4) {
+                    float4 p[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) p[u] = A.pos[min(j + u, j1 - 1)];
+                    if (__any(n > LIST - 4)) evaluate();
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        float d[3];
+                        const float dr2 = separation(p[u], im, dy, dz, d);
+                        if (j + u < j1 && dr2 < 1.0f && dr2 > 1e-18f) {
+                            list[n][t] = j + u;
+                            row[n++][t] = (uint8_t)(im | ((dy + 1) << 2) | (dz << 4));
+                        }
                     }
                 }
             };
@@ -475,11 +489,14 @@ hipError_t launch_slice_stress(const SliceArgs& a, double* pair_tab, double* bon
         const int nb = std::max(1, a.nbeads);
         // whole 256s of slots per workgroup, about kSliceBlocks workgroups
         const int per = (nb + kSliceBlocks * 256 - 1) / (kSliceBlocks * 256) * 256;
-        if (tab * sizeof(double) <= kSliceLdsBytes)
-            hipLaunchKernelGGL(k_slice_pairs<true>, dim3((nb + per - 1) / per), dim3(256), copies * tab * sizeof(double),
-                               s, a, pair_tab, per, win, copies);
+        const dim3 gr((nb + per - 1) / per), bl(256);
+        const size_t lds = copies * tab * sizeof(double);
+        if (tab * sizeof(double) > kSliceLdsBytes)
+            hipLaunchKernelGGL((k_slice_pairs<false, kSliceListLong>), gr, bl, 0, s, a, pair_tab, per, 0, 1);
+        else if (lds + slice_list_bytes(kSliceListLong) <= 65536)
+            hipLaunchKernelGGL((k_slice_pairs<true, kSliceListLong>), gr, bl, lds, s, a, pair_tab, per, win, copies);
         else
-            hipLaunchKernelGGL(k_slice_pairs<false>, dim3((nb + per - 1) / per), dim3(256), 0, s, a, pair_tab, per, 0, 1);
+            hipLaunchKernelGGL((k_slice_pairs<true, kSliceListShort>), gr, bl, lds, s, a, pair_tab, per, win, copies);
         hipLaunchKernelGGL(k_slice_mirror, dim3((unsigned)(((size_t)a.nslice * a.nidx + 255) / 256)), dim3(256), 0, s, a,
                            pair_tab);
     }

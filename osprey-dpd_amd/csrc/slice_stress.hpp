@@ -32,7 +32,7 @@ struct SliceArgs {
 // atomics
 constexpr size_t kSliceLdsBytes = 49152;
 // the pair window is repeated in LDS up to this size, for fewer lanes on one address
-constexpr size_t kSliceCopyBytes = 32768;
+constexpr size_t kSliceCopyBytes = 16384;
 // workgroups of the pair pass (each adds its window to the table once per z layer it touches;
 // 512, 1024, 2048 of them: 230, 198, 196 us a call on the 48x48x32 bilayer)
 // and of the bonded tables per window

@@ -44,3 +44,28 @@ def test_tables_match_the_oracle(cells, nt, n, nslices):
                                                ((bp, O.slice_stress_bondpairs(box, ids, t, x, nslices, unpbc=u, topo=topo)),)):
         assert np.linalg.norm(got - ref) <= 1e-5 * np.linalg.norm(ref)
         assert np.abs(got.sum(0) - ref.sum(0)).max() <= 1e-5 * np.abs(ref.sum(0)).max()
+
+
+@pytest.mark.parametrize("nslices", [6, 560, 6000], ids=["long-lists", "short-lists", "no-window"])
+def test_lists_that_overflow(nslices):
+    """A clump of 600 beads in two cells beside the x face (some 150 partners a bead in the half
+    shell, where a list holds 28 or 12) in a box that is thin elsewhere, with a window beside
+    which the long lists fit, one beside which only the short do, and none."""
+    cells, n = (6, 5, 8), 900
+    rng = np.random.default_rng(3)
+    L = np.array(cells, float)
+    x = rng.uniform(0, 1, (n, 3)) * L
+    x[:600] = (np.array([5.2, 2.1, 3.6]) + rng.uniform(0, 1, (600, 3)) * [1.2, 0.8, 0.9]) % L
+    t = rng.integers(0, 3, n).astype(np.int32)
+    v = rng.normal(0, 1, (n, 3))
+    a = np.array([[25.0, 30.0, 40.0], [30.0, 20.0, 35.0], [40.0, 35.0, 15.0]])
+    g = np.full((3, 3), 4.5)
+    ids = np.arange(1, n + 1, dtype=np.int32)
+    print("lists", nslices, flush=True)
+    e = D.Engine(cells, a, g, seed=9)
+    e.upload(ids, t, x, v)
+    pair, _ = e.slice_stress(nslices)
+    pr, _ = O.slice_stress(O.Box(cells, a, g, seed=9), ids, t, x, v, 0, nslices)
+    pr = pr.reshape(nslices, 3, 3, 9)
+    pr = (0.5 * (pr + pr.transpose(0, 2, 1, 3))).reshape(nslices, 9, 9)
+    assert np.linalg.norm(pair - pr) <= 1e-5 * np.linalg.norm(pr)
