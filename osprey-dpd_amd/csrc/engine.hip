@@ -887,7 +887,13 @@ void set_schedule(dpd_engine* e, int s)
 // fit the 26-bit list entries, the full-shell kernel beyond
 int default_schedule(const dpd_engine* e)
 {
-    return e->n <= (int64_t)kHitSlotMask ? size_schedule(e->n) : kFullShellSchedule;
+    return e->n <= (int64_t)kHitSlotMask ? size_schedule(e->n, e->nbonded > 0) : kFullShellSchedule;
+}
+
+// the automatic choice again, where the beads or the topology have changed
+void auto_schedule(dpd_engine* e)
+{
+    if (e->pair_auto) set_schedule(e, default_schedule(e));
 }
 
 void set_step_constants(BoxHost& b)
@@ -1318,9 +1324,7 @@ int commit_beads(dpd_engine* e, int64_t step0)
     e->jumps = 0;
     e->obs_valid = false;
     e->committed = true;
-    if (e->pair_auto) {
-        set_schedule(e, default_schedule(e));
-    }
+    auto_schedule(e);
     return report(e, false);
 }
 
@@ -1413,6 +1417,7 @@ int commit_topology(dpd_engine* e)
     e->nbonded = (int)nb;
     hipLaunchKernelGGL(k_clear_bonded_flag, dim3(grid(n, 256)), dim3(256), 0, e->stream, (int)n, e->pos[e->cur],
                        e->bead[e->cur], e->slot_of);
+    auto_schedule(e);
     mark_bonded(e);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(e->stream));
@@ -1651,6 +1656,7 @@ int dpd_upload_beads(dpd_engine* e, int64_t n, const int32_t* id, const int32_t*
     if ((rc = commit_beads(e, step0))) return rc;
     if (keep_topo) return commit_topology(e);
     e->nbonds = e->nangles = e->nbonded = 0;
+    auto_schedule(e);
     return DPD_OK;
 }
 
@@ -1971,7 +1977,7 @@ int dpd_set_pair_kernel(dpd_engine* e, int32_t kernel)
     if (e->pair_auto) set_schedule(e, e->committed ? default_schedule(e) : kFullShellSchedule);
     else if (kernel == DPD_PAIR_FULLSHELL) set_schedule(e, kFullShellSchedule);
     else if (kSchedule[e->sched].kernel != DPD_PAIR_HITLIST)
-        set_schedule(e, e->committed ? size_schedule(e->n) : kDefaultSchedule);
+        set_schedule(e, e->committed ? size_schedule(e->n, e->nbonded > 0) : kDefaultSchedule);
     return DPD_OK;
 }
 
@@ -2122,7 +2128,7 @@ int tune_trials(dpd_engine* e, int32_t nsteps, const std::vector<int>& trials, d
 int dpd_autotune(dpd_engine* e, int32_t nsteps, int32_t* chosen, double* ms_per_step)
 {
     if (!e) return DPD_ERR_PARAM;
-    const int hit = size_schedule(e->n);
+    const int hit = size_schedule(e->n, e->nbonded > 0);
     const std::vector<int> trials = {hit, kFullShellSchedule};
     double ms[2] = {0.0, 0.0};
     int best = 0;

@@ -601,12 +601,18 @@ constexpr Schedule kSchedule[kSchedules] = {
     {DPD_PAIR_HITLIST, 256, 8, 8, 9, "hitlist-split9-t256-c8"},
 };
 constexpr int kDefaultSchedule = 2;
-// The automatic choice for n beads: nine lanes per bead while one thread per bead would leave
-// most of the 1024 SIMDs without a wavefront, three lanes while it would leave them one or two,
-// then one (microseconds per step at 9, 3 and 1 lanes, density 3: chains 24.0k beads 28.6, 32.5,
-// 40.1; 41k 34.1, 35.6, 42.9; 66k 37.7, 37.4, 42.6; 98k 47.3, 43.5, 45.6; 140k 55.8, 52.8, 50.2;
-// water 5.2k 21.9, 25.6, 34.9; 41k 33.7, 32.2, 39.5; 98k 48.1, 39.0, 40.6; 140k 58.9, 49.7, 44.9).
-constexpr int size_schedule(int64_t n) { return n <= 45000 ? 6 : (n <= 105000 ? 5 : kDefaultSchedule); }
+// The automatic choice for n beads.  Nine lanes per bead while that leaves most of the 1024
+// SIMDs a wavefront or two; fewer beads of an engine without bonded terms, whose launch also
+// files the beads, by atomics for seven beads a wavefront.  Three lanes while their wavefronts
+// fit the SIMDs at once (four each); one with the longest lists while its do, then one with a
+// fifth wavefront.  Microseconds per step at 9, 3, 1 (lists of 32) and 1 (of 24) lanes, density 3:
+// water 10.1k beads 19.9, 20.5; 12.3k 21.8, 20.8; 98k 41.2, 31.8, 32.0; 108k 43, 38.0, 31.9,
+// 32.8; 256k -, -, 42.0, 42.8; 273k -, -, 54.7, 47.0; chains 41k 24.5, 25.8; 66k 31.1, 30.1;
+// 89k 37, 34.0, 35.7; 118k 43, 41.3, 36.7; 256k -, -, 47.0, 49.0; 292k -, -, 59.6, 52.3.
+constexpr int size_schedule(int64_t n, bool bonded)
+{
+    return n <= (bonded ? 50000 : 11000) ? 6 : (n <= 100000 ? 5 : (n <= 4 * 1024 * 64 ? 3 : kDefaultSchedule));
+}
 constexpr int kFullShellSchedule = 4;
 
 // hit-list launch of schedule S on a grid of workgroups of its thread count

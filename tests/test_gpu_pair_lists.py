@@ -40,14 +40,29 @@ def test_lists_match_the_oracle(sched, cells, n, clump):
     assert np.allclose(pe, per, rtol=1e-5)
 
 
-@pytest.mark.parametrize("n,name", [(45000, "hitlist-split9-t256-c8"), (45001, "hitlist-split3-t256-c12"),
-                                    (105000, "hitlist-split3-t256-c12"), (105001, "hitlist-t256-c24")])
-def test_automatic_schedule_by_bead_count(n, name):
+@pytest.mark.parametrize("n,bonds,name", [
+    (11000, 0, "hitlist-split9-t256-c8"), (11001, 0, "hitlist-split3-t256-c12"), (50000, 9, "hitlist-split9-t256-c8"),
+    (50001, 9, "hitlist-split3-t256-c12"), (100000, 0, "hitlist-split3-t256-c12"), (100001, 9, "hitlist-t256-c32"),
+    (262144, 0, "hitlist-t256-c32"), (262145, 0, "hitlist-t256-c24")])
+def test_automatic_schedule_by_bead_count(n, bonds, name):
     cells = (40, 30, 30)
     ids, t, x, v = random_state(cells, n, 2, seed=5)
+    u = x.copy()
+    h, tl = np.arange(bonds), np.arange(bonds) + 20
+    u[tl] = u[h] + [0.4, 0.1, 0.0]
+    x = np.mod(u, np.array(cells, float))
+    topo = (h, tl, np.full(bonds, 50.0), np.full(bonds, 0.5))
     e = D.Engine(cells, A2, G2, seed=3, pair_kernel=D.PAIR_AUTO)
-    e.upload(ids, t, x, v)
+    e.upload(ids, t, x, v, unpbc=u)
+    if bonds:
+        e.upload_topology(*topo)
     assert D.schedule_name(e.schedule) == name
     F, _, _ = e.compute_forces(step=2)
-    fr, _, _ = O.forces(O.Box(cells, A2, G2, seed=3), ids, t, x, v, step=2)
+    T = O.Topo(*topo, [], [], [], []) if bonds else None
+    fr, _, _ = O.forces(O.Box(cells, A2, G2, seed=3), ids, t, x, v, step=2, unpbc=u, topo=T)
     assert force_errors(F, fr)[0] < 1e-5
+    if bonds:   # without the topology the choice is that of free beads
+        e.upload(ids, t, x, v, unpbc=u)
+        e.upload_topology()
+        free = 6 if n <= 11000 else (5 if n <= 100000 else (3 if n <= 262144 else 2))
+        assert e.schedule == free
