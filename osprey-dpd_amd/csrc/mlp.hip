@@ -15,10 +15,10 @@
 // What bounds it: the latency of a chain of small products (0.7 GFLOP an iteration at 1,638
 // rows and 256 hidden units), so what counts is the number of launches and of passes over
 // memory.  That iteration took 26 launches and 123 us with a kernel for each product, partial
-// sum, column sum and elementwise step; it takes 30 us, 14 of it in k_mlp_rows and 12 in
+// sum, column sum and elementwise step; it takes 22 us, 14 of it in k_mlp_rows and 8 in
 // k_mlp_update.  With operands in [column][k] order, of which a wavefront's load touches 16
 // rows, the two took 25 and 20 us.  Many rows are bound by L2: 20,000 of 256 units 43 and
-// 61 us (k_mlp_update reads 330 MB of fragments at 5.4 TB/s), 429 us before.
+// 42 us (k_mlp_update reads 330 MB of fragments at 7.8 TB/s), 429 us before.
 //
 // Sums are split over K in the same parts and added in the same order whatever the kernel
 // (split_k), and each part is one chain of matrix instructions, so results do not depend on
@@ -88,6 +88,24 @@ __device__ inline void in_steps(int k0, int k1, const F& f)
     for (; k + 64 <= k1; k += 64) f(std::integral_constant<int, 4>{}, k);
     if (k + 32 <= k1) { f(std::integral_constant<int, 2>{}, k); k += 32; }
     if (k < k1) f(std::integral_constant<int, 1>{}, k);
+}
+
+// f(steps, s) over the 16-term steps s0 .. s1 - 1 in ascending order, eight at a time and what
+// is left at once
+template <class F>
+__device__ inline void in_rounds(int s0, int s1, const F& f)
+{
+    int s = s0;
+    for (; s + 8 <= s1; s += 8) f(std::integral_constant<int, 8>{}, s);
+    switch (s1 - s) {
+    case 1: f(std::integral_constant<int, 1>{}, s); break;
+    case 2: f(std::integral_constant<int, 2>{}, s); break;
+    case 3: f(std::integral_constant<int, 3>{}, s); break;
+    case 4: f(std::integral_constant<int, 4>{}, s); break;
+    case 5: f(std::integral_constant<int, 5>{}, s); break;
+    case 6: f(std::integral_constant<int, 6>{}, s); break;
+    case 7: f(std::integral_constant<int, 7>{}, s); break;
+    }
 }
 
 // standardisation of inputs and targets
@@ -310,85 +328,97 @@ __device__ inline float adam(const UpdateArgs& A, int64_t i, float g)
 }
 
 // The gradients of 16 x 16 blocks of a weight matrix, or of 16 biases, and their update:
-// blocks of W2, of W3, of W1, then tiles of b2, b1, b3.  Of the 16 wavefronts P share a block (P
-// the parts of its sum over the rows, as a power of two up to 16) and take parts p, p + P, ...;
-// 16 / P blocks side by side share a workgroup.  The parts are added in order through LDS.
+// tiles of b2, b1, b3, then blocks of W3, of W1, of W2.  Of a workgroup's wavefronts P share a
+// block (P the parts of its sum over the rows, as a power of two up to their number) and take
+// parts p, p + P, ...; blocks side by side fill the workgroup.  The parts are added in order
+// through LDS.
 // Bias gradients are column sums in slabs of kColSlab rows: in each, 16 sums over every 16th
 // row, added in order, and the slabs in order.
+// What bounds it: round trips to L2 one after another, so a wavefront has eight steps' operands
+// in flight and what is left of a part in one round more (four, two and one at a time took 12.2
+// us at 1,638 rows and 256 units, this 10.4, both in workgroups of sixteen wavefronts; smaller
+// ones 8.5); the longest chains, those of the biases, come first.  2 x 2 blocks a wavefront,
+// which read half as much, were no faster at 6,000 rows and 512 units (36.6 us at best against
+// 33.3): with a quarter of the wavefronts less is in flight.  Loading Adam's moments before the
+// product kept more registers and was slower for small nets (100 rows of 64: 13.3 us against
+// 9.6).
 constexpr int kColSlab = 128;
-inline __host__ __device__ int update_share(const SplitK& k)
+inline __host__ __device__ int update_share(const SplitK& k, int waves)
 {
     int P = 1;
-    while (P < k.parts && P < 16) P *= 2;
+    while (P < k.parts && P < waves) P *= 2;
     return P;
 }
-inline __host__ __device__ int update_groups(const SplitK& k, int blocks) { return (blocks + 16 / update_share(k) - 1) / (16 / update_share(k)); }
+inline __host__ __device__ int update_groups(const SplitK& k, int waves, int blocks)
+{
+    const int per = waves / update_share(k, waves);
+    return (blocks + per - 1) / per;
+}
 __global__ __launch_bounds__(1024) void k_mlp_update(UpdateArgs A)
 {
-    __shared__ __align__(16) float part[16][256];
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6, r = lane & 15;
+    extern __shared__ __align__(16) float part[];   // [wavefronts][256]
+    const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6), r = lane & 15, waves = blockDim.x >> 6;
     const int H = A.H, nt = H >> 4, nb = A.Mp >> 4;
-    const int n2 = update_groups(A.g2, nt * nt), n3 = update_groups(A.g3, nt), n1 = update_groups(A.g1, nt);
+    const int nbias = 2 * nt + 1, n3 = update_groups(A.g3, waves, nt), n1 = update_groups(A.g1, waves, nt);
     int job = blockIdx.x;
-    if (job < n2 + n3 + n1) {
-        const bool is2 = job < n2, is3 = !is2 && job < n2 + n3;
+    if (job >= nbias) {
+        job -= nbias;
+        const bool is3 = job < n3, is2 = job >= n3 + n1;
         const SplitK k = is2 ? A.g2 : (is3 ? A.g3 : A.g1);
-        job -= is2 ? 0 : (is3 ? n2 : n2 + n3);
-        const int P = update_share(k), per = 16 / P, blocks = is2 ? nt * nt : nt;
+        job -= is2 ? n3 + n1 : (is3 ? 0 : n3);
+        const int P = update_share(k, waves), per = waves / P, blocks = is2 ? nt * nt : nt;
         // block x of the matrix: k tile tm, n tile tn
         auto tm = [&](int x) { return is2 ? x / nt : (is3 ? x : 0); };
         auto tn = [&](int x) { return is2 ? x % nt : (is3 ? 0 : x); };
         const int x = min(job * per + w / P, blocks - 1);   // (past the last: it again, not stored)
         const uint16_t* a = (is2 ? A.H1F : (is3 ? A.H2F : A.XF)) + ((size_t)tm(x) * nb * 64 + lane) * 4;
         const uint16_t* b = (is2 ? A.dZ2F : (is3 ? A.dYF : A.dZ1F)) + ((size_t)tn(x) * nb * 64 + lane) * 4;
-        float g[4] = {0.f, 0.f, 0.f, 0.f};   // entries t % 256 of blocks t / 256 + 4 v
+        float g[4] = {0.f, 0.f, 0.f, 0.f};   // entries t + v * blockDim of the workgroup's blocks
         for (int z0 = 0; z0 < k.parts; z0 += P) {
             const int z = z0 + w % P;
             if (z < k.parts) {
                 floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-                in_steps(z * k.per, min(A.Mp, (z + 1) * k.per), [&](auto steps, int kk) {
+                in_rounds(z * k.per >> 4, min(A.Mp, (z + 1) * k.per) >> 4, [&](auto steps, int s) {
                     constexpr int U = decltype(steps)::value;
                     bf16x4 fa[U], fb[U];
 #pragma unroll
                     for (int u = 0; u < U; ++u) {
-                        fa[u] = frag(a + (size_t)((kk >> 4) + u) * 256);
-                        fb[u] = frag(b + (size_t)((kk >> 4) + u) * 256);
+                        fa[u] = frag(a + (size_t)(s + u) * 256);
+                        fb[u] = frag(b + (size_t)(s + u) * 256);
                     }
 #pragma unroll
                     for (int u = 0; u < U; ++u) acc = mfma(fa[u], fb[u], acc);
                 });
-                *reinterpret_cast<floatx4*>(&part[w][lane * 4]) = acc;
+                *reinterpret_cast<floatx4*>(part + w * 256 + lane * 4) = acc;
             }
             __syncthreads();
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                const int c = t / 256 + 4 * v;
+                const int c = (t + v * (int)blockDim.x) >> 8, e = (t + v * (int)blockDim.x) & 255;
                 if (c < per)
-                    for (int u = 0; u < min(P, k.parts - z0); ++u) g[v] += part[c * P + u][t % 256];
+                    for (int u = 0; u < min(P, k.parts - z0); ++u) g[v] += part[(c * P + u) * 256 + e];
             }
             __syncthreads();
         }
-        const int e = t % 256, m = 4 * (e >> 6) + (e & 3), n = (e >> 2) & 15;
         const int64_t o = is2 ? A.w2 : (is3 ? A.w3 : A.w1);
         const int K = is2 || is3 ? H : 16, N = is3 ? 16 : H;
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const int c = t / 256 + 4 * v, y = job * per + c;
+            const int c = (t + v * (int)blockDim.x) >> 8, e = (t + v * (int)blockDim.x) & 255, y = job * per + c;
             if (c >= per || y >= blocks) continue;
-            const int row = tm(y) * 16 + m, col = tn(y) * 16 + n;
+            const int row = tm(y) * 16 + 4 * (e >> 6) + (e & 3), col = tn(y) * 16 + ((e >> 2) & 15);
             const int64_t i = o + (int64_t)row * N + col;
             if (A.grad) A.grad[i] = g[v];
             else store_weight(A.wf, A.wt, o, row, col, K, N, adam(A, i, g[v]));
         }
         return;
     }
-    job -= n2 + n3 + n1;
     const float* d = job < nt ? A.dZ2 : (job < 2 * nt ? A.dZ1 : A.dY);
     const int64_t i0 = job < nt ? A.b2 + job * 16 : (job < 2 * nt ? A.b1 + (job - nt) * 16 : A.b3);
     d += ((size_t)(job < 2 * nt ? job % nt : 0) * nb * 64 + lane) * 4;
     const int slabs = (A.Mp + kColSlab - 1) / kColSlab;
     float g = 0.f;
-    for (int z0 = 0; z0 < slabs; z0 += 16) {
+    for (int z0 = 0; z0 < slabs; z0 += waves) {
         const int z = z0 + w;
         if (z < slabs) {
             // lane (q, r): rows 4q .. 4q+3 of every 16, column r
@@ -402,11 +432,11 @@ __global__ __launch_bounds__(1024) void k_mlp_update(UpdateArgs A)
             float p = 0.f;
 #pragma unroll
             for (int u = 0; u < 16; ++u) p += __shfl(s[u & 3], (u >> 2) * 16 + r);
-            if (lane < 16) part[w][lane] = p;
+            if (lane < 16) part[w * 16 + lane] = p;
         }
         __syncthreads();
         if (t < 16)
-            for (int u = 0; u < min(16, slabs - z0); ++u) g += part[u][t];
+            for (int u = 0; u < min(waves, slabs - z0); ++u) g += part[u * 16 + t];
         __syncthreads();
     }
     if (t < 16) {
@@ -595,9 +625,17 @@ void launch_update(dpd_mlp* m, int Mp, bool store, float lr, float c1, float c2)
     a.mask = m->mask;
     a.wf = m->wf; a.wt = m->wt;
     a.lr = lr; a.c1 = c1; a.c2 = c2;
-    const int nt = m->H / 16;
-    const int groups = update_groups(a.g2, nt * nt) + update_groups(a.g3, nt) + update_groups(a.g1, nt);
-    hipLaunchKernelGGL(k_mlp_update, dim3(groups + 2 * nt + 1), dim3(1024), 0, m->stream, a);
+    // Eight wavefronts a workgroup: short enough for several to share a compute unit, so one
+    // loads while another adds its parts.  Four where a sum has few parts to share out (unless
+    // there are fewer than 16 blocks of W2 to lay side by side), or where blocks are many;
+    // sixteen where blocks are few and the chains of the bias sums and of W3 are what is waited
+    // for (us with 4 / 8 / 16: 400 rows of 128 units 4.8 / 6.4 / 6.6, 6,000 of 768 66 / 77 /
+    // 102; 100 of 32 6.3 / 5.7 / 6.4, 1,638 of 256 10.0 / 8.5 / 10.4, 6,000 of 512 33.8 / 33.3
+    // / 37.1; 6,000 of 128 25.1 / 16.2 / 12.9.  Sixteen and four steps at a time, for every size:
+    // 7.2, 99; 5.8, 12.1, 41.5; 14.7).
+    const int nt = m->H / 16, waves = m->H > 512 || (Mp <= 512 && m->H >= 64) ? 4 : (Mp > 1024 && m->H <= 128 ? 16 : 8);
+    const int groups = update_groups(a.g3, waves, nt) + update_groups(a.g1, waves, nt) + update_groups(a.g2, waves, nt * nt);
+    hipLaunchKernelGGL(k_mlp_update, dim3(2 * nt + 1 + groups), dim3(64 * waves), sizeof(float) * 256 * waves, m->stream, a);
 }
 
 void refresh_bf16(dpd_mlp* m)

@@ -1,7 +1,9 @@
 """GPU tests of the surrogate network's kernels at the edges of their tiles: batches around a
 16-row workgroup and a 128-row slab of the bias sums, hidden layers of one column tile, of a
 ragged number of tiles per wavefront and of the largest size, the narrowest and widest inputs
-and outputs, and batches of more than 256 workgroups (eight wavefronts instead of sixteen)."""
+and outputs, and batches of more than 256 workgroups (eight wavefronts instead of sixteen); and
+where the update changes from four wavefronts to eight and to sixteen, with parts of its sums
+of one to eight steps and longer."""
 import numpy as np
 import pytest
 
@@ -19,7 +21,9 @@ TOL = 2.0 ** -8
 
 @pytest.mark.parametrize("nin,H,nout,n", [
     (1, 16, 1, 1), (7, 16, 2, 15), (16, 48, 16, 16), (3, 128, 5, 17), (6, 144, 2, 127), (6, 272, 2, 129),
-    (7, 256, 2, 2100), (5, 528, 3, 40), (7, 1024, 2, 33), (2, 144, 1, 4112), (4, 272, 2, 4130)])
+    (7, 256, 2, 2100), (5, 528, 3, 40), (7, 1024, 2, 33), (2, 144, 1, 4112), (4, 272, 2, 4130),
+    (4, 64, 2, 512), (6, 512, 2, 513), (3, 528, 2, 520), (7, 128, 2, 1024), (7, 128, 2, 1025), (5, 144, 2, 1030),
+    (2, 32, 1, 1456), (2, 16, 1, 1100)])
 def test_edges_of_the_tiles(nin, H, nout, n):
     rng = np.random.default_rng(nin + H + n)
     net = Surrogate(nin, H, nout, seed=4)
