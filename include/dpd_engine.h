@@ -235,7 +235,8 @@ int dpd_renormalise_momenta(dpd_engine* e, int32_t box);
  * (tensor element 3a + b = F_a dx_b; F on the first bead, dx = first - second) to the
  * slices its two beads span: the whole of it to their slice when both lie in one, else
  * the share width / |dz| to each slice crossed and the fractions of that to the two end
- * slices.  pair_out[nslices][nt][nt][9] (may be NULL) holds the pair forces of the
+ * slices.  A pair with |dz| <= 1e-5 has half in each bead's own slice, under (its type, the
+ * other's).  pair_out[nslices][nt][nt][9] (may be NULL) holds the pair forces of the
  * current state -- positions, predicted velocities and pair stream of the last force
  * evaluation, i.e. the last step's forces after dpd_step and the uploaded state at
  * step0 after dpd_commit -- with each pair's share split equally between (ti, tj) and

@@ -29,18 +29,33 @@ namespace dpd {
 
 namespace {
 
+// The slice of an interaction at z (in slices), the two beside a border it lies on.  z is wrapped
+// into [0, Lz): the indices are in range; the clamp only guards the table against a position
+// rounded onto Lz.
+template <class Add>
+__device__ inline void flat_split(int nslice, double z, const Add& add)
+{
+    const int i = min(max((int)z, 0), nslice - 1);
+    if (z - (double)i > 0.00001) {
+        add(i, 1.0);
+    } else {
+        add(i, 0.5);
+        add(i > 0 ? i - 1 : nslice - 1, 0.5);
+    }
+}
+
 // The z-slice split of one interaction (see orc_slice_add for the rule) between z1 and z2,
-// dz = z1 - z2 unwrapped: add(slice, share) for every slice spanned.
+// dz = z1 - z2 unwrapped: add(slice, share) for every slice spanned.  A flat interaction
+// (|dz| <= kFlat) lies at z1, whatever z2 is.
+constexpr double kFlat = 0.00001;
 template <class Add>
 __device__ inline void slice_split(int nslice, double Lz, double z1, double z2, double dz, const Add& add)
 {
     const double width = Lz / nslice, inv = nslice / Lz;
     double zd = dz, zu, zl;
-    if (zd > 0.00001) { zu = z1 * inv; zl = z2 * inv; }
-    else if (zd < -0.00001) { zd = -zd; zu = z2 * inv; zl = z1 * inv; }
+    if (zd > kFlat) { zu = z1 * inv; zl = z2 * inv; }
+    else if (zd < -kFlat) { zd = -zd; zu = z2 * inv; zl = z1 * inv; }
     else { zu = zl = z1 * inv; }
-    // z is wrapped into [0, Lz): the slice indices are in range; the clamp only guards
-    // the table against a position rounded onto Lz
     int iu = min(max((int)zu, 0), nslice - 1), il = min(max((int)zl, 0), nslice - 1);
     const double ru = zu - (double)iu, rl = zl - (double)il;
     if (iu == il) {
@@ -80,6 +95,12 @@ __device__ inline double wrapped_z(const SliceArgs& A, int slot)
 // pairs) of the slices from s0 on, lane l adding to copy l mod copies.  The sums of types ti <= tj
 // go to their components a <= b of out; k_slice_mirror spreads them afterwards.  Without WIN
 // (no window fits LDS) the pairs add to out themselves.
+// Seen from either bead a pair spans the same slices, unless it is flat: then each bead has half
+// of it in its own slices, under (its type, the other's).  So j's half is moved there from i's,
+// and what (ti, tj) gets beyond half of the sum, and (tj, ti) lacks, is left in out's entry of
+// types (tj, ti), ti < tj.  One pair in 1e5 is flat; these go straight to out, after the others of
+// their lists (a call on the 48x48x32 bilayer 206 us; with the halves told apart within the loop
+// over all pairs 215, after each pair 207).
 // LIST: listed partners per thread; when one of the lanes that scan has no room for four more,
 // they evaluate their lists together.  28 where they fit 64 KB beside the window, else 12 (a
 // call on the 48x48x32 bilayer with 64 slices, and one of 48x40x20 with 250: 108 and 151 us,
@@ -134,40 +155,67 @@ __global__ __launch_bounds__(256) void k_slice_pairs(SliceArgs A, double* __rest
                 d[2] = (pi.z - (float)dz * B.w[2]) - pj.z;
                 return d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
             };
+            // the pair of listed partner h: its sums, the partner's z, dz and the types
+            struct Pair {
+                double f[6], zj, dz;
+                int lo, hi;
+            };
+            auto pair_of = [&](int h) {
+                const int j = list[h][t], code = row[h][t];
+                const int im = code & 3, dy = ((code >> 2) & 3) - 1, dz = code >> 4;
+                const float4 pj = A.pos[j], vj = A.vp[j];
+                float d[3];
+                const float dr2 = separation(pj, im, dy, dz, d);
+                const int tj = bead_type(__float_as_int(pj.w));
+                const int tt = ti * kMaxTypes + tj;
+                const float dxdv = d[0] * (vi.x - vj.x) + d[1] * (vi.y - vj.y) + d[2] * (vi.z - vj.z);
+                const float s = pair_scalar(dr2, dxdv, A.table[tt], A.table[2 * kTypeStride + tt],
+                                            A.table[kTypeStride + tt], idi, (uint32_t)__float_as_int(vj.w),
+                                            B.invrootdt, K, nullptr);
+                int cz = c[2] + dz;
+                cz -= cz >= B.n[2] ? B.n[2] : 0;
+                const double sx = (double)s * d[0], sy = (double)s * d[1], sz = (double)s * d[2];
+                return Pair{{sx * d[0], sx * d[1], sx * d[2], sy * d[1], sy * d[2], sz * d[2]},
+                            (double)cz * B.wd[2] + (double)pj.z, (double)d[2], min(ti, tj), max(ti, tj)};
+            };
             auto evaluate = [&]() {
+                int flat = 0;   // flat pairs, to the list's front
                 for (int h = 0; h < n; ++h) {
-                    const int j = list[h][t], code = row[h][t];
-                    const int im = code & 3, dy = ((code >> 2) & 3) - 1, dz = code >> 4;
-                    const float4 pj = A.pos[j], vj = A.vp[j];
-                    float d[3];
-                    const float dr2 = separation(pj, im, dy, dz, d);
-                    const int tj = bead_type(__float_as_int(pj.w));
-                    const int tt = ti * kMaxTypes + tj;
-                    const float dxdv = d[0] * (vi.x - vj.x) + d[1] * (vi.y - vj.y) + d[2] * (vi.z - vj.z);
-                    const float s = pair_scalar(dr2, dxdv, A.table[tt], A.table[2 * kTypeStride + tt],
-                                                A.table[kTypeStride + tt], idi, (uint32_t)__float_as_int(vj.w),
-                                                B.invrootdt, K, nullptr);
-                    int cz = c[2] + dz;
-                    cz -= cz >= B.n[2] ? B.n[2] : 0;
-                    const double zj = (double)cz * B.wd[2] + (double)pj.z;
-                    const double sx = (double)s * d[0], sy = (double)s * d[1], sz = (double)s * d[2];
-                    const double f[6] = {sx * d[0], sx * d[1], sx * d[2], sy * d[1], sy * d[2], sz * d[2]};
-                    const int lo = min(ti, tj), hi = max(ti, tj);
-                    slice_split(A.nslice, Lz, zi, zj, (double)d[2], [&](int sl, double share) {
+                    const Pair p = pair_of(h);
+                    slice_split(A.nslice, Lz, zi, p.zj, p.dz, [&](int sl, double share) {
                         if constexpr (WIN) {
                             int w = sl - s0;
                             w -= w >= A.nslice ? A.nslice : 0;
                             w += w < 0 ? A.nslice : 0;
                             w = min(w, win - 1);   // (holds: keeps a bad state's sums in the table)
-                            double* q = mine + (w * ntri + hi * (hi + 1) / 2 + lo) * 6;
+                            double* q = mine + (w * ntri + p.hi * (p.hi + 1) / 2 + p.lo) * 6;
 #pragma unroll
-                            for (int m = 0; m < 6; ++m) atomicAdd(q + m, f[m] * share);
+                            for (int m = 0; m < 6; ++m) atomicAdd(q + m, p.f[m] * share);
                         } else {
-                            double* q = out + ((size_t)sl * A.nidx + lo * A.ntypes + hi) * 9;
+                            double* q = out + ((size_t)sl * A.nidx + p.lo * A.ntypes + p.hi) * 9;
 #pragma unroll
-                            for (int m = 0; m < 6; ++m) atomicAdd(q + kTri[m], f[m] * share);
+                            for (int m = 0; m < 6; ++m) atomicAdd(q + kTri[m], p.f[m] * share);
                         }
                     });
+                    if (fabs(p.dz) <= kFlat) {
+                        list[flat][t] = list[h][t];
+                        row[flat++][t] = row[h][t];
+                    }
+                }
+                for (int h = 0; h < flat; ++h) {
+                    const Pair p = pair_of(h);
+                    for (int of_j = 0; of_j < 2; ++of_j)
+                        flat_split(A.nslice, inv * (of_j ? p.zj : zi), [&](int sl, double share) {
+                            const double sum = of_j ? 0.5 * share : -0.5 * share;
+                            const double more = (ti == p.lo) == (of_j == 0) ? 0.25 * share : -0.25 * share;
+                            double* q = out + ((size_t)sl * A.nidx + p.lo * A.ntypes + p.hi) * 9;
+                            double* r = out + ((size_t)sl * A.nidx + p.hi * A.ntypes + p.lo) * 9;
+#pragma unroll
+                            for (int m = 0; m < 6; ++m) {
+                                atomicAdd(q + kTri[m], p.f[m] * sum);
+                                if (p.lo != p.hi) atomicAdd(r + kTri[m], p.f[m] * more);
+                            }
+                        });
                 }
                 n = 0;
             };
@@ -225,8 +273,8 @@ __global__ __launch_bounds__(256) void k_slice_pairs(SliceArgs A, double* __rest
     }
 }
 
-// the pair table's other halves: types (tj, ti) beside (ti, tj), half of the sum each, and the
-// components below the diagonal
+// the pair table's other halves: types (tj, ti) beside (ti, tj), half of the sum each and the
+// flat pairs' difference, and the components below the diagonal
 __global__ __launch_bounds__(256) void k_slice_mirror(SliceArgs A, double* __restrict__ out)
 {
     const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -236,11 +284,14 @@ __global__ __launch_bounds__(256) void k_slice_mirror(SliceArgs A, double* __res
     double* a = out + q * 9;
     double* b = out + (q - lo * A.ntypes - hi + hi * A.ntypes + lo) * 9;
     const double share = lo == hi ? 1.0 : 0.5;
-    double v[6];
-    for (int m = 0; m < 6; ++m) v[m] = a[kTri[m]] * share;
-    for (int m = 0; m < 9; ++m) a[m] = v[kSym[m]];
+    double v[6], more[6];
+    for (int m = 0; m < 6; ++m) {
+        v[m] = a[kTri[m]] * share;
+        more[m] = lo != hi ? b[kTri[m]] : 0.0;
+    }
+    for (int m = 0; m < 9; ++m) a[m] = v[kSym[m]] + more[kSym[m]];
     if (lo != hi)
-        for (int m = 0; m < 9; ++m) b[m] = v[kSym[m]];
+        for (int m = 0; m < 9; ++m) b[m] = v[kSym[m]] - more[kSym[m]];
 }
 
 // Tables of bonds and bond pairs: workgroup (b, w) adds the interactions it takes (every
