@@ -8,7 +8,8 @@
 //               (without bonded terms the previous pair launch's epilogue does this)
 //   k_sort      the counting sort and the move into the new cell-sorted SoA buffers, beads
 //               of a cell in ascending bead index (deterministic layout); above 8192 groups
-//               of 64 cell keys k_group_scan goes before it
+//               of 64 cell keys k_group_scan goes before it, and with dense cells k_move
+//               after it does the move
 //   pair kernel DPD pair forces (src/CNTCell.cpp:1144-1555)
 //               and in the same launch the bonded terms (k_bonded with the full-shell kernel):
 //               bonds and angles (src/Bond.cpp:111-162, src/BondPair.cpp:138-286) summed for
@@ -373,6 +374,90 @@ __global__ __launch_bounds__(1024) void k_group_scan(int ngroups, int* __restric
     scan_block(gcnt, gstart, ngroups, ex, wsum, &carry);
 }
 
+// A bead as the sort finds it, and what it takes to move it
+struct Bead {
+    float4 p, v, f;
+    int key;
+};
+struct Move {
+    Buffers S, D;
+    const float4* frc;
+    float4* vp;
+    int* slot_of;
+    double4* upos;
+    int write_vp;
+};
+
+template <int MODE>
+__device__ inline Bead load_bead(const Move& M, int s)
+{
+    return Bead{M.S.pos[s], M.S.vel[s], MODE == kRebin ? M.S.fold[s] : M.frc[s], M.S.key[s]};
+}
+
+// Bead q, found as x, to slot dst of the new order under key k: repeats the advance that filed it.
+template <int MODE, bool MULTI>
+__device__ inline void move_bead(const Move& M, const BoxDev* boxes, const BoxDev& B0, const Bead& x, int k, int q, int dst)
+{
+    const Buffers &S = M.S, &D = M.D;
+    const float4 p = x.p, f = x.f;
+    float4 v = x.v;
+    const BoxDev& B = box_of<MULTI>(boxes, B0, __float_as_int(p.w));
+    if (MODE == kEndBegin) {
+        // UpdateMom of the step that ends (the same sum as k_advance)
+        v.x = kick(v.x, f.x, B.hdt);
+        v.y = kick(v.y, f.y, B.hdt);
+        v.z = kick(v.z, f.z, B.hdt);
+    }
+    int c[3];
+    key_cell(x.key - B.koff, B, c);
+    const float o[3] = {p.x, p.y, p.z};
+    const int img[3] = {0, 0, 0};   // m.img is the change of image this step
+    float d[3] = {0.f, 0.f, 0.f};
+    if (MODE != kRebin) {
+        d[0] = drift(v.x, f.x, B);
+        d[1] = drift(v.y, f.y, B);
+        d[2] = drift(v.z, f.z, B);
+    }
+    Moved m;
+    advance(o, c, img, d, B, m);
+    const int wd = (__float_as_int(p.w) & ~kCellXBits) | ((m.c[0] & 3) << kCellXShift);
+    D.pos[dst] = make_float4(m.o[0], m.o[1], m.o[2], __int_as_float(wd));
+    if (MODE == kRebin) {
+        D.vel[dst] = v;
+        D.fold[dst] = f;
+    } else {
+        // the first half of the next UpdateMom: v + dt/2 F, so the force need not be kept
+        D.vel[dst] = make_float4(kick(v.x, f.x, B.hdt), kick(v.y, f.y, B.hdt), kick(v.z, f.z, B.hdt), v.w);
+    }
+    D.bead[dst] = q;
+    // the image counts live by bead index: only a bead that crosses the box changes them,
+    // and only its own thread writes them
+    const bool bonded = __float_as_int(p.w) & kBondedBit, crosses = m.img[0] | m.img[1] | m.img[2];
+    if ((MULTI && bonded) || crosses) {
+        int4 im = S.img[q];
+        im.x += m.img[0]; im.y += m.img[1]; im.z += m.img[2];
+        if (crosses) S.img[q] = im;
+        if (MULTI && bonded)
+            M.upos[q] = make_double4((double)(m.c[0] + im.x * B.n[0]) * B.wd[0] + (double)m.o[0],
+                                     (double)(m.c[1] + im.y * B.n[1]) * B.wd[1] + (double)m.o[1],
+                                     (double)(m.c[2] + im.z * B.n[2]) * B.wd[2] + (double)m.o[2],
+                                     (double)bead_box(wd));
+    }
+    D.key[dst] = k;
+    D.code[dst] = scan_code(m.o, m.c, B);
+    if (MODE == kRebin) {
+        M.vp[dst] = v;
+    } else {
+        // (equal to the new velocity's bits when lambda dt = dt/2: the steps then read that)
+        if (M.write_vp)
+            M.vp[dst] = make_float4(kick(v.x, f.x, B.lamdt), kick(v.y, f.y, B.lamdt), kick(v.z, f.z, B.lamdt), v.w);
+    }
+    // the slot of each bead is read for bonded beads only (bond and angle terms); a scattered
+    // 4-byte store per bead costs a partial-line write each, so the others are skipped once
+    // the topology has flagged the bonded ones (an upload re-binning writes every bead)
+    if (MODE == kRebin || bonded) M.slot_of[q] = dst;
+}
+
 // The counting sort and the move in one launch: workgroup g takes the 64 cell keys of scan
 // group g, finds where its beads go (the counts of the groups before it, then a scan of its 64
 // cells), collects them from their bins and moves them there, in every cell by ascending bead
@@ -381,7 +466,8 @@ __global__ __launch_bounds__(1024) void k_group_scan(int ngroups, int* __restric
 // The beads before the group are gstart[g] (k_group_scan) or, with it null, the sum of gcnt.
 // Clears cnt; gcnt and nspill are read by other workgroups, so those of the sort before (`clear`)
 // are cleared instead.
-// Groups of more than kSortList beads, or with a spill, go through `order` in global memory.
+// Groups of more than kSortList beads, or with a spill, go through `order` in global memory: a few
+// of them, for engines whose groups are that full on average take the DENSE form.
 // What bounds it: in small boxes the three round trips to memory (counts, bins, beads), 4.8 us
 // where three launches (cell starts, placement by rank, move), each a chain of its own, took 14;
 // in large ones HBM, about 110 bytes a bead: 786,432 beads 19.8 us (4.4 TB/s) against 28,
@@ -390,8 +476,10 @@ __global__ __launch_bounds__(1024) void k_group_scan(int ngroups, int* __restric
 // A workgroup takes one group: four wavefronts move its 192 beads (at three a cell) at once.
 // Workgroups are dealt to the XCDs in eight contiguous ranges, as the pair launch deals beads:
 // 96^3 342 us a step, dealt in turn 352.
+// DENSE: no bead is moved here, but the cell of every kMoveSlots-th slot noted in `order` (k_move).
 constexpr int kSortList = 1024;
-template <int MODE, bool MULTI>
+constexpr int kMoveSlots = 256;
+template <int MODE, bool MULTI, bool DENSE>
 __global__ __launch_bounds__(256) void k_sort(int n, int ngroups, int per_xcd, Buffers S, Buffers D,
                                               const float4* __restrict__ frc, float4* __restrict__ vp,
                                               const BoxDev* boxes, BoxDev B0, Intake I, const int* __restrict__ gstart,
@@ -401,7 +489,7 @@ __global__ __launch_bounds__(256) void k_sort(int n, int ngroups, int per_xcd, B
 {
     __shared__ int first[kGroupKeys + 1];   // of each cell among the group's beads
     __shared__ int old[kGroupKeys];         // of each cell in the old order
-    __shared__ int slot[kSortList], ids[kSortList];
+    __shared__ int slot[DENSE ? 1 : kSortList], ids[DENSE ? 1 : kSortList];
     __shared__ int wsum[4], spilled;
     const int g = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
     if (g >= ngroups) return;
@@ -445,73 +533,16 @@ __global__ __launch_bounds__(256) void k_sort(int n, int ngroups, int per_xcd, B
         for (int h = kGroupKeys / 2; h > 0; h >>= 1) c += first[c + h] <= j ? h : 0;
         return c;
     };
+    if constexpr (DENSE) {
+        int* cell = reinterpret_cast<int*>(order);
+        for (int b = (start + kMoveSlots - 1) / kMoveSlots + t; b * kMoveSlots < start + total; b += 256)
+            cell[b] = k0 + cell_of(b * kMoveSlots - start);
+        return;
+    }
     auto bin = [&](int c) { return I.bins + bin_at(old[c], k0 + c); };
-    struct Bead {
-        float4 p, v, f;
-        int key;
-    };
-    auto load = [&](int s) {
-        return Bead{S.pos[s], S.vel[s], MODE == kRebin ? S.fold[s] : frc[s], S.key[s]};
-    };
-    auto move = [&](const Bead& x, int k, int q, int dst) {
-        const float4 p = x.p, f = x.f;
-        float4 v = x.v;
-        const BoxDev& B = box_of<MULTI>(boxes, B0, __float_as_int(p.w));
-        if (MODE == kEndBegin) {
-            // UpdateMom of the step that ends (the same sum as k_advance)
-            v.x = kick(v.x, f.x, B.hdt);
-            v.y = kick(v.y, f.y, B.hdt);
-            v.z = kick(v.z, f.z, B.hdt);
-        }
-        int c[3];
-        key_cell(x.key - B.koff, B, c);
-        const float o[3] = {p.x, p.y, p.z};
-        const int img[3] = {0, 0, 0};   // m.img is the change of image this step
-        float d[3] = {0.f, 0.f, 0.f};
-        if (MODE != kRebin) {
-            d[0] = drift(v.x, f.x, B);
-            d[1] = drift(v.y, f.y, B);
-            d[2] = drift(v.z, f.z, B);
-        }
-        Moved m;
-        advance(o, c, img, d, B, m);
-        const int wd = (__float_as_int(p.w) & ~kCellXBits) | ((m.c[0] & 3) << kCellXShift);
-        D.pos[dst] = make_float4(m.o[0], m.o[1], m.o[2], __int_as_float(wd));
-        if (MODE == kRebin) {
-            D.vel[dst] = v;
-            D.fold[dst] = f;
-        } else {
-            // the first half of the next UpdateMom: v + dt/2 F, so the force need not be kept
-            D.vel[dst] = make_float4(kick(v.x, f.x, B.hdt), kick(v.y, f.y, B.hdt), kick(v.z, f.z, B.hdt), v.w);
-        }
-        D.bead[dst] = q;
-        // the image counts live by bead index: only a bead that crosses the box changes them,
-        // and only its own thread writes them
-        const bool bonded = __float_as_int(p.w) & kBondedBit, crosses = m.img[0] | m.img[1] | m.img[2];
-        if ((MULTI && bonded) || crosses) {
-            int4 im = S.img[q];
-            im.x += m.img[0]; im.y += m.img[1]; im.z += m.img[2];
-            if (crosses) S.img[q] = im;
-            if (MULTI && bonded)
-                upos[q] = make_double4((double)(m.c[0] + im.x * B.n[0]) * B.wd[0] + (double)m.o[0],
-                                       (double)(m.c[1] + im.y * B.n[1]) * B.wd[1] + (double)m.o[1],
-                                       (double)(m.c[2] + im.z * B.n[2]) * B.wd[2] + (double)m.o[2],
-                                       (double)bead_box(wd));
-        }
-        D.key[dst] = k;
-        D.code[dst] = scan_code(m.o, m.c, B);
-        if (MODE == kRebin) {
-            vp[dst] = v;
-        } else {
-            // (equal to the new velocity's bits when lambda dt = dt/2: the steps then read that)
-            if (write_vp)
-                vp[dst] = make_float4(kick(v.x, f.x, B.lamdt), kick(v.y, f.y, B.lamdt), kick(v.z, f.z, B.lamdt), v.w);
-        }
-        // the slot of each bead is read for bonded beads only (bond and angle terms); a scattered
-        // 4-byte store per bead costs a partial-line write each, so the others are skipped once
-        // the topology has flagged the bonded ones (an upload re-binning writes every bead)
-        if (MODE == kRebin || bonded) slot_of[q] = dst;
-    };
+    const Move M{S, D, frc, vp, slot_of, upos, write_vp};
+    auto load = [&](int q) { return load_bead<MODE>(M, q); };
+    auto move = [&](const Bead& x, int k, int q, int dst) { move_bead<MODE, MULTI>(M, boxes, B0, x, k, q, dst); };
     if (total <= kSortList && !spilled) {
         // the first 256 beads are loaded before their indices are exchanged
         Bead b0;
@@ -560,6 +591,81 @@ __global__ __launch_bounds__(256) void k_sort(int n, int ngroups, int per_xcd, B
         for (int e = first[c]; e < first[c + 1]; ++e) r += list[e].x < x.x;
         move(load(x.y), k0 + c, x.x, start + first[c] + r);
     }
+}
+
+// The move for engines of dense cells, after k_sort's cell starts: a workgroup takes kMoveSlots
+// slots of the new order, whatever cells these belong to.  It collects the bead indices of their
+// cells (the first and the last reach past its slots) tile by tile in LDS, and each thread counts
+// those below its bead's.
+// What bounds it: the round trips (cells, bins, bead indices) and, in cells of hundreds, the
+// counting.  A step of 81,000 beads in 10^3 cells of width 3 takes 156 us, 136 of them the pair
+// launch (318 where each scan group's workgroup moves its 5,000 beads alone, one round trip after
+// the other), 41,472 in 6^3 of width 4 264 us (1,053), the same in 3^3 of width 8 2.5 ms (20.4).
+constexpr int kMoveTile = 1024;
+template <int MODE, bool MULTI>
+__global__ __launch_bounds__(kMoveSlots) void k_move(int n, int nkeys, int nblocks, int per_xcd, Move M,
+                                                     const BoxDev* boxes, BoxDev B0, Intake I,
+                                                     const int* __restrict__ cstart, const int* __restrict__ cell)
+{
+    __shared__ int ids[kMoveTile], src[kMoveSlots];
+    __shared__ int last, over;
+    const int blk = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if (blk >= nblocks) return;
+    const int t = threadIdx.x, d0 = blk * kMoveSlots, d1 = min(n, d0 + kMoveSlots), j = min(d0 + t, d1 - 1);
+    const bool active = d0 + t < d1;
+    // the cell k of slot j: the last one that starts at it or before
+    const int kl = cell[blk];
+    int k = kl;
+    for (int hi = d1 < n ? cell[blk + 1] : nkeys - 1; k < hi;) {
+        const int mid = (k + hi + 1) >> 1;
+        if (cstart[mid] <= j) k = mid;
+        else hi = mid - 1;
+    }
+    const int c0 = cstart[k], c1 = cstart[k + 1];
+    // the source of the bead of rank r in cell q's bin (-1: spilled)
+    auto in_bin = [&](int q, int r) {
+        const int a = I.cstart[q];
+        return r < bin_room(I.cstart[q + 1] - a) ? I.bins[bin_at(a, q) + r] : -1;
+    };
+    // f(slot, source) of the spilled beads that belong to slots [a, b)
+    auto spilled = [&](int a, int b, const auto& f) {
+        for (int i = t, m = min(*I.nspill, I.cap); i < m; i += kMoveSlots) {
+            const int4 x = I.spill[i];
+            const int s = cstart[x.x] + x.y;
+            if (s >= a && s < b) f(s, x.z);
+        }
+        __syncthreads();
+    };
+    if (t == 0) over = 0;
+    if (d0 + t == d1 - 1) last = k;
+    __syncthreads();
+    if (active) {
+        const int s = in_bin(k, j - c0);
+        src[t] = s;
+        if (s < 0) over = 1;
+    }
+    __syncthreads();
+    if (over) spilled(d0, d1, [&](int s, int from) { src[s - d0] = from; });
+    const int s = src[j - d0];
+    const Bead x = load_bead<MODE>(M, s);
+    const int q = M.S.bead[s];
+    const int kr = last, e0 = cstart[kl], e1 = cstart[kr + 1], l0 = e0, r0 = cstart[kr];
+    int rank = 0;
+    for (int a = e0; a < e1; a += kMoveTile) {
+        const int b = min(a + kMoveTile, e1);
+        __syncthreads();   // ids and over are read no more
+        if (t == 0) over = 0;
+        __syncthreads();
+        for (int i = a + t; i < b; i += kMoveSlots) {
+            const int from = i < d0 ? in_bin(kl, i - l0) : (i < d1 ? src[i - d0] : in_bin(kr, i - r0));
+            if (from < 0) over = 1;
+            else ids[i - a] = M.S.bead[from];
+        }
+        __syncthreads();
+        if (over) spilled(a, b, [&](int i, int from) { ids[i - a] = M.S.bead[from]; });
+        for (int i = max(a, c0); i < min(b, c1); ++i) rank += ids[i - a] < q;
+    }
+    if (active) move_bead<MODE, MULTI>(M, boxes, B0, x, k, q, c0 + rank);
 }
 
 // REBIN leaves the uploaded force in fold; the canonical state needs it in frc too
@@ -1006,6 +1112,12 @@ void launch_advance(dpd_engine* e, const Buffers& S, const Intake& I)
 // more the sum, quadratic in all, costs more than a launch of one workgroup that scans them
 // (a step of 4,096 groups 122.2 us, with the scan 123.7; of 13,824 355 us, with the scan 342).
 constexpr int kDirectGroups = 8192;
+// Above kDenseGroup beads a group on average (wide cells, or many beads in few of them) k_sort
+// leaves the move to k_move, which spreads it over the chip by slots.  Microseconds a step moved
+// by groups and by slots, water at density 3: 192 beads a group (unit cells, 24,000 beads) 22.9,
+// 26.1; 862 (186,000 beads) 64.1, 61.2, (862,000) 165.7, 170.4; 1,029 (222,000) 83.3, 73.3; 1,536
+// (98,000) 99.3, 79.1, (786,000) 229, 210.
+constexpr int kDenseGroup = 896;
 template <int MODE, bool MULTI>
 void sort_step_t(dpd_engine* e, bool advanced)
 {
@@ -1017,10 +1129,21 @@ void sort_step_t(dpd_engine* e, bool advanced)
         n > kAdvanceOnce ? launch_advance<MODE, MULTI, 2>(e, S, I) : launch_advance<MODE, MULTI, 1>(e, S, I);
     const bool scan = e->ngroups > kDirectGroups;
     if (scan) hipLaunchKernelGGL(k_group_scan, dim3(1), dim3(1024), 0, e->stream, e->ngroups, I.gcnt, e->gstart);
-    const int per = grid(e->ngroups, 8);
-    hipLaunchKernelGGL((k_sort<MODE, MULTI>), dim3(8 * per), dim3(256), 0, e->stream, n, e->ngroups, per, S, D, e->frc,
-                       e->vp, e->dboxes, B0, I, scan ? e->gstart : nullptr, e->cstart[e->cur ^ 1],
-                       e->counts[e->cur ^ 1], e->slot_of, e->upos, (MODE == kRebin || !vp_is_vel(e)) ? 1 : 0, e->dstep, e->order);
+    const int per = grid(e->ngroups, 8), write_vp = (MODE == kRebin || !vp_is_vel(e)) ? 1 : 0;
+    const int *gstart = scan ? e->gstart : nullptr;
+    int *cstart = e->cstart[e->cur ^ 1], *clear = e->counts[e->cur ^ 1];
+    const dim3 gr(8 * per), bl(256);
+    if (n > (int64_t)kDenseGroup * e->ngroups) {
+        hipLaunchKernelGGL((k_sort<MODE, MULTI, true>), gr, bl, 0, e->stream, n, e->ngroups, per, S, D, e->frc, e->vp,
+                           e->dboxes, B0, I, gstart, cstart, clear, e->slot_of, e->upos, write_vp, e->dstep, e->order);
+        const Move M{S, D, e->frc, e->vp, e->slot_of, e->upos, write_vp};
+        const int nb = grid(n, kMoveSlots), pm = grid(nb, 8);
+        hipLaunchKernelGGL((k_move<MODE, MULTI>), dim3(8 * pm), dim3(kMoveSlots), 0, e->stream, n, e->nkeys, nb, pm, M,
+                           e->dboxes, B0, I, cstart, reinterpret_cast<const int*>(e->order));
+    } else {
+        hipLaunchKernelGGL((k_sort<MODE, MULTI, false>), gr, bl, 0, e->stream, n, e->ngroups, per, S, D, e->frc, e->vp,
+                           e->dboxes, B0, I, gstart, cstart, clear, e->slot_of, e->upos, write_vp, e->dstep, e->order);
+    }
     e->cur ^= 1;
 }
 
