@@ -1918,21 +1918,10 @@ void launch_gather(dpd_engine* e, const float4* frc, double* x, double* u, doubl
         hipLaunchKernelGGL(k_gather<false>, gr, bl, 0, e->stream, n, bufs(e, e->cur), frc, e->dboxes, B0, x, u, v, f);
 }
 
-}  // namespace
-
-extern "C" {
-
-int dpd_compute_forces(dpd_engine* e, int64_t step, uint32_t flags, double* f_out, double* virial, double* pe)
+// dpd_compute_forces with the tables as they are
+int evaluate_forces(dpd_engine* e, int64_t step, double* f_out, double* virial, double* pe)
 {
-    if (!e) return DPD_ERR_PARAM;
-    if (!e->committed) return fail(e, DPD_ERR_STATE, "no beads uploaded");
-    HIPCHK(hipSetDevice(e->device));
     int rc;
-    std::vector<bool> saved;
-    if (flags & DPD_NO_THERMOSTAT) {
-        for (auto& b : e->boxes) { saved.push_back(b.thermostat_on); b.thermostat_on = false; }
-        if ((rc = upload_tables(e))) return rc;
-    }
     // beside the trajectory: force and time of the next dpd_step stay as they are
     hipLaunchKernelGGL(k_set_step, dim3(1), dim3(64), 0, e->stream, e->dstep + 1, step);
     // the uploaded state is sorted with vp = v: evaluate at it (after dpd_step, vp is the
@@ -1961,11 +1950,27 @@ int dpd_compute_forces(dpd_engine* e, int64_t step, uint32_t flags, double* f_ou
             pe[i] = 0.0;
             for (size_t b = 0; b < e->boxes.size(); ++b) pe[i] += h[b * kObsStride + O_PEP + i];
         }
-    if (flags & DPD_NO_THERMOSTAT) {
-        for (size_t b = 0; b < e->boxes.size(); ++b) e->boxes[b].thermostat_on = saved[b];
-        if ((rc = upload_tables(e))) return rc;
-    }
     return DPD_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int dpd_compute_forces(dpd_engine* e, int64_t step, uint32_t flags, double* f_out, double* virial, double* pe)
+{
+    if (!e) return DPD_ERR_PARAM;
+    if (!e->committed) return fail(e, DPD_ERR_STATE, "no beads uploaded");
+    HIPCHK(hipSetDevice(e->device));
+    if (!(flags & DPD_NO_THERMOSTAT)) return evaluate_forces(e, step, f_out, virial, pe);
+    // the thermostat is back whatever the evaluation ends with
+    std::vector<bool> saved;
+    for (auto& b : e->boxes) { saved.push_back(b.thermostat_on); b.thermostat_on = false; }
+    int rc = upload_tables(e);
+    if (!rc) rc = evaluate_forces(e, step, f_out, virial, pe);
+    for (size_t b = 0; b < e->boxes.size(); ++b) e->boxes[b].thermostat_on = saved[b];
+    const int back = upload_tables(e);
+    return rc ? rc : back;
 }
 
 int dpd_observables_box(dpd_engine* e, int32_t box, dpd_obs* out)
