@@ -214,7 +214,8 @@ int32_t dpd_get_schedule(const dpd_engine* e);
 int dpd_autotune_schedules(dpd_engine* e, int32_t nsteps, int32_t* chosen, double* ms_per_step);
 /* Apply a schedule recorded by the autotuner (a file of one JSON object per line, written
  * by dpd_amd.tune, keyed by the number of boxes (1, or 2 for any batch), beads per box as a
- * power-of-two range [beads_lo, beads_hi), bead types and whether there are bonds) to a
+ * power-of-two range [beads_lo, beads_hi), for a batch all beads as one [total_lo, total_hi)
+ * (a line without it holds for any), bead types and whether there are bonds) to a
  * committed engine of that shape; *chosen (may be NULL) gets the schedule set, -1 when the
  * file holds none for this shape (the engine is then left as it was). */
 int dpd_apply_tuning(dpd_engine* e, const char* path, int32_t* chosen);

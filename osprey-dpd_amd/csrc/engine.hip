@@ -2138,25 +2138,31 @@ int dpd_apply_tuning(dpd_engine* e, const char* path, int32_t* chosen)
     if (!fh) return fail(e, DPD_ERR_IO, std::string("cannot open ") + path);
     // the engine's shape, as dpd_amd.tune keys it
     const int64_t nbox = (int64_t)e->boxes.size();
-    const int64_t per = std::max<int64_t>(1, e->n / nbox);
-    int64_t lo = 1;
-    while (lo * 2 <= per) lo *= 2;
-    const int64_t key[5] = {nbox == 1 ? 1 : 2, lo, 2 * lo, e->boxes[0].p.ntypes, (e->nbonds + e->nangles) > 0};
-    const char* names[6] = {"\"nbox\":", "\"beads_lo\":", "\"beads_hi\":", "\"ntypes\":", "\"bonded\":", "\"schedule\":"};
+    auto bucket = [](int64_t n) {
+        int64_t lo = 1;
+        while (lo * 2 <= n) lo *= 2;
+        return lo;
+    };
+    const int64_t lo = bucket(e->n / nbox), tot = bucket(e->n);
+    const int64_t key[7] = {nbox == 1 ? 1 : 2, lo, 2 * lo, e->boxes[0].p.ntypes, (e->nbonds + e->nangles) > 0, tot, 2 * tot};
+    const char* names[8] = {"\"nbox\":",   "\"beads_lo\":", "\"beads_hi\":", "\"ntypes\":",
+                            "\"bonded\":", "\"total_lo\":", "\"total_hi\":", "\"schedule\":"};
     char line[4096];
     int found = -1;
     while (found < 0 && std::fgets(line, sizeof(line), fh)) {
-        int64_t v[6];
+        int64_t v[8];
         bool ok = true;
-        for (int k = 0; k < 6 && ok; ++k) {
+        for (int k = 0; k < 8 && ok; ++k) {
             const char* p = std::strstr(line, names[k]);
-            if (!p) { ok = false; break; }
-            v[k] = std::strtoll(p + std::strlen(names[k]), nullptr, 10);
+            if (p) v[k] = std::strtoll(p + std::strlen(names[k]), nullptr, 10);
+            // all beads of a batch: a line without them holds for any, and one box has its own
+            else if (k == 5 || k == 6) v[k] = key[k];
+            else ok = false;
         }
         if (!ok) continue;
         bool match = true;
-        for (int k = 0; k < 5; ++k) match = match && v[k] == key[k];
-        if (match && v[5] >= 0 && v[5] < kSchedules) found = (int)v[5];
+        for (int k = 0; k < (nbox == 1 ? 5 : 7); ++k) match = match && v[k] == key[k];
+        if (match && v[7] >= 0 && v[7] < kSchedules) found = (int)v[7];
     }
     std::fclose(fh);
     if (found >= 0) {

@@ -609,6 +609,9 @@ constexpr int kDefaultSchedule = 2;
 // water 10.1k beads 19.9, 20.5; 12.3k 21.8, 20.8; 98k 41.2, 31.8, 32.0; 108k 43, 38.0, 31.9,
 // 32.8; 256k -, -, 42.0, 42.8; 273k -, -, 54.7, 47.0; chains 41k 24.5, 25.8; 66k 31.1, 30.1;
 // 89k 37, 34.0, 35.7; 118k 43, 41.3, 36.7; 256k -, -, 47.0, 49.0; 292k -, -, 59.6, 52.3.
+// A batch goes by all its beads, however many boxes they are in (bonded, boxes of 11,300 each: 4
+// of them 31.6, 34.4, 39.4, 40.2; 8 42.0, 41.0, 43.6, 43.9; 16 63, 58.6, 51.3, 52.0; 24 86, 78,
+// 72.9, 65.4).
 constexpr int size_schedule(int64_t n, bool bonded)
 {
     return n <= (bonded ? 50000 : 11000) ? 6 : (n <= 100000 ? 5 : (n <= 4 * 1024 * 64 ? 3 : kDefaultSchedule));
