@@ -1334,6 +1334,8 @@ int commit_beads(dpd_engine* e, int64_t step0)
     }
     if (n > ((int64_t)1 << 30) || (int64_t)nbr * kGroupKeys > ((int64_t)1 << 30))
         return fail(e, DPD_ERR_PARAM, "batch too large");
+    // from here on what the device holds changes: without a state until all of it is there
+    e->committed = false;
     drop_graphs(e);
     int rc;
     // hit-list workgroups of a batch: slots of one box each (a box's beads are the slots
@@ -1371,15 +1373,18 @@ int commit_beads(dpd_engine* e, int64_t step0)
         e->cleared = nk + 2 * ng;
         if ((rc = clear_counts(e))) return rc;
     }
-    if (new_cells || n != e->n || !e->filed) {
+    // (a call that ended without the arrays by bead left n at 0)
+    const bool new_beads = n != e->n;
+    if (new_cells || new_beads) {
         // spill (int4 a bead), order (int2 a bead), bins
+        e->n = 0;
         const size_t nbins = bin_at((int)n, e->nkeys);
         if ((rc = dalloc(e, &e->filed, (6 * (size_t)n + nbins + 3) / 4))) return rc;
         e->spill = e->filed;
         e->order = reinterpret_cast<int2*>(e->filed + n);
         e->bins = reinterpret_cast<int*>(e->order + n);
     }
-    if (n != e->n) {
+    if (new_beads) {
         std::vector<Part> parts;
         for (int b = 0; b < 2; ++b)
             for (const Part& q : {part(&e->pos[b], n), part(&e->vel[b], n), part(&e->fold[b], n), part(&e->bead[b], n),
@@ -1390,8 +1395,8 @@ int commit_beads(dpd_engine* e, int64_t step0)
             parts.push_back(q);
         if ((rc = dalloc_parts(e, &e->per_bead, parts))) return rc;
         for (int b = 0; b < 2; ++b) HIPCHK(hipMemsetAsync(e->code[b] + n, 0, sizeof(uint32_t) * kCodePad, e->stream));
-        e->n = n;
     }
+    e->n = n;
     if ((rc = upload_boxes(e))) return rc;
     std::vector<float4> hp(n), hv(n), hf(n);
     std::vector<int> hb(n);
@@ -1516,6 +1521,7 @@ int commit_topology(dpd_engine* e)
         }
     drop_graphs(e);
     int rc;
+    e->committed = false;   // (until the topology and the beads' marks agree)
     e->nbonded = 0;
     const size_t nb = bonded.size();
     if ((rc = dalloc(e, &e->bond_ent, bent.size())) || (rc = dalloc(e, &e->bond_par, bpar.size())) ||
@@ -1544,6 +1550,7 @@ int commit_topology(dpd_engine* e)
     mark_bonded(e);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(e->stream));
+    e->committed = true;
     return DPD_OK;
 }
 
