@@ -804,6 +804,7 @@ int dpd_mlp_train(dpd_mlp* m, int64_t n, const double* x, const double* y, int32
     int rc;
     if ((rc = ensure_rows(m, Mp, true)) || (rc = upload_batch(m, n, x, y, Mp))) return rc;
     if (m->loss_cap < iters) {
+        m->loss_cap = 0;
         if ((rc = malloc_dev(m, &m->loss, iters))) return rc;
         m->loss_cap = iters;
     }

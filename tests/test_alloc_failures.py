@@ -1,7 +1,7 @@
 """Device memory that runs out, without a GPU: the library's host code runs on a stand-in for the
 HIP runtime (hip_stub.c) whose k-th allocation fails, for every k a call makes.  A call that
 fails says so, leaves an engine without a state (no later call uses arrays that are gone or too
-small), and the same engine takes the next upload."""
+small), and the same engine or network takes the next."""
 import os
 import subprocess
 import sys
@@ -88,6 +88,33 @@ print("allocations:", n)
 assert n > 8
 """
 
+NETWORK = PRELUDE + """
+from dpd_amd.mlp import MLPError, Surrogate
+X, Y = rng.normal(0, 1, (40, 7)), rng.normal(0, 1, (40, 2))
+k = 0
+while True:
+    m = Surrogate(7, 32, 2)
+    m.train(X[:20], Y[:20], iters=4)
+    stub.stub_fail(k)
+    try:
+        m.train(X, Y, iters=9)
+        done = True
+    except MLPError:
+        done = False
+    stub.stub_fail(-1)
+    # (fewer rows and iterations than the call that failed had made room for)
+    m.train(X[:20], Y[:20], iters=4)
+    m.gradients(X, Y)
+    m.predict(X)
+    assert stub.stub_outside() == 0, k
+    m.close()
+    if done:
+        break
+    k += 1
+print("allocations:", k)
+assert k > 10
+"""
+
 
 @pytest.fixture(scope="module")
 def stub(tmp_path_factory):
@@ -96,7 +123,7 @@ def stub(tmp_path_factory):
     return path
 
 
-@pytest.mark.parametrize("script", [BEADS, BATCH], ids=["one-box", "batch"])
-def test_engine_after_a_failed_upload(stub, script):
+@pytest.mark.parametrize("script", [BEADS, BATCH, NETWORK], ids=["one-box", "batch", "network"])
+def test_after_a_failed_call(stub, script):
     r = subprocess.run([sys.executable, "-c", script, stub, ROOT], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
