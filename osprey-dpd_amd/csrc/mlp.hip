@@ -1,6 +1,6 @@
 // mlp.hip -- surrogate network: BF16 matrix-core forward/backward and FP32 Adam on gfx950.
 //
-// Two kernels an iteration.  k_mlp_rows takes 16 rows of the batch through the whole forward
+// Two launches an iteration (three for few rows of a wide network).  k_mlp_rows takes 16 rows of the batch through the whole forward
 // and backward chain (a workgroup, activations in registers and one LDS buffer) and leaves the
 // factors of the weight gradients; k_mlp_update makes every gradient entry and applies Adam to
 // it.  Every matrix product runs on v_mfma_f32_16x16x16_bf16 (BF16 operands, FP32
@@ -142,6 +142,7 @@ struct RowArgs {
     // training: the gradients' factors as fragments over the rows, and in FP32 for the biases
     uint16_t *H1F, *H2F, *dZ1F, *dZ2F, *dYF;
     float *dZ1, *dZ2, *dY;
+    float* h2;                   // in two launches: the second hidden layer between them
     double* loss;
     // prediction: y[n][nout]
     double* out;
@@ -151,7 +152,15 @@ struct RowArgs {
 // Rows [16 b, 16 b + 16) through the network and, with TRAIN, back: WAVES wavefronts, wavefront
 // w computing the 16-column tiles w, w + WAVES, ... (TPW of them at most) of every hidden layer.
 // One LDS buffer holds the layer that the next product reads; the weights come from L2.
-template <int WAVES, int TPW, bool TRAIN>
+// PART: few rows of a wide network in two launches (training, TPW 1), a row block's tiles of the
+// two large products spread over blockIdx.y.  kToHidden goes to the second hidden layer,
+// kFromHidden from there; what comes before its product every workgroup does itself, and the first
+// one stores.  In one launch these rows wait for the weights on their way into one compute unit
+// (1,024 units: 4 MB in some 75 us); an iteration of 16 rows takes 45 us instead of 89 at 1,024
+// units, 38 instead of 69 at 768 and 31 instead of 52 at 528 (a kernel for each product took 74, 67
+// and 65), with the same results to the bit.
+enum Part { kWhole, kToHidden, kFromHidden };
+template <int WAVES, int TPW, bool TRAIN, Part PART = kWhole>
 __global__ __launch_bounds__(64 * WAVES) void k_mlp_rows(RowArgs A)
 {
     extern __shared__ __align__(16) uint16_t act[];   // [16][H + 4]
@@ -162,18 +171,23 @@ __global__ __launch_bounds__(64 * WAVES) void k_mlp_rows(RowArgs A)
     const int H = A.H, nt = H >> 4, ld = H + 4, Mp = A.Mp;
     const int row0 = blockIdx.x * 16;
     const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+    static_assert(PART == kWhole || (TRAIN && TPW == 1), "two launches: one tile a wavefront");
+    const bool whole = PART == kWhole, stores = whole || blockIdx.y == 0;
+    // the first of this wavefront's tiles
+    const int w0 = whole ? w : (int)blockIdx.y * WAVES + w;
     float h1[TPW][4], h2[TPW][4];
     // this lane's place in this workgroup's fragment of a tile of columns
     auto mine = [&](int tile) { return (((size_t)tile * (Mp >> 4) + blockIdx.x) * 64 + lane) * 4; };
-    auto hidden = [&](int tile, const floatx4& z, const float* bias, float (&h)[4], uint16_t* HF) {
+    auto hidden = [&](int tile, const floatx4& z, const float* bias, float (&h)[4], uint16_t* HF, bool keep = true,
+                      bool store = true) {
         const int n = tile * 16 + r;
         const float b = bias[n];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             h[i] = row0 + q + i < A.n ? tanhf(z[i] + b) : 0.0f;
-            act[(q + i) * ld + n] = f2bf(h[i]);
+            if (keep) act[(q + i) * ld + n] = f2bf(h[i]);
         }
-        if (TRAIN) *reinterpret_cast<uint2*>(HF + mine(tile)) = pack4(h);
+        if (TRAIN && store) *reinterpret_cast<uint2*>(HF + mine(tile)) = pack4(h);
     };
     // act (16 x H) times a weight matrix's fragments: this wavefront's tiles
     auto product = [&](const uint16_t* WF, floatx4 (&s)[TPW]) {
@@ -181,7 +195,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_mlp_rows(RowArgs A)
             floatx4 acc[TPW];
 #pragma unroll
             for (int j = 0; j < TPW; ++j) acc[j] = zero;
-            in_steps(z * A.k2.per, min(H, (z + 1) * A.k2.per), [&](auto steps, int k) {
+            auto some = [&](auto steps, int k) {
                 constexpr int U = decltype(steps)::value;
                 bf16x4 b[U][TPW];
 #pragma unroll
@@ -189,7 +203,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_mlp_rows(RowArgs A)
 #pragma unroll
                     for (int j = 0; j < TPW; ++j) {
                         // (a wavefront without this tile repeats the last one)
-                        const int tile = min(w + WAVES * j, nt - 1);
+                        const int tile = min(w0 + WAVES * j, nt - 1);
                         b[u][j] = frag(WF + (((size_t)tile * nt + (k >> 4) + u) * 64 + lane) * 4);
                     }
 #pragma unroll
@@ -198,27 +212,48 @@ __global__ __launch_bounds__(64 * WAVES) void k_mlp_rows(RowArgs A)
 #pragma unroll
                     for (int j = 0; j < TPW; ++j) acc[j] = mfma(a, b[u][j], acc[j]);
                 }
-            });
+            };
+            const int k0 = z * A.k2.per, k1 = min(H, (z + 1) * A.k2.per);
+            if constexpr (PART == kWhole) in_steps(k0, k1, some);
+            else in_rounds(k0 >> 4, k1 >> 4, [&](auto steps, int s16) { some(steps, 16 * s16); });
 #pragma unroll
             for (int j = 0; j < TPW; ++j) s[j] = z ? s[j] + acc[j] : acc[j];
         }
     };
     // hidden layer 1
-    {
-        const bf16x4 a = frag(A.X + (size_t)(row0 + r) * 16 + q);
+    auto layer1 = [&](int tile) {
+        return mfma(frag(A.X + (size_t)(row0 + r) * 16 + q), frag(A.W1 + (tile * 64 + lane) * 4), zero);
+    };
+    floatx4 s[TPW];
+    if constexpr (PART == kWhole) {
 #pragma unroll
         for (int j = 0; j < TPW; ++j) {
             const int tile = w + WAVES * j;
-            if (tile < nt) hidden(tile, mfma(a, frag(A.W1 + (tile * 64 + lane) * 4), zero), A.b1, h1[j], A.H1F);
+            if (tile < nt) hidden(tile, layer1(tile), A.b1, h1[j], A.H1F);
+        }
+        __syncthreads();
+        product(A.W2, s);
+        __syncthreads();   // act is read no more
+#pragma unroll
+        for (int j = 0; j < TPW; ++j)
+            if (w + WAVES * j < nt) hidden(w + WAVES * j, s[j], A.b2, h2[j], A.H2F);
+    } else if constexpr (PART == kToHidden) {
+        for (int tile = w; tile < nt; tile += WAVES) hidden(tile, layer1(tile), A.b1, h1[0], A.H1F, true, stores);
+        __syncthreads();
+        product(A.W2, s);
+        if (w0 < nt) {
+            hidden(w0, s[0], A.b2, h2[0], A.H2F, false);
+            *reinterpret_cast<float4*>(A.h2 + mine(w0)) = make_float4(h2[0][0], h2[0][1], h2[0][2], h2[0][3]);
+        }
+        return;
+    } else {
+        for (int tile = w; tile < nt; tile += WAVES) {
+            const float4 h = *reinterpret_cast<const float4*>(A.h2 + mine(tile));
+            const float v[4] = {h.x, h.y, h.z, h.w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) act[(q + i) * ld + tile * 16 + r] = f2bf(v[i]);
         }
     }
-    __syncthreads();
-    floatx4 s[TPW];
-    product(A.W2, s);
-    __syncthreads();   // act is read no more
-#pragma unroll
-    for (int j = 0; j < TPW; ++j)
-        if (w + WAVES * j < nt) hidden(w + WAVES * j, s[j], A.b2, h2[j], A.H2F);
     __syncthreads();
     // output layer: a part of its sum per wavefront
     for (int z = w; z < A.k3.parts; z += WAVES) {
@@ -245,8 +280,10 @@ __global__ __launch_bounds__(64 * WAVES) void k_mlp_rows(RowArgs A)
             const float e = valid ? y - A.T[(size_t)row * A.nout + n] : 0.0f;
             const float g = e / (float)(A.n * A.nout);
             dyb[m][n] = f2bf(g);
-            A.dYF[(size_t)blockIdx.x * 256 + t] = f2bf(g);
-            A.dY[(size_t)blockIdx.x * 256 + t] = g;
+            if (stores) {
+                A.dYF[(size_t)blockIdx.x * 256 + t] = f2bf(g);
+                A.dY[(size_t)blockIdx.x * 256 + t] = g;
+            }
             l = valid ? 0.5 * (double)e * (double)e / (double)(A.n * A.nout) : 0.0;
         } else if (valid) {
 #pragma clang fp contract(off)
@@ -258,13 +295,13 @@ __global__ __launch_bounds__(64 * WAVES) void k_mlp_rows(RowArgs A)
     for (int off = 32; off > 0; off >>= 1) l += __shfl_down(l, off, 64);
     if (lane == 0) lsum[w] = l;
     __syncthreads();
-    if (t == 0) {
+    if (t == 0 && stores) {
         double v = 0.0;
         for (int i = 0; i < WAVES; ++i) v += lsum[i];
         atomicAdd(A.loss, v);
     }
     // back through the output layer
-    auto back = [&](int tile, const floatx4& dh, const float (&h)[4], bool keep, uint16_t* dZF, float* dZ) {
+    auto back = [&](int tile, const floatx4& dh, const float (&h)[4], bool keep, uint16_t* dZF, float* dZ, bool store = true) {
         const int n = tile * 16 + r;
         float g[4];
 #pragma unroll
@@ -272,22 +309,32 @@ __global__ __launch_bounds__(64 * WAVES) void k_mlp_rows(RowArgs A)
             g[i] = dh[i] * (1.0f - h[i] * h[i]);
             if (keep) act[(q + i) * ld + n] = f2bf(g[i]);
         }
+        if (!store) return;
         *reinterpret_cast<uint2*>(dZF + mine(tile)) = pack4(g);
         *reinterpret_cast<float4*>(dZ + mine(tile)) = make_float4(g[0], g[1], g[2], g[3]);
     };
-    {
-        const bf16x4 a = frag(&dyb[r][q]);
+    const bf16x4 dy = frag(&dyb[r][q]);
+    auto layer3 = [&](int tile) { return mfma(dy, frag(A.W3t + (tile * 64 + lane) * 4), zero); };
+    if constexpr (PART == kWhole) {
 #pragma unroll
         for (int j = 0; j < TPW; ++j) {
             const int tile = w + WAVES * j;
-            if (tile < nt) back(tile, mfma(a, frag(A.W3t + (tile * 64 + lane) * 4), zero), h2[j], true, A.dZ2F, A.dZ2);
+            if (tile < nt) back(tile, layer3(tile), h2[j], true, A.dZ2F, A.dZ2);
+        }
+    } else {
+        for (int tile = w; tile < nt; tile += WAVES) {
+            const float4 h = *reinterpret_cast<const float4*>(A.h2 + mine(tile));
+            const float v[4] = {h.x, h.y, h.z, h.w};
+            back(tile, layer3(tile), v, true, A.dZ2F, A.dZ2, stores);
         }
     }
     __syncthreads();
     product(A.W2t, s);
+    if constexpr (PART != kWhole)
+        if (w0 < nt) hidden(w0, layer1(w0), A.b1, h1[0], A.H1F, false, false);
 #pragma unroll
     for (int j = 0; j < TPW; ++j)
-        if (w + WAVES * j < nt) back(w + WAVES * j, s[j], h1[j], false, A.dZ1F, A.dZ1);
+        if (w0 + WAVES * j < nt) back(w0 + WAVES * j, s[j], h1[j], false, A.dZ1F, A.dZ1);
 }
 
 struct UpdateArgs {
@@ -475,7 +522,7 @@ struct dpd_mlp {
     // gradients are made of; its raw rows
     int cap = 0, train_cap = 0;
     uint16_t *X = nullptr, *XF = nullptr, *H1F = nullptr, *H2F = nullptr, *dZ1F = nullptr, *dZ2F = nullptr, *dYF = nullptr;
-    float *T = nullptr, *dZ1 = nullptr, *dZ2 = nullptr, *dY = nullptr;
+    float *T = nullptr, *dZ1 = nullptr, *dZ2 = nullptr, *dY = nullptr, *h2 = nullptr;
     double *raw = nullptr, *out = nullptr;
     double* loss = nullptr;
     int loss_cap = 0;
@@ -525,6 +572,15 @@ Layout layout(const dpd_mlp* m)
     return L;
 }
 
+// Training of few rows of a wide network takes k_mlp_rows in two launches: of more than kWideUnits
+// units, up to as many rows as leave every workgroup of the two a compute unit of its own.  us an
+// iteration in one launch and in two: 100 rows of 528 units 54, 33, 800 56, 35; 600 of 768 73, 41;
+// 500 of 1,024 96, 50.  (At 512 units one launch was at 37 for 512 rows and never behind a kernel
+// for each product; nor was it past the line, 700 rows of 768 73 and 147, 600 of 1,024 97 and 164.)
+constexpr int kWideUnits = 512, kFewWaves = 8;
+inline int few_parts(int H) { return (H / 16 + kFewWaves - 1) / kFewWaves; }
+inline int few_rows(int H) { return 256 / few_parts(H) * 16; }
+
 // room for `rows` padded rows; what only training needs when it is first asked for
 int ensure_rows(dpd_mlp* m, int rows, bool train)
 {
@@ -542,7 +598,8 @@ int ensure_rows(dpd_mlp* m, int rows, bool train)
         const size_t h = (size_t)rows * m->H, o = (size_t)rows * 16;
         if ((rc = malloc_dev(m, &m->H1F, h)) || (rc = malloc_dev(m, &m->H2F, h)) || (rc = malloc_dev(m, &m->dZ1F, h)) ||
             (rc = malloc_dev(m, &m->dZ2F, h)) || (rc = malloc_dev(m, &m->dYF, o)) || (rc = malloc_dev(m, &m->dZ1, h)) ||
-            (rc = malloc_dev(m, &m->dZ2, h)) || (rc = malloc_dev(m, &m->dY, o)))
+            (rc = malloc_dev(m, &m->dZ2, h)) || (rc = malloc_dev(m, &m->dY, o)) ||
+            (rc = malloc_dev(m, &m->h2, m->H > kWideUnits ? (size_t)std::min(rows, few_rows(m->H)) * m->H : 0)))
             return rc;
         m->train_cap = rows;
     }
@@ -593,15 +650,23 @@ void launch_rows(dpd_mlp* m, int n, int Mp, double* loss)
     a.b1 = m->w + L.b1; a.b2 = m->w + L.b2; a.b3 = m->w + L.b3;
     a.H1F = m->H1F; a.H2F = m->H2F; a.dZ1F = m->dZ1F; a.dZ2F = m->dZ2F; a.dYF = m->dYF;
     a.dZ1 = m->dZ1; a.dZ2 = m->dZ2; a.dY = m->dY;
+    a.h2 = m->h2;
     a.loss = loss;
     a.out = m->out;
     a.S = scaling(m);
     // Eight wavefronts a workgroup where there is one tile of columns for each, or where
     // workgroups wait for a compute unit anyway; otherwise sixteen, which halve the chain of
-    // each (training, 16 against 8: 1,638 rows of 256 13.8 / 16.1 us, 500 of 512 25.5 / 30.1,
-    // 300 of 1,024 74 / 78; 20,000 of 256 45.6 / 43.3, 6,000 of 512 51.7 / 45.1).
+    // each (training, 16 against 8: 1,638 rows of 256 13.8 / 16.1 us, 500 of 512 25.5 / 30.1;
+    // 20,000 of 256 45.6 / 43.3, 6,000 of 512 51.7 / 45.1).
     const int tiles = m->H / 16;
     const bool train = loss != nullptr, many = Mp / 16 > 256;
+    if (train && m->H > kWideUnits && Mp <= few_rows(m->H)) {
+        const dim3 grid(Mp / 16, few_parts(m->H)), block(64 * kFewWaves);
+        const size_t lds = sizeof(uint16_t) * 16 * (m->H + 4);
+        hipLaunchKernelGGL((k_mlp_rows<kFewWaves, 1, true, kToHidden>), grid, block, lds, m->stream, a);
+        hipLaunchKernelGGL((k_mlp_rows<kFewWaves, 1, true, kFromHidden>), grid, block, lds, m->stream, a);
+        return;
+    }
     if (tiles <= 8) launch_rows_t<8, 1>(a, train, m->stream);
     else if (tiles <= 16) many ? launch_rows_t<8, 2>(a, train, m->stream) : launch_rows_t<16, 1>(a, train, m->stream);
     else if (tiles <= 32) many ? launch_rows_t<8, 4>(a, train, m->stream) : launch_rows_t<16, 2>(a, train, m->stream);
@@ -720,7 +785,7 @@ void dpd_mlp_destroy(dpd_mlp* m)
     if (!m) return;
     if (m->stream) (void)hipStreamSynchronize(m->stream);
     void* ptrs[] = {m->w, m->grad, m->mom, m->var, m->mask, m->wf, m->wt, m->X, m->XF, m->T, m->raw, m->out, m->H1F,
-                    m->H2F, m->dZ1F, m->dZ2F, m->dYF, m->dZ1, m->dZ2, m->dY, m->loss};
+                    m->H2F, m->dZ1F, m->dZ2F, m->dYF, m->dZ1, m->dZ2, m->dY, m->h2, m->loss};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     if (m->stream) (void)hipStreamDestroy(m->stream);
