@@ -1362,7 +1362,7 @@ int commit_beads(dpd_engine* e, int64_t step0)
         e->ngroups = nbr;
         e->nkeys = nbr * kGroupKeys;
         // (each part starts at a multiple of four: the counts are read four at a time)
-        const size_t nk = (size_t)e->nkeys, ng = (size_t)(nbr + 4) / 4 * 4, nc = (nk + 1 + kCstartPad + 3) / 4 * 4;
+        const size_t nk = (size_t)e->nkeys, ng = (size_t)(nbr + 4) / 4 * 4, nc = (nk + 1 + 3) / 4 * 4;
         if ((rc = dalloc(e, &e->cells, nk + 3 * ng + 2 * nc))) return rc;
         e->cnt = e->cells;
         e->counts[0] = e->cells + nk;

@@ -320,10 +320,10 @@ __device__ inline uint64_t run_lanes(uint64_t starts)
 // whole wavefront, by every lane with the `from` of a slot of its own or its neighbours.  Slots
 // are cell-sorted and few beads leave their cell, so the lanes of a run of equal `from` whose
 // bead stays are counted with one atomic, and so are those of a run of equal groups; a bead that
-// leaves counts by itself.  (One atomic per bead would serialise: an atomic on a shared address
-// costs about 100 ns in turn.  The pair launch of 96^3 cells took 451 us that way against 268
-// with a loop over the wavefront's distinct keys, whose 300 instructions were 8% of the launch;
-// 252 us with runs.)
+// leaves counts by itself.  (One atomic per bead would serialise: those on one address, the
+// 192 of a scan group's count, take 12 to 15 ns each in turn.  The pair launch of 96^3 cells took
+// 451 us that way against 268 with a loop over the wavefront's distinct keys, whose 300
+// instructions were 8% of the launch; 252 us with runs.)
 __device__ inline void file_bead(const Intake& I, int from, int to, int s, bool act)
 {
     int start = 0, room = 0;
@@ -356,13 +356,15 @@ __device__ inline void file_bead(const Intake& I, int from, int to, int s, bool 
 
 // Accumulators of a call's sums: each box has spread + 1 rows of kObsStride (spread + 1 a power
 // of two), of which a workgroup adds to one; k_report adds the rows up.  FP64 atomics on one
-// address take about 15 ns in turn: with one row the 10,368 workgroups of k_finish took 134 us in
-// a 96^3 box, 42 with sixteen.
+// address take 12 to 15 ns in turn: with one row the 10,368 workgroups of k_finish took 134 us in
+// a 96^3 box, 42 with sixteen.  Batches of more than kSpreadBoxes boxes have one row a box (256
+// bytes; k_report reads a row for each): their workgroups spread over the boxes, and where these
+// are large they wait, in k_finish of 17 boxes of 48^3 99 us, 77 for 16 of them with 16 rows.
 struct Sums {
     double* acc;
     int spread;
 };
-constexpr int kSpread = 15;   // (engines of up to kSpreadBoxes boxes; more share no rows anyway)
+constexpr int kSpread = 15;
 constexpr int kSpreadBoxes = 16;
 
 // Add per-thread FP64 values v[0..N) to slots base .. base + N - 1 of the threads' boxes (< 0:

@@ -1,13 +1,13 @@
 // mlp.hip -- surrogate network: BF16 matrix-core forward/backward and FP32 Adam on gfx950.
 //
-// Two launches an iteration (three for few rows of a wide network).  k_mlp_rows takes 16 rows of the batch through the whole forward
-// and backward chain (a workgroup, activations in registers and one LDS buffer) and leaves the
-// factors of the weight gradients; k_mlp_update makes every gradient entry and applies Adam to
-// it.  Every matrix product runs on v_mfma_f32_16x16x16_bf16 (BF16 operands, FP32
-// accumulation).  Operand fragment layout of that instruction for lane l (0..63): A holds
-// A[l%16][4(l/16) .. 4(l/16)+3], B holds B[4(l/16) .. 4(l/16)+3][l%16], and the accumulator
-// holds C[4(l/16)+i][l%16], i = 0..3.  Everything a product reads from memory is stored as
-// fragments: 64 lanes x 4 values, [16 columns][16 of k][lane][4], one 512-byte load per
+// Two launches an iteration (three for few rows of a wide network).  k_mlp_rows takes 16 rows of
+// the batch through the whole forward and backward chain (a workgroup, activations in registers
+// and one LDS buffer) and leaves the factors of the weight gradients; k_mlp_update makes every
+// gradient entry and applies Adam to it.  Every matrix product runs on v_mfma_f32_16x16x16_bf16
+// (BF16 operands, FP32 accumulation).  Operand fragment layout of that instruction for lane l
+// (0..63): A holds A[l%16][4(l/16) .. 4(l/16)+3], B holds B[4(l/16) .. 4(l/16)+3][l%16], and the
+// accumulator holds C[4(l/16)+i][l%16], i = 0..3.  Everything a product reads from memory is
+// stored as fragments: 64 lanes x 4 values, [16 columns][16 of k][lane][4], one 512-byte load per
 // wavefront.  A result leaves in that layout too, as the fragment of a product over its rows,
 // which is what the weight gradients are.  Weights are kept in BF16 as fragments of W and, for
 // the way back, of W transposed.

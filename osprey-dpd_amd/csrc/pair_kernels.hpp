@@ -168,11 +168,8 @@ typedef __attribute__((address_space(3))) uint32_t lds_u32;
 typedef uint32_t code2_t __attribute__((ext_vector_type(2), aligned(4)));
 // four scan codes from one 4-byte-aligned 16-byte load
 typedef uint32_t code4_t __attribute__((ext_vector_type(4), aligned(4)));
-// cell starts: a row's four and two, from 4-byte-aligned loads
-typedef int int4u __attribute__((ext_vector_type(4), aligned(4)));
+// a cell's start and end, from one 4-byte-aligned load
 typedef int int2u __attribute__((ext_vector_type(2), aligned(4)));
-// entries of padding after the cell starts (a row's four are loaded at once)
-constexpr int kCstartPad = 4;
 
 // The candidate test in integer code units (u = w / kCodeUnits): the four bytes of code minus
 // code, as one 32-bit difference, squared and added by one v_dot4_i32_i8.  Bytes hold positions
