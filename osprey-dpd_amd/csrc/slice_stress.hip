@@ -15,7 +15,7 @@
 // pairs in a window of the slices that one layer of cells reaches (a workgroup takes slots of
 // one z layer at a time, and the slots are sorted by z), bonds and bond pairs in windows of
 // the whole table.  Bilayer 48x48x32, 221k beads, 64 slices (global atomics per pair and bond
-// -> now): pairs 13,700 -> 80 us, bonds 715 -> 15, bond pairs 1,767 -> 28.  The atomics are
+// -> now): pairs 13,700 -> 88 us, bonds 715 -> 15, bond pairs 1,767 -> 28.  The atomics are
 // then 30 us of the pairs; the rest is their scan and evaluation, with few wavefronts to hide a
 // load (177 us with one position loaded at a time and lists of 12 that a lane evaluated alone
 // whenever they were full).
