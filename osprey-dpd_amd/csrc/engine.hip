@@ -849,7 +849,10 @@ struct BoxHost {
     bool has_f = false;
     std::vector<int32_t> bh, bt, pf, ps;
     std::vector<double> bk, bl0, pk, pphi;
-    int64_t bead_off = 0;
+    // what the device holds of it, which is not what is staged until the next commit: its beads
+    // from bead_off on, its bonds and bond pairs from bond_off and pair_off on
+    int64_t bead_off = 0, nbeads = 0;
+    int bond_off = 0, nbonds = 0, pair_off = 0, npairs = 0;
 };
 
 struct dpd_engine {
@@ -1258,7 +1261,7 @@ int finish_obs(dpd_engine* e)
         const dpd_params& p = e->boxes[b].p;
         dpd_obs& o = e->obs[b];
         o.step = e->step;
-        o.nbeads = e->boxes[b].n;
+        o.nbeads = e->boxes[b].nbeads;
         const double V = (double)p.nx * p.wx * (double)p.ny * p.wy * (double)p.nz * p.wz;
         for (int d = 0; d < 3; ++d) { o.sum_v2[d] = a[O_V2 + d]; o.momentum[d] = a[O_MOM + d]; }
         for (int i = 0; i < 9; ++i) o.stress[i] = a[O_VIR + i] / V;
@@ -1320,23 +1323,31 @@ int enqueue_steps(dpd_engine* e, int64_t nsteps, bool obs, int timing)
 // Assemble the staged boxes into device buffers and sort them.
 int commit_beads(dpd_engine* e, int64_t step0)
 {
-    int64_t n = 0;
-    int nbr = 0;
+    int64_t n = 0, groups = 0;
     for (size_t b = 0; b < e->boxes.size(); ++b) {
-        BoxHost& h = e->boxes[b];
+        const BoxHost& h = e->boxes[b];
         if (h.n == 0) return fail(e, DPD_ERR_STATE, "box " + std::to_string(b) + " has no beads");
-        h.bead_off = n;
-        h.B.koff = nbr * kGroupKeys;
-        h.B.goff = nbr;
-        h.B.box = (int)b;
-        nbr += h.B.ngroups;
+        groups += h.B.ngroups;
         n += h.n;
     }
-    if (n > ((int64_t)1 << 30) || (int64_t)nbr * kGroupKeys > ((int64_t)1 << 30))
+    if (n > ((int64_t)1 << 30) || groups * kGroupKeys > ((int64_t)1 << 30))
         return fail(e, DPD_ERR_PARAM, "batch too large");
     // from here on what the device holds changes: without a state until all of it is there
     e->committed = false;
     drop_graphs(e);
+    const int nbr = (int)groups;
+    n = groups = 0;
+    for (size_t b = 0; b < e->boxes.size(); ++b) {
+        BoxHost& h = e->boxes[b];
+        h.bead_off = n;
+        h.nbeads = h.n;
+        h.bond_off = h.nbonds = h.pair_off = h.npairs = 0;
+        h.B.koff = (int)groups * kGroupKeys;
+        h.B.goff = (int)groups;
+        h.B.box = (int)b;
+        groups += h.B.ngroups;
+        n += h.n;
+    }
     int rc;
     // hit-list workgroups of a batch: slots of one box each (a box's beads are the slots
     // [bead_off, bead_off + n) since the sort keys are ordered by box)
@@ -1470,9 +1481,13 @@ int commit_topology(dpd_engine* e)
     std::vector<int> bp(n + 1, 0), ap(n + 1, 0);
     std::vector<int> H, Tl, F, Sd;
     std::vector<double> K, L0, M, P;
-    for (const BoxHost& h : e->boxes) {
+    for (BoxHost& h : e->boxes) {
         const int off = (int)h.bead_off;
         const int boff = (int)H.size();
+        h.bond_off = boff;
+        h.nbonds = (int)h.bh.size();
+        h.pair_off = (int)F.size();
+        h.npairs = (int)h.pf.size();
         for (size_t b = 0; b < h.bh.size(); ++b) {
             H.push_back(h.bh[b] + off); Tl.push_back(h.bt[b] + off);
             K.push_back(h.bk[b]); L0.push_back(h.bl0[b]);
@@ -1667,13 +1682,12 @@ int slice_tables(dpd_engine* e, int32_t box, int32_t nslices, double* tab, size_
     a.slot_of = e->slot_of;
     a.bond_bead = e->bond_bead;
     a.bond_par = e->bond_par;
-    a.b0 = 0;
-    for (int32_t b = 0; b < box; ++b) a.b0 += (int)e->boxes[b].bh.size();
-    a.b1 = a.b0 + (int)h.bh.size();
+    a.b0 = h.bond_off;
+    a.b1 = a.b0 + h.nbonds;
     a.ang_bead = e->ang_bead;
     a.ang_par = e->ang_par;
     a.a0 = a.a1 = 0;
-    a.nbeads = (int)h.n;
+    a.nbeads = (int)h.nbeads;
     a.nslice = nslices;
     a.ntypes = nt;
     a.nidx = nt * nt;
@@ -2002,7 +2016,7 @@ int dpd_download_box(dpd_engine* e, int32_t box, double* x, double* unpbc, doubl
     launch_gather(e, e->frc, x ? g : nullptr, unpbc ? g + 3 * n : nullptr, v ? g + 6 * n : nullptr, f ? g + 9 * n : nullptr);
     HIPCHK(hipGetLastError());
     const int64_t off = box < 0 ? 0 : e->boxes[box].bead_off;
-    const int64_t cnt = box < 0 ? e->n : e->boxes[box].n;
+    const int64_t cnt = box < 0 ? e->n : e->boxes[box].nbeads;
     const size_t b3 = sizeof(double) * 3 * cnt;
     if (x) HIPCHK(hipMemcpyAsync(x, g + 3 * off, b3, hipMemcpyDeviceToHost, e->stream));
     if (unpbc) HIPCHK(hipMemcpyAsync(unpbc, g + 3 * n + 3 * off, b3, hipMemcpyDeviceToHost, e->stream));
@@ -2408,10 +2422,10 @@ int dpd_energy_output(dpd_engine* e, int32_t box, double* out3)
     a.bond_par = e->bond_par;
     a.ang_bead = e->ang_bead;
     a.ang_par = e->ang_par;
-    a.b0 = a.a0 = 0;
-    for (int32_t b = 0; b < box; ++b) { a.b0 += (int)e->boxes[b].bh.size(); a.a0 += (int)e->boxes[b].pf.size(); }
-    a.b1 = e->nbonds > 0 ? a.b0 + (int)h.bh.size() : a.b0;
-    a.a1 = e->nangles > 0 ? a.a0 + (int)h.pf.size() : a.a0;
+    a.b0 = h.bond_off;
+    a.b1 = a.b0 + h.nbonds;
+    a.a0 = h.pair_off;
+    a.a1 = a.a0 + h.npairs;
     a.ntypes = h.B.ntypes;
     HIPCHK(launch_energy_output(a, e->slice, e->stream));
     HIPCHK(hipMemcpyAsync(out3, e->slice, sizeof(double) * 3, hipMemcpyDeviceToHost, e->stream));
@@ -2443,9 +2457,8 @@ int dpd_slice_stress_bondpairs(dpd_engine* e, int32_t box, int32_t nslices, doub
     a.slot_of = e->slot_of;
     a.ang_bead = e->ang_bead;
     a.ang_par = e->ang_par;
-    a.a0 = 0;
-    for (int32_t b = 0; b < box; ++b) a.a0 += (int)e->boxes[b].pf.size();
-    a.a1 = e->nangles > 0 ? a.a0 + (int)h.pf.size() : a.a0;
+    a.a0 = h.pair_off;
+    a.a1 = a.a0 + h.npairs;
     a.nslice = nslices;
     a.ntypes = nt;
     a.nidx = nt * nt * nt;

@@ -368,7 +368,8 @@ class Batch(Engine):
             raise DpdError(rc, msg)
         self.nbox = len(boxes)
         self.box_ntypes = [np.asarray(b["a"]).shape[0] for b in boxes]
-        self.box_n = [0] * self.nbox
+        self.box_n = [0] * self.nbox      # beads on the device; staged ones take effect at commit
+        self._staged_n = [0] * self.nbox
         self.n = 0
 
     def _ntypes(self, box):
@@ -381,7 +382,7 @@ class Batch(Engine):
         x, v, f, u = _f64(x, (n, 3)), _f64(v, (n, 3)), _f64(f, (n, 3)), _f64(unpbc, (n, 3))
         self._check(lib().dpd_upload_box(self.h, int(box), n, _ptr(ids), _ptr(types), _ptr(x), _ptr(u),
                                          _ptr(v), _ptr(f)))
-        self.box_n[box] = n
+        self._staged_n[box] = n
 
     def upload_box_topology(self, box, head=(), tail=(), k=(), l0=(), first=(), second=(), modulus=(),
                             phi0=()):
@@ -394,6 +395,7 @@ class Batch(Engine):
 
     def commit(self, step0=0):
         self._check(lib().dpd_commit(self.h, int(step0)))
+        self.box_n = list(self._staged_n)
         self.n = sum(self.box_n)
 
     def download_box(self, box):
